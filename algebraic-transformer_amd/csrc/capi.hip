@@ -123,12 +123,17 @@ AttnWs attn_ws(int dtype, int B, int H, int T, int D) {
 // Vp = V rounded up to 8 (16-byte aligned rows).
 struct HeadWs {
   size_t partial, obj_part, bwd, dh_part, de_part, total;
+  size_t flag, E3, h3;  // f32 hidden states
   size_t res_ut, res_l, res_total;
   int Npad, Vp, dh_split;
   alg::HeadDePlan de;
 };
+size_t head_de_part_bytes(const alg::HeadDePlan& de) {
+  return de.split > 1 ? (size_t)(de.tiles - de.full) * de.split * alg::HT_M * alg::HT_N * sizeof(float) : 0;
+}
 HeadWs head_ws(int N, int d, int V, int pass, bool residual) {
   HeadWs w;
+  w.flag = w.E3 = w.h3 = 0;
   w.Npad = alg::head_token_pad(N);
   w.Vp = alg::head_vocab_pitch(V);
   w.partial = 0;
@@ -140,31 +145,34 @@ HeadWs head_ws(int N, int d, int V, int pass, bool residual) {
   const size_t part_bytes = w.dh_split > 1 ? (size_t)w.dh_split * N * d * sizeof(float) : 0;
   w.de = alg::head_de_plan(N, d, V);
   w.de_part = w.dh_part + align256(part_bytes);
-  const size_t de_bytes =
-      w.de.split > 1 ? (size_t)(w.de.tiles - w.de.full) * w.de.split * alg::HT_M * alg::HT_N * sizeof(float) : 0;
-  w.total = pass == 0 ? w.bwd : w.de_part + align256(de_bytes);
+  w.total = pass == 0 ? w.bwd : w.de_part + align256(head_de_part_bytes(w.de));
   w.res_ut = 0;
   w.res_l = align256((size_t)w.Npad * w.Vp * 2);
   w.res_total = w.res_l + align256((size_t)N * sizeof(float));
   return w;
 }
 
-// f32 hidden states (head_f32.hip, the reference's recompute schedule in f32): [partials f32
-// nvt*N over 128-entry vocabulary tiles][obj parts] (+ bwd: dZ f32 N*Vp, then the f32 partials
-// split*N*d of a vocabulary-split dh product). No residual.
+// f32 hidden states (the reference's recompute schedule in f32): [partials f32 nvt*N over
+// 128-entry vocabulary tiles][obj parts][flag i32: an input is not finite][E and h as three bf16
+// planes each] (+ bwd: dZ as three bf16 planes Npad*Vp, or f32 N*Vp where the flag is set; then
+// the f32 partials split*N*d of a vocabulary-split dh product; then the f32 tiles of the
+// token-split dE tail). No residual.
 HeadWs head_ws_f32(int N, int d, int V, int pass) {
   HeadWs w;
-  w.Npad = N;
+  w.Npad = alg::head_token_pad(N);
   w.Vp = alg::head_vocab_pitch(V);
   w.partial = 0;
   w.obj_part = align256((size_t)alg::head_f32_vocab_tiles(V) * N * sizeof(float));
-  w.bwd = w.obj_part + align256((size_t)alg::head_stat_blocks(N) * sizeof(float));
-  w.dh_split = alg::head_f32_dh_split(N, d, V);
-  w.dh_part = w.bwd + align256((size_t)N * w.Vp * sizeof(float));
+  w.flag = w.obj_part + align256((size_t)alg::head_stat_blocks(N) * sizeof(float));
+  w.E3 = w.flag + 256;
+  w.h3 = w.E3 + align256((size_t)V * d * 6);
+  w.bwd = w.h3 + align256((size_t)N * d * 6);
+  w.dh_split = alg::head_dh_split(N, d, V);
+  w.dh_part = w.bwd + align256((size_t)w.Npad * w.Vp * 6);
   const size_t part_bytes = w.dh_split > 1 ? (size_t)w.dh_split * N * d * sizeof(float) : 0;
-  w.de = alg::HeadDePlan{0, 0, 1, 0};
-  w.de_part = 0;
-  w.total = pass == 0 ? w.bwd : w.dh_part + align256(part_bytes);
+  w.de = alg::head_de_plan(N, d, V);
+  w.de_part = w.dh_part + align256(part_bytes);
+  w.total = pass == 0 ? w.bwd : w.de_part + align256(head_de_part_bytes(w.de));
   w.res_ut = w.res_l = w.res_total = 0;
   return w;
 }
@@ -597,9 +605,7 @@ static HeadStreamWs head_stream_ws(int dtype, int N, int d, int V, int vocab_chu
   w.de_part = w.acc + (nchunks > 1 ? align256((size_t)N * d * sizeof(float)) : 0);
   size_t de_bytes = 0;
   for (int vc : {w.chunk, V - (nchunks - 1) * w.chunk}) {
-    const alg::HeadDePlan pl = alg::head_de_plan(N, d, vc);
-    if (pl.split > 1)
-      de_bytes = std::max(de_bytes, (size_t)(pl.tiles - pl.full) * pl.split * alg::HT_M * alg::HT_N * sizeof(float));
+    de_bytes = std::max(de_bytes, head_de_part_bytes(alg::head_de_plan(N, d, vc)));
   }
   w.has_de_part = de_bytes > 0;
   w.total = w.de_part + align256(de_bytes);
@@ -649,6 +655,14 @@ static alg::HeadParams head_params(int dtype, int N, int d, int V, const void* h
   return p;
 }
 
+// f32 hidden states: the bf16 planes of the workspace that the products run on.
+static void use_split_planes(alg::HeadParams& p, void* workspace, const HeadWs& ws) {
+  char* w = static_cast<char*>(workspace);
+  p.split_bad = reinterpret_cast<int*>(w + ws.flag);
+  p.E = reinterpret_cast<bf16*>(w + ws.E3);
+  p.h = reinterpret_cast<bf16*>(w + ws.h3);
+}
+
 int alg_head_fwd(alg_stream_t stream, int dtype, int N, int d, int V, const void* h, const void* E,
                  const int32_t* targets, int n, float c, float* stat, float* zt, float* pt, float* obj,
                  void* residual, void* workspace, size_t workspace_bytes) {
@@ -664,7 +678,10 @@ int alg_head_fwd(alg_stream_t stream, int dtype, int N, int d, int V, const void
     return fail(ALG_ERR_INVALID, "workspace too small: need %zu bytes", ws.total);
   alg::HeadParams p = head_params(dtype, N, d, V, h, E, targets, n, c, workspace, ws);
   p.stat = stat; p.zt = zt; p.pt = pt; p.obj = obj;
-  if (f32) return hip_status(alg::launch_head_fwd_f32(p, (hipStream_t)stream), "alg_head_fwd");
+  if (f32) {
+    use_split_planes(p, workspace, ws);
+    return hip_status(alg::launch_head_fwd_f32(p, (hipStream_t)stream), "alg_head_fwd");
+  }
   if (residual) {
     p.ut = reinterpret_cast<bf16*>(static_cast<char*>(residual) + ws.res_ut);
     p.lsum = reinterpret_cast<float*>(static_cast<char*>(residual) + ws.res_l);
@@ -847,11 +864,17 @@ int alg_head_bwd(alg_stream_t stream, int dtype, int N, int d, int V, const void
   p.dE = dE;
   p.dE_f32 = dE_dtype == ALG_DTYPE_F32;
   if (f32) {
+    use_split_planes(p, workspace, ws);
+    p.dzt = reinterpret_cast<bf16*>(w + ws.bwd);
     p.dz32 = reinterpret_cast<float*>(w + ws.bwd);
     p.dh32 = static_cast<float*>(dh);
     p.dh_split = ws.dh_split;
-    p.dh_kchunk = alg::head_f32_dh_kchunk(V, ws.dh_split);
+    p.dh_kchunk = alg::head_dh_kchunk(V, ws.dh_split);
     p.dh_part = ws.dh_split > 1 ? reinterpret_cast<float*>(w + ws.dh_part) : nullptr;
+    p.de_full = ws.de.full;
+    p.de_split = ws.de.split;
+    p.de_kchunk = ws.de.kchunk;
+    p.de_part = ws.de.split > 1 ? reinterpret_cast<float*>(w + ws.de_part) : nullptr;
     return hip_status(alg::launch_head_bwd_f32(p, (hipStream_t)stream), "alg_head_bwd");
   }
   if (residual) {

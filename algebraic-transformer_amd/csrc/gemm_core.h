@@ -52,6 +52,9 @@ struct GemmOperand {
   // gives each wave matching W1 and W2 columns. 0: plain operand. Logical tile columns start at
   // mn0, stored ones at mn0 / 2.
   long split = 0;
+  // Elements between the planes of an operand kept as the exact sum of three bf16 matrices
+  // (the f32 products, SPLIT3 of gemm_mainloop). 0: one plane.
+  long plane = 0;
 };
 
 // Stored element offset, relative to a tile's stored first column, of logical chunk c
@@ -113,12 +116,13 @@ struct OperandTile {
   // per-lane offset only, not the scalar one), so chunks past the allocation read as zeros.
   template <bool CHECKED = false, int J0 = 0, int J1 = PER_WAVE>
   static __device__ __forceinline__ void copy(bf16* tile, const GemmOperand& op, const uint32_t (&off)[2], int wave,
-                                              int mn0, int k0) {
+                                              int mn0, int k0, long plane = 0) {
     const int r0 = (MODE == KMAJOR) ? mn0 : k0;
     const int c0 = (MODE == KMAJOR) ? k0 : (op.split ? mn0 / 2 : mn0);
+    const bf16* src = op.ptr + plane;
     if constexpr (!CHECKED) {
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(op.ptr + ((long)r0 * op.ld + c0)), (short)0, 0x7FFFFFFF, BUF_RSRC_WORD3);
+          (void*)(src + ((long)r0 * op.ld + c0)), (short)0, 0x7FFFFFFF, BUF_RSRC_WORD3);
 #pragma unroll
       for (int j = J0; j < J1; ++j) {
         const int J = wave * PER_WAVE + j;
@@ -133,14 +137,15 @@ struct OperandTile {
         const long rest = op.extent - first;
         const int nrec = rest <= 0 ? 0 : (int)(rest >= 0x3FFFFFFF ? 0x7FFFFFFE : 2 * rest);
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(op.ptr + (rest <= 0 ? 0 : first)), (short)0, nrec, BUF_RSRC_WORD3);
+            (void*)(src + (rest <= 0 ? 0 : first)), (short)0, nrec, BUF_RSRC_WORD3);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS_PTR(void, tile + J * 512), 16, off[j & 1], 0, 0, 0);
       }
     }
   }
   // Synchronous copy with zero fill (edge tiles, partial last k tile): elements outside the
   // stored matrix, or at k >= K, are zero (per element, so rows may end inside a chunk).
-  static __device__ __forceinline__ void copy_zero_fill(bf16* tile, const GemmOperand& op, int mn0, int k0, int K) {
+  static __device__ __forceinline__ void copy_zero_fill(bf16* tile, const GemmOperand& op, int mn0, int k0, int K,
+                                                        long plane = 0) {
     for (int p = threadIdx.x; p < ROWS * CPR; p += NT) {
       const int row = p / CPR, c = p - row * CPR;
       const int grow = (MODE == KMAJOR) ? mn0 + row : k0 + row;
@@ -150,7 +155,7 @@ struct OperandTile {
       const int nv = row_ok ? min(8, col_end - gcol) : 0;  // live elements of this chunk
       const long scol = (MODE != KMAJOR && op.split) ? mn0 / 2 + split_chunk_offset(op, c) : gcol;
       uint4 v = make_uint4(0, 0, 0, 0);
-      if (nv > 0) v = *reinterpret_cast<const uint4*>(op.ptr + (long)grow * op.ld + scol);
+      if (nv > 0) v = *reinterpret_cast<const uint4*>(op.ptr + plane + (long)grow * op.ld + scol);
       if (nv < 8) {  // keep elements [0, nv): two bf16 per 32-bit word
         unsigned int* w = reinterpret_cast<unsigned int*>(&v);
 #pragma unroll
@@ -220,9 +225,19 @@ __device__ __forceinline__ void wave_coords(int& wm, int& wn) {
   wn = wave % C::WN;
 }
 
+// f32 products on the bf16 matrix cores: an f32 value is the exact sum of three bf16 values
+// (8 significant bits each, nearest first), and the product of two such sums drops only the
+// terms of planes (1,2), (2,1) and (2,2), together under 2^-25 of the product. The six kept terms run
+// as six passes over k, smallest first, so the large (0,0) pass alone sets the rounding of the
+// f32 accumulator: plane of A and of B for each pass, one hex digit each.
+constexpr int SPLIT3_PASSES = 6;
+__device__ __forceinline__ int split3_a(int pass) { return (0x001102 >> (4 * pass)) & 15; }
+__device__ __forceinline__ int split3_b(int pass) { return (0x010120 >> (4 * pass)) & 15; }
+
 // Accumulate the (m0, n0) tile over k in [kbeg, K). acc[mb][nb] is the wave's 32x32 block at
-// rows wm*WTM + mb*32 and columns wn*WTN + nb*32 of the workgroup tile.
-template <int AM, int BM, class C>
+// rows wm*WTM + mb*32 and columns wn*WTN + nb*32 of the workgroup tile. SPLIT3: the operands
+// are three planes each and the loop runs the six passes above back to back.
+template <int AM, int BM, class C, bool SPLIT3 = false>
 __device__ __forceinline__ void gemm_mainloop(GemmStage<AM, BM, C>& s0, GemmStage<AM, BM, C>& s1,
                                               const GemmOperand& A, const GemmOperand& B, int m0, int n0, int kbeg,
                                               int K, floatx16 (&acc)[C::MB][C::NB]) {
@@ -252,7 +267,9 @@ __device__ __forceinline__ void gemm_mainloop(GemmStage<AM, BM, C>& s0, GemmStag
       for (int j = 0; j < C::NB; ++j) acc[i][j] = mfma_bf16(f.a[i], f.b[j], acc[i][j]);
   };
   const int klen = K - kbeg;
-  const int kmain = klen >= 2 * GT_K ? klen - klen % (2 * GT_K) : 0;  // pipelined part
+  // Pipelined part of the k range (of every pass: six passes make an even number of k steps of
+  // any number per pass).
+  const int kmain = SPLIT3 ? klen - klen % GT_K : klen >= 2 * GT_K ? klen - klen % (2 * GT_K) : 0;
   const bool a_full = (AM == KMAJOR ? A.rows_valid : A.cols_valid) >= m0 + C::TM;
   const bool b_full = (BM == KMAJOR ? B.rows_valid : B.cols_valid) >= n0 + C::TN;
   if (kmain > 0) {
@@ -260,7 +277,8 @@ __device__ __forceinline__ void gemm_mainloop(GemmStage<AM, BM, C>& s0, GemmStag
     TA::lane_offsets(A, aoff);
     TB::lane_offsets(B, boff);
     const int wave_u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nk = kmain / GT_K;  // even, >= 2
+    const int nk1 = kmain / GT_K;                        // k steps of one pass
+    const int nk = SPLIT3 ? SPLIT3_PASSES * nk1 : nk1;   // even, >= 2
     // One k step, software-pipelined over its four 16-deep sub-steps: fragments of sub-step
     // ks+1 are read while ks multiplies. f0 holds sub-step 0 of `cur` on entry and sub-step 0
     // of `nxt` on exit. The barrier (after this wave's copies into `nxt` have landed, vmcnt)
@@ -269,9 +287,18 @@ __device__ __forceinline__ void gemm_mainloop(GemmStage<AM, BM, C>& s0, GemmStag
     // whole k step to land before the next barrier waits for it.
     auto pipelined = [&](auto checked) {
       constexpr bool CHK = decltype(checked)::value;
+      // Tiles are copied in the order 0, 1, 2, ...; the split form keeps its place in the
+      // passes instead of dividing.
+      int pass = 0, kp = 0;
       auto copy_tile = [&](GemmStage<AM, BM, C>& st, int kt) {
-        TA::template copy<CHK>(st.a, A, aoff, wave_u, m0, kbeg + kt * GT_K);
-        TB::template copy<CHK>(st.b, B, boff, wave_u, n0, kbeg + kt * GT_K);
+        if constexpr (SPLIT3) {
+          TA::template copy<CHK>(st.a, A, aoff, wave_u, m0, kbeg + kp * GT_K, split3_a(pass) * A.plane);
+          TB::template copy<CHK>(st.b, B, boff, wave_u, n0, kbeg + kp * GT_K, split3_b(pass) * B.plane);
+          if (++kp == nk1) { kp = 0; ++pass; }
+        } else {
+          TA::template copy<CHK>(st.a, A, aoff, wave_u, m0, kbeg + kt * GT_K);
+          TB::template copy<CHK>(st.b, B, boff, wave_u, n0, kbeg + kt * GT_K);
+        }
       };
       constexpr int NG = TA::PER_WAVE + TB::PER_WAVE;  // copy instructions per wave and tile
       Frags f0, f1;
@@ -337,15 +364,17 @@ __device__ __forceinline__ void gemm_mainloop(GemmStage<AM, BM, C>& s0, GemmStag
   }
   // Remaining partial k tiles (and short k ranges): register copies with zero fill.
   for (int k0 = kbeg + kmain; k0 < K; k0 += GT_K) {
-    __syncthreads();
-    TA::copy_zero_fill(s0.a, A, m0, k0, K);
-    TB::copy_zero_fill(s0.b, B, n0, k0, K);
-    __syncthreads();
+    for (int pass = 0; pass < (SPLIT3 ? SPLIT3_PASSES : 1); ++pass) {
+      __syncthreads();
+      TA::copy_zero_fill(s0.a, A, m0, k0, K, SPLIT3 ? split3_a(pass) * A.plane : 0);
+      TB::copy_zero_fill(s0.b, B, n0, k0, K, SPLIT3 ? split3_b(pass) * B.plane : 0);
+      __syncthreads();
 #pragma unroll
-    for (int ks = 0; ks < GT_K / 16; ++ks) {
-      Frags f;
-      load(s0, ks, f);
-      mma(f);
+      for (int ks = 0; ks < GT_K / 16; ++ks) {
+        Frags f;
+        load(s0, ks, f);
+        mma(f);
+      }
     }
   }
 }

@@ -57,8 +57,10 @@ __device__ __forceinline__ int ustage_at(int tl, int vl) {
 }
 
 // Stores the staged block: token rows tok0 + (0..WTN-1), vocabulary entries v0 + (0..WTM-1) of
-// out (row pitch Vp, Npad rows). AUX is the store's cache policy.
-template <int AUX>
+// out (row pitch Vp, Npad rows). AUX is the store's cache policy. EDGE: chunks at or past Vp are
+// dropped (Vp is a multiple of 8, so a chunk lies inside a row or past it; token rows always lie
+// inside the Npad rows).
+template <int AUX, bool EDGE = false>
 __device__ __forceinline__ void store_staged_tokmajor(const bf16* ub, bf16* out, int Npad, int Vp, int tok0, int v0,
                                                       int lane) {
   const size_t ubase = (size_t)tok0 * Vp + v0;
@@ -78,8 +80,17 @@ __device__ __forceinline__ void store_staged_tokmajor(const bf16* ub, bf16* out,
   for (int j = 0; j < HC::WTN / RPS; ++j) {
     const int tl = RPS * j + lane / UCH;
     const u32x4 v = *reinterpret_cast<const u32x4*>(ub + ustage_at(tl, ch * 8));
-    __builtin_amdgcn_raw_buffer_store_b128(v, urs, voff + RPS * j * Vp * 2, 0, AUX);
+    if (!EDGE || v0 + ch * 8 < Vp) __builtin_amdgcn_raw_buffer_store_b128(v, urs, voff + RPS * j * Vp * 2, 0, AUX);
   }
+}
+
+// A row-major (N, d) or (V, d) operand of the head's products: bf16, or with SPLIT the three
+// bf16 planes of an f32 matrix.
+template <bool SPLIT>
+__device__ __forceinline__ GemmOperand head_operand(const bf16* ptr, int rows, int d, long plane) {
+  GemmOperand o{ptr, d, rows, d, (long)rows * d};
+  if constexpr (SPLIT) o.plane = plane;
+  return o;
 }
 
 // z^T = E h^T with the forward epilogue (row sums, target logit, optional U residual).
@@ -95,8 +106,12 @@ __device__ __forceinline__ float select_row(const floatx16 (&acc)[HC::MB][HC::NB
   return z;
 }
 
-template <int L2N>
+// SPLIT: f32 h and E as three bf16 planes each (gemm_mainloop's six passes); no residual, and
+// the row sums are kept per 128 vocabulary entries, the tiling of the f32 kernels that run
+// instead when an input is not finite (p.split_bad).
+template <int L2N, bool SPLIT>
 __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
+  if (SPLIT && *p.split_bad) return;
   __shared__ __attribute__((aligned(16))) GemmStage<KMAJOR, KMAJOR, HC> s0, s1;
   __shared__ float red[HC::WM][HT_N];
   const int nbm = (p.V + HT_M - 1) / HT_M, nbn = p.Npad / HT_N;
@@ -104,23 +119,27 @@ __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
   xcd_tile(blockIdx.x, nbm, nbn, tm, tn);
   const int m0 = tm * HT_M;  // vocab
   const int n0 = tn * HT_N;  // tokens
-  GemmOperand A{p.E, p.d, p.V, p.d, (long)p.V * p.d}, B{p.h, p.d, p.N, p.d, (long)p.N * p.d};
+  const GemmOperand A = head_operand<SPLIT>(p.E, p.V, p.d, (long)p.V * p.d);
+  const GemmOperand B = head_operand<SPLIT>(p.h, p.N, p.d, (long)p.N * p.d);
   floatx16 acc[HC::MB][HC::NB];
-  gemm_mainloop<KMAJOR, KMAJOR, HC>(s0, s1, A, B, m0, n0, 0, p.d, acc);
+  gemm_mainloop<KMAJOR, KMAJOR, HC, SPLIT>(s0, s1, A, B, m0, n0, 0, p.d, acc);
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
   wave_coords<HC>(wm, wn);
   const float inv_c = p.inv_c, clamp = p.clamp;
   const int vrow0 = m0 + wm * HC::WTM;  // first vocab row of this wave
-  // Interior tile (every row and column live); WITH_U also stores the residual. U is
-  // token-major (element (tok, v) at tok * Vp + v), staged per wave and written with 16-byte
-  // stores marked non-temporal so the 1 GB stream of U does not evict the E / h panels the
-  // GEMM is reusing from L2.
+  // WITH_U also stores the residual. U is token-major (element (tok, v) at tok * Vp + v),
+  // staged per wave and written with 16-byte stores marked non-temporal so the 1 GB stream of U
+  // does not evict the E / h panels the GEMM is reusing from L2. EDGE (tiles that reach past V
+  // or N): rows past V add nothing to the sums; U's rows up to Npad and its columns up to Vp
+  // are all written, as finite values wherever h is finite (operand rows past the end read as
+  // zeros). Edge tiles once stored U an element at a time, 2 bytes a lane: at N = 1000 their
+  // quarter of the tiles took most of the kernel.
   constexpr int NWAVES = HC::THREADS / 64;
   static_assert(NWAVES * UWAVE * 2 <= 2 * (int)sizeof(s0), "staging fits the pipeline buffers");
   static_assert((NWAVES / 2) * UWAVE * 2 <= (int)sizeof(s0) || NWAVES == 1, "half the waves per stage");
-  auto interior = [&](auto with_u) {
-    constexpr bool WITH_U = decltype(with_u)::value;
+  auto epilogue = [&](auto with_u, auto edge) {
+    constexpr bool WITH_U = decltype(with_u)::value, EDGE = decltype(edge)::value;
     bf16* ub = nullptr;
     if constexpr (WITH_U) {
       __syncthreads();  // every wave is done reading the pipeline buffers
@@ -132,7 +151,8 @@ __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
     for (int nb = 0; nb < HC::NB; ++nb) {
       const int col = wn * HC::WTN + nb * 32 + l32;
       const int tok = n0 + col;
-      const int dt = p.targets[tok] - vrow0 - 4 * h;  // target row relative to this lane's rows
+      const int tgt = !EDGE || tok < p.N ? p.targets[tok] : -1;
+      const int dt = tgt - vrow0 - 4 * h;  // target row relative to this lane's rows
       float part = 0.0f;
 #pragma unroll
       for (int mb = 0; mb < HC::MB; ++mb) {
@@ -145,7 +165,7 @@ __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
             const float x = fminf(z * inv_c, clamp);  // fused_head.py:98
             float r;
             const float w = pow2n<L2N>(rho_fast(x, r), p.log2n);
-            part += w;
+            part += !EDGE || vrow0 + mb * 32 + 8 * g + 4 * h + e < p.V ? w : 0.0f;
             u[e] = w * r;
           }
           if constexpr (WITH_U) {
@@ -159,7 +179,7 @@ __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
       // The lane holds rows mb*32 + 8g + e (+4h) of the block: the target's row is one of them
       // when its offset dt has bit 2 clear and lies in [0, WTM). That is rare (WTM of V rows
       // per token), so the select runs behind a wave-uniform branch, skipped by every wave
-      // where no lane hits.
+      // where no lane hits. (A target past V may hit a row past V; the statistics ignore it.)
       const bool mine = (unsigned)dt < (unsigned)HC::WTM && !(dt & 4);
       if (__builtin_amdgcn_ballot_w64(mine)) {
         int dsel = dt;
@@ -171,46 +191,30 @@ __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
       if (h == 0) red[wm][col] = part;
     }
     // Rows of this wave's block: tokens n0 + wn*64 + (0..63), vocabulary vrow0 + (0..127).
-    if constexpr (WITH_U) store_staged_tokmajor<BUF_NT>(ub, p.ut, p.Npad, p.Vp, n0 + wn * HC::WTN, vrow0, lane);
+    if constexpr (WITH_U) store_staged_tokmajor<BUF_NT, EDGE>(ub, p.ut, p.Npad, p.Vp, n0 + wn * HC::WTN, vrow0, lane);
   };
-  if (m0 + HT_M <= p.V && n0 + HT_N <= p.N) {
-    if (p.ut) interior(std::true_type{});
-    else interior(std::false_type{});
+  const bool inside = m0 + HT_M <= p.V && n0 + HT_N <= p.N;
+  if (!SPLIT && p.ut) {
+    if (inside) epilogue(std::true_type{}, std::false_type{});
+    else epilogue(std::true_type{}, std::true_type{});
   } else {
-#pragma unroll
-    for (int nb = 0; nb < HC::NB; ++nb) {
-      const int col = wn * HC::WTN + nb * 32 + l32;
-      const int tok = n0 + col;
-      const bool live = tok < p.N;
-      const int tgt = live ? p.targets[tok] : -1;
-      float part = 0.0f;
-#pragma unroll
-      for (int mb = 0; mb < HC::MB; ++mb) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int v = vrow0 + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
-          const float z = acc[mb][nb][i];
-          const float x = fminf(z * inv_c, clamp);
-          float r;
-          const float w = pow2n<L2N>(rho_fast(x, r), p.log2n);
-          if (v < p.V) {
-            part += w;
-            if (p.ut && live) p.ut[(size_t)tok * p.Vp + v] = f2bf(w * r);
-          }
-          if (v == tgt) p.zt[tok] = z;
-        }
-      }
-      part += xor32(part);
-      if (h == 0) red[wm][col] = part;
-    }
+    if (inside) epilogue(std::false_type{}, std::false_type{});
+    else epilogue(std::false_type{}, std::true_type{});
   }
   __syncthreads();
   for (int t = threadIdx.x; t < HT_N; t += NT) {
     const int tok = n0 + t;
-    float s = 0.0f;
+    if (tok >= p.N) continue;
+    if constexpr (SPLIT) {
 #pragma unroll
-    for (int w = 0; w < HC::WM; ++w) s += red[w][t];
-    if (tok < p.N) p.partial[(size_t)tm * p.N + tok] = s;
+      for (int w = 0; w < HC::WM; ++w)
+        if (m0 + w * HC::WTM < p.V) p.partial[(size_t)(tm * HC::WM + w) * p.N + tok] = red[w][t];
+    } else {
+      float s = 0.0f;
+#pragma unroll
+      for (int w = 0; w < HC::WM; ++w) s += red[w][t];
+      p.partial[(size_t)tm * p.N + tok] = s;
+    }
   }
 }
 
@@ -477,34 +481,54 @@ __device__ __forceinline__ bf16* wave_stage(Stage& s0, Stage& s1, int wm, int wn
          (wi % (NWAVES / 2)) * UWAVE;
 }
 
-// Recompute schedules: z^T again, dZ^T = bf16(s (p - y) r), token-major. L2N > 0 fixes
-// n = 2^L2N at compile time (0: taken from the parameters). Interior tiles stage each wave's
-// block and write whole token rows with 16-byte stores (default cache policy: the dh and dE
-// products read dZ right after); edge tiles store element by element.
-template <int L2N>
+// Recompute schedules: z^T again, dZ^T = s (p - y) r, token-major: rounded to bf16, or (SPLIT,
+// f32 hidden states) as three bf16 planes whose sum is the f32 value. L2N > 0 fixes
+// n = 2^L2N at compile time (0: taken from the parameters). Each wave's block is staged and
+// written in whole token rows with 16-byte stores (default cache policy: the dh and dE products
+// read dZ right after); edge tiles write the rows up to Npad and the columns up to Vp too, of
+// which nothing is read.
+template <int L2N, bool SPLIT>
 __global__ __launch_bounds__(NT, 1) void head_dz_kernel(HeadParams p) {
+  if (SPLIT && *p.split_bad) return;
   __shared__ __attribute__((aligned(16))) GemmStage<KMAJOR, KMAJOR, HC> s0, s1;
   const int nbm = (p.V + HT_M - 1) / HT_M, nbn = p.Npad / HT_N;
   int tm, tn;
   xcd_tile(blockIdx.x, nbm, nbn, tm, tn);
   const int m0 = tm * HT_M, n0 = tn * HT_N;
-  GemmOperand A{p.E, p.d, p.V, p.d, (long)p.V * p.d}, B{p.h, p.d, p.N, p.d, (long)p.N * p.d};
+  const GemmOperand A = head_operand<SPLIT>(p.E, p.V, p.d, (long)p.V * p.d);
+  const GemmOperand B = head_operand<SPLIT>(p.h, p.N, p.d, (long)p.N * p.d);
   floatx16 acc[HC::MB][HC::NB];
-  gemm_mainloop<KMAJOR, KMAJOR, HC>(s0, s1, A, B, m0, n0, 0, p.d, acc);
+  gemm_mainloop<KMAJOR, KMAJOR, HC, SPLIT>(s0, s1, A, B, m0, n0, 0, p.d, acc);
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
   wave_coords<HC>(wm, wn);
   const float scale = head_grad_scale(p);
   const float inv_c = p.inv_c, clamp = p.clamp;
   const int vrow0 = m0 + wm * HC::WTM;  // first vocab row of this wave
-  if (m0 + HT_M <= p.V && n0 + HT_N <= p.N) {
-    __syncthreads();  // every wave is done reading the pipeline buffers
-    bf16* ub = wave_stage(s0, s1, wm, wn);
+  __syncthreads();  // every wave is done reading the pipeline buffers
+  bf16* ub = wave_stage(s0, s1, wm, wn);
+  auto epilogue = [&](auto edge) {
+    constexpr bool EDGE = decltype(edge)::value;
 #pragma unroll
     for (int nb = 0; nb < HC::NB; ++nb) {
       const int tok = n0 + wn * HC::WTN + nb * 32 + l32;
-      const int dt = p.targets[tok] - p.v_off - vrow0 - 4 * h;  // target row relative to this lane's rows
-      const float st = p.stat[tok];
+      const bool live = !EDGE || tok < p.N;
+      const int dt = (live ? p.targets[tok] - p.v_off : -1) - vrow0 - 4 * h;  // target row relative to this lane's rows
+      const float st = live ? p.stat[tok] : 0.0f;
+      // The target entry, (t - 1) r s (y = 1), lies in this wave's rows for few tokens (WTM of V
+      // rows), so it is formed behind a wave-uniform branch, as the forward selects the target
+      // logit; every entry is formed with y = 0 and the target's replaced.
+      const bool mine = (unsigned)dt < (unsigned)HC::WTM && !(dt & 4);
+      const bool some = __builtin_amdgcn_ballot_w64(mine);
+      float utgt = 0.0f;
+      int dsel = dt;
+      if (some) {
+        asm volatile("" : "+v"(dsel));  // keeps the select inside the branch (not speculated)
+        const float x = fminf(select_row(acc, nb, dsel) * inv_c, clamp);
+        float r;
+        const float t = pow2n<L2N>(rho_fast(x, r) * st, p.log2n);
+        utgt = (t - 1.0f) * r * scale;
+      }
 #pragma unroll
       for (int mb = 0; mb < HC::MB; ++mb) {
 #pragma unroll
@@ -523,42 +547,71 @@ __global__ __launch_bounds__(NT, 1) void head_dz_kernel(HeadParams p) {
           *reinterpret_cast<u32x2*>(ub + ustage_at(nb * 32 + l32, mb * 32 + 8 * g + 4 * h)) = pk;
         }
       }
-      // The target entry, (t - 1) r s (y = 1): rare (WTM of V rows per token), so it is formed
-      // again behind a wave-uniform branch, as the forward selects the target logit, and
-      // overwrites its staged slot (the same lane wrote it above; LDS keeps a wave's order).
-      const bool mine = (unsigned)dt < (unsigned)HC::WTM && !(dt & 4);
-      if (__builtin_amdgcn_ballot_w64(mine)) {
-        int dsel = dt;
-        asm volatile("" : "+v"(dsel));  // keeps the select inside the branch (not speculated)
-        const float x = fminf(select_row(acc, nb, dsel) * inv_c, clamp);
-        float r;
-        const float t = pow2n<L2N>(rho_fast(x, r) * st, p.log2n);
-        if (mine) ub[ustage_at(nb * 32 + l32, dsel + 4 * h)] = f2bf((t - 1.0f) * r * scale);
+      // The staged slot is overwritten (the same lane wrote it above; LDS keeps a wave's order).
+      if (some && mine) ub[ustage_at(nb * 32 + l32, dsel + 4 * h)] = f2bf(utgt);
+    }
+    store_staged_tokmajor<0, EDGE>(ub, p.dzt, p.Npad, p.Vp, n0 + wn * HC::WTN, vrow0, lane);
+  };
+  // SPLIT: blocks of 32 tokens x 64 vocabulary entries, whose three planes fit the wave's share
+  // of the buffers together, so each value is formed once and split in registers.
+  auto epilogue_split = [&]() {
+    constexpr int SV = 64, SCH = SV / 8, PLANE = 32 * SV;
+    static_assert(3 * PLANE <= UWAVE && HC::WTM % SV == 0, "three planes fit the wave's share");
+    auto at = [](int tl, int vl) { return tl * SV + (((vl >> 3) ^ (tl & (SCH - 1))) << 3) + (vl & 7); };
+#pragma unroll
+    for (int nb = 0; nb < HC::NB; ++nb) {
+      const int tok0 = n0 + wn * HC::WTN + nb * 32, tok = tok0 + l32;
+      const bool live = tok < p.N;
+      const int dt = (live ? p.targets[tok] - p.v_off : -1) - vrow0 - 4 * h;
+      const float st = live ? p.stat[tok] : 0.0f;
+#pragma unroll
+      for (int vb = 0; vb < HC::WTM / SV; ++vb) {
+#pragma unroll
+        for (int m2 = 0; m2 < SV / 32; ++m2) {
+          const int mb = vb * (SV / 32) + m2;
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            float u[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float x = fminf(acc[mb][nb][4 * g + e] * inv_c, clamp);
+              float r;
+              const float t = pow2n<L2N>(rho_fast(x, r) * st, p.log2n);
+              u[e] = (t - (dt == mb * 32 + 8 * g + e ? 1.0f : 0.0f)) * r * scale;
+            }
+#pragma unroll
+            for (int pl = 0; pl < 3; ++pl) {
+              u32x2 pk;
+              pk[0] = pack_bf16x2(u[0], u[1]);
+              pk[1] = pack_bf16x2(u[2], u[3]);
+              *reinterpret_cast<u32x2*>(ub + pl * PLANE + at(l32, m2 * 32 + 8 * g + 4 * h)) = pk;
+#pragma unroll
+              for (int e = 0; e < 4; ++e)  // what this plane leaves: bf16 is the high half of an f32
+                u[e] -= __builtin_bit_cast(float, e & 1 ? pk[e >> 1] & 0xffff0000u : pk[e >> 1] << 16);
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);  // one 32 x 32 block's values at a time in registers
+        }
+        const int v0 = vrow0 + vb * SV, ch = lane % SCH;
+        if (v0 + ch * 8 < p.Vp) {
+#pragma unroll
+          for (int pl = 0; pl < 3; ++pl) {
+            bf16* out = p.dzt + ((size_t)pl * p.Npad + tok0) * p.Vp + v0 + ch * 8;
+#pragma unroll
+            for (int j = 0; j < 32 * SCH / 64; ++j) {
+              const int tl = (64 / SCH) * j + lane / SCH;
+              *reinterpret_cast<u32x4*>(out + (size_t)tl * p.Vp) =
+                  *reinterpret_cast<const u32x4*>(ub + pl * PLANE + at(tl, ch * 8));
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    store_staged_tokmajor<0>(ub, p.dzt, p.Npad, p.Vp, n0 + wn * HC::WTN, vrow0, lane);
-    return;
-  }
-#pragma unroll
-  for (int nb = 0; nb < HC::NB; ++nb) {
-    const int tok = n0 + wn * HC::WTN + nb * 32 + l32;
-    const bool live = tok < p.N;
-    const int tgt = live ? p.targets[tok] : -1;
-    const float st = live ? p.stat[tok] : 0.0f;
-#pragma unroll
-    for (int mb = 0; mb < HC::MB; ++mb) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int v = vrow0 + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
-        if (v >= p.V) continue;
-        const float x = fminf(acc[mb][nb][i] * inv_c, clamp);
-        float r;
-        const float t = pow2n<L2N>(rho_fast(x, r) * st, p.log2n);
-        const float y = (v + p.v_off == tgt) ? 1.0f : 0.0f;
-        if (live) p.dzt[(size_t)tok * p.Vp + v] = f2bf((t - y) * r * scale);  // token-major
-      }
-    }
-  }
+  };
+  if constexpr (SPLIT) epilogue_split();
+  else if (m0 + HT_M <= p.V && n0 + HT_N <= p.N) epilogue(std::false_type{});
+  else epilogue(std::true_type{});
 }
 
 // Residual schedule: hs = bf16(s h / l) (the row scale of dE = U'^T (s h / l)).
@@ -618,8 +671,11 @@ __device__ __forceinline__ void store_block_bf16(const floatx16 (&acc)[HC::MB][H
 // vocabulary chunks, p.dh_accum 1 or 2): the tile of the f32 accumulator p.dh_part is read
 // whole after the main loop (all loads issued before the first add) and added to the product,
 // which then goes back to the accumulator (dh_accum 1) or, rounded, to dh (dh_accum 2).
-template <bool ACC>
+// SPLIT (f32 hidden states): dZ and E as three bf16 planes each, the f32 result or its
+// vocabulary partials in p.dh_part.
+template <bool ACC, bool SPLIT>
 __global__ __launch_bounds__(NT, 1) void head_dh_kernel(HeadParams p) {
+  if (SPLIT && *p.split_bad) return;
   __shared__ __attribute__((aligned(16))) GemmStage<KMAJOR, MNMAJOR, HC> s0, s1;
   const int nbm = p.Npad / HT_M, nbn = (p.d + HT_N - 1) / HT_N;
   int tr, tn;
@@ -631,13 +687,15 @@ __global__ __launch_bounds__(NT, 1) void head_dh_kernel(HeadParams p) {
   const int n0 = tn * HT_N;  // d
   const int kbeg = min(p.V, split * p.dh_kchunk), kend = min(p.V, kbeg + p.dh_kchunk);
   const bf16* a = p.ut ? p.ut : p.dzt;
-  GemmOperand A{a, p.Vp, p.N, p.V, (long)p.Npad * p.Vp}, B{p.E, p.d, p.V, p.d, (long)p.V * p.d};
+  const long apad = (long)p.Npad * p.Vp;
+  const GemmOperand A{a, p.Vp, p.N, p.V, apad, 0, SPLIT ? apad : 0};
+  const GemmOperand B = head_operand<SPLIT>(p.E, p.V, p.d, (long)p.V * p.d);
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
   wave_coords<HC>(wm, wn);
   float* part = p.dh_part ? p.dh_part + (size_t)split * p.N * p.d : nullptr;
   floatx16 acc[HC::MB][HC::NB];
-  gemm_mainloop<KMAJOR, MNMAJOR, HC>(s0, s1, A, B, m0, n0, kbeg, kend, acc);
+  gemm_mainloop<KMAJOR, MNMAJOR, HC, SPLIT>(s0, s1, A, B, m0, n0, kbeg, kend, acc);
   if constexpr (ACC) {
     // One 32 x 32 block at a time: its 16 loads are issued together, then added, and (dh_accum
     // 1) stored back to the accumulator.
@@ -723,7 +781,10 @@ __global__ __launch_bounds__(256) void head_dh_reduce_kernel(HeadParams p) {
 // XCD's share (U panels streamed once); the rest compute token range (id - de_full) % de_split
 // of tile de_full + (id - de_full) / de_split into an f32 tile of de_part, which
 // head_de_tail_kernel sums.
+// SPLIT (f32 hidden states): dZ and h as three bf16 planes each.
+template <bool SPLIT>
 __global__ __launch_bounds__(NT, 1) void head_de_kernel(HeadParams p) {
+  if (SPLIT && *p.split_bad) return;
   __shared__ __attribute__((aligned(16))) GemmStage<MNMAJOR, MNMAJOR, HC> s0, s1;
   const int nbn = (p.d + HT_N - 1) / HT_N;
   const int bid = blockIdx.x;
@@ -741,9 +802,11 @@ __global__ __launch_bounds__(NT, 1) void head_de_kernel(HeadParams p) {
   const int n0 = tn * HT_N;  // d
   const bf16* a = p.ut ? p.ut : p.dzt;
   const bf16* b = p.ut ? p.hs : p.h;
-  GemmOperand A{a, p.Vp, p.N, p.V, (long)p.Npad * p.Vp}, B{b, p.d, p.N, p.d, (long)p.N * p.d};
+  const long apad = (long)p.Npad * p.Vp;
+  const GemmOperand A{a, p.Vp, p.N, p.V, apad, 0, SPLIT ? apad : 0};
+  const GemmOperand B = head_operand<SPLIT>(b, p.N, p.d, (long)p.N * p.d);
   floatx16 acc[HC::MB][HC::NB];
-  gemm_mainloop<MNMAJOR, MNMAJOR, HC>(s0, s1, A, B, m0, n0, kbeg, kend, acc);
+  gemm_mainloop<MNMAJOR, MNMAJOR, HC, SPLIT>(s0, s1, A, B, m0, n0, kbeg, kend, acc);
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
   wave_coords<HC>(wm, wn);
@@ -787,6 +850,7 @@ __global__ __launch_bounds__(NT, 1) void head_de_kernel(HeadParams p) {
 // dE of a split tile: the de_split token-range tiles summed in range order, 32 rows of the
 // tile per workgroup (grid: split tiles x HT_M / 32).
 __global__ __launch_bounds__(256) void head_de_tail_kernel(HeadParams p) {
+  if (p.split_bad && *p.split_bad) return;  // dE came whole from the f32 kernel
   const int nbn = (p.d + HT_N - 1) / HT_N;
   const int lin = p.de_full + blockIdx.x;
   const int tm = lin / nbn, tn = lin - tm * nbn;
@@ -871,8 +935,8 @@ hipError_t launch_head_fwd(const HeadParams& p, hipStream_t st) {
   const int tiles = head_vocab_tiles(p.V) * (p.Npad / HT_N);
   {
     KTimer t("head_fwd", st);
-    if (p.log2n == 3) hipLaunchKernelGGL(head_fwd_kernel<3>, dim3(tiles), dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL(head_fwd_kernel<0>, dim3(tiles), dim3(NT), 0, st, p);
+    if (p.log2n == 3) hipLaunchKernelGGL((head_fwd_kernel<3, false>), dim3(tiles), dim3(NT), 0, st, p);
+    else hipLaunchKernelGGL((head_fwd_kernel<0, false>), dim3(tiles), dim3(NT), 0, st, p);
   }
   return launch_head_stats(p, head_vocab_tiles(p.V), st);
 }
@@ -908,8 +972,8 @@ static void launch_head_dh(const HeadParams& p, hipStream_t st) {
   {
     KTimer t("head_dh", st);
     const dim3 grid((p.Npad / HT_M) * dtiles * p.dh_split);
-    if (p.dh_accum) hipLaunchKernelGGL(head_dh_kernel<true>, grid, dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL(head_dh_kernel<false>, grid, dim3(NT), 0, st, p);
+    if (p.dh_accum) hipLaunchKernelGGL((head_dh_kernel<true, false>), grid, dim3(NT), 0, st, p);
+    else hipLaunchKernelGGL((head_dh_kernel<false, false>), grid, dim3(NT), 0, st, p);
   }
   if (p.dh_split > 1) {
     const size_t chunks = (size_t)p.N * p.d / 8;
@@ -922,23 +986,30 @@ static void launch_head_dh(const HeadParams& p, hipStream_t st) {
 // dE = (U' or dZ)^T (hs or h), with the token split of head_de_plan when p carries one.
 static void launch_head_de(const HeadParams& p, hipStream_t st) {
   const int de_tiles = head_vocab_tiles(p.V) * ((p.d + HT_N - 1) / HT_N);
-  if (p.de_split > 1 && p.de_part) {
-    const int tail = de_tiles - p.de_full;
-    { KTimer t("head_de", st); hipLaunchKernelGGL(head_de_kernel, dim3(p.de_full + tail * p.de_split), dim3(NT), 0, st, p); }
-    { KTimer t("head_de_tail", st); hipLaunchKernelGGL(head_de_tail_kernel, dim3(tail, HT_M / 32), dim3(256), 0, st, p); }
-  } else {
-    HeadParams q = p;
+  HeadParams q = p;
+  const bool split = p.de_split > 1 && p.de_part;
+  if (!split) {
     q.de_full = de_tiles;
     q.de_split = 1;
-    { KTimer t("head_de", st); hipLaunchKernelGGL(head_de_kernel, dim3(de_tiles), dim3(NT), 0, st, q); }
+  }
+  const int tail = de_tiles - q.de_full;
+  {
+    KTimer t("head_de", st);
+    const dim3 grid(q.de_full + tail * q.de_split);
+    if (p.split_bad) hipLaunchKernelGGL(head_de_kernel<true>, grid, dim3(NT), 0, st, q);
+    else hipLaunchKernelGGL(head_de_kernel<false>, grid, dim3(NT), 0, st, q);
+  }
+  if (split) {
+    KTimer t("head_de_tail", st);
+    hipLaunchKernelGGL(head_de_tail_kernel, dim3(tail, HT_M / 32), dim3(256), 0, st, q);
   }
 }
 
 static void launch_head_dz(const HeadParams& p, hipStream_t st) {
   const int tiles = head_vocab_tiles(p.V) * (p.Npad / HT_N);
   KTimer t("head_dz", st);
-  if (p.log2n == 3) hipLaunchKernelGGL(head_dz_kernel<3>, dim3(tiles), dim3(NT), 0, st, p);
-  else hipLaunchKernelGGL(head_dz_kernel<0>, dim3(tiles), dim3(NT), 0, st, p);
+  if (p.log2n == 3) hipLaunchKernelGGL((head_dz_kernel<3, false>), dim3(tiles), dim3(NT), 0, st, p);
+  else hipLaunchKernelGGL((head_dz_kernel<0, false>), dim3(tiles), dim3(NT), 0, st, p);
 }
 
 hipError_t launch_head_bwd(const HeadParams& p, hipStream_t st) {
@@ -952,6 +1023,76 @@ hipError_t launch_head_bwd(const HeadParams& p, hipStream_t st) {
   launch_head_dh(p, st);
   launch_head_de(p, st);
   return hipGetLastError();
+}
+
+// f32 hidden states on the bf16 matrix cores (p.E, p.h, p.dzt: three planes each; p.split_bad
+// set): every launch returns at once when an input was not finite, and the f32 kernels of
+// head_f32.hip, launched after it, run instead.
+//
+// f32 values into three bf16 planes, each the bf16 nearest to what the planes before it leave;
+// with 8 significant bits a plane the third leaves nothing (values under 2^-110 aside, whose
+// last planes would be subnormal). An infinity or NaN, or a value that rounds to infinity in
+// bf16, has no such planes: it sets *bad. Bound by memory: 4 bytes read and 6 written an element.
+__global__ __launch_bounds__(256) void head_split3_kernel(const float* src, bf16* dst, size_t n, int* bad) {
+  bool off = false;
+  for (size_t c = (size_t)blockIdx.x * 256 + threadIdx.x; c < n / 8; c += (size_t)gridDim.x * 256) {
+    const float4 x = reinterpret_cast<const float4*>(src)[2 * c], y = reinterpret_cast<const float4*>(src)[2 * c + 1];
+    float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) {
+      bf16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        o[e] = f2bf(v[e]);
+        const float b = (float)o[e];
+        if (pl == 0) off |= !(__builtin_fabsf(b) < INFINITY);
+        v[e] -= b;
+      }
+      *reinterpret_cast<bf16x8*>(dst + pl * n + 8 * c) = o;
+    }
+  }
+  if (__builtin_amdgcn_ballot_w64(off) && (threadIdx.x & 63) == 0) *bad = 1;
+}
+
+__global__ void head_split_clear_kernel(int* bad) { *bad = 0; }
+
+// Planes of h and E, and *p.split_bad.
+static void launch_head_split3(const HeadParams& p, hipStream_t st) {
+  KTimer t("head_split3", st);
+  int* bad = const_cast<int*>(p.split_bad);
+  hipLaunchKernelGGL(head_split_clear_kernel, dim3(1), dim3(1), 0, st, bad);
+  auto split = [&](const float* src, const bf16* dst, size_t n) {
+    const int blocks = (int)std::min<size_t>((n / 8 + 255) / 256, 4096);
+    hipLaunchKernelGGL(head_split3_kernel, dim3(blocks), dim3(256), 0, st, src, const_cast<bf16*>(dst), n, bad);
+  };
+  split(p.h32, p.h, (size_t)p.N * p.d);
+  split(p.E32, p.E, (size_t)p.V * p.d);
+}
+
+void launch_head_fwd_split(const HeadParams& p, hipStream_t st) {
+  launch_head_split3(p, st);
+  const int tiles = head_vocab_tiles(p.V) * (p.Npad / HT_N);
+  KTimer t("head_fwd_split", st);
+  if (p.log2n == 3) hipLaunchKernelGGL((head_fwd_kernel<3, true>), dim3(tiles), dim3(NT), 0, st, p);
+  else hipLaunchKernelGGL((head_fwd_kernel<0, true>), dim3(tiles), dim3(NT), 0, st, p);
+}
+
+void launch_head_bwd_split(const HeadParams& p, hipStream_t st) {
+  launch_head_split3(p, st);
+  const int tiles = head_vocab_tiles(p.V) * (p.Npad / HT_N);
+  {
+    KTimer t("head_dz_split", st);
+    if (p.log2n == 3) hipLaunchKernelGGL((head_dz_kernel<3, true>), dim3(tiles), dim3(NT), 0, st, p);
+    else hipLaunchKernelGGL((head_dz_kernel<0, true>), dim3(tiles), dim3(NT), 0, st, p);
+  }
+  {
+    HeadParams q = p;
+    if (p.dh_split == 1) q.dh_part = p.dh32;
+    KTimer t("head_dh_split", st);
+    const dim3 grid((p.Npad / HT_M) * ((p.d + HT_N - 1) / HT_N) * p.dh_split);
+    hipLaunchKernelGGL((head_dh_kernel<false, true>), grid, dim3(NT), 0, st, q);
+  }
+  launch_head_de(p, st);
 }
 
 HeadParams head_vocab_chunk(const HeadParams& p, int v0, int vc) {

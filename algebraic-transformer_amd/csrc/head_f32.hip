@@ -163,8 +163,10 @@ __global__ __launch_bounds__(F_NT) void head_fwd_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   __shared__ float red[F_WM][F_TN];
   const int nbm = (p.V + F_TM - 1) / F_TM, nbn = (p.N + F_TN - 1) / F_TN;
+  if (p.split_bad && !*p.split_bad) return;
+  for (int bid = blockIdx.x; bid < nbm * nbn; bid += gridDim.x) {
   int tm, tn;
-  xcd_tile(blockIdx.x, nbm, nbn, tm, tn);
+  xcd_tile(bid, nbm, nbn, tm, tn);
   const int m0 = tm * F_TM, n0 = tn * F_TN;
   const F32Op A{p.E32, p.d, p.V, p.d}, B{p.h32, p.d, p.N, p.d};
   floatx16 acc[2][2];
@@ -195,6 +197,8 @@ __global__ __launch_bounds__(F_NT) void head_fwd_f32_kernel(HeadParams p) {
     const int tok = n0 + t;
     if (tok < p.N) p.partial[(size_t)tm * p.N + tok] = red[0][t] + red[1][t];
   }
+  __syncthreads();  // the next tile reuses the LDS
+  }
 }
 
 // Backward, logit gradient: z = h E^T (m = tokens, n = vocabulary, so the f32 stores run along
@@ -202,8 +206,10 @@ __global__ __launch_bounds__(F_NT) void head_fwd_f32_kernel(HeadParams p) {
 __global__ __launch_bounds__(F_NT) void head_dz_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   const int nbm = (p.N + F_TM - 1) / F_TM, nbn = (p.V + F_TN - 1) / F_TN;
+  if (p.split_bad && !*p.split_bad) return;
+  for (int bid = blockIdx.x; bid < nbm * nbn; bid += gridDim.x) {
   int tm, tn;
-  xcd_tile(blockIdx.x, nbm, nbn, tm, tn);
+  xcd_tile(bid, nbm, nbn, tm, tn);
   const int m0 = tm * F_TM, n0 = tn * F_TN;
   const F32Op A{p.h32, p.d, p.N, p.d}, B{p.E32, p.d, p.V, p.d};
   floatx16 acc[2][2];
@@ -228,6 +234,7 @@ __global__ __launch_bounds__(F_NT) void head_dz_f32_kernel(HeadParams p) {
         p.dz32[(size_t)tok * p.Vp + v] = (t - y) * r * scale;
       }
     }
+  }
 }
 
 // dh = dZ E: A = dZ stored [token][v] (k contiguous), B = E stored [v][d] (n contiguous). With
@@ -235,8 +242,10 @@ __global__ __launch_bounds__(F_NT) void head_dz_f32_kernel(HeadParams p) {
 __global__ __launch_bounds__(F_NT) void head_dh_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   const int nbm = (p.N + F_TM - 1) / F_TM, nbn = (p.d + F_TN - 1) / F_TN;
+  if (p.split_bad && !*p.split_bad) return;
+  for (int bid = blockIdx.x; bid < nbm * p.dh_split * nbn; bid += gridDim.x) {
   int tr, tn;
-  xcd_tile_rowmajor(blockIdx.x, nbm * p.dh_split, nbn, tr, tn);
+  xcd_tile_rowmajor(bid, nbm * p.dh_split, nbn, tr, tn);
   const int tm = tr / p.dh_split, split = tr - tm * p.dh_split;
   const int m0 = tm * F_TM, n0 = tn * F_TN;
   const int kbeg = min(p.V, split * p.dh_kchunk), kend = min(p.V, kbeg + p.dh_kchunk);
@@ -259,6 +268,7 @@ __global__ __launch_bounds__(F_NT) void head_dh_f32_kernel(HeadParams p) {
         else out[(size_t)tok * p.d + col] = acc[mb][nb][i];
       }
     }
+  }
 }
 
 // dh = sum over the vocabulary splits of the partials, added in split order.
@@ -278,8 +288,10 @@ __global__ __launch_bounds__(256) void head_dh_f32_reduce_kernel(HeadParams p) {
 __global__ __launch_bounds__(F_NT) void head_de_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   const int nbm = (p.V + F_TM - 1) / F_TM, nbn = (p.d + F_TN - 1) / F_TN;
+  if (p.split_bad && !*p.split_bad) return;
+  for (int bid = blockIdx.x; bid < nbm * nbn; bid += gridDim.x) {
   int tm, tn;
-  xcd_tile_rowmajor(blockIdx.x, nbm, nbn, tm, tn);
+  xcd_tile_rowmajor(bid, nbm, nbn, tm, tn);
   const int m0 = tm * F_TM, n0 = tn * F_TN;
   const F32Op A{p.dz32, p.Vp, p.V, p.N}, B{p.h32, p.d, p.d, p.N};
   floatx16 acc[2][2];
@@ -300,6 +312,7 @@ __global__ __launch_bounds__(F_NT) void head_de_f32_kernel(HeadParams p) {
         else reinterpret_cast<bf16*>(p.dE)[o] = f2bf(acc[mb][nb][i]);
       }
     }
+  }
 }
 
 // Evaluation head: z^T = E h^T as in the forward; per token and vocabulary tile the largest
@@ -382,35 +395,34 @@ __global__ __launch_bounds__(F_NT) void head_eval_f32_kernel(HeadParams p) {
 
 int head_f32_vocab_tiles(int V) { return (V + F_TM - 1) / F_TM; }
 
-// Vocabulary splits of the dh product: double them while the product has fewer than about
-// 1024 workgroups (4 per CU) and each split keeps at least 256 vocabulary entries.
-int head_f32_dh_split(int N, int d, int V) {
-  const long tiles = (long)((N + F_TM - 1) / F_TM) * ((d + F_TN - 1) / F_TN);
-  int s = 1;
-  while (s < 32 && tiles * s < 1024 && V / (2 * s) >= 256) s *= 2;
-  return s;
-}
 // Vocabulary entries per split: a multiple of the k step (so every split starts 16-byte aligned).
 int head_f32_dh_kchunk(int V, int split) { return ((V + split - 1) / split + F_TK - 1) / F_TK * F_TK; }
 
+// Workgroups of an f32 kernel: one per tile, or, where the split kernels have done the work unless
+// an input was not finite, at most four per CU looping over the tiles (a launch that returns at
+// once costs its workgroups).
+static dim3 f32_grid(const HeadParams& p, int tiles) { return dim3(p.split_bad ? std::min(tiles, 1024) : tiles); }
+
 hipError_t launch_head_fwd_f32(const HeadParams& p, hipStream_t st) {
   const int tiles = head_f32_vocab_tiles(p.V) * ((p.N + F_TN - 1) / F_TN);
+  if (p.split_bad) launch_head_fwd_split(p, st);
   {
     KTimer t("head_fwd_f32", st);
-    hipLaunchKernelGGL(head_fwd_f32_kernel, dim3(tiles), dim3(F_NT), 0, st, p);
+    hipLaunchKernelGGL(head_fwd_f32_kernel, f32_grid(p, tiles), dim3(F_NT), 0, st, p);
   }
   return launch_head_stats(p, head_f32_vocab_tiles(p.V), st);
 }
 
 hipError_t launch_head_bwd_f32(const HeadParams& p, hipStream_t st) {
   const int ntok = (p.N + F_TM - 1) / F_TM, nd = (p.d + F_TN - 1) / F_TN;
+  if (p.split_bad) launch_head_bwd_split(p, st);
   {
     KTimer t("head_dz_f32", st);
-    hipLaunchKernelGGL(head_dz_f32_kernel, dim3(ntok * head_f32_vocab_tiles(p.V)), dim3(F_NT), 0, st, p);
+    hipLaunchKernelGGL(head_dz_f32_kernel, f32_grid(p, ntok * head_f32_vocab_tiles(p.V)), dim3(F_NT), 0, st, p);
   }
   {
     KTimer t("head_dh_f32", st);
-    hipLaunchKernelGGL(head_dh_f32_kernel, dim3(ntok * nd * p.dh_split), dim3(F_NT), 0, st, p);
+    hipLaunchKernelGGL(head_dh_f32_kernel, f32_grid(p, ntok * nd * p.dh_split), dim3(F_NT), 0, st, p);
   }
   if (p.dh_split > 1) {
     const size_t chunks = (size_t)p.N * p.d / 4;
@@ -420,7 +432,7 @@ hipError_t launch_head_bwd_f32(const HeadParams& p, hipStream_t st) {
   }
   {
     KTimer t("head_de_f32", st);
-    hipLaunchKernelGGL(head_de_f32_kernel, dim3(head_f32_vocab_tiles(p.V) * nd), dim3(F_NT), 0, st, p);
+    hipLaunchKernelGGL(head_de_f32_kernel, f32_grid(p, head_f32_vocab_tiles(p.V) * nd), dim3(F_NT), 0, st, p);
   }
   return hipGetLastError();
 }

@@ -55,7 +55,10 @@ struct HeadParams {
   int* pidx;            // eval: (ceil(V/HT_M), N) its vocabulary index
   float* logprob;       // eval: (N,) log p(target)
   int* argmax;          // eval: (N,) argmax_v z
-  // f32 hidden states (the head_f32 kernels; the bf16 pointers above are then unused):
+  // f32 hidden states. With split_bad set, h, E and dzt above are three bf16 planes each (the
+  // products run on the bf16 matrix cores) and the f32 kernels run only where *split_bad says
+  // that an input was not finite; without it the f32 kernels always run and h, E, dzt are unused.
+  const int* split_bad;
   const float* h32;     // (N, d)
   const float* E32;     // (V, d), already cast to f32
   float* dz32;          // recompute workspace (N, Vp): s (p - y) r, token-major

@@ -41,8 +41,9 @@ hipError_t launch_head_eval(const HeadParams& p, hipStream_t st);
 hipError_t launch_head_stats(const HeadParams& p, int vocab_tiles, hipStream_t st);
 hipError_t launch_head_eval_stats(const HeadParams& p, int vocab_tiles, hipStream_t st);
 int head_f32_vocab_tiles(int V);
-int head_f32_dh_split(int N, int d, int V);
 int head_f32_dh_kchunk(int V, int split);
+void launch_head_fwd_split(const HeadParams& p, hipStream_t st);
+void launch_head_bwd_split(const HeadParams& p, hipStream_t st);
 hipError_t launch_head_fwd_f32(const HeadParams& p, hipStream_t st);
 hipError_t launch_head_bwd_f32(const HeadParams& p, hipStream_t st);
 hipError_t launch_head_bwd_f32_streamed(const HeadParams& p, int chunk, hipStream_t st);

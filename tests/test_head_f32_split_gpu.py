@@ -1,0 +1,97 @@
+"""The f32 head's products on the bf16 matrix cores (three bf16 planes an operand, csrc/head.hip):
+sizes at the edges of the 256 x 256 tiles, of the 64-deep k steps and of the vocabulary and token
+splits, against the float64 dense oracle at the f32 bars; inputs that are not finite, which the f32
+kernels take, against those kernels (the streamed schedule runs them always) and numpy.
+"""
+
+import numpy as np
+import pytest
+
+from helpers import rel_l2
+from oracle import head as OH
+from oracle.numerics import head_clamp
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+# (N, d, V): one k step, a partial one, several; N and V one past, at and under a tile; d past a
+# tile; splits of the dh product (V >= 1024) and of the dE tail (N >= 2048).
+SHAPES = [(256, 64, 256), (257, 72, 513), (255, 128, 255), (513, 264, 1032), (100, 200, 4100), (2050, 192, 700)]
+
+
+def _run(h, E, t, e_dtype=torch.float32, g=1.0):
+    from algebraic_amd.kernels.fused_head import fused_head
+    th = torch.tensor(h, device="cuda", requires_grad=True)
+    tE = torch.tensor(E, device="cuda").to(e_dtype).requires_grad_(True)
+    obj, pt = fused_head(th, tE, torch.tensor(t, device="cuda"), kind="alg_ce", n=8, c=2.0, block_n=len(h))
+    dh, dE = torch.autograd.grad(obj * g, (th, tE))
+    f = lambda x: x.detach().float().cpu().numpy().astype(np.float64)
+    return float(obj.detach()), f(pt), f(dh), f(dE)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_split_products_match_dense(shape):
+    N, d, V = shape
+    print(f"f32 head split N{N} d{d} V{V}", flush=True)
+    rng = np.random.default_rng(N + d + V)
+    h = rng.standard_normal((N, d)).astype(np.float32)
+    E = (rng.standard_normal((V, d)) * 0.15).astype(np.float32)
+    E[0] *= 1e-12  # rows of very different sizes keep their relative precision
+    t = rng.integers(0, V, N).astype(np.int32)
+    obj, pt, dh, dE = _run(h, E, t, g=0.7)
+    obj_r, pt_r = OH.dense_forward(h, E, t, n=8, c=2.0)
+    dh_r, dE_r = OH.dense_backward(h, E, t, 0.7, n=8, c=2.0)
+    np.testing.assert_allclose(obj, obj_r, rtol=1e-5)
+    np.testing.assert_allclose(pt, pt_r, rtol=1e-5)
+    # A plane dropped or taken twice shows as 2^-9, 2^-17 or 2^-25 of the whole; the f32 sums
+    # themselves stay within the f32 bar.
+    assert rel_l2(dh, dh_r) < 3e-6
+    assert rel_l2(dE, dE_r) < 3e-6
+
+
+def test_small_values_keep_their_precision():
+    """Gradient scales down to 1e-20: the planes hold the same 24 bits there."""
+    rng = np.random.default_rng(3)
+    h = rng.standard_normal((300, 128)).astype(np.float32)
+    E = (rng.standard_normal((500, 128)) * 0.15).astype(np.float32)
+    t = rng.integers(0, 500, 300).astype(np.int32)
+    _, _, dh, dE = _run(h, E, t, g=1e-20)
+    dh_r, dE_r = OH.dense_backward(h, E, t, 1e-20, n=8, c=2.0)
+    assert rel_l2(dh, dh_r) < 3e-6 and rel_l2(dE, dE_r) < 3e-6
+
+
+@pytest.mark.parametrize("where", ["h_inf", "h_nan", "E_inf", "E_huge"])
+def test_not_finite_inputs(where, monkeypatch):
+    from algebraic_amd.kernels import fused_head as FH
+    rng = np.random.default_rng(7)
+    N, d, V = 300, 128, 600
+    h = rng.standard_normal((N, d)).astype(np.float32)
+    E = (rng.standard_normal((V, d)) * 0.15).astype(np.float32)
+    t = rng.integers(0, V, N).astype(np.int32)
+    if where == "h_inf":
+        h[17, 5] = np.inf
+    elif where == "h_nan":
+        h[17, 5] = np.nan
+    elif where == "E_inf":
+        E[33, 2] = -np.inf
+    else:
+        E[33, 2] = 3.4e38  # finite, but not in bf16
+    obj, pt, dh, dE = _run(h, E, t)
+    monkeypatch.setattr(FH, "SCHEDULE", "streamed")
+    obj_s, pt_s, dh_s, dE_s = _run(h, E, t)
+    np.testing.assert_equal(obj, obj_s)
+    np.testing.assert_equal(pt, pt_s)
+    for got, want in ((dh, dh_s), (dE, dE_s)):
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+        np.testing.assert_allclose(got, want, rtol=1e-4, atol=1e-9)
+    # The formula in numpy f32: min(z/c, X) takes X for a NaN logit.
+    with np.errstate(all="ignore"):
+        z = (h.astype(np.float64) @ E.T.astype(np.float64)).astype(np.float32)
+        x = np.fmin(z / np.float32(2), np.float32(head_clamp(V, 8)))
+        rad = 1 + x * x
+        w = ((x + rad * (1 / np.sqrt(rad))) ** 8).astype(np.float64)
+        pt_r = w[np.arange(N), t] / w.sum(1)
+    same = np.isfinite(pt_r)
+    assert same.sum() >= N - 1 if where.startswith("h") else True
+    rows = same & (np.arange(N) != 17)
+    np.testing.assert_allclose(pt[rows], pt_r[rows], rtol=1e-4, atol=1e-12)
