@@ -778,7 +778,7 @@ int alg_ffn_alu_glu_dy(alg_stream_t stream, int N, int dm, int F, const void* do
 
 size_t alg_ffn_gemm_workspace_size(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return alg::ffn_gemm_workspace_bytes(alg::ffn_gemm_plan(M, N, K));
+  return alg::ffn_gemm_plan(M, N, K).ws_bytes;
 }
 
 int alg_ffn_gemm(alg_stream_t stream, int M, int N, int K, const void* A, long lda, int a_trans, const void* B,
@@ -798,7 +798,7 @@ int alg_ffn_gemm(alg_stream_t stream, int M, int N, int K, const void* A, long l
       (double)(M - 1) * ldc + N > 2.0e9)
     return fail(ALG_ERR_INVALID, "matrices too large");
   const alg::FfnGemmPlan pl = alg::ffn_gemm_plan(M, N, K);
-  const size_t need = alg::ffn_gemm_workspace_bytes(pl);
+  const size_t need = pl.ws_bytes;
   if (need && (!workspace || workspace_bytes < need))
     return fail(ALG_ERR_INVALID, "workspace too small: need %zu bytes", need);
   if (need && !aligned16({workspace})) return fail(ALG_ERR_INVALID, "workspace must be 16-byte aligned");
@@ -809,7 +809,7 @@ int alg_ffn_gemm(alg_stream_t stream, int M, int N, int K, const void* A, long l
   g.C = static_cast<bf16*>(C);
   g.ldc = ldc;
   g.M = M; g.N = N; g.K = K;
-  g.full = pl.full; g.split = pl.split; g.kchunk = pl.kchunk;
+  g.tile = pl.tile; g.full = pl.full; g.split = pl.split; g.kchunk = pl.kchunk;
   g.part = need ? static_cast<float*>(workspace) : nullptr;
   // A stored (M, K) is k-contiguous; B stored (N, K) is k-contiguous.
   return hip_status(alg::launch_ffn_gemm(g, a_trans ? alg::MNMAJOR : alg::KMAJOR, b_trans ? alg::KMAJOR : alg::MNMAJOR,

@@ -41,6 +41,8 @@ namespace alg {
 // vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
 constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
 constexpr int VMCNT0 = vmcnt_imm(0);
+// vmcnt(n) and lgkmcnt(0).
+constexpr int vmcnt_lgkm0_imm(int n) { return vmcnt_imm(n) & ~0x0F00; }
 }  // namespace alg
 
 namespace alg {

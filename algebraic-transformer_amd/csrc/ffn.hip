@@ -10,6 +10,7 @@
 // d_act = round(dy gate), d_up = round(d_act (0.5 (1 + u) + 0.5 u r^2)) (u, r recomputed from
 // up), stored as one (N, 2F) matrix [d_gate | d_up] so dh2 and [dw_g | dw_u] are one product
 // each. The remaining products (y w_d, dh2, the weight gradients) are plain GEMMs.
+#include <algorithm>
 #include <cmath>
 
 #include "gemm_core.h"
@@ -20,8 +21,9 @@
 
 namespace alg {
 
-typedef HeadGemm FC;  // 256 x 256 tiles, 8 waves (2 x 4)
-constexpr int FNT = FC::THREADS;
+typedef HeadGemm FC;                    // 256 x 256 tiles, 8 waves (2 x 4)
+typedef GemmCfg<128, 128, 2, 2> FC128;  // products that fill less of the chip
+typedef GemmCfg<64, 64, 2, 2> FC64;
 
 namespace {
 
@@ -41,136 +43,156 @@ __device__ __forceinline__ float alu_f32(float z, float beta, float& u, float& r
 
 __device__ __forceinline__ float rb(float x) { return (float)f2bf(x); }
 
-// Each wave stages its 128 x 64 block of bf16 values in its own 16 KiB share of the (idle)
-// pipeline buffers, rows of 8 16-byte chunks XOR-swizzled by the row, so the accumulator's
+// Each wave stages its WTM x WTN block of bf16 values in its own share of the (idle) pipeline
+// buffers, rows of WTN / 8 16-byte chunks XOR-swizzled by the row, so the accumulator's
 // column-per-lane writes spread over the banks and the 16-byte row reads stay aligned; the
 // global loads and stores of the epilogue then move 8 consecutive columns per lane.
-__device__ __forceinline__ int stage_at(int r, int c) { return r * 64 + ((((c >> 3) ^ (r & 7)) & 7) << 3) + (c & 7); }
+template <int W>
+__device__ __forceinline__ int stage_at(int r, int c) {
+  return r * W + (((c >> 3) ^ (r & (W / 8 - 1))) << 3) + (c & 7);
+}
 
-template <class Stage>
-__device__ __forceinline__ bf16* wave_stage(Stage& s0, Stage& s1, int wm, int wn) {
-  static_assert(FC::WM * FC::WN == 8 && FC::WTM == 128 && FC::WTN == 64, "staging assumes 8 waves of 128 x 64");
-  static_assert(sizeof(Stage) >= 4 * 128 * 64 * sizeof(bf16), "a stage holds four waves' blocks");
-  const int wi = wm * FC::WN + wn;  // 8 waves: 0..3 in s0, 4..7 in s1
-  return reinterpret_cast<bf16*>(wi < 4 ? static_cast<void*>(&s0) : static_cast<void*>(&s1)) + (wi & 3) * 128 * 64;
+// Tile (m0, n0) of A B over k in [kbeg, kend), handed to epi(acc, stage) with this wave's
+// staging share, free of readers.
+template <int AM, int BM, class C, class Epi>
+__device__ __forceinline__ void ffn_tile(const GemmOperand& A, const GemmOperand& B, int m0, int n0, int kbeg, int kend,
+                                         Epi epi) {
+  floatx16 acc[C::MB][C::NB];
+  constexpr int BLOCK = C::WTM * C::WTN;
+  int wm, wn;
+  wave_coords<C>(wm, wn);
+  const int wi = wm * C::WN + wn;
+  if constexpr (C::THREADS == 512) {
+    __shared__ __attribute__((aligned(16))) GemmStage<AM, BM, C> s0, s1;
+    static_assert(sizeof(s0) >= 4 * BLOCK * sizeof(bf16), "a stage holds four waves' blocks");
+    gemm_mainloop<AM, BM, C>(s0, s1, A, B, m0, n0, kbeg, kend, acc);
+    __syncthreads();  // every wave is done reading the pipeline buffers
+    epi(acc, reinterpret_cast<bf16*>(wi < 4 ? static_cast<void*>(&s0) : static_cast<void*>(&s1)) + (wi & 3) * BLOCK);
+  } else {
+    __shared__ __attribute__((aligned(16))) GemmStage<AM, BM, C> s0, s1, s2, s3;
+    static_assert(sizeof(s0) >= 2 * BLOCK * sizeof(bf16), "a stage holds two waves' blocks");
+    gemm_ring<AM, BM, C>(s0, s1, s2, s3, A, B, m0, n0, kbeg, kend, acc);
+    __syncthreads();
+    epi(acc, reinterpret_cast<bf16*>(wi < 2 ? static_cast<void*>(&s0) : static_cast<void*>(&s1)) + (wi & 1) * BLOCK);
+  }
 }
 
 }  // namespace
 
-__global__ __launch_bounds__(FNT, 1) void ffn_gate_up_kernel(FfnParams p) {
-  __shared__ __attribute__((aligned(16))) GemmStage<KMAJOR, MNMAJOR, FC> s0, s1;
-  const int nbm = (p.N + HT_M - 1) / HT_M, nbn = 2 * p.F / HT_N;
+template <class C>
+__global__ __launch_bounds__(C::THREADS, 2) void ffn_gate_up_kernel(FfnParams p) {
+  const int nbm = (p.N + C::TM - 1) / C::TM, nbn = 2 * p.F / C::TN;
   int tm, tn;
   xcd_tile(blockIdx.x, nbm, nbn, tm, tn);
-  const int m0 = tm * HT_M, n0 = tn * HT_N;  // tokens, logical [gate | up] columns
+  const int m0 = tm * C::TM, n0 = tn * C::TN;  // tokens, logical [gate | up] columns
   GemmOperand A{p.h2, p.d, p.N, p.d, (long)p.N * p.d};
   GemmOperand B{p.w_gu, 2L * p.F, p.d, 2 * p.F, 2L * p.d * p.F, (long)p.F};
-  floatx16 acc[FC::MB][FC::NB];
-  gemm_mainloop<KMAJOR, MNMAJOR, FC>(s0, s1, A, B, m0, n0, 0, p.d, acc);
-  const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
-  int wm, wn;
-  wave_coords<FC>(wm, wn);
-  // acc[.][0] is gate column f0 + l32, acc[.][1] up column f0 + l32 (f0 = n0/2 + 32 wn).
-  __syncthreads();  // every wave is done reading the pipeline buffers
-  bf16* stg = wave_stage(s0, s1, wm, wn);  // [row][0..31] gate, [row][32..63] up
+  ffn_tile<KMAJOR, MNMAJOR, C>(A, B, m0, n0, 0, p.d, [&](const floatx16 (&acc)[C::MB][C::NB], bf16* stg) {
+    static_assert(C::NB == 2, "a wave's two column blocks are gate and up");
+    const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
+    int wm, wn;
+    wave_coords<C>(wm, wn);
+    // acc[.][0] is gate column f0 + l32, acc[.][1] up column f0 + l32 (f0 = n0/2 + 32 wn);
+    // staged as [row][0..31] gate, [row][32..63] up.
 #pragma unroll
-  for (int mb = 0; mb < FC::MB; ++mb) {
+    for (int mb = 0; mb < C::MB; ++mb) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
-      stg[stage_at(row, l32)] = f2bf(acc[mb][0][i]);
-      stg[stage_at(row, 32 + l32)] = f2bf(acc[mb][1][i]);
+      for (int i = 0; i < 16; ++i) {
+        const int row = mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+        stg[stage_at<64>(row, l32)] = f2bf(acc[mb][0][i]);
+        stg[stage_at<64>(row, 32 + l32)] = f2bf(acc[mb][1][i]);
+      }
     }
-  }
-  // 128 rows x 4 chunks of 8 columns: lane -> (row, chunk).
-  const int f0 = n0 / 2 + wn * 32;
+    // WTM rows x 4 chunks of 8 columns: lane -> (row, chunk).
+    const int f0 = n0 / 2 + wn * 32;
 #pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int idx = it * 64 + lane, row = idx >> 2, ch = idx & 3;
-    const int tok = m0 + wm * FC::WTM + row;
-    const bf16x8 gv = *reinterpret_cast<const bf16x8*>(stg + stage_at(row, 8 * ch));
-    const bf16x8 uv = *reinterpret_cast<const bf16x8*>(stg + stage_at(row, 32 + 8 * ch));
-    bf16x8 yv;
+    for (int it = 0; it < C::WTM / 16; ++it) {
+      const int idx = it * 64 + lane, row = idx >> 2, ch = idx & 3;
+      const int tok = m0 + wm * C::WTM + row;
+      const bf16x8 gv = *reinterpret_cast<const bf16x8*>(stg + stage_at<64>(row, 8 * ch));
+      const bf16x8 uv = *reinterpret_cast<const bf16x8*>(stg + stage_at<64>(row, 32 + 8 * ch));
+      bf16x8 yv;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float u, r;
-      const float act = rb(alu_f32((float)uv[e], p.beta, u, r));
-      yv[e] = f2bf(__fmul_rn((float)gv[e], act));
+      for (int e = 0; e < 8; ++e) {
+        float u, r;
+        const float act = rb(alu_f32((float)uv[e], p.beta, u, r));
+        yv[e] = f2bf(__fmul_rn((float)gv[e], act));
+      }
+      if (tok < p.N) {
+        const size_t o = (size_t)tok * p.F + f0 + 8 * ch;
+        *reinterpret_cast<bf16x8*>(p.y + o) = yv;
+        *reinterpret_cast<bf16x8*>(p.gate + o) = gv;
+        *reinterpret_cast<bf16x8*>(p.up + o) = uv;
+      }
     }
-    if (tok < p.N) {
-      const size_t o = (size_t)tok * p.F + f0 + 8 * ch;
-      *reinterpret_cast<bf16x8*>(p.y + o) = yv;
-      *reinterpret_cast<bf16x8*>(p.gate + o) = gv;
-      *reinterpret_cast<bf16x8*>(p.up + o) = uv;
-    }
-  }
+  });
 }
 
-__global__ __launch_bounds__(FNT, 1) void ffn_dy_kernel(FfnParams p) {
-  __shared__ __attribute__((aligned(16))) GemmStage<KMAJOR, KMAJOR, FC> s0, s1;
-  const int nbm = (p.N + HT_M - 1) / HT_M, nbn = (p.F + HT_N - 1) / HT_N;
+template <class C>
+__global__ __launch_bounds__(C::THREADS, 2) void ffn_dy_kernel(FfnParams p) {
+  const int nbm = (p.N + C::TM - 1) / C::TM, nbn = (p.F + C::TN - 1) / C::TN;
   int tm, tn;
   xcd_tile(blockIdx.x, nbm, nbn, tm, tn);
-  const int m0 = tm * HT_M, n0 = tn * HT_N;  // tokens, columns f
+  const int m0 = tm * C::TM, n0 = tn * C::TN;  // tokens, columns f
   GemmOperand A{p.dout, p.dm, p.N, p.dm, (long)p.N * p.dm};
   GemmOperand B{p.w_d, p.dm, p.F, p.dm, (long)p.F * p.dm};  // w_d (F, dm): [f][k]
-  floatx16 acc[FC::MB][FC::NB];
-  gemm_mainloop<KMAJOR, KMAJOR, FC>(s0, s1, A, B, m0, n0, 0, p.dm, acc);
-  const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
-  int wm, wn;
-  wave_coords<FC>(wm, wn);
-  __syncthreads();  // every wave is done reading the pipeline buffers
-  bf16* stg = wave_stage(s0, s1, wm, wn);  // this wave's dy block, [row][0..63]
+  ffn_tile<KMAJOR, KMAJOR, C>(A, B, m0, n0, 0, p.dm, [&](const floatx16 (&acc)[C::MB][C::NB], bf16* stg) {
+    constexpr int W = C::WTN, CH = W / 8;  // this wave's dy block, [row][0..W)
+    const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
+    int wm, wn;
+    wave_coords<C>(wm, wn);
 #pragma unroll
-  for (int mb = 0; mb < FC::MB; ++mb) {
+    for (int mb = 0; mb < C::MB; ++mb) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+      for (int i = 0; i < 16; ++i) {
+        const int row = mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
 #pragma unroll
-      for (int nb = 0; nb < FC::NB; ++nb) stg[stage_at(row, nb * 32 + l32)] = f2bf(acc[mb][nb][i]);
+        for (int nb = 0; nb < C::NB; ++nb) stg[stage_at<W>(row, nb * 32 + l32)] = f2bf(acc[mb][nb][i]);
+      }
     }
-  }
-  // 128 rows x 8 chunks of 8 columns: lane -> (row, chunk), in groups of GRP chunks per lane
-  // whose gate/up loads are issued together (out-of-range chunks read chunk 0 and are not
-  // stored): behind a per-chunk range check each load got a branch and a wait of its own.
-  const int f0 = n0 + wn * FC::WTN;
-  constexpr int GRP = 8;
+    // WTM rows x CH chunks of 8 columns: lane -> (row, chunk), in groups of GRP chunks per lane
+    // whose gate/up loads are issued together (out-of-range chunks read chunk 0 and are not
+    // stored): behind a per-chunk range check each load got a branch and a wait of its own.
+    const int f0 = n0 + wn * W;
+    constexpr int PER = C::WTM * CH / 64, GRP = PER < 8 ? PER : 8;
 #pragma unroll 1
-  for (int g0 = 0; g0 < 16; g0 += GRP) {
-    bf16x8 gvs[GRP], uvs[GRP];
+    for (int g0 = 0; g0 < PER; g0 += GRP) {
+      bf16x8 gvs[GRP], uvs[GRP];
 #pragma unroll
-    for (int k = 0; k < GRP; ++k) {
-      const int idx = (g0 + k) * 64 + lane, row = idx >> 3, ch = idx & 7;
-      const int tok = m0 + wm * FC::WTM + row, f = f0 + 8 * ch;
-      const size_t o = tok < p.N && f < p.F ? (size_t)tok * p.F + f : 0;
-      gvs[k] = *reinterpret_cast<const bf16x8*>(p.gate + o);
-      uvs[k] = *reinterpret_cast<const bf16x8*>(p.up + o);
+      for (int k = 0; k < GRP; ++k) {
+        const int idx = (g0 + k) * 64 + lane, row = idx / CH, ch = idx % CH;
+        const int tok = m0 + wm * C::WTM + row, f = f0 + 8 * ch;
+        const size_t o = tok < p.N && f < p.F ? (size_t)tok * p.F + f : 0;
+        gvs[k] = *reinterpret_cast<const bf16x8*>(p.gate + o);
+        uvs[k] = *reinterpret_cast<const bf16x8*>(p.up + o);
+      }
+#pragma unroll
+      for (int k = 0; k < GRP; ++k) asm volatile("" : "+v"(gvs[k]), "+v"(uvs[k]));  // loads before the checks
+#pragma unroll
+      for (int k = 0; k < GRP; ++k) {
+        const int idx = (g0 + k) * 64 + lane, row = idx / CH, ch = idx % CH;
+        const int tok = m0 + wm * C::WTM + row, f = f0 + 8 * ch;
+        if (tok >= p.N || f >= p.F) continue;  // F is a multiple of 128: chunks are whole
+        const bf16x8 dyv = *reinterpret_cast<const bf16x8*>(stg + stage_at<W>(row, 8 * ch));
+        const bf16x8 gv = gvs[k], uv = uvs[k];
+        bf16x8 dg, du;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float dy = (float)dyv[e];
+          float u, r;
+          const float act = rb(alu_f32((float)uv[e], p.beta, u, r));
+          const float d_act = rb(__fmul_rn(dy, (float)gv[e]));
+          const float deriv =
+              __fadd_rn(__fmul_rn(0.5f, __fadd_rn(1.0f, u)), __fmul_rn(__fmul_rn(0.5f, u), __fmul_rn(r, r)));
+          dg[e] = f2bf(__fmul_rn(dy, act));
+          du[e] = f2bf(__fmul_rn(d_act, deriv));
+        }
+        const size_t od = (size_t)tok * 2 * p.F + f;
+        *reinterpret_cast<bf16x8*>(p.d_gu + od) = dg;
+        *reinterpret_cast<bf16x8*>(p.d_gu + od + p.F) = du;
+      }
     }
-#pragma unroll
-    for (int k = 0; k < GRP; ++k) asm volatile("" : "+v"(gvs[k]), "+v"(uvs[k]));  // loads before the checks
-#pragma unroll
-  for (int k = 0; k < GRP; ++k) {
-    const int idx = (g0 + k) * 64 + lane, row = idx >> 3, ch = idx & 7;
-    const int tok = m0 + wm * FC::WTM + row, f = f0 + 8 * ch;
-    if (tok >= p.N || f >= p.F) continue;  // F is a multiple of 128: chunks are whole
-    const bf16x8 dyv = *reinterpret_cast<const bf16x8*>(stg + stage_at(row, 8 * ch));
-    const bf16x8 gv = gvs[k], uv = uvs[k];
-    bf16x8 dg, du;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float dy = (float)dyv[e];
-      float u, r;
-      const float act = rb(alu_f32((float)uv[e], p.beta, u, r));
-      const float d_act = rb(__fmul_rn(dy, (float)gv[e]));
-      const float deriv = __fadd_rn(__fmul_rn(0.5f, __fadd_rn(1.0f, u)), __fmul_rn(__fmul_rn(0.5f, u), __fmul_rn(r, r)));
-      dg[e] = f2bf(__fmul_rn(dy, act));
-      du[e] = f2bf(__fmul_rn(d_act, deriv));
-    }
-    const size_t od = (size_t)tok * 2 * p.F + f;
-    *reinterpret_cast<bf16x8*>(p.d_gu + od) = dg;
-    *reinterpret_cast<bf16x8*>(p.d_gu + od + p.F) = du;
-  }
-  }
+  });
 }
 
 // Plain products of the block (model.py:185-193: y w_d in the forward; [d_gate | d_up] [w_g |
@@ -179,10 +201,9 @@ __global__ __launch_bounds__(FNT, 1) void ffn_dy_kernel(FfnParams p) {
 // Workgroups below g.full compute whole tiles, row-major inside each XCD's share; the rest
 // compute k range (id - full) % split of tile full + (id - full) / split into an f32 tile of
 // g.part, which ffn_gemm_tail_kernel sums in range order (ffn_gemm_plan).
-template <int AM, int BM>
-__global__ __launch_bounds__(FNT, 1) void ffn_gemm_kernel(FfnGemmParams g) {
-  __shared__ __attribute__((aligned(16))) GemmStage<AM, BM, FC> s0, s1;
-  const int nbn = (g.N + HT_N - 1) / HT_N;
+template <int AM, int BM, class C>
+__global__ __launch_bounds__(C::THREADS, 2) void ffn_gemm_kernel(FfnGemmParams g) {
+  const int nbn = (g.N + C::TN - 1) / C::TN;
   const int bid = blockIdx.x;
   int lin, kbeg = 0, kend = g.K, unit = -1;
   if (bid < g.full) {
@@ -194,78 +215,66 @@ __global__ __launch_bounds__(FNT, 1) void ffn_gemm_kernel(FfnGemmParams g) {
     kend = min(g.K, kbeg + g.kchunk);
   }
   const int tm = lin / nbn, tn = lin - tm * nbn;
-  const int m0 = tm * HT_M, n0 = tn * HT_N;
-  floatx16 acc[FC::MB][FC::NB];
-  gemm_mainloop<AM, BM, FC>(s0, s1, g.A, g.B, m0, n0, kbeg, kend, acc);
-  const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
-  int wm, wn;
-  wave_coords<FC>(wm, wn);
-  if (unit >= 0) {  // one k range of a split tile: the whole f32 tile, row-major
-    float* part = g.part + (size_t)unit * HT_M * HT_N;
+  const int m0 = tm * C::TM, n0 = tn * C::TN;
+  ffn_tile<AM, BM, C>(g.A, g.B, m0, n0, kbeg, kend, [&](const floatx16 (&acc)[C::MB][C::NB], bf16* stg) {
+    constexpr int W = C::WTN, CH = W / 8;
+    const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
+    int wm, wn;
+    wave_coords<C>(wm, wn);
+    if (unit >= 0) {  // one k range of a split tile: the whole f32 tile, row-major
+      float* part = g.part + (size_t)unit * C::TM * C::TN;
 #pragma unroll
-    for (int mb = 0; mb < FC::MB; ++mb)
+      for (int mb = 0; mb < C::MB; ++mb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = wm * FC::WTM + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+        for (int i = 0; i < 16; ++i) {
+          const int r = wm * C::WTM + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
 #pragma unroll
-        for (int nb = 0; nb < FC::NB; ++nb) part[r * HT_N + wn * FC::WTN + nb * 32 + l32] = acc[mb][nb][i];
-      }
-    return;
-  }
-  if (m0 + HT_M <= g.M && n0 + HT_N <= g.N) {  // interior tile: staged 16-byte row stores
-    __syncthreads();  // every wave is done reading the pipeline buffers
-    bf16* stg = wave_stage(s0, s1, wm, wn);
+          for (int nb = 0; nb < C::NB; ++nb) part[r * C::TN + wn * W + nb * 32 + l32] = acc[mb][nb][i];
+        }
+      return;
+    }
+    // Staged 16-byte row stores; N is a multiple of 8, so a chunk lies inside a row or past it.
 #pragma unroll
-    for (int mb = 0; mb < FC::MB; ++mb) {
+    for (int mb = 0; mb < C::MB; ++mb) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int row = mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
 #pragma unroll
-        for (int nb = 0; nb < FC::NB; ++nb) stg[stage_at(row, nb * 32 + l32)] = f2bf(acc[mb][nb][i]);
+        for (int nb = 0; nb < C::NB; ++nb) stg[stage_at<W>(row, nb * 32 + l32)] = f2bf(acc[mb][nb][i]);
       }
     }
-    bf16* out = g.C + (size_t)(m0 + wm * FC::WTM) * g.ldc + n0 + wn * FC::WTN;
+    const int mw = m0 + wm * C::WTM, nw = n0 + wn * W;
+    bf16* out = g.C + (size_t)mw * g.ldc + nw;
+    const bool inside = m0 + C::TM <= g.M && n0 + C::TN <= g.N;
 #pragma unroll 4
-    for (int it = 0; it < 16; ++it) {
-      const int idx = it * 64 + lane, row = idx >> 3, ch = idx & 7;
-      *reinterpret_cast<bf16x8*>(out + (size_t)row * g.ldc + 8 * ch) =
-          *reinterpret_cast<const bf16x8*>(stg + stage_at(row, 8 * ch));
+    for (int it = 0; it < C::WTM * CH / 64; ++it) {
+      const int idx = it * 64 + lane, row = idx / CH, ch = idx % CH;
+      if (inside || (mw + row < g.M && nw + 8 * ch < g.N))
+        *reinterpret_cast<bf16x8*>(out + (size_t)row * g.ldc + 8 * ch) =
+            *reinterpret_cast<const bf16x8*>(stg + stage_at<W>(row, 8 * ch));
     }
-    return;
-  }
-#pragma unroll
-  for (int mb = 0; mb < FC::MB; ++mb) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int m = m0 + wm * FC::WTM + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
-      if (m >= g.M) continue;
-#pragma unroll
-      for (int nb = 0; nb < FC::NB; ++nb) {
-        const int n = n0 + wn * FC::WTN + nb * 32 + l32;
-        if (n < g.N) g.C[(size_t)m * g.ldc + n] = f2bf(acc[mb][nb][i]);
-      }
-    }
-  }
+  });
 }
 
 // C of a split tile: its split f32 range tiles summed in range order, 32 rows of the tile per
-// workgroup (grid: split tiles x HT_M / 32). N is a multiple of 8, so 8 columns that start
+// workgroup (grid: split tiles x TM / 32). N is a multiple of 8, so 8 columns that start
 // inside the matrix lie inside it.
+template <class C>
 __global__ __launch_bounds__(256) void ffn_gemm_tail_kernel(FfnGemmParams g) {
-  const int nbn = (g.N + HT_N - 1) / HT_N;
+  const int nbn = (g.N + C::TN - 1) / C::TN;
   const int lin = g.full + blockIdx.x;
   const int tm = lin / nbn, tn = lin - tm * nbn;
-  const float* part = g.part + (size_t)blockIdx.x * g.split * HT_M * HT_N;
+  const float* part = g.part + (size_t)blockIdx.x * g.split * C::TM * C::TN;
 #pragma unroll
-  for (int c = 0; c < 32 * HT_N / 8 / 256; ++c) {
+  for (int c = 0; c < 32 * C::TN / 8 / 256; ++c) {
     const int e = (threadIdx.x + 256 * c) * 8;
-    const int r = blockIdx.y * 32 + e / HT_N, col = e % HT_N;
-    const int m = tm * HT_M + r, n = tn * HT_N + col;
+    const int r = blockIdx.y * 32 + e / C::TN, col = e % C::TN;
+    const int m = tm * C::TM + r, n = tn * C::TN + col;
     if (m >= g.M || n >= g.N) continue;
-    const size_t o = (size_t)r * HT_N + col;
+    const size_t o = (size_t)r * C::TN + col;
     float4 a = *reinterpret_cast<const float4*>(part + o), b = *reinterpret_cast<const float4*>(part + o + 4);
     for (int k = 1; k < g.split; ++k) {
-      const float* q = part + (size_t)k * HT_M * HT_N + o;
+      const float* q = part + (size_t)k * C::TM * C::TN + o;
       const float4 x = *reinterpret_cast<const float4*>(q), y = *reinterpret_cast<const float4*>(q + 4);
       a.x += x.x; a.y += x.y; a.z += x.z; a.w += x.w;
       b.x += y.x; b.y += y.y; b.z += y.z; b.w += y.w;
@@ -278,69 +287,133 @@ __global__ __launch_bounds__(256) void ffn_gemm_tail_kernel(FfnGemmParams g) {
   }
 }
 
-// Split plan: the tiles past the last complete round of 256 workgroups (all of them when there
-// are fewer than 256) are split over k into S ranges when that is cheaper. Cost model, from
-// the head products' measured rates: a round of 256 x 256 tiles costs 23.4 ns per k step of
-// one element (48 us for K = 2048), and each split range tile costs its f32 tile written,
-// read and summed (512 KiB at about 5 TB/s over the chip, 0.1 us) plus 5 us for the summing
-// launch. A range keeps at least 1024 of K (so every range is non-empty).
+// Time in us of `units` workgroups of a tile configuration over k steps of K in all, fitted to
+// the products of one short sequence and of the 1b block (M N K, measured us for tiles of 256 /
+// 128 / 64, each in a captured graph with its launch):
+//   1024  768 2048   39.3 / 20.8 / 11.0     768 4096 1024   25.4 / 14.7 / 19.6
+//   1024  768 4096   69.5 / 37.2 / 19.2    2048  768 1024   23.2 / 12.6 /  8.3
+//    512  512 2048   37.5 / 20.2 / 10.5    2048 2048 2048   41.8 / 25.1 / 36.7
+// A 256 tile needs 14.8 ns per k alone on the chip and 23.4 ns when all CUs hold one (power); 128
+// tiles 8 to 10 ns; 64 tiles 4 ns while a CU holds one, 8 ns for two. Small tiles move two or four
+// times the operand bytes per multiplication, so they win only while the larger ones leave
+// CUs idle.
+static double ffn_tile_time(int tile, int units, double K) {
+  const double fill = std::min(1.0, units / 256.0), rounds = std::ceil(units / 256.0);
+  if (tile == 256) return 9.0 + rounds * K * (0.0148 + 0.0086 * fill);
+  if (tile == 128) return 4.4 + rounds * K * (0.008 + 0.002 * fill);
+  return 2.8 + K * (units <= 512 ? 0.004 + 0.004 * std::max(0, units - 256) / 256.0 : std::ceil(units / 512.0) * 0.008);
+}
+
+static int ffn_tiles(int tile, int M, int N) { return ((M + tile - 1) / tile) * ((N + tile - 1) / tile); }
+
+// Tile of an unsplit product with an epilogue of its own (allowed: 256, 128 and, if `min_tile`
+// lets it, 64).
+static int ffn_epilogue_tile(int M, int N, int K, int min_tile) {
+  int best = 256;
+  for (int t = 128; t >= min_tile; t /= 2)
+    if (ffn_tile_time(t, ffn_tiles(t, M, N), K) < ffn_tile_time(best, ffn_tiles(best, M, N), K)) best = t;
+  return best;
+}
+
+// Plan of a plain product. With 256 x 256 tiles, those past the last complete round of 256
+// workgroups (all of them when there are fewer than 256) are split over k into S ranges when that
+// is cheaper. Cost model, from the head products' measured rates: a round of 256 x 256 tiles
+// costs 23.4 ns per k step of one element (48 us for K = 2048), and each split range tile costs
+// its f32 tile written, read and summed (512 KiB at about 5 TB/s over the chip, 0.1 us) plus 5 us
+// for the summing launch. A range keeps at least 1024 of K (so every range is non-empty). The
+// workspace is that of this split. A product that fills less of the chip runs on smaller tiles
+// when ffn_tile_time says so; 64 x 64 tiles are split over k (ranges of at least 512) as far as
+// the same workspace goes, which pays where few tiles have a long k (304 1024 4096: 26.9 us
+// whole, 15.0 us in four ranges).
 FfnGemmPlan ffn_gemm_plan(int M, int N, int K) {
   FfnGemmPlan pl;
-  pl.tiles = ((M + HT_M - 1) / HT_M) * ((N + HT_N - 1) / HT_N);
+  pl.tile = 256;
+  pl.tiles = ffn_tiles(256, M, N);
   pl.full = pl.tiles;
   pl.split = 1;
   pl.kchunk = 0;
+  pl.ws_bytes = 0;
   const int base = pl.tiles / 256 * 256, tail = pl.tiles - base;
-  if (tail == 0) return pl;
-  auto cost = [&](int s) {
-    const double rounds = std::ceil(tail * (double)s / 256.0);
-    return rounds * (K / (double)s) * 0.0234 + (s > 1 ? tail * s * 0.1 + 5.0 : 0.0);
-  };
-  int best = 1;
-  double best_cost = cost(1);
-  for (int s = 2; s <= 8 && K / s >= 1024; ++s) {
-    const double c = cost(s);
-    if (c < best_cost - 1e-9) { best = s; best_cost = c; }
+  if (tail) {
+    auto cost = [&](int s) {
+      const double rounds = std::ceil(tail * (double)s / 256.0);
+      return rounds * (K / (double)s) * 0.0234 + (s > 1 ? tail * s * 0.1 + 5.0 : 0.0);
+    };
+    int best = 1;
+    double best_cost = cost(1);
+    for (int s = 2; s <= 8 && K / s >= 1024; ++s) {
+      const double c = cost(s);
+      if (c < best_cost - 1e-9) { best = s; best_cost = c; }
+    }
+    if (best > 1) {
+      pl.full = base;
+      pl.split = best;
+      pl.kchunk = ((K + best - 1) / best + 127) / 128 * 128;
+      pl.ws_bytes = (size_t)tail * best * 256 * 256 * sizeof(float);
+    }
   }
-  if (best == 1) return pl;
-  pl.full = base;
-  pl.split = best;
-  pl.kchunk = ((K + best - 1) / best + 127) / 128 * 128;
+  if (base) return pl;  // a whole round of 256 tiles: the chip is full
+  double best_time = pl.split == 1 ? ffn_tile_time(256, pl.tiles, K)
+                                   : ffn_tile_time(256, pl.tiles * pl.split, pl.kchunk) + 5.0;
+  auto consider = [&](int tile, int s) {
+    const int tiles = ffn_tiles(tile, M, N);
+    const int chunk = s > 1 ? ((K + s - 1) / s + 127) / 128 * 128 : K;
+    const double t = ffn_tile_time(tile, tiles * s, chunk) + (s > 1 ? 5.0 : 0.0);
+    if (t >= best_time) return;
+    best_time = t;
+    pl.tile = tile;
+    pl.tiles = tiles;
+    pl.full = s > 1 ? 0 : tiles;
+    pl.split = s;
+    pl.kchunk = s > 1 ? chunk : 0;
+  };
+  consider(128, 1);
+  consider(64, 1);
+  const size_t plane = (size_t)ffn_tiles(64, M, N) * 64 * 64 * sizeof(float);
+  for (int s = 2; s <= 8 && K / s >= 512 && s * plane <= pl.ws_bytes; s *= 2) consider(64, s);
   return pl;
 }
 
-size_t ffn_gemm_workspace_bytes(const FfnGemmPlan& pl) {
-  return pl.split > 1 ? (size_t)(pl.tiles - pl.full) * pl.split * HT_M * HT_N * sizeof(float) : 0;
-}
-
-hipError_t launch_ffn_gemm(const FfnGemmParams& g, int a_mode, int b_mode, hipStream_t st) {
-  const int tiles = ((g.M + HT_M - 1) / HT_M) * ((g.N + HT_N - 1) / HT_N);
-  const int grid = g.split > 1 ? g.full + (tiles - g.full) * g.split : tiles;
+template <class C>
+static void launch_ffn_gemm_cfg(const FfnGemmParams& g, int a_mode, int b_mode, hipStream_t st) {
+  const int tiles = ((g.M + C::TM - 1) / C::TM) * ((g.N + C::TN - 1) / C::TN);
+  const dim3 grid(g.split > 1 ? g.full + (tiles - g.full) * g.split : tiles), nt(C::THREADS);
   {
     KTimer t("ffn_gemm", st);
-    if (a_mode == KMAJOR && b_mode == KMAJOR) hipLaunchKernelGGL((ffn_gemm_kernel<KMAJOR, KMAJOR>), dim3(grid), dim3(FNT), 0, st, g);
-    else if (a_mode == KMAJOR) hipLaunchKernelGGL((ffn_gemm_kernel<KMAJOR, MNMAJOR>), dim3(grid), dim3(FNT), 0, st, g);
-    else if (b_mode == KMAJOR) hipLaunchKernelGGL((ffn_gemm_kernel<MNMAJOR, KMAJOR>), dim3(grid), dim3(FNT), 0, st, g);
-    else hipLaunchKernelGGL((ffn_gemm_kernel<MNMAJOR, MNMAJOR>), dim3(grid), dim3(FNT), 0, st, g);
+    if (a_mode == KMAJOR && b_mode == KMAJOR) hipLaunchKernelGGL((ffn_gemm_kernel<KMAJOR, KMAJOR, C>), grid, nt, 0, st, g);
+    else if (a_mode == KMAJOR) hipLaunchKernelGGL((ffn_gemm_kernel<KMAJOR, MNMAJOR, C>), grid, nt, 0, st, g);
+    else if (b_mode == KMAJOR) hipLaunchKernelGGL((ffn_gemm_kernel<MNMAJOR, KMAJOR, C>), grid, nt, 0, st, g);
+    else hipLaunchKernelGGL((ffn_gemm_kernel<MNMAJOR, MNMAJOR, C>), grid, nt, 0, st, g);
   }
   if (g.split > 1) {
     KTimer t("ffn_gemm_tail", st);
-    hipLaunchKernelGGL(ffn_gemm_tail_kernel, dim3(tiles - g.full, HT_M / 32), dim3(256), 0, st, g);
+    hipLaunchKernelGGL(ffn_gemm_tail_kernel<C>, dim3(tiles - g.full, C::TM / 32), dim3(256), 0, st, g);
   }
+}
+
+hipError_t launch_ffn_gemm(const FfnGemmParams& g, int a_mode, int b_mode, hipStream_t st) {
+  if (g.tile == 64) launch_ffn_gemm_cfg<FC64>(g, a_mode, b_mode, st);
+  else if (g.tile == 128) launch_ffn_gemm_cfg<FC128>(g, a_mode, b_mode, st);
+  else launch_ffn_gemm_cfg<FC>(g, a_mode, b_mode, st);
   return hipGetLastError();
 }
 
 hipError_t launch_ffn_fwd(const FfnParams& p, hipStream_t st) {
-  const int tiles = ((p.N + HT_M - 1) / HT_M) * (2 * p.F / HT_N);
   KTimer t("ffn_gate_up", st);
-  hipLaunchKernelGGL(ffn_gate_up_kernel, dim3(tiles), dim3(FNT), 0, st, p);
+  if (ffn_epilogue_tile(p.N, 2 * p.F, p.d, 128) == 128)
+    hipLaunchKernelGGL(ffn_gate_up_kernel<FC128>, dim3(ffn_tiles(128, p.N, 2 * p.F)), dim3(FC128::THREADS), 0, st, p);
+  else
+    hipLaunchKernelGGL(ffn_gate_up_kernel<FC>, dim3(ffn_tiles(256, p.N, 2 * p.F)), dim3(FC::THREADS), 0, st, p);
   return hipGetLastError();
 }
 
 hipError_t launch_ffn_dy(const FfnParams& p, hipStream_t st) {
-  const int tiles = ((p.N + HT_M - 1) / HT_M) * ((p.F + HT_N - 1) / HT_N);
   KTimer t("ffn_dy", st);
-  hipLaunchKernelGGL(ffn_dy_kernel, dim3(tiles), dim3(FNT), 0, st, p);
+  const int tile = ffn_epilogue_tile(p.N, p.F, p.dm, 64);
+  const dim3 grid(ffn_tiles(tile, p.N, p.F));
+  if (tile == 64) hipLaunchKernelGGL(ffn_dy_kernel<FC64>, grid, dim3(FC64::THREADS), 0, st, p);
+  else if (tile == 128) hipLaunchKernelGGL(ffn_dy_kernel<FC128>, grid, dim3(FC128::THREADS), 0, st, p);
+  else hipLaunchKernelGGL(ffn_dy_kernel<FC>, grid, dim3(FC::THREADS), 0, st, p);
   return hipGetLastError();
 }
 

@@ -15,6 +15,7 @@
 // XOR swizzle that keeps the fragment reads free of bank conflicts:
 //   k-contiguous rows (128 B):      chunk c of row r lives at chunk c ^ ((r >> 1) & 7)
 //   mn-contiguous rows (2*TMN B):   chunk c of row r lives at chunk c ^ (4 * (r & 3))
+//     (rows of 128 B: c ^ (4 * ((r >> 1) & 1)), two rows to a period of the banks)
 // The pipelined loop covers the largest multiple of 128 in the k range; a remaining partial
 // k tile is copied through registers with zero fill. Tiles that reach past the matrix edge in
 // m or n stay on the pipelined loop with range-checked copies: every copy instruction gets a
@@ -79,7 +80,7 @@ struct OperandTile {
   static constexpr int READS_PER_FRAG = MODE == KMAJOR ? 1 : 2;  // LDS instructions per fragment
 
   static __device__ __forceinline__ int swz(int row) {
-    return MODE == KMAJOR ? ((row >> 1) & 7) : 4 * (row & 3);
+    return MODE == KMAJOR ? ((row >> 1) & 7) : CPR == 8 ? 4 * ((row >> 1) & 1) : 4 * (row & 3);
   }
   // Element offset of logical (row, chunk) inside the tile.
   static __device__ __forceinline__ int at(int row, int chunk) { return (row * CPR + (chunk ^ swz(row))) * 8; }
@@ -375,6 +376,101 @@ __device__ __forceinline__ void gemm_mainloop(GemmStage<AM, BM, C>& s0, GemmStag
         load(s0, ks, f);
         mma(f);
       }
+    }
+  }
+}
+
+// Main loop for products too small to fill the chip with 256 x 256 tiles: smaller tiles, 4 waves,
+// a ring of four LDS stages. Such a launch is bound by the latency of its copies (a tile has few
+// k steps, its operands come from HBM once, and one or two workgroups run on a CU), so tile
+// kt + 3 is requested while tile kt multiplies and a wave waits only for the copies of the tile
+// it reads next; one barrier per k step both publishes that tile and frees the stage the next
+// request fills. The stages are separate __shared__ objects, as above.
+constexpr int RING = 4;
+template <int AM, int BM, class C>
+__device__ __forceinline__ void gemm_ring(GemmStage<AM, BM, C>& s0, GemmStage<AM, BM, C>& s1,
+                                          GemmStage<AM, BM, C>& s2, GemmStage<AM, BM, C>& s3, const GemmOperand& A,
+                                          const GemmOperand& B, int m0, int n0, int kbeg, int K,
+                                          floatx16 (&acc)[C::MB][C::NB]) {
+  typedef GemmStage<AM, BM, C> Stage;
+  typedef OperandTile<AM, C::TM, C::THREADS> TA;
+  typedef OperandTile<BM, C::TN, C::THREADS> TB;
+  const int lane = threadIdx.x & 63;
+  int wm, wn;
+  wave_coords<C>(wm, wn);
+#pragma unroll
+  for (int i = 0; i < C::MB; ++i)
+#pragma unroll
+    for (int j = 0; j < C::NB; ++j) acc[i][j] = floatx16{};
+  struct Frags {
+    bf16x8 a[C::MB], b[C::NB];
+  };
+  auto load = [&](const Stage& st, int ks, Frags& f) {
+#pragma unroll
+    for (int j = 0; j < C::NB; ++j) f.b[j] = TB::frag(st.b, wn * C::WTN + j * 32, ks, lane);
+#pragma unroll
+    for (int i = 0; i < C::MB; ++i) f.a[i] = TA::frag(st.a, wm * C::WTM + i * 32, ks, lane);
+  };
+  auto mma = [&](const Frags& f) {
+#pragma unroll
+    for (int i = 0; i < C::MB; ++i)
+#pragma unroll
+      for (int j = 0; j < C::NB; ++j) acc[i][j] = mfma_bf16(f.a[i], f.b[j], acc[i][j]);
+  };
+  const int nk = K > kbeg ? (K - kbeg) / GT_K : 0;
+  const bool a_full = (AM == KMAJOR ? A.rows_valid : A.cols_valid) >= m0 + C::TM;
+  const bool b_full = (BM == KMAJOR ? B.rows_valid : B.cols_valid) >= n0 + C::TN;
+  auto pipelined = [&](auto checked) {
+    constexpr bool CHK = decltype(checked)::value;
+    constexpr int NG = TA::PER_WAVE + TB::PER_WAVE;
+    uint32_t aoff[2], boff[2];
+    TA::lane_offsets(A, aoff);
+    TB::lane_offsets(B, boff);
+    const int wave_u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    auto copy_tile = [&](Stage& st, int kt) {
+      TA::template copy<CHK>(st.a, A, aoff, wave_u, m0, kbeg + kt * GT_K);
+      TB::template copy<CHK>(st.b, B, boff, wave_u, n0, kbeg + kt * GT_K);
+    };
+    auto step = [&](const Stage& cur, Stage& fill, int kt) {
+      // Tile kt has landed once at most the two younger tiles' copies are outstanding. This
+      // wave's reads of tile kt - 1 are complete too before any wave refills its stage.
+      if (kt + 2 < nk) __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(2 * NG));
+      else __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(0));
+      asm volatile("s_barrier" ::: "memory");
+      if (kt + 3 < nk) copy_tile(fill, kt + 3);
+      Frags f0, f1;
+      load(cur, 0, f0);
+      load(cur, 1, f1);
+      mma(f0);
+      load(cur, 2, f0);
+      mma(f1);
+      load(cur, 3, f1);
+      mma(f0);
+      mma(f1);
+    };
+    if (nk > 0) copy_tile(s0, 0);
+    if (nk > 1) copy_tile(s1, 1);
+    if (nk > 2) copy_tile(s2, 2);
+    for (int kt = 0; kt < nk; kt += RING) {
+      step(s0, s3, kt);
+      if (kt + 1 < nk) step(s1, s0, kt + 1);
+      if (kt + 2 < nk) step(s2, s1, kt + 2);
+      if (kt + 3 < nk) step(s3, s2, kt + 3);
+    }
+  };
+  if (a_full && b_full) pipelined(std::false_type{});
+  else pipelined(std::true_type{});
+  // The remaining partial k tile: register copies with zero fill.
+  if (const int k0 = kbeg + nk * GT_K; k0 < K) {
+    __syncthreads();
+    TA::copy_zero_fill(s0.a, A, m0, k0, K);
+    TB::copy_zero_fill(s0.b, B, n0, k0, K);
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < GT_K / 16; ++ks) {
+      Frags f;
+      load(s0, ks, f);
+      mma(f);
     }
   }
 }

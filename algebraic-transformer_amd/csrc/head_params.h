@@ -93,6 +93,7 @@ struct FfnGemmParams {
   long ldc;
   int M, N, K;
   float* part;          // f32 tiles of the split tiles (ffn_gemm_plan), or nullptr
+  int tile;             // tile side: 256, 128 or 64 (ffn_gemm_plan)
   int full;             // tiles computed whole
   int split;            // k ranges per remaining tile
   int kchunk;           // k per range (a multiple of 128)
