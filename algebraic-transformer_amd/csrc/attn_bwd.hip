@@ -34,9 +34,6 @@
 namespace alg {
 
 constexpr int BWD_BK = 128;  // keys per workgroup
-// Queries per streamed tile: 64, or 32 where 64 would not fit in LDS (f32 with D=128).
-template <typename T, int D>
-constexpr int bwd_bq() { return (sizeof(T) == 4 && D == 128) ? 32 : 64; }
 // Rows per pre-kernel workgroup, and per block of the sink-gradient partials: the bf16 dQ
 // kernel writes one partial per 128-query workgroup, the f32 pre kernel one per 128 rows.
 constexpr int SINK_ROWS = 128;
@@ -134,54 +131,58 @@ __global__ __launch_bounds__(256) void attn_bwd_pre_kernel(AttnBwdParams p, int 
 // ---------------------------------------------------------------------------
 // main
 // ---------------------------------------------------------------------------
-// Registers <-> LDS staging of an R-row tile of a (T, D) matrix (16-byte chunks; rows >= T
-// read as zero).
-template <typename T, int D, int R>
+// Registers <-> padded LDS staging of an R-row tile of a (T, D) f32 matrix in 16-byte chunks, PER
+// per thread of 256.
+template <int D, int R>
 struct RowTile {
-  static constexpr int CH = 16 / sizeof(T);
-  static constexpr int CPR = D / CH;
-  static constexpr int PER = (R * CPR + 255) / 256;  // chunks per thread
+  static constexpr int CPR = D / 4;
+  static constexpr int PER = R * CPR / 256;
+  static_assert(PER * 256 == R * CPR, "whole chunks per thread");
   // Rows past T load the last row instead (clamped, unconditional loads that nothing waits
   // for until the tile is stored). The query tiles' rows past T carry stat = 0, so their
   // weights and score gradients are exactly zero and the finite stand-in values add nothing.
-  static __device__ __forceinline__ void load(uint4 (&r)[PER], const T* src, int r0, int T_, int ld) {
+  static __device__ __forceinline__ void load(floatx4 (&r)[PER], const float* src, int r0, int T_, int ld) {
 #pragma unroll
     for (int c = 0; c < PER; ++c) {
-      const int idx = threadIdx.x + c * 256;
-      const int row = min(idx / CPR, R - 1), col = (idx - (idx / CPR) * CPR) * CH;
-      r[c] = *reinterpret_cast<const uint4*>(src + (size_t)min(r0 + row, T_ - 1) * ld + col);
+      const int idx = threadIdx.x + c * 256, row = idx / CPR, col = (idx % CPR) * 4;
+      r[c] = *reinterpret_cast<const floatx4*>(src + (size_t)min(r0 + row, T_ - 1) * ld + col);
     }
   }
-  // bf16 tiles are unpadded and swizzled (swz_at); f32 tiles are row-major with `pitch`.
-  static __device__ __forceinline__ void store(T* dst, int pitch, const uint4 (&r)[PER]) {
+  static __device__ __forceinline__ void store(float* dst, int pitch, const floatx4 (&r)[PER]) {
 #pragma unroll
     for (int c = 0; c < PER; ++c) {
-      const int idx = threadIdx.x + c * 256;
-      const int row = idx / CPR, col = (idx - row * CPR) * CH;
-      if (row < R) {
-        if constexpr (sizeof(T) == 2) *reinterpret_cast<uint4*>(dst + swz_at<CPR>(row, col)) = r[c];
-        else *reinterpret_cast<uint4*>(dst + row * pitch + col) = r[c];
-      }
+      const int idx = threadIdx.x + c * 256, row = idx / CPR, col = (idx % CPR) * 4;
+      *reinterpret_cast<floatx4*>(dst + row * pitch + col) = r[c];
     }
   }
 };
 
-template <typename T, int D, int MODE, int L2N>
-__global__ __launch_bounds__(256, 1) void attn_bwd_kernel(AttnBwdParams p) {
+// f32 main kernel: one workgroup = 64 keys of one head against its 64-query tiles. Bound by the
+// f32 matrix instructions (64 cycles for 32 x 32 x 2), so it is cut for balance and for two
+// waves per SIMD: wave (kg, sub) forms the 32 keys kg x 32 queries sub block of each tile (S, dP,
+// dV += P^T dO, dK += dS^T Q), the halves of dK and dV that the two waves of a key group hold
+// are added through LDS at the end, and for dQ each wave takes 32 queries and half of D. At
+// D = 64 the LDS (70 KB) lets two workgroups run on a CU. Against 128 keys per workgroup with one
+// wave per SIMD and the next tile's registers spilled (us, B H T D): 2 12 1024 64: 219 -> 119;
+// 4 12 2048 64: 726 -> 607; 8 16 1024 64: 496 -> 432; 1 4 300 64: 70 -> 40; 2 12 1024 128:
+// 526 -> 212. (Two workgroups per key block, its query tiles dealt between them, took 2 12 1024 64
+// to 109 us, but dQ's addends then arrive in an order that changes from call to call.)
+constexpr int F32_BK = 64, F32_BQ = 64;
+// Barrier for LDS alone: __syncthreads() also waits for every global access in flight, here the
+// dQ atomics and the next tile's loads.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+template <int D, int MODE, int L2N>
+__global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_f32_kernel(AttnBwdParams p) {
   static_assert(D == 64 || D == 128, "head_dim");
-  constexpr bool BF = sizeof(T) == 2;
-  constexpr int BWD_BQ = bwd_bq<T, D>();
-  // f32 tiles: padded row-major; bf16 tiles: unpadded, swizzled (CPR / SCPR chunks per row).
   constexpr int PITCH = D + F32_PAD;
-  constexpr int SPITCH = BWD_BQ + F32_PAD;
-  constexpr int CPR = D / 8, SCPR = BWD_BQ / 8;
+  constexpr int SPITCH = F32_BQ + F32_PAD;
   constexpr int NDB = D / 32;
-  __shared__ __attribute__((aligned(16))) T Ks[BF ? BWD_BK * D : BWD_BK * PITCH];
-  __shared__ __attribute__((aligned(16))) T Qs[BF ? BWD_BQ * D : BWD_BQ * PITCH];
-  __shared__ __attribute__((aligned(16))) T dOs[BF ? BWD_BQ * D : BWD_BQ * PITCH];
-  __shared__ __attribute__((aligned(16))) T dSs[BF ? BWD_BK * BWD_BQ : BWD_BK * SPITCH];
-  __shared__ __attribute__((aligned(16))) float st_s[BWD_BQ];
-  __shared__ __attribute__((aligned(16))) float di_s[BWD_BQ];
+  __shared__ __attribute__((aligned(16))) float Ks[F32_BK * PITCH];
+  __shared__ __attribute__((aligned(16))) float Qs[F32_BQ * PITCH];
+  __shared__ __attribute__((aligned(16))) float dOs[F32_BQ * PITCH];
+  __shared__ __attribute__((aligned(16))) float dSs[F32_BK * SPITCH];
+  __shared__ __attribute__((aligned(16))) float st_s[F32_BQ];
+  __shared__ __attribute__((aligned(16))) float di_s[F32_BQ];
 
   if (p.flag) {
     const bool in_range = *p.flag != 0;
@@ -189,65 +190,56 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_kernel(AttnBwdParams p) {
   }
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int kg = wave & 1, sub = wave >> 1;
   const int T_ = p.T;
-  // One 128-key block of one head. The in-range kernel takes one per workgroup from its 2-D
+  // One 64-key block of one head. The in-range kernel takes one per workgroup from its 2-D
   // grid; the fallbacks loop over them (grid-stride), key block 0 (the most causal work) first.
   auto run = [&](int bh, int kblk) __attribute__((always_inline)) {
-  const int k0 = kblk * BWD_BK;
+  const int k0 = kblk * F32_BK;
   const size_t base = (size_t)bh * T_ * D;  // internal (B, H, T, D) buffers (dq_acc)
   const size_t hb = head_base(bh, p.H, T_, D, p.layout);
   const int ld = row_stride(p.H, D, p.layout);
-  const T* Q = reinterpret_cast<const T*>(p.q) + hb;
-  const T* K = reinterpret_cast<const T*>(p.k) + hb;
-  const T* V = reinterpret_cast<const T*>(p.v) + hb;
-  const T* dO = reinterpret_cast<const T*>(p.dO) + hb;
+  const float* Q = reinterpret_cast<const float*>(p.q) + hb;
+  const float* K = reinterpret_cast<const float*>(p.k) + hb;
+  const float* V = reinterpret_cast<const float*>(p.v) + hb;
+  const float* dO = reinterpret_cast<const float*>(p.dO) + hb;
   const float* stat = p.stat + (size_t)bh * T_;
   const float* di = p.di + (size_t)bh * T_;
   float* dq_acc = p.dq_acc + base;
-  const int wk0 = k0 + wave * 32;    // this wave's first key
+  const int wk0 = k0 + kg * 32;      // this wave's first key
   const int mykey = wk0 + l32;
   const int log2n = p.log2n;
+  const int nq = ceil_div(T_, F32_BQ);
+  const int q_first = k0 / F32_BQ;
 
   {
-    typedef RowTile<T, D, BWD_BK> KT;
-    uint4 kr[KT::PER];
+    typedef RowTile<D, F32_BK> KT;
+    floatx4 kr[KT::PER];
     KT::load(kr, K, k0, T_, ld);
     KT::store(Ks, PITCH, kr);
   }
 
-  // K and V fragments as B operands of S = Q K^T and dP = dO V^T.
-  constexpr int NF = BF ? D / 16 : D / 8;
-  typedef typename std::conditional<BF, bf16x8, floatx4>::type Frag;
-  Frag kf[NF], vf[NF];
+  // V fragments as the B operand of dP = dO V^T (K's, of S = Q K^T, are read from LDS, which the
+  // registers of two waves per SIMD need and the f32 MFMAs hide). Keys past T load the last row;
+  // the mask removes them.
+  constexpr int NF = D / 8;
+  floatx4 vf[NF];
 #pragma unroll
-  for (int s = 0; s < NF; ++s) {
-    if constexpr (BF) {
-      bf16x8 z = {};
-      const size_t o = (size_t)mykey * ld + 16 * s + 8 * h;
-      kf[s] = mykey < T_ ? ld8(reinterpret_cast<const bf16*>(K) + o) : z;
-      vf[s] = mykey < T_ ? ld8(reinterpret_cast<const bf16*>(V) + o) : z;
-    } else {
-      floatx4 z = {};
-      const size_t o = (size_t)mykey * ld + 8 * s + 4 * h;
-      kf[s] = mykey < T_ ? *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(K) + o) : z;
-      vf[s] = mykey < T_ ? *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(V) + o) : z;
-    }
-  }
+  for (int s = 0; s < NF; ++s)
+    vf[s] = *reinterpret_cast<const floatx4*>(V + (size_t)min(mykey, T_ - 1) * ld + 8 * s + 4 * h);
   floatx16 dk[NDB], dv[NDB];
 #pragma unroll
   for (int db = 0; db < NDB; ++db) { dk[db] = floatx16{}; dv[db] = floatx16{}; }
 
-  const int nq = ceil_div(T_, BWD_BQ);
-  const int qstart = k0 / BWD_BQ;
   // Q/dO/stat/di tiles are prefetched into registers one iteration ahead and written to
   // LDS between the dS barrier and the dQ phase (which reads only dS and K).
-  typedef RowTile<T, D, BWD_BQ> QT;
-  uint4 qr[QT::PER], dr[QT::PER];
+  typedef RowTile<D, F32_BQ> QT;
+  floatx4 qr[QT::PER], dr[QT::PER];
   float str = 0.0f, dir = 0.0f;
   auto prefetch = [&](int qbase) {
     QT::load(qr, Q, qbase, T_, ld);
     QT::load(dr, dO, qbase, T_, ld);
-    if (threadIdx.x < BWD_BQ) {  // raw loads; rows past T are zeroed when committed
+    if (threadIdx.x < F32_BQ) {  // raw loads; rows past T are zeroed when committed
       const int q = min(qbase + (int)threadIdx.x, T_ - 1);
       str = stat[q];
       dir = di[q];
@@ -256,220 +248,165 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_kernel(AttnBwdParams p) {
   auto commit = [&](int qbase) {
     QT::store(Qs, PITCH, qr);
     QT::store(dOs, PITCH, dr);
-    if (threadIdx.x < BWD_BQ) {
+    if (threadIdx.x < F32_BQ) {
       const bool live = qbase + (int)threadIdx.x < T_;  // stat = 0 removes rows past T
       st_s[threadIdx.x] = live ? str : 0.0f;
       di_s[threadIdx.x] = live ? dir : 0.0f;
     }
   };
-  prefetch(qstart * BWD_BQ);
-  commit(qstart * BWD_BQ);
+  prefetch(q_first * F32_BQ);
+  commit(q_first * F32_BQ);
   __syncthreads();
-  for (int qt = qstart; qt < nq; ++qt) {
-    const int qbase = qt * BWD_BQ;
+  for (int qt = q_first; qt < nq; ++qt) {
+    const int qbase = qt * F32_BQ;
     const bool more = qt + 1 < nq;
-    if (more) prefetch(qbase + BWD_BQ);
-    // One 32-query block against this wave's 32 keys: S, dP, P, dS, dV += P^T dO,
-    // dK += dS^T Q, dS staged in LDS for the dQ phase.
-    auto sub_block = [&](int sub, bool diag) {
-      const int sq0 = qbase + sub * 32;
-      T* dsrow = dSs + (wave * 32 + l32) * SPITCH + sub * 32;
-        const T* qrow = Qs + (sub * 32 + l32) * PITCH;
-        const T* dorow = dOs + (sub * 32 + l32) * PITCH;
-        floatx16 s = {}, dp = {};
-  #pragma unroll
-        for (int st = 0; st < NF; ++st) {
-          if constexpr (BF) {
-            const int at = swz_at<CPR>(sub * 32 + l32, 16 * st + 8 * h);
-            bf16x8 qa = *reinterpret_cast<const bf16x8*>(Qs + at);
-            s = mfma_bf16(qa, kf[st], s);
-            bf16x8 da = *reinterpret_cast<const bf16x8*>(dOs + at);
-            dp = mfma_bf16(da, vf[st], dp);
-          } else {
-            floatx4 qa = *reinterpret_cast<const floatx4*>(qrow + 8 * st + 4 * h);
-            floatx4 da = *reinterpret_cast<const floatx4*>(dorow + 8 * st + 4 * h);
-  #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              s = mfma_f32(qa[u], kf[st][u], s);
-              dp = mfma_f32(da[u], vf[st][u], dp);
-            }
-          }
-        }
-        float pv[16], dsv[16];
-  #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const floatx4 stq = *reinterpret_cast<const floatx4*>(st_s + sub * 32 + 8 * g + 4 * h);
-          const floatx4 diq = *reinterpret_cast<const floatx4*>(di_s + sub * 32 + 8 * g + 4 * h);
-  #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int i = 4 * g + e;
-            float x = s[i];
-            float r, pw;
-            if constexpr (MODE == MODE_INRANGE) {
-              pw = pow2n<L2N>(rho_fast(x, r), log2n) * stq[e];
-            } else if constexpr (MODE == MODE_CLIPPED) {
-              x = fminf(x, p.clamp);
-              float t = rho_fast(x, r);
-              if (p.inv_stat) {
-                for (int k2 = 0; k2 < log2n; ++k2) t = t * t;
-                pw = t * stq[e];
-              } else {
-                t = t * stq[e];
-                for (int k2 = 0; k2 < log2n; ++k2) t = t * t;
-                pw = t;
-              }
-            } else {
-              const int q = sq0 + 8 * g + 4 * h + e;
-              if (diag && mykey > q) x = 0.0f;
-              const float t = p.fast_rho ? rho_fast(x, r) : rho_exact(x, r);
-              pw = pow2n<L2N>(t * stq[e], log2n);
-            }
-            float dsx = pw * (dp[i] - diq[e]) * r;
-            if constexpr (MODE == MODE_CLIPPED) dsx = s[i] < p.clamp ? dsx : 0.0f;
-            if (diag) {
-              const int q = sq0 + 8 * g + 4 * h + e;
-              if (mykey > q) { pw = 0.0f; dsx = 0.0f; }
-            }
-            pv[i] = pw;
-            dsv[i] = dsx;
-          }
-        }
-        if constexpr (BF) {
-          bf16x8 pa0, pa1, da0, da1;
-  #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            pa0[j] = f2bf(pv[j]); pa1[j] = f2bf(pv[8 + j]);
-            da0[j] = f2bf(dsv[j]); da1[j] = f2bf(dsv[8 + j]);
-          }
-          const bf16* qt_ = reinterpret_cast<const bf16*>(Qs);
-          const bf16* dot_ = reinterpret_cast<const bf16*>(dOs);
-  #pragma unroll
-          for (int db = 0; db < NDB; ++db) {
-            const int r0 = sub * 32 + 4 * h;
-            bf16x8 ob0 = swz_tr_frag<CPR>(dot_, r0, r0 + 8, db * 32, lane);
-            bf16x8 ob1 = swz_tr_frag<CPR>(dot_, r0 + 16, r0 + 24, db * 32, lane);
-            dv[db] = mfma_bf16(pa0, ob0, dv[db]);
-            dv[db] = mfma_bf16(pa1, ob1, dv[db]);
-            bf16x8 qb0 = swz_tr_frag<CPR>(qt_, r0, r0 + 8, db * 32, lane);
-            bf16x8 qb1 = swz_tr_frag<CPR>(qt_, r0 + 16, r0 + 24, db * 32, lane);
-            dk[db] = mfma_bf16(da0, qb0, dk[db]);
-            dk[db] = mfma_bf16(da1, qb1, dk[db]);
-          }
-          // Stage dS (rounded, as the dq/dk operands are) in LDS as [key][query].
-  #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            bf16x4 v4;
-  #pragma unroll
-            for (int e = 0; e < 4; ++e) v4[e] = f2bf(dsv[4 * g + e]);
-            *reinterpret_cast<bf16x4*>(dSs + swz_at<SCPR>(wave * 32 + l32, sub * 32 + 8 * g + 4 * h)) = v4;
-          }
-        } else {
-          const float* qt_ = reinterpret_cast<const float*>(Qs);
-          const float* dot_ = reinterpret_cast<const float*>(dOs);
-  #pragma unroll
-          for (int db = 0; db < NDB; ++db) {
-  #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const int qr = sub * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
-              dv[db] = mfma_f32(pv[i], dot_[qr * PITCH + db * 32 + l32], dv[db]);
-              dk[db] = mfma_f32(dsv[i], qt_[qr * PITCH + db * 32 + l32], dk[db]);
-            }
-          }
-  #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            floatx4 v4;
-  #pragma unroll
-            for (int e = 0; e < 4; ++e) v4[e] = dsv[4 * g + e];
-            *reinterpret_cast<floatx4*>(dsrow + 8 * g + 4 * h) = v4;
-          }
-        }
-    };
-    if (wk0 < T_ && qbase >= wk0 + 31) {  // every query follows every key: no masking
+    if (more) prefetch(qbase + F32_BQ);
+    const int sq0 = qbase + sub * 32;
+    float* dsrow = dSs + (kg * 32 + l32) * SPITCH + sub * 32;
+    // This wave's 32 x 32 block: S, dP, P, dS, dV += P^T dO, dK += dS^T Q, dS staged in LDS for
+    // the dQ phase.
+    auto block = [&]() __attribute__((always_inline)) {
+      const float* qrow = Qs + (sub * 32 + l32) * PITCH;
+      const float* krow = Ks + (kg * 32 + l32) * PITCH;
+      const float* dorow = dOs + (sub * 32 + l32) * PITCH;
+      floatx16 s = {}, dp = {};
 #pragma unroll
-      for (int sub = 0; sub < BWD_BQ / 32; ++sub) sub_block(sub, false);
-    } else {
+      for (int st = 0; st < NF; ++st) {
+        const floatx4 qa = *reinterpret_cast<const floatx4*>(qrow + 8 * st + 4 * h);
+        const floatx4 da = *reinterpret_cast<const floatx4*>(dorow + 8 * st + 4 * h);
+        const floatx4 ka = *reinterpret_cast<const floatx4*>(krow + 8 * st + 4 * h);
 #pragma unroll
-      for (int sub = 0; sub < BWD_BQ / 32; ++sub) {
-        const int sq0 = qbase + sub * 32;
-        if (sq0 + 31 < wk0 || wk0 >= T_) {  // all queries precede all keys of this wave
-          T* dsrow = dSs + (wave * 32 + l32) * SPITCH + sub * 32;
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            if constexpr (BF) {
-              bf16x4 z = {};
-              *reinterpret_cast<bf16x4*>(dSs + swz_at<SCPR>(wave * 32 + l32, sub * 32 + 8 * g + 4 * h)) = z;
-            }
-            else { floatx4 z = {}; *reinterpret_cast<floatx4*>(dsrow + 8 * g + 4 * h) = z; }
-          }
-        } else {
-          sub_block(sub, wk0 + 31 > sq0);
+        for (int u = 0; u < 4; ++u) {
+          s = mfma_f32(qa[u], ka[u], s);
+          dp = mfma_f32(da[u], vf[st][u], dp);
         }
       }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const floatx4 stq = *reinterpret_cast<const floatx4*>(st_s + sub * 32 + 8 * g + 4 * h);
+        const floatx4 diq = *reinterpret_cast<const floatx4*>(di_s + sub * 32 + 8 * g + 4 * h);
+        floatx4 v4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = 4 * g + e;
+          const int q = sq0 + 8 * g + 4 * h + e;
+          float x = s[i];
+          float r, pw;
+          if constexpr (MODE == MODE_INRANGE) {
+            pw = pow2n<L2N>(rho_fast(x, r), log2n) * stq[e];
+          } else if constexpr (MODE == MODE_CLIPPED) {
+            x = fminf(x, p.clamp);
+            float t = rho_fast(x, r);
+            if (p.inv_stat) {
+              for (int k2 = 0; k2 < log2n; ++k2) t = t * t;
+              pw = t * stq[e];
+            } else {
+              t = t * stq[e];
+              for (int k2 = 0; k2 < log2n; ++k2) t = t * t;
+              pw = t;
+            }
+          } else {
+            if (mykey > q) x = 0.0f;
+            const float t = p.fast_rho ? rho_fast(x, r) : rho_exact(x, r);
+            pw = pow2n<L2N>(t * stq[e], log2n);
+          }
+          float dsx = pw * (dp[i] - diq[e]) * r;
+          if constexpr (MODE == MODE_CLIPPED) dsx = s[i] < p.clamp ? dsx : 0.0f;
+          if (mykey > q) { pw = 0.0f; dsx = 0.0f; }
+          s[i] = pw;
+          dp[i] = v4[e] = dsx;
+        }
+        *reinterpret_cast<floatx4*>(dsrow + 8 * g + 4 * h) = v4;
+      }
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int qrw = sub * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+          dv[db] = mfma_f32(s[i], dOs[qrw * PITCH + db * 32 + l32], dv[db]);
+          dk[db] = mfma_f32(dp[i], Qs[qrw * PITCH + db * 32 + l32], dk[db]);
+        }
+      }
+    };
+    if (sq0 + 31 < wk0 || wk0 >= T_) {  // all queries precede all keys of this wave
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        floatx4 z = {};
+        *reinterpret_cast<floatx4*>(dsrow + 8 * g + 4 * h) = z;
+      }
+    } else {
+      block();
     }
-    __syncthreads();
-    if (more) commit(qbase + BWD_BQ);
-    // dQ tile = dS K over this workgroup's keys; each wave takes 32 queries x DBW blocks.
+    lds_barrier();
+    if (more) commit(qbase + F32_BQ);
+    // dQ tile = dS K over this workgroup's keys; each wave takes 32 queries and half of D.
     {
-      constexpr int NQH = BWD_BQ / 32;         // 32-query slices of the tile
-      constexpr int WPH = 4 / NQH;             // waves per slice
-      constexpr int DBW = NDB / WPH;           // 32-wide d blocks per wave
-      static_assert(DBW >= 1, "tile shape");
-      const int qs = wave / WPH;
-      const int db0 = (wave % WPH) * DBW;
+      constexpr int DBW = NDB / 2;  // 32-wide d blocks per wave
+      const int qs = wave >> 1, db0 = (wave & 1) * DBW;
       floatx16 dqa[DBW];
 #pragma unroll
       for (int j = 0; j < DBW; ++j) dqa[j] = floatx16{};
-      if constexpr (BF) {
-        const bf16* ds_ = reinterpret_cast<const bf16*>(dSs);
-        const bf16* k_ = reinterpret_cast<const bf16*>(Ks);
-        // DBW >= 2 independent accumulator chains keep the MFMA pipe busy.
+      // The operands of 8 MFMA steps are read together, one group ahead of their MFMAs.
+      constexpr int G = 8;
+      float a[2][G], b[2][G][DBW];
+      auto operands = [&](int ks0, int to) __attribute__((always_inline)) {
 #pragma unroll
-        for (int ks = 0; ks < BWD_BK / 16; ++ks) {
-          const int klo = ks * 16 + 8 * h;
-          bf16x8 a0 = swz_tr_frag<SCPR>(ds_, klo, klo + 4, qs * 32, lane);
+        for (int u = 0; u < G; ++u) {
+          const int key = 2 * (ks0 + u) + h;
+          a[to][u] = dSs[key * SPITCH + qs * 32 + l32];
 #pragma unroll
-          for (int j = 0; j < DBW; ++j) {
-            bf16x8 b0 = swz_tr_frag<CPR>(k_, klo, klo + 4, (db0 + j) * 32, lane);
-            dqa[j] = mfma_bf16(a0, b0, dqa[j]);
-          }
+          for (int j = 0; j < DBW; ++j) b[to][u][j] = Ks[key * PITCH + (db0 + j) * 32 + l32];
         }
-      } else {
-        const float* ds_ = reinterpret_cast<const float*>(dSs);
-        const float* k_ = reinterpret_cast<const float*>(Ks);
-#pragma unroll 8
-        for (int ks = 0; ks < BWD_BK / 2; ++ks) {
-          const int key = 2 * ks + h;
-          const float a = ds_[key * SPITCH + qs * 32 + l32];
+      };
+      operands(0, 0);
 #pragma unroll
-          for (int j = 0; j < DBW; ++j) dqa[j] = mfma_f32(a, k_[key * PITCH + (db0 + j) * 32 + l32], dqa[j]);
-        }
+      for (int ks0 = 0; ks0 < F32_BK / 2; ks0 += G) {
+        if (ks0 + G < F32_BK / 2) operands(ks0 + G, (ks0 / G + 1) & 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+#pragma unroll
+          for (int j = 0; j < DBW; ++j) dqa[j] = mfma_f32(a[(ks0 / G) & 1][u], b[(ks0 / G) & 1][u][j], dqa[j]);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      {
-        // Buffer atomics over this slice's rows: the row offset is part of the range-checked
-        // VGPR offset, so rows at or past T (beyond num_records) are dropped by the hardware;
-        // the d-block offset is the scalar offset.
-        const int rowbase = qbase + qs * 32;
-        const int live_rows = max(0, T_ - rowbase);
-        const __amdgpu_buffer_rsrc_t dqr = __builtin_amdgcn_make_buffer_rsrc(
-            dq_acc + (size_t)rowbase * D, (short)0, live_rows * D * 4, BUF_RSRC_WORD3);
-        const int lane_off = (4 * h * D + l32) * 4;
+      // Buffer atomics over this slice's rows: the row offset is part of the range-checked
+      // VGPR offset, so rows at or past T (beyond num_records) are dropped by the hardware;
+      // the d-block offset is the scalar offset.
+      const int rowbase = qbase + qs * 32;
+      const int live_rows = max(0, T_ - rowbase);
+      const __amdgpu_buffer_rsrc_t dqr = __builtin_amdgcn_make_buffer_rsrc(
+          dq_acc + (size_t)rowbase * D, (short)0, live_rows * D * 4, BUF_RSRC_WORD3);
+      const int lane_off = (4 * h * D + l32) * 4;
 #pragma unroll
-        for (int j = 0; j < DBW; ++j) {
+      for (int j = 0; j < DBW; ++j) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(dqa[j][i], dqr,
-                                                            lane_off + (8 * (i >> 2) + (i & 3)) * D * 4,
-                                                            (db0 + j) * 128, 0);
-        }
+        for (int i = 0; i < 16; ++i)
+          __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(dqa[j][i], dqr, lane_off + (8 * (i >> 2) + (i & 3)) * D * 4,
+                                                          (db0 + j) * 128, 0);
       }
     }
-    __syncthreads();
+    lds_barrier();
   }
 
-  // dK = n * acc, dV = acc (flash.py:591-597), rounded to the input dtype.
+  // The two halves (queries sub = 0, 1) of a key group's dK and dV: sub 1 leaves its registers in
+  // the query tiles' LDS, sub 0 adds them.
+  static_assert(2 * NDB * 16 * 64 <= F32_BQ * PITCH, "a half fits a query tile");
+  auto slot = [&](int db, int i) { return ((kg * NDB + db) * 16 + i) * 64 + lane; };
+  if (sub == 1) {
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        Qs[slot(db, i)] = dk[db][i];
+        dOs[slot(db, i)] = dv[db][i];
+      }
+  }
+  __syncthreads();
+  if (sub == 1) return;
+  // dK = n * acc, dV = acc (flash.py:591-597).
   const float slope = (float)(1 << log2n);
-  T* DK = reinterpret_cast<T*>(p.dk) + hb;
-  T* DV = reinterpret_cast<T*>(p.dv) + hb;
+  float* DK = reinterpret_cast<float*>(p.dk) + hb;
+  float* DV = reinterpret_cast<float*>(p.dv) + hb;
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
 #pragma unroll
@@ -477,8 +414,8 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_kernel(AttnBwdParams p) {
       const int key = wk0 + 8 * (i >> 2) + 4 * h + (i & 3);
       if (key < T_) {
         const size_t o = (size_t)key * ld + db * 32 + l32;
-        DK[o] = (T)(dk[db][i] * slope);
-        DV[o] = (T)(dv[db][i]);
+        DK[o] = (dk[db][i] + Qs[slot(db, i)]) * slope;
+        DV[o] = dv[db][i] + dOs[slot(db, i)];
       }
     }
   }
@@ -486,10 +423,10 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_kernel(AttnBwdParams p) {
   if constexpr (MODE == MODE_INRANGE) {
     run(blockIdx.x, blockIdx.y);
   } else {
-    const int nbh = p.B * p.H, total = nbh * ceil_div(T_, BWD_BK);
+    const int nbh = p.B * p.H, total = nbh * ceil_div(T_, F32_BK);
     for (int L = blockIdx.x; L < total; L += gridDim.x) {
       run(L % nbh, L / nbh);
-      __syncthreads();  // the next block's K tile overwrites LDS
+      __syncthreads();  // the next block's tiles overwrite LDS
     }
   }
 }
@@ -1613,27 +1550,31 @@ static hipError_t launch_bwd_bf16(const AttnBwdParams& p, int mode, bool dq, hip
   return p.layout ? launch_bwd_bf16_l<D, 1>(p, mode, dq, st) : launch_bwd_bf16_l<D, 0>(p, mode, dq, st);
 }
 
-// f32: the key-stationary kernel with dQ atomics.
+// f32: the key-stationary kernel with dQ atomics. Up to 512 key blocks, the in-range launch asks
+// for LDS it does not use, so that a CU takes one workgroup at a time: the first 256, the longest
+// key blocks, then start on a CU each and the short ones follow, where two to a CU put long
+// blocks together and left CUs idle (384 key blocks, B H T D: 2 12 1024 64 142 -> 119 us,
+// 1 12 2048 64 253 -> 210). With more blocks than that, two to a CU hide each other's waits
+// (1536, 4 12 2048 64: 607 us, one to a CU 672).
 template <int D>
 static hipError_t launch_bwd_f32(const AttnBwdParams& p, int mode, hipStream_t st) {
-  const int nbh = p.B * p.H, nkb = ceil_div(p.T, BWD_BK);
+  const int nbh = p.B * p.H, nkb = ceil_div(p.T, F32_BK);
   dim3 block(256);
   switch (mode) {
     case MODE_INRANGE: {
       KTimer t("attn_bwd_inrange", st);
       dim3 grid(nbh, nkb);
-      if (p.log2n == 4) hipLaunchKernelGGL((attn_bwd_kernel<float, D, MODE_INRANGE, 4>), grid, block, 0, st, p);
-      else hipLaunchKernelGGL((attn_bwd_kernel<float, D, MODE_INRANGE, 0>), grid, block, 0, st, p);
+      const int pad = D == 64 && (long)nbh * nkb <= 512 ? 16 << 10 : 0;  // 70 + 16 KB: over half of 160
+      if (p.log2n == 4) hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_INRANGE, 4>), grid, block, pad, st, p);
+      else hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_INRANGE, 0>), grid, block, pad, st, p);
     } break;
     case MODE_CLIPPED: {
       KTimer t("attn_bwd_clipped", st);
-      hipLaunchKernelGGL((attn_bwd_kernel<float, D, MODE_CLIPPED, 0>), dim3(fallback_grid(p, nbh * nkb)), block, 0, st,
-                         p);
+      hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_CLIPPED, 0>), dim3(fallback_grid(p, nbh * nkb)), block, 0, st, p);
     } break;
     case MODE_SHIFTED: {
       KTimer t("attn_bwd_shifted", st);
-      hipLaunchKernelGGL((attn_bwd_kernel<float, D, MODE_SHIFTED, 0>), dim3(fallback_grid(p, nbh * nkb)), block, 0, st,
-                         p);
+      hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_SHIFTED, 0>), dim3(fallback_grid(p, nbh * nkb)), block, 0, st, p);
     } break;
     default: return hipErrorInvalidValue;
   }
