@@ -125,9 +125,13 @@ struct HeadWs {
   size_t partial, obj_part, bwd, dh_part, de_part, total;
   size_t flag, E3, h3;  // f32 hidden states
   size_t res_ut, res_l, res_total;
-  int Npad, Vp, dh_split;
+  int Npad, Vp;
+  alg::HeadDhPlan dh;
   alg::HeadDePlan de;
 };
+size_t head_dh_part_bytes(const alg::HeadDhPlan& dh, int N, int d) {
+  return dh.split > 1 ? (size_t)dh.split * N * d * sizeof(float) : 0;
+}
 size_t head_de_part_bytes(const alg::HeadDePlan& de) {
   return de.split > 1 ? (size_t)(de.tiles - de.full) * de.split * alg::HT_M * alg::HT_N * sizeof(float) : 0;
 }
@@ -137,14 +141,14 @@ HeadWs head_ws(int N, int d, int V, int pass, bool residual) {
   w.Npad = alg::head_token_pad(N);
   w.Vp = alg::head_vocab_pitch(V);
   w.partial = 0;
-  w.obj_part = align256((size_t)alg::head_vocab_tiles(V) * N * sizeof(float));
+  const int vtile = alg::head_logit_tile(N, V);
+  w.obj_part = align256((size_t)alg::ceil_div(V, vtile) * N * sizeof(float));
   w.bwd = w.obj_part + align256((size_t)alg::head_stat_blocks(N) * sizeof(float));
   const size_t bwd_bytes = residual ? (size_t)N * d * 2 : (size_t)w.Npad * w.Vp * 2;
-  w.dh_split = alg::head_dh_split(N, d, V);
+  w.dh = alg::head_dh_plan(N, d, V, 1);
   w.dh_part = w.bwd + align256(bwd_bytes);
-  const size_t part_bytes = w.dh_split > 1 ? (size_t)w.dh_split * N * d * sizeof(float) : 0;
-  w.de = alg::head_de_plan(N, d, V);
-  w.de_part = w.dh_part + align256(part_bytes);
+  w.de = alg::head_de_plan(N, d, V, 1);
+  w.de_part = w.dh_part + align256(head_dh_part_bytes(w.dh, N, d));
   w.total = pass == 0 ? w.bwd : w.de_part + align256(head_de_part_bytes(w.de));
   w.res_ut = 0;
   w.res_l = align256((size_t)w.Npad * w.Vp * 2);
@@ -153,25 +157,32 @@ HeadWs head_ws(int N, int d, int V, int pass, bool residual) {
 }
 
 // f32 hidden states (the reference's recompute schedule in f32): [partials f32 nvt*N over
-// 128-entry vocabulary tiles][obj parts][flag i32: an input is not finite][E and h as three bf16
-// planes each] (+ bwd: dZ as three bf16 planes Npad*Vp, or f32 N*Vp where the flag is set; then
-// the f32 partials split*N*d of a vocabulary-split dh product; then the f32 tiles of the
-// token-split dE tail). No residual.
+// 128-entry vocabulary tiles][obj parts], with split products (head_f32_split) [flag i32: an input
+// is not finite][E and h as three bf16 planes each] (+ bwd: dZ, f32 N*Vp or with split products
+// three bf16 planes Npad*Vp; then the f32 partials split*N*d of a vocabulary-split dh product;
+// then the f32 tiles of the token-split dE tail). No residual.
 HeadWs head_ws_f32(int N, int d, int V, int pass) {
   HeadWs w;
-  w.Npad = alg::head_token_pad(N);
+  const bool split = alg::head_f32_split(N);
+  w.Npad = split ? alg::head_token_pad(N) : N;
   w.Vp = alg::head_vocab_pitch(V);
   w.partial = 0;
   w.obj_part = align256((size_t)alg::head_f32_vocab_tiles(V) * N * sizeof(float));
   w.flag = w.obj_part + align256((size_t)alg::head_stat_blocks(N) * sizeof(float));
-  w.E3 = w.flag + 256;
-  w.h3 = w.E3 + align256((size_t)V * d * 6);
-  w.bwd = w.h3 + align256((size_t)N * d * 6);
-  w.dh_split = alg::head_dh_split(N, d, V);
-  w.dh_part = w.bwd + align256((size_t)w.Npad * w.Vp * 6);
-  const size_t part_bytes = w.dh_split > 1 ? (size_t)w.dh_split * N * d * sizeof(float) : 0;
-  w.de = alg::head_de_plan(N, d, V);
-  w.de_part = w.dh_part + align256(part_bytes);
+  w.E3 = w.flag + (split ? 256 : 0);
+  w.h3 = w.E3 + (split ? align256((size_t)V * d * 6) : 0);
+  w.bwd = w.h3 + (split ? align256((size_t)N * d * 6) : 0);
+  w.dh_part = w.bwd + align256((size_t)w.Npad * w.Vp * (split ? 6 : 4));
+  if (split) {
+    w.dh = alg::head_dh_plan(N, d, V, alg::SPLIT3_PASSES);
+    w.de = alg::head_de_plan(N, d, V, alg::SPLIT3_PASSES);
+  } else {
+    w.dh.tile = 128;
+    w.dh.split = alg::head_f32_dh_split(N, d, V);
+    w.dh.kchunk = alg::head_f32_dh_kchunk(V, w.dh.split);
+    w.de = alg::HeadDePlan{128, 0, 0, 1, 0};
+  }
+  w.de_part = w.dh_part + align256(head_dh_part_bytes(w.dh, N, d));
   w.total = pass == 0 ? w.bwd : w.de_part + align256(head_de_part_bytes(w.de));
   w.res_ut = w.res_l = w.res_total = 0;
   return w;
@@ -181,8 +192,8 @@ HeadWs head_ws_f32(int N, int d, int V, int pass) {
 struct HeadEvalWs {
   size_t partial, pmax, pidx, total;
 };
-HeadEvalWs head_eval_ws(int N, int V, bool f32) {
-  const size_t cells = (size_t)(f32 ? alg::head_f32_vocab_tiles(V) : alg::head_vocab_tiles(V)) * N;
+HeadEvalWs head_eval_ws(int N, int d, int V, bool f32) {
+  const size_t cells = (size_t)(f32 ? alg::head_f32_vocab_tiles(V) : alg::ceil_div(V, alg::head_logit_tile(N, V))) * N;
   HeadEvalWs w;
   w.partial = 0;
   w.pmax = align256(cells * sizeof(float));
@@ -566,7 +577,7 @@ size_t alg_head_workspace_size(int dtype, int N, int d, int V, int pass) {
   if (dtype != ALG_DTYPE_BF16 && dtype != ALG_DTYPE_F32) return 0;
   const bool f32 = dtype == ALG_DTYPE_F32;
   // pass 0: forward; 1: backward without a residual; 2: backward with a residual; 3: eval
-  if (pass == 3) return head_eval_ws(N, V, f32).total;
+  if (pass == 3) return head_eval_ws(N, d, V, f32).total;
   if (f32) return pass == 2 ? 0 : head_ws_f32(N, d, V, pass ? 1 : 0).total;  // no residual in f32
   return head_ws(N, d, V, pass ? 1 : 0, pass == 2).total;
 }
@@ -605,7 +616,7 @@ static HeadStreamWs head_stream_ws(int dtype, int N, int d, int V, int vocab_chu
   w.de_part = w.acc + (nchunks > 1 ? align256((size_t)N * d * sizeof(float)) : 0);
   size_t de_bytes = 0;
   for (int vc : {w.chunk, V - (nchunks - 1) * w.chunk}) {
-    de_bytes = std::max(de_bytes, head_de_part_bytes(alg::head_de_plan(N, d, vc)));
+    de_bytes = std::max(de_bytes, head_de_part_bytes(alg::head_de_plan(N, d, vc, 1)));
   }
   w.has_de_part = de_bytes > 0;
   w.total = w.de_part + align256(de_bytes);
@@ -663,6 +674,18 @@ static void use_split_planes(alg::HeadParams& p, void* workspace, const HeadWs& 
   p.h = reinterpret_cast<bf16*>(w + ws.h3);
 }
 
+static void use_head_plans(alg::HeadParams& p, char* w, const HeadWs& ws) {
+  p.dh_tile = ws.dh.tile;
+  p.dh_split = ws.dh.split;
+  p.dh_kchunk = ws.dh.kchunk;
+  p.dh_part = ws.dh.split > 1 ? reinterpret_cast<float*>(w + ws.dh_part) : nullptr;
+  p.de_tile = ws.de.tile;
+  p.de_full = ws.de.full;
+  p.de_split = ws.de.split;
+  p.de_kchunk = ws.de.kchunk;
+  p.de_part = ws.de.split > 1 ? reinterpret_cast<float*>(w + ws.de_part) : nullptr;
+}
+
 int alg_head_fwd(alg_stream_t stream, int dtype, int N, int d, int V, const void* h, const void* E,
                  const int32_t* targets, int n, float c, float* stat, float* zt, float* pt, float* obj,
                  void* residual, void* workspace, size_t workspace_bytes) {
@@ -679,7 +702,7 @@ int alg_head_fwd(alg_stream_t stream, int dtype, int N, int d, int V, const void
   alg::HeadParams p = head_params(dtype, N, d, V, h, E, targets, n, c, workspace, ws);
   p.stat = stat; p.zt = zt; p.pt = pt; p.obj = obj;
   if (f32) {
-    use_split_planes(p, workspace, ws);
+    if (alg::head_f32_split(N)) use_split_planes(p, workspace, ws);
     return hip_status(alg::launch_head_fwd_f32(p, (hipStream_t)stream), "alg_head_fwd");
   }
   if (residual) {
@@ -826,7 +849,7 @@ int alg_head_eval(alg_stream_t stream, int dtype, int N, int d, int V, const voi
   const bool f32 = dtype == ALG_DTYPE_F32;
   if (!h || !E || !targets || !logprob) return fail(ALG_ERR_INVALID, "null argument");
   if (!aligned16({h, E, workspace})) return fail(ALG_ERR_INVALID, "matrices must be 16-byte aligned");
-  const HeadEvalWs ws = head_eval_ws(N, V, f32);
+  const HeadEvalWs ws = head_eval_ws(N, d, V, f32);
   if (!workspace || workspace_bytes < ws.total)
     return fail(ALG_ERR_INVALID, "workspace too small: need %zu bytes", ws.total);
   const HeadWs hw = f32 ? head_ws_f32(N, d, V, 0) : head_ws(N, d, V, 0, false);
@@ -864,17 +887,11 @@ int alg_head_bwd(alg_stream_t stream, int dtype, int N, int d, int V, const void
   p.dE = dE;
   p.dE_f32 = dE_dtype == ALG_DTYPE_F32;
   if (f32) {
-    use_split_planes(p, workspace, ws);
+    if (alg::head_f32_split(N)) use_split_planes(p, workspace, ws);
     p.dzt = reinterpret_cast<bf16*>(w + ws.bwd);
     p.dz32 = reinterpret_cast<float*>(w + ws.bwd);
     p.dh32 = static_cast<float*>(dh);
-    p.dh_split = ws.dh_split;
-    p.dh_kchunk = alg::head_dh_kchunk(V, ws.dh_split);
-    p.dh_part = ws.dh_split > 1 ? reinterpret_cast<float*>(w + ws.dh_part) : nullptr;
-    p.de_full = ws.de.full;
-    p.de_split = ws.de.split;
-    p.de_kchunk = ws.de.kchunk;
-    p.de_part = ws.de.split > 1 ? reinterpret_cast<float*>(w + ws.de_part) : nullptr;
+    use_head_plans(p, w, ws);
     return hip_status(alg::launch_head_bwd_f32(p, (hipStream_t)stream), "alg_head_bwd");
   }
   if (residual) {
@@ -885,13 +902,7 @@ int alg_head_bwd(alg_stream_t stream, int dtype, int N, int d, int V, const void
     p.dzt = reinterpret_cast<bf16*>(w + ws.bwd);
   }
   p.dh = static_cast<bf16*>(dh);
-  p.dh_split = ws.dh_split;
-  p.dh_kchunk = alg::head_dh_kchunk(V, ws.dh_split);
-  p.dh_part = ws.dh_split > 1 ? reinterpret_cast<float*>(w + ws.dh_part) : nullptr;
-  p.de_full = ws.de.full;
-  p.de_split = ws.de.split;
-  p.de_kchunk = ws.de.kchunk;
-  p.de_part = ws.de.split > 1 ? reinterpret_cast<float*>(w + ws.de_part) : nullptr;
+  use_head_plans(p, w, ws);
   return hip_status(alg::launch_head_bwd(p, (hipStream_t)stream), "alg_head_bwd");
 }
 

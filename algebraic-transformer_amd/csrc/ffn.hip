@@ -57,24 +57,11 @@ __device__ __forceinline__ int stage_at(int r, int c) {
 template <int AM, int BM, class C, class Epi>
 __device__ __forceinline__ void ffn_tile(const GemmOperand& A, const GemmOperand& B, int m0, int n0, int kbeg, int kend,
                                          Epi epi) {
+  static_assert(gemm_share<AM, BM, C>() >= C::WTM * C::WTN, "a wave's block fits its share");
   floatx16 acc[C::MB][C::NB];
-  constexpr int BLOCK = C::WTM * C::WTN;
-  int wm, wn;
-  wave_coords<C>(wm, wn);
-  const int wi = wm * C::WN + wn;
-  if constexpr (C::THREADS == 512) {
-    __shared__ __attribute__((aligned(16))) GemmStage<AM, BM, C> s0, s1;
-    static_assert(sizeof(s0) >= 4 * BLOCK * sizeof(bf16), "a stage holds four waves' blocks");
-    gemm_mainloop<AM, BM, C>(s0, s1, A, B, m0, n0, kbeg, kend, acc);
-    __syncthreads();  // every wave is done reading the pipeline buffers
-    epi(acc, reinterpret_cast<bf16*>(wi < 4 ? static_cast<void*>(&s0) : static_cast<void*>(&s1)) + (wi & 3) * BLOCK);
-  } else {
-    __shared__ __attribute__((aligned(16))) GemmStage<AM, BM, C> s0, s1, s2, s3;
-    static_assert(sizeof(s0) >= 2 * BLOCK * sizeof(bf16), "a stage holds two waves' blocks");
-    gemm_ring<AM, BM, C>(s0, s1, s2, s3, A, B, m0, n0, kbeg, kend, acc);
-    __syncthreads();
-    epi(acc, reinterpret_cast<bf16*>(wi < 2 ? static_cast<void*>(&s0) : static_cast<void*>(&s1)) + (wi & 1) * BLOCK);
-  }
+  bf16* stage = gemm_tile<AM, BM, C>(A, B, m0, n0, kbeg, kend, acc);
+  __syncthreads();  // every wave is done reading the pipeline buffers
+  epi(acc, stage);
 }
 
 }  // namespace
@@ -287,23 +274,6 @@ __global__ __launch_bounds__(256) void ffn_gemm_tail_kernel(FfnGemmParams g) {
   }
 }
 
-// Time in us of `units` workgroups of a tile configuration over k steps of K in all, fitted to
-// the products of one short sequence and of the 1b block (M N K, measured us for tiles of 256 /
-// 128 / 64, each in a captured graph with its launch):
-//   1024  768 2048   39.3 / 20.8 / 11.0     768 4096 1024   25.4 / 14.7 / 19.6
-//   1024  768 4096   69.5 / 37.2 / 19.2    2048  768 1024   23.2 / 12.6 /  8.3
-//    512  512 2048   37.5 / 20.2 / 10.5    2048 2048 2048   41.8 / 25.1 / 36.7
-// A 256 tile needs 14.8 ns per k alone on the chip and 23.4 ns when all CUs hold one (power); 128
-// tiles 8 to 10 ns; 64 tiles 4 ns while a CU holds one, 8 ns for two. Small tiles move two or four
-// times the operand bytes per multiplication, so they win only while the larger ones leave
-// CUs idle.
-static double ffn_tile_time(int tile, int units, double K) {
-  const double fill = std::min(1.0, units / 256.0), rounds = std::ceil(units / 256.0);
-  if (tile == 256) return 9.0 + rounds * K * (0.0148 + 0.0086 * fill);
-  if (tile == 128) return 4.4 + rounds * K * (0.008 + 0.002 * fill);
-  return 2.8 + K * (units <= 512 ? 0.004 + 0.004 * std::max(0, units - 256) / 256.0 : std::ceil(units / 512.0) * 0.008);
-}
-
 static int ffn_tiles(int tile, int M, int N) { return ((M + tile - 1) / tile) * ((N + tile - 1) / tile); }
 
 // Tile of an unsplit product with an epilogue of its own (allowed: 256, 128 and, if `min_tile`
@@ -311,7 +281,7 @@ static int ffn_tiles(int tile, int M, int N) { return ((M + tile - 1) / tile) * 
 static int ffn_epilogue_tile(int M, int N, int K, int min_tile) {
   int best = 256;
   for (int t = 128; t >= min_tile; t /= 2)
-    if (ffn_tile_time(t, ffn_tiles(t, M, N), K) < ffn_tile_time(best, ffn_tiles(best, M, N), K)) best = t;
+    if (gemm_tile_time(t, ffn_tiles(t, M, N), K) < gemm_tile_time(best, ffn_tiles(best, M, N), K)) best = t;
   return best;
 }
 
@@ -322,7 +292,7 @@ static int ffn_epilogue_tile(int M, int N, int K, int min_tile) {
 // its f32 tile written, read and summed (512 KiB at about 5 TB/s over the chip, 0.1 us) plus 5 us
 // for the summing launch. A range keeps at least 1024 of K (so every range is non-empty). The
 // workspace is that of this split. A product that fills less of the chip runs on smaller tiles
-// when ffn_tile_time says so; 64 x 64 tiles are split over k (ranges of at least 512) as far as
+// when gemm_tile_time says so; 64 x 64 tiles are split over k (ranges of at least 512) as far as
 // the same workspace goes, which pays where few tiles have a long k (304 1024 4096: 26.9 us
 // whole, 15.0 us in four ranges).
 FfnGemmPlan ffn_gemm_plan(int M, int N, int K) {
@@ -353,12 +323,12 @@ FfnGemmPlan ffn_gemm_plan(int M, int N, int K) {
     }
   }
   if (base) return pl;  // a whole round of 256 tiles: the chip is full
-  double best_time = pl.split == 1 ? ffn_tile_time(256, pl.tiles, K)
-                                   : ffn_tile_time(256, pl.tiles * pl.split, pl.kchunk) + 5.0;
+  double best_time = pl.split == 1 ? gemm_tile_time(256, pl.tiles, K)
+                                   : gemm_tile_time(256, pl.tiles * pl.split, pl.kchunk) + 5.0;
   auto consider = [&](int tile, int s) {
     const int tiles = ffn_tiles(tile, M, N);
     const int chunk = s > 1 ? ((K + s - 1) / s + 127) / 128 * 128 : K;
-    const double t = ffn_tile_time(tile, tiles * s, chunk) + (s > 1 ? 5.0 : 0.0);
+    const double t = gemm_tile_time(tile, tiles * s, chunk) + (s > 1 ? 5.0 : 0.0);
     if (t >= best_time) return;
     best_time = t;
     pl.tile = tile;

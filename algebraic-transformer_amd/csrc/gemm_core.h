@@ -387,7 +387,7 @@ __device__ __forceinline__ void gemm_mainloop(GemmStage<AM, BM, C>& s0, GemmStag
 // it reads next; one barrier per k step both publishes that tile and frees the stage the next
 // request fills. The stages are separate __shared__ objects, as above.
 constexpr int RING = 4;
-template <int AM, int BM, class C>
+template <int AM, int BM, class C, bool SPLIT3 = false>
 __device__ __forceinline__ void gemm_ring(GemmStage<AM, BM, C>& s0, GemmStage<AM, BM, C>& s1,
                                           GemmStage<AM, BM, C>& s2, GemmStage<AM, BM, C>& s3, const GemmOperand& A,
                                           const GemmOperand& B, int m0, int n0, int kbeg, int K,
@@ -417,7 +417,8 @@ __device__ __forceinline__ void gemm_ring(GemmStage<AM, BM, C>& s0, GemmStage<AM
 #pragma unroll
       for (int j = 0; j < C::NB; ++j) acc[i][j] = mfma_bf16(f.a[i], f.b[j], acc[i][j]);
   };
-  const int nk = K > kbeg ? (K - kbeg) / GT_K : 0;
+  const int nk1 = K > kbeg ? (K - kbeg) / GT_K : 0;  // k steps of one pass
+  const int nk = SPLIT3 ? SPLIT3_PASSES * nk1 : nk1;
   const bool a_full = (AM == KMAJOR ? A.rows_valid : A.cols_valid) >= m0 + C::TM;
   const bool b_full = (BM == KMAJOR ? B.rows_valid : B.cols_valid) >= n0 + C::TN;
   auto pipelined = [&](auto checked) {
@@ -427,9 +428,16 @@ __device__ __forceinline__ void gemm_ring(GemmStage<AM, BM, C>& s0, GemmStage<AM
     TA::lane_offsets(A, aoff);
     TB::lane_offsets(B, boff);
     const int wave_u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int pass = 0, kp = 0;  // as in gemm_mainloop: tiles are copied in order
     auto copy_tile = [&](Stage& st, int kt) {
-      TA::template copy<CHK>(st.a, A, aoff, wave_u, m0, kbeg + kt * GT_K);
-      TB::template copy<CHK>(st.b, B, boff, wave_u, n0, kbeg + kt * GT_K);
+      if constexpr (SPLIT3) {
+        TA::template copy<CHK>(st.a, A, aoff, wave_u, m0, kbeg + kp * GT_K, split3_a(pass) * A.plane);
+        TB::template copy<CHK>(st.b, B, boff, wave_u, n0, kbeg + kp * GT_K, split3_b(pass) * B.plane);
+        if (++kp == nk1) { kp = 0; ++pass; }
+      } else {
+        TA::template copy<CHK>(st.a, A, aoff, wave_u, m0, kbeg + kt * GT_K);
+        TB::template copy<CHK>(st.b, B, boff, wave_u, n0, kbeg + kt * GT_K);
+      }
     };
     auto step = [&](const Stage& cur, Stage& fill, int kt) {
       // Tile kt has landed once at most the two younger tiles' copies are outstanding. This
@@ -461,19 +469,48 @@ __device__ __forceinline__ void gemm_ring(GemmStage<AM, BM, C>& s0, GemmStage<AM
   if (a_full && b_full) pipelined(std::false_type{});
   else pipelined(std::true_type{});
   // The remaining partial k tile: register copies with zero fill.
-  if (const int k0 = kbeg + nk * GT_K; k0 < K) {
-    __syncthreads();
-    TA::copy_zero_fill(s0.a, A, m0, k0, K);
-    TB::copy_zero_fill(s0.b, B, n0, k0, K);
-    __syncthreads();
+  if (const int k0 = kbeg + nk1 * GT_K; k0 < K) {
+    for (int pass = 0; pass < (SPLIT3 ? SPLIT3_PASSES : 1); ++pass) {
+      __syncthreads();
+      TA::copy_zero_fill(s0.a, A, m0, k0, K, SPLIT3 ? split3_a(pass) * A.plane : 0);
+      TB::copy_zero_fill(s0.b, B, n0, k0, K, SPLIT3 ? split3_b(pass) * B.plane : 0);
+      __syncthreads();
 #pragma unroll
-    for (int ks = 0; ks < GT_K / 16; ++ks) {
-      Frags f;
-      load(s0, ks, f);
-      mma(f);
+      for (int ks = 0; ks < GT_K / 16; ++ks) {
+        Frags f;
+        load(s0, ks, f);
+        mma(f);
+      }
     }
   }
 }
+
+// Tile (m0, n0) over k in [kbeg, K) with the main loop of configuration C. Returns this wave's
+// share of the pipeline buffers (16 KiB with 8 waves, a stage with 4), which an epilogue may use
+// once it has passed a barrier.
+template <int AM, int BM, class C, bool SPLIT3 = false>
+__device__ __forceinline__ bf16* gemm_tile(const GemmOperand& A, const GemmOperand& B, int m0, int n0, int kbeg, int K,
+                                           floatx16 (&acc)[C::MB][C::NB]) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if constexpr (C::THREADS == 512) {
+    __shared__ __attribute__((aligned(16))) GemmStage<AM, BM, C> s0, s1;
+    gemm_mainloop<AM, BM, C, SPLIT3>(s0, s1, A, B, m0, n0, kbeg, K, acc);
+    return reinterpret_cast<bf16*>(wave < 4 ? static_cast<void*>(&s0) : static_cast<void*>(&s1)) +
+           (wave & 3) * (sizeof(s0) / sizeof(bf16) / 4);
+  } else {
+    static_assert(C::THREADS == 256, "4 or 8 waves");
+    __shared__ __attribute__((aligned(16))) GemmStage<AM, BM, C> s0, s1, s2, s3;
+    gemm_ring<AM, BM, C, SPLIT3>(s0, s1, s2, s3, A, B, m0, n0, kbeg, K, acc);
+    return reinterpret_cast<bf16*>(wave < 2 ? (wave == 0 ? static_cast<void*>(&s0) : static_cast<void*>(&s1))
+                                            : (wave == 2 ? static_cast<void*>(&s2) : static_cast<void*>(&s3)));
+  }
+}
+// Elements of that share.
+template <int AM, int BM, class C>
+constexpr int gemm_share() {
+  return (int)(sizeof(GemmStage<AM, BM, C>) / sizeof(bf16)) / (C::THREADS == 512 ? 4 : 1);
+}
+
 
 // Map a linear workgroup id to (tile_m, tile_n) so that the workgroups one XCD runs
 // (ids congruent mod 8 are dispatched to the same XCD) cover a compact group of tiles

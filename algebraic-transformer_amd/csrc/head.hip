@@ -34,8 +34,10 @@
 
 namespace alg {
 
-typedef HeadGemm HC;
-constexpr int NT = HC::THREADS;
+typedef HeadGemm HC;                    // 256 x 256 tiles, 8 waves (2 x 4)
+typedef GemmCfg<128, 128, 2, 2> HC128;  // products that fill less of the chip
+template <class C>
+constexpr int head_waves_per_simd() { return C::THREADS == 512 ? 1 : 2; }
 
 __device__ __forceinline__ float head_w(float z, const HeadParams& p, float& r) {
   const float x = fminf(z * p.inv_c, p.clamp);  // fused_head.py:98
@@ -49,25 +51,25 @@ __device__ __forceinline__ float head_w(float z, const HeadParams& p, float& r) 
 // into its own share of the idle pipeline buffers as [tok][v] rows, 16-byte chunks
 // XOR-swizzled by the token, then stores it with 16-byte stores that cover whole token rows
 // (full cache lines) per instruction.
-constexpr int UCH = HC::WTM / 8;          // 16-byte chunks per staged token row
-constexpr int UWAVE = HC::WTM * HC::WTN;  // staged elements per wave
-static_assert(UCH <= 64 && 64 % UCH == 0 && (UCH & (UCH - 1)) == 0, "staged row width");
+template <class C>
 __device__ __forceinline__ int ustage_at(int tl, int vl) {
-  return tl * HC::WTM + (((vl >> 3) ^ (tl & (UCH - 1))) << 3) + (vl & 7);
+  constexpr int UCH = C::WTM / 8;  // 16-byte chunks per staged token row
+  static_assert(UCH <= 64 && 64 % UCH == 0 && (UCH & (UCH - 1)) == 0, "staged row width");
+  return tl * C::WTM + (((vl >> 3) ^ (tl & (UCH - 1))) << 3) + (vl & 7);
 }
 
 // Stores the staged block: token rows tok0 + (0..WTN-1), vocabulary entries v0 + (0..WTM-1) of
 // out (row pitch Vp, Npad rows). AUX is the store's cache policy. EDGE: chunks at or past Vp are
 // dropped (Vp is a multiple of 8, so a chunk lies inside a row or past it; token rows always lie
 // inside the Npad rows).
-template <int AUX, bool EDGE = false>
+template <class C, int AUX, bool EDGE = false>
 __device__ __forceinline__ void store_staged_tokmajor(const bf16* ub, bf16* out, int Npad, int Vp, int tok0, int v0,
                                                       int lane) {
   const size_t ubase = (size_t)tok0 * Vp + v0;
   const size_t rest = ((size_t)Npad * Vp - ubase) * 2;  // bytes of out from the base
   const __amdgpu_buffer_rsrc_t urs = __builtin_amdgcn_make_buffer_rsrc(
       out + ubase, (short)0, (int)std::min<size_t>(rest, 0x7fffffff), BUF_RSRC_WORD3);
-  constexpr int RPS = 64 / UCH;  // token rows per store instruction
+  constexpr int UCH = C::WTM / 8, RPS = 64 / UCH;  // token rows per store instruction
   const int ch = lane % UCH;
   const int voff = ((lane / UCH) * Vp + ch * 8) * 2;
   // The row offset goes into the per-lane offset and the scalar offset stays the constant
@@ -77,9 +79,9 @@ __device__ __forceinline__ void store_staged_tokmajor(const bf16* ub, bf16* out,
   // reused the data registers of the store just issued, and on gfx950 the store wrote the
   // new values (measured: about 0.1 % of the U entries replaced by address arithmetic).
 #pragma unroll
-  for (int j = 0; j < HC::WTN / RPS; ++j) {
+  for (int j = 0; j < C::WTN / RPS; ++j) {
     const int tl = RPS * j + lane / UCH;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(ub + ustage_at(tl, ch * 8));
+    const u32x4 v = *reinterpret_cast<const u32x4*>(ub + ustage_at<C>(tl, ch * 8));
     if (!EDGE || v0 + ch * 8 < Vp) __builtin_amdgcn_raw_buffer_store_b128(v, urs, voff + RPS * j * Vp * 2, 0, AUX);
   }
 }
@@ -97,10 +99,11 @@ __device__ __forceinline__ GemmOperand head_operand(const bf16* ptr, int rows, i
 // L2N > 0 fixes n = 2^L2N at compile time (0: taken from the parameters).
 // acc[mb][nb][4g + e] for the row offset dt = mb*32 + 8g + e (bit 2 of dt, the lane half,
 // already matched).
-__device__ __forceinline__ float select_row(const floatx16 (&acc)[HC::MB][HC::NB], int nb, int dt) {
+template <class C>
+__device__ __forceinline__ float select_row(const floatx16 (&acc)[C::MB][C::NB], int nb, int dt) {
   float z = 0.0f;
 #pragma unroll
-  for (int mb = 0; mb < HC::MB; ++mb)
+  for (int mb = 0; mb < C::MB; ++mb)
 #pragma unroll
     for (int i = 0; i < 16; ++i) z = dt == mb * 32 + 8 * (i >> 2) + (i & 3) ? acc[mb][nb][i] : z;
   return z;
@@ -109,25 +112,24 @@ __device__ __forceinline__ float select_row(const floatx16 (&acc)[HC::MB][HC::NB
 // SPLIT: f32 h and E as three bf16 planes each (gemm_mainloop's six passes); no residual, and
 // the row sums are kept per 128 vocabulary entries, the tiling of the f32 kernels that run
 // instead when an input is not finite (p.split_bad).
-template <int L2N, bool SPLIT>
-__global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
+template <class C, int L2N, bool SPLIT>
+__global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_fwd_kernel(HeadParams p) {
   if (SPLIT && *p.split_bad) return;
-  __shared__ __attribute__((aligned(16))) GemmStage<KMAJOR, KMAJOR, HC> s0, s1;
-  __shared__ float red[HC::WM][HT_N];
-  const int nbm = (p.V + HT_M - 1) / HT_M, nbn = p.Npad / HT_N;
+  __shared__ float red[C::WM][C::TN];
+  const int nbm = (p.V + C::TM - 1) / C::TM, nbn = (p.N + C::TN - 1) / C::TN;
   int tm, tn;
   xcd_tile(blockIdx.x, nbm, nbn, tm, tn);
-  const int m0 = tm * HT_M;  // vocab
-  const int n0 = tn * HT_N;  // tokens
+  const int m0 = tm * C::TM;  // vocab
+  const int n0 = tn * C::TN;  // tokens
   const GemmOperand A = head_operand<SPLIT>(p.E, p.V, p.d, (long)p.V * p.d);
   const GemmOperand B = head_operand<SPLIT>(p.h, p.N, p.d, (long)p.N * p.d);
-  floatx16 acc[HC::MB][HC::NB];
-  gemm_mainloop<KMAJOR, KMAJOR, HC, SPLIT>(s0, s1, A, B, m0, n0, 0, p.d, acc);
+  floatx16 acc[C::MB][C::NB];
+  bf16* ub = gemm_tile<KMAJOR, KMAJOR, C, SPLIT>(A, B, m0, n0, 0, p.d, acc);
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
-  wave_coords<HC>(wm, wn);
+  wave_coords<C>(wm, wn);
   const float inv_c = p.inv_c, clamp = p.clamp;
-  const int vrow0 = m0 + wm * HC::WTM;  // first vocab row of this wave
+  const int vrow0 = m0 + wm * C::WTM;  // first vocab row of this wave
   // WITH_U also stores the residual. U is token-major (element (tok, v) at tok * Vp + v),
   // staged per wave and written with 16-byte stores marked non-temporal so the 1 GB stream of U
   // does not evict the E / h panels the GEMM is reusing from L2. EDGE (tiles that reach past V
@@ -135,27 +137,19 @@ __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
   // are all written, as finite values wherever h is finite (operand rows past the end read as
   // zeros). Edge tiles once stored U an element at a time, 2 bytes a lane: at N = 1000 their
   // quarter of the tiles took most of the kernel.
-  constexpr int NWAVES = HC::THREADS / 64;
-  static_assert(NWAVES * UWAVE * 2 <= 2 * (int)sizeof(s0), "staging fits the pipeline buffers");
-  static_assert((NWAVES / 2) * UWAVE * 2 <= (int)sizeof(s0) || NWAVES == 1, "half the waves per stage");
+  static_assert(C::WTM * C::WTN <= gemm_share<KMAJOR, KMAJOR, C>(), "a wave's block fits its share");
   auto epilogue = [&](auto with_u, auto edge) {
     constexpr bool WITH_U = decltype(with_u)::value, EDGE = decltype(edge)::value;
-    bf16* ub = nullptr;
-    if constexpr (WITH_U) {
-      __syncthreads();  // every wave is done reading the pipeline buffers
-      const int wi = wm * HC::WN + wn;
-      ub = reinterpret_cast<bf16*>(wi < NWAVES / 2 ? static_cast<void*>(&s0) : static_cast<void*>(&s1)) +
-           (wi % (NWAVES / 2)) * UWAVE;
-    }
+    if constexpr (WITH_U) __syncthreads();  // every wave is done reading the pipeline buffers
 #pragma unroll
-    for (int nb = 0; nb < HC::NB; ++nb) {
-      const int col = wn * HC::WTN + nb * 32 + l32;
+    for (int nb = 0; nb < C::NB; ++nb) {
+      const int col = wn * C::WTN + nb * 32 + l32;
       const int tok = n0 + col;
       const int tgt = !EDGE || tok < p.N ? p.targets[tok] : -1;
       const int dt = tgt - vrow0 - 4 * h;  // target row relative to this lane's rows
       float part = 0.0f;
 #pragma unroll
-      for (int mb = 0; mb < HC::MB; ++mb) {
+      for (int mb = 0; mb < C::MB; ++mb) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           float u[4];
@@ -172,7 +166,7 @@ __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
             u32x2 pk;
             pk[0] = pack_bf16x2(u[0], u[1]);
             pk[1] = pack_bf16x2(u[2], u[3]);
-            *reinterpret_cast<u32x2*>(ub + ustage_at(nb * 32 + l32, mb * 32 + 8 * g + 4 * h)) = pk;
+            *reinterpret_cast<u32x2*>(ub + ustage_at<C>(nb * 32 + l32, mb * 32 + 8 * g + 4 * h)) = pk;
           }
         }
       }
@@ -180,20 +174,20 @@ __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
       // when its offset dt has bit 2 clear and lies in [0, WTM). That is rare (WTM of V rows
       // per token), so the select runs behind a wave-uniform branch, skipped by every wave
       // where no lane hits. (A target past V may hit a row past V; the statistics ignore it.)
-      const bool mine = (unsigned)dt < (unsigned)HC::WTM && !(dt & 4);
+      const bool mine = (unsigned)dt < (unsigned)C::WTM && !(dt & 4);
       if (__builtin_amdgcn_ballot_w64(mine)) {
         int dsel = dt;
         asm volatile("" : "+v"(dsel));  // keeps the select inside the branch (not speculated)
-        const float z = select_row(acc, nb, dsel);
+        const float z = select_row<C>(acc, nb, dsel);
         if (mine) p.zt[tok] = z;
       }
       part += xor32(part);
       if (h == 0) red[wm][col] = part;
     }
     // Rows of this wave's block: tokens n0 + wn*64 + (0..63), vocabulary vrow0 + (0..127).
-    if constexpr (WITH_U) store_staged_tokmajor<BUF_NT, EDGE>(ub, p.ut, p.Npad, p.Vp, n0 + wn * HC::WTN, vrow0, lane);
+    if constexpr (WITH_U) store_staged_tokmajor<C, BUF_NT, EDGE>(ub, p.ut, p.Npad, p.Vp, n0 + wn * C::WTN, vrow0, lane);
   };
-  const bool inside = m0 + HT_M <= p.V && n0 + HT_N <= p.N;
+  const bool inside = m0 + C::TM <= p.V && n0 + C::TN <= p.N;
   if (!SPLIT && p.ut) {
     if (inside) epilogue(std::true_type{}, std::false_type{});
     else epilogue(std::true_type{}, std::true_type{});
@@ -202,17 +196,17 @@ __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
     else epilogue(std::false_type{}, std::true_type{});
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < HT_N; t += NT) {
+  for (int t = threadIdx.x; t < C::TN; t += C::THREADS) {
     const int tok = n0 + t;
     if (tok >= p.N) continue;
-    if constexpr (SPLIT) {
+    if constexpr (SPLIT && C::WTM == 128) {
 #pragma unroll
-      for (int w = 0; w < HC::WM; ++w)
-        if (m0 + w * HC::WTM < p.V) p.partial[(size_t)(tm * HC::WM + w) * p.N + tok] = red[w][t];
+      for (int w = 0; w < C::WM; ++w)
+        if (m0 + w * C::WTM < p.V) p.partial[(size_t)(tm * C::WM + w) * p.N + tok] = red[w][t];
     } else {
       float s = 0.0f;
 #pragma unroll
-      for (int w = 0; w < HC::WM; ++w) s += red[w][t];
+      for (int w = 0; w < C::WM; ++w) s += red[w][t];
       p.partial[(size_t)tm * p.N + tok] = s;
     }
   }
@@ -227,28 +221,27 @@ __global__ __launch_bounds__(NT, 1) void head_fwd_kernel(HeadParams p) {
 // first index (the argmax), the sum of w' relative to that logit, and the target logit.
 // Nothing per (token, vocab) pair is stored; head_eval_stats_kernel combines the tiles.
 
-template <int L2N>
-__global__ __launch_bounds__(NT, 1) void head_eval_kernel(HeadParams p) {
-  __shared__ __attribute__((aligned(16))) GemmStage<KMAJOR, KMAJOR, HC> s0, s1;
-  __shared__ float red[HC::WM][HT_N];
-  __shared__ float redm[HC::WM][HT_N];
-  __shared__ int redi[HC::WM][HT_N];
-  const int nbm = (p.V + HT_M - 1) / HT_M, nbn = p.Npad / HT_N;
+template <class C, int L2N>
+__global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_eval_kernel(HeadParams p) {
+  __shared__ float red[C::WM][C::TN];
+  __shared__ float redm[C::WM][C::TN];
+  __shared__ int redi[C::WM][C::TN];
+  const int nbm = (p.V + C::TM - 1) / C::TM, nbn = (p.N + C::TN - 1) / C::TN;
   int tm, tn;
   xcd_tile(blockIdx.x, nbm, nbn, tm, tn);
-  const int m0 = tm * HT_M;  // vocab
-  const int n0 = tn * HT_N;  // tokens
+  const int m0 = tm * C::TM;  // vocab
+  const int n0 = tn * C::TN;  // tokens
   GemmOperand A{p.E, p.d, p.V, p.d, (long)p.V * p.d}, B{p.h, p.d, p.N, p.d, (long)p.N * p.d};
-  floatx16 acc[HC::MB][HC::NB];
-  gemm_mainloop<KMAJOR, KMAJOR, HC>(s0, s1, A, B, m0, n0, 0, p.d, acc);
+  floatx16 acc[C::MB][C::NB];
+  gemm_tile<KMAJOR, KMAJOR, C>(A, B, m0, n0, 0, p.d, acc);
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
-  wave_coords<HC>(wm, wn);
+  wave_coords<C>(wm, wn);
   const float inv_c = p.inv_c;
-  const int vrow0 = m0 + wm * HC::WTM;
+  const int vrow0 = m0 + wm * C::WTM;
 #pragma unroll
-  for (int nb = 0; nb < HC::NB; ++nb) {
-    const int col = wn * HC::WTN + nb * 32 + l32;
+  for (int nb = 0; nb < C::NB; ++nb) {
+    const int col = wn * C::WTN + nb * 32 + l32;
     const int tok = n0 + col;
     const int tgt = tok < p.N ? p.targets[tok] : -1;
     // Pass 1: this lane's largest logit and its first index (the lane's vocabulary rows
@@ -256,7 +249,7 @@ __global__ __launch_bounds__(NT, 1) void head_eval_kernel(HeadParams p) {
     float zm = -INFINITY;
     int im = EVAL_NO_INDEX;
 #pragma unroll
-    for (int mb = 0; mb < HC::MB; ++mb) {
+    for (int mb = 0; mb < C::MB; ++mb) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int v = vrow0 + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
@@ -272,7 +265,7 @@ __global__ __launch_bounds__(NT, 1) void head_eval_kernel(HeadParams p) {
     const float sh = eval_rho(-zm * inv_c);
     float part = 0.0f;
 #pragma unroll
-    for (int mb = 0; mb < HC::MB; ++mb) {
+    for (int mb = 0; mb < C::MB; ++mb) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int v = vrow0 + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
@@ -291,16 +284,16 @@ __global__ __launch_bounds__(NT, 1) void head_eval_kernel(HeadParams p) {
     if (h == 0) { red[wm][col] = mine + other; redm[wm][col] = zm; redi[wm][col] = im; }
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < HT_N; t += NT) {
+  for (int t = threadIdx.x; t < C::TN; t += C::THREADS) {
     const int tok = n0 + t;
     float m = -INFINITY;
     int ix = EVAL_NO_INDEX;
 #pragma unroll
-    for (int w = 0; w < HC::WM; ++w)  // waves cover increasing vocabulary rows
+    for (int w = 0; w < C::WM; ++w)  // waves cover increasing vocabulary rows
       if (redi[w][t] != EVAL_NO_INDEX && eval_better(redm[w][t], redi[w][t], m, ix)) { m = redm[w][t]; ix = redi[w][t]; }
     float s = 0.0f;
 #pragma unroll
-    for (int w = 0; w < HC::WM; ++w)
+    for (int w = 0; w < C::WM; ++w)
       if (red[w][t] != 0.0f) s += red[w][t] * eval_rescale<L2N>(redm[w][t], m, inv_c, p.log2n);
     if (tok < p.N) {
       p.partial[(size_t)tm * p.N + tok] = s;
@@ -470,67 +463,54 @@ __global__ __launch_bounds__(256) void head_obj_kernel(HeadParams p, int nblocks
   if (threadIdx.x == 0) p.obj[0] = red[0] / (float)p.N;
 }
 
-// This wave's share of the pipeline buffers (idle after the main loop; the caller has passed
-// a barrier after which no wave reads them): half the waves stage in s0, half in s1.
-template <class Stage>
-__device__ __forceinline__ bf16* wave_stage(Stage& s0, Stage& s1, int wm, int wn) {
-  constexpr int NWAVES = HC::THREADS / 64, UWAVE = HC::WTM * HC::WTN;
-  static_assert((NWAVES / 2) * UWAVE * 2 <= (int)sizeof(Stage), "half the waves per stage");
-  const int wi = wm * HC::WN + wn;
-  return reinterpret_cast<bf16*>(wi < NWAVES / 2 ? static_cast<void*>(&s0) : static_cast<void*>(&s1)) +
-         (wi % (NWAVES / 2)) * UWAVE;
-}
-
 // Recompute schedules: z^T again, dZ^T = s (p - y) r, token-major: rounded to bf16, or (SPLIT,
 // f32 hidden states) as three bf16 planes whose sum is the f32 value. L2N > 0 fixes
 // n = 2^L2N at compile time (0: taken from the parameters). Each wave's block is staged and
 // written in whole token rows with 16-byte stores (default cache policy: the dh and dE products
 // read dZ right after); edge tiles write the rows up to Npad and the columns up to Vp too, of
 // which nothing is read.
-template <int L2N, bool SPLIT>
-__global__ __launch_bounds__(NT, 1) void head_dz_kernel(HeadParams p) {
+template <class C, int L2N, bool SPLIT>
+__global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_dz_kernel(HeadParams p) {
   if (SPLIT && *p.split_bad) return;
-  __shared__ __attribute__((aligned(16))) GemmStage<KMAJOR, KMAJOR, HC> s0, s1;
-  const int nbm = (p.V + HT_M - 1) / HT_M, nbn = p.Npad / HT_N;
+  const int nbm = (p.V + C::TM - 1) / C::TM, nbn = (p.N + C::TN - 1) / C::TN;
   int tm, tn;
   xcd_tile(blockIdx.x, nbm, nbn, tm, tn);
-  const int m0 = tm * HT_M, n0 = tn * HT_N;
+  const int m0 = tm * C::TM, n0 = tn * C::TN;
   const GemmOperand A = head_operand<SPLIT>(p.E, p.V, p.d, (long)p.V * p.d);
   const GemmOperand B = head_operand<SPLIT>(p.h, p.N, p.d, (long)p.N * p.d);
-  floatx16 acc[HC::MB][HC::NB];
-  gemm_mainloop<KMAJOR, KMAJOR, HC, SPLIT>(s0, s1, A, B, m0, n0, 0, p.d, acc);
+  floatx16 acc[C::MB][C::NB];
+  bf16* ub = gemm_tile<KMAJOR, KMAJOR, C, SPLIT>(A, B, m0, n0, 0, p.d, acc);
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
-  wave_coords<HC>(wm, wn);
+  wave_coords<C>(wm, wn);
   const float scale = head_grad_scale(p);
   const float inv_c = p.inv_c, clamp = p.clamp;
-  const int vrow0 = m0 + wm * HC::WTM;  // first vocab row of this wave
+  const int vrow0 = m0 + wm * C::WTM;  // first vocab row of this wave
   __syncthreads();  // every wave is done reading the pipeline buffers
-  bf16* ub = wave_stage(s0, s1, wm, wn);
   auto epilogue = [&](auto edge) {
     constexpr bool EDGE = decltype(edge)::value;
 #pragma unroll
-    for (int nb = 0; nb < HC::NB; ++nb) {
-      const int tok = n0 + wn * HC::WTN + nb * 32 + l32;
+    for (int nb = 0; nb < C::NB; ++nb) {
+      const int tok = n0 + wn * C::WTN + nb * 32 + l32;
       const bool live = !EDGE || tok < p.N;
       const int dt = (live ? p.targets[tok] - p.v_off : -1) - vrow0 - 4 * h;  // target row relative to this lane's rows
       const float st = live ? p.stat[tok] : 0.0f;
       // The target entry, (t - 1) r s (y = 1), lies in this wave's rows for few tokens (WTM of V
       // rows), so it is formed behind a wave-uniform branch, as the forward selects the target
       // logit; every entry is formed with y = 0 and the target's replaced.
-      const bool mine = (unsigned)dt < (unsigned)HC::WTM && !(dt & 4);
+      const bool mine = (unsigned)dt < (unsigned)C::WTM && !(dt & 4);
       const bool some = __builtin_amdgcn_ballot_w64(mine);
       float utgt = 0.0f;
       int dsel = dt;
       if (some) {
         asm volatile("" : "+v"(dsel));  // keeps the select inside the branch (not speculated)
-        const float x = fminf(select_row(acc, nb, dsel) * inv_c, clamp);
+        const float x = fminf(select_row<C>(acc, nb, dsel) * inv_c, clamp);
         float r;
         const float t = pow2n<L2N>(rho_fast(x, r) * st, p.log2n);
         utgt = (t - 1.0f) * r * scale;
       }
 #pragma unroll
-      for (int mb = 0; mb < HC::MB; ++mb) {
+      for (int mb = 0; mb < C::MB; ++mb) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           float u[4];
@@ -544,28 +524,28 @@ __global__ __launch_bounds__(NT, 1) void head_dz_kernel(HeadParams p) {
           u32x2 pk;
           pk[0] = pack_bf16x2(u[0], u[1]);
           pk[1] = pack_bf16x2(u[2], u[3]);
-          *reinterpret_cast<u32x2*>(ub + ustage_at(nb * 32 + l32, mb * 32 + 8 * g + 4 * h)) = pk;
+          *reinterpret_cast<u32x2*>(ub + ustage_at<C>(nb * 32 + l32, mb * 32 + 8 * g + 4 * h)) = pk;
         }
       }
       // The staged slot is overwritten (the same lane wrote it above; LDS keeps a wave's order).
-      if (some && mine) ub[ustage_at(nb * 32 + l32, dsel + 4 * h)] = f2bf(utgt);
+      if (some && mine) ub[ustage_at<C>(nb * 32 + l32, dsel + 4 * h)] = f2bf(utgt);
     }
-    store_staged_tokmajor<0, EDGE>(ub, p.dzt, p.Npad, p.Vp, n0 + wn * HC::WTN, vrow0, lane);
+    store_staged_tokmajor<C, 0, EDGE>(ub, p.dzt, p.Npad, p.Vp, n0 + wn * C::WTN, vrow0, lane);
   };
   // SPLIT: blocks of 32 tokens x 64 vocabulary entries, whose three planes fit the wave's share
   // of the buffers together, so each value is formed once and split in registers.
   auto epilogue_split = [&]() {
     constexpr int SV = 64, SCH = SV / 8, PLANE = 32 * SV;
-    static_assert(3 * PLANE <= UWAVE && HC::WTM % SV == 0, "three planes fit the wave's share");
+    static_assert(3 * PLANE <= gemm_share<KMAJOR, KMAJOR, C>() && C::WTM % SV == 0, "three planes fit the wave's share");
     auto at = [](int tl, int vl) { return tl * SV + (((vl >> 3) ^ (tl & (SCH - 1))) << 3) + (vl & 7); };
 #pragma unroll
-    for (int nb = 0; nb < HC::NB; ++nb) {
-      const int tok0 = n0 + wn * HC::WTN + nb * 32, tok = tok0 + l32;
+    for (int nb = 0; nb < C::NB; ++nb) {
+      const int tok0 = n0 + wn * C::WTN + nb * 32, tok = tok0 + l32;
       const bool live = tok < p.N;
       const int dt = (live ? p.targets[tok] - p.v_off : -1) - vrow0 - 4 * h;
       const float st = live ? p.stat[tok] : 0.0f;
 #pragma unroll
-      for (int vb = 0; vb < HC::WTM / SV; ++vb) {
+      for (int vb = 0; vb < C::WTM / SV; ++vb) {
 #pragma unroll
         for (int m2 = 0; m2 < SV / 32; ++m2) {
           const int mb = vb * (SV / 32) + m2;
@@ -610,7 +590,7 @@ __global__ __launch_bounds__(NT, 1) void head_dz_kernel(HeadParams p) {
     }
   };
   if constexpr (SPLIT) epilogue_split();
-  else if (m0 + HT_M <= p.V && n0 + HT_N <= p.N) epilogue(std::false_type{});
+  else if (m0 + C::TM <= p.V && n0 + C::TN <= p.N) epilogue(std::false_type{});
   else epilogue(std::true_type{});
 }
 
@@ -635,27 +615,27 @@ __global__ __launch_bounds__(256) void head_hscale_kernel(HeadParams p) {
 // in `stage` (this wave's share of the idle pipeline buffers) as [row][col] rows of WTN
 // elements, 16-byte chunks XOR-swizzled by the row, and written back with 16-byte stores
 // that cover whole 128-byte row segments. f(r) is the scale of block row r.
-template <class RowScale>
-__device__ __forceinline__ void store_block_bf16(const floatx16 (&acc)[HC::MB][HC::NB], bf16* stage, bf16* out,
+template <class C, class RowScale>
+__device__ __forceinline__ void store_block_bf16(const floatx16 (&acc)[C::MB][C::NB], bf16* stage, bf16* out,
                                                  long ld, RowScale f) {
-  constexpr int CH = HC::WTN / 8;  // 16-byte chunks per staged row
+  constexpr int CH = C::WTN / 8;  // 16-byte chunks per staged row
   static_assert(CH <= 64 && 64 % CH == 0 && (CH & (CH - 1)) == 0, "staged row width");
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
-  auto at = [](int r, int c) { return r * HC::WTN + (((c >> 3) ^ (r & (CH - 1))) << 3) + (c & 7); };
+  auto at = [](int r, int c) { return r * C::WTN + (((c >> 3) ^ (r & (CH - 1))) << 3) + (c & 7); };
 #pragma unroll
-  for (int mb = 0; mb < HC::MB; ++mb) {
+  for (int mb = 0; mb < C::MB; ++mb) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int r = mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
       const float fr = f(r);
 #pragma unroll
-      for (int nb = 0; nb < HC::NB; ++nb) stage[at(r, nb * 32 + l32)] = f2bf(acc[mb][nb][i] * fr);
+      for (int nb = 0; nb < C::NB; ++nb) stage[at(r, nb * 32 + l32)] = f2bf(acc[mb][nb][i] * fr);
     }
   }
   constexpr int RPS = 64 / CH;  // rows per store instruction
   const int c = lane % CH;
 #pragma unroll
-  for (int j = 0; j < HC::WTM / RPS; ++j) {
+  for (int j = 0; j < C::WTM / RPS; ++j) {
     const int r = RPS * j + lane / CH;
     const u32x4 v = *reinterpret_cast<const u32x4*>(stage + at(r, c * 8));
     *reinterpret_cast<u32x4*>(out + (long)r * ld + c * 8) = v;
@@ -673,18 +653,17 @@ __device__ __forceinline__ void store_block_bf16(const floatx16 (&acc)[HC::MB][H
 // which then goes back to the accumulator (dh_accum 1) or, rounded, to dh (dh_accum 2).
 // SPLIT (f32 hidden states): dZ and E as three bf16 planes each, the f32 result or its
 // vocabulary partials in p.dh_part.
-template <bool ACC, bool SPLIT>
-__global__ __launch_bounds__(NT, 1) void head_dh_kernel(HeadParams p) {
+template <class C, bool ACC, bool SPLIT>
+__global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_dh_kernel(HeadParams p) {
   if (SPLIT && *p.split_bad) return;
-  __shared__ __attribute__((aligned(16))) GemmStage<KMAJOR, MNMAJOR, HC> s0, s1;
-  const int nbm = p.Npad / HT_M, nbn = (p.d + HT_N - 1) / HT_N;
+  const int nbm = (p.N + C::TM - 1) / C::TM, nbn = (p.d + C::TN - 1) / C::TN;
   int tr, tn;
   xcd_tile_rowmajor(blockIdx.x, nbm * p.dh_split, nbn, tr, tn);  // U panels streamed once
   // Split-major: the workgroups an XCD runs together share one vocabulary range, so its E
   // rows are read by every token tile there from L2 (C2: dh 0.658 -> 0.639 ms).
   const int split = tr / nbm, tm = tr - split * nbm;
-  const int m0 = tm * HT_M;  // tokens
-  const int n0 = tn * HT_N;  // d
+  const int m0 = tm * C::TM;  // tokens
+  const int n0 = tn * C::TN;  // d
   const int kbeg = min(p.V, split * p.dh_kchunk), kend = min(p.V, kbeg + p.dh_kchunk);
   const bf16* a = p.ut ? p.ut : p.dzt;
   const long apad = (long)p.Npad * p.Vp;
@@ -692,19 +671,19 @@ __global__ __launch_bounds__(NT, 1) void head_dh_kernel(HeadParams p) {
   const GemmOperand B = head_operand<SPLIT>(p.E, p.V, p.d, (long)p.V * p.d);
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
-  wave_coords<HC>(wm, wn);
+  wave_coords<C>(wm, wn);
   float* part = p.dh_part ? p.dh_part + (size_t)split * p.N * p.d : nullptr;
-  floatx16 acc[HC::MB][HC::NB];
-  gemm_mainloop<KMAJOR, MNMAJOR, HC, SPLIT>(s0, s1, A, B, m0, n0, kbeg, kend, acc);
+  floatx16 acc[C::MB][C::NB];
+  bf16* stage = gemm_tile<KMAJOR, MNMAJOR, C, SPLIT>(A, B, m0, n0, kbeg, kend, acc);
   if constexpr (ACC) {
     // One 32 x 32 block at a time: its 16 loads are issued together, then added, and (dh_accum
     // 1) stored back to the accumulator.
     const bool back = p.dh_accum == 1;
 #pragma unroll
-    for (int mb = 0; mb < HC::MB; ++mb)
+    for (int mb = 0; mb < C::MB; ++mb)
 #pragma unroll
-      for (int nb = 0; nb < HC::NB; ++nb) {
-        const int r0 = m0 + wm * HC::WTM + mb * 32 + 4 * h, col = n0 + wn * HC::WTN + nb * 32 + l32;
+      for (int nb = 0; nb < C::NB; ++nb) {
+        const int r0 = m0 + wm * C::WTM + mb * 32 + 4 * h, col = n0 + wn * C::WTN + nb * 32 + l32;
         float* blk = part + (size_t)r0 * p.d + col;
         float pv[16];
 #pragma unroll
@@ -723,27 +702,27 @@ __global__ __launch_bounds__(NT, 1) void head_dh_kernel(HeadParams p) {
   }
   const float s = p.ut ? head_grad_scale(p) : 1.0f;
   const bool to_dh = !part || ACC;  // bf16 output (ACC here: the last chunk)
-  if (to_dh && m0 + HT_M <= p.N && n0 + HT_N <= p.d) {
+  if (to_dh && m0 + C::TM <= p.N && n0 + C::TN <= p.d) {
     // Interior tile, bf16 output: the row scales s/l once per row (the expression of
     // head_hscale_kernel), then the staged 16-byte stores.
-    __shared__ float fsc[HT_M];
-    for (int t = threadIdx.x; t < HT_M; t += NT) fsc[t] = p.ut ? s / p.lsum[m0 + t] : 1.0f;
+    __shared__ float fsc[C::TM];
+    for (int t = threadIdx.x; t < C::TM; t += C::THREADS) fsc[t] = p.ut ? s / p.lsum[m0 + t] : 1.0f;
     __syncthreads();  // fsc is written and every wave is done with the pipeline buffers
-    const int r0 = wm * HC::WTM;
-    store_block_bf16(acc, wave_stage(s0, s1, wm, wn), p.dh + (size_t)(m0 + r0) * p.d + n0 + wn * HC::WTN, p.d,
+    const int r0 = wm * C::WTM;
+    store_block_bf16<C>(acc, stage, p.dh + (size_t)(m0 + r0) * p.d + n0 + wn * C::WTN, p.d,
                      [&](int r) { return fsc[r0 + r]; });
     return;
   }
 #pragma unroll
-  for (int mb = 0; mb < HC::MB; ++mb) {
+  for (int mb = 0; mb < C::MB; ++mb) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int tok = m0 + wm * HC::WTM + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+      const int tok = m0 + wm * C::WTM + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
       if (tok >= p.N) continue;
       const float f = p.ut ? s / p.lsum[tok] : 1.0f;
 #pragma unroll
-      for (int nb = 0; nb < HC::NB; ++nb) {
-        const int col = n0 + wn * HC::WTN + nb * 32 + l32;
+      for (int nb = 0; nb < C::NB; ++nb) {
+        const int col = n0 + wn * C::WTN + nb * 32 + l32;
         if (col >= p.d) continue;
         const size_t o = (size_t)tok * p.d + col;
         if (to_dh) p.dh[o] = f2bf(acc[mb][nb][i] * f);
@@ -782,11 +761,10 @@ __global__ __launch_bounds__(256) void head_dh_reduce_kernel(HeadParams p) {
 // of tile de_full + (id - de_full) / de_split into an f32 tile of de_part, which
 // head_de_tail_kernel sums.
 // SPLIT (f32 hidden states): dZ and h as three bf16 planes each.
-template <bool SPLIT>
-__global__ __launch_bounds__(NT, 1) void head_de_kernel(HeadParams p) {
+template <class C, bool SPLIT>
+__global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_de_kernel(HeadParams p) {
   if (SPLIT && *p.split_bad) return;
-  __shared__ __attribute__((aligned(16))) GemmStage<MNMAJOR, MNMAJOR, HC> s0, s1;
-  const int nbn = (p.d + HT_N - 1) / HT_N;
+  const int nbn = (p.d + C::TN - 1) / C::TN;
   const int bid = blockIdx.x;
   int lin, kbeg = 0, kend = p.N, unit = -1;
   if (bid < p.de_full) {
@@ -798,46 +776,46 @@ __global__ __launch_bounds__(NT, 1) void head_de_kernel(HeadParams p) {
     kend = min(p.N, kbeg + p.de_kchunk);
   }
   const int tm = lin / nbn, tn = lin - tm * nbn;
-  const int m0 = tm * HT_M;  // vocab
-  const int n0 = tn * HT_N;  // d
+  const int m0 = tm * C::TM;  // vocab
+  const int n0 = tn * C::TN;  // d
   const bf16* a = p.ut ? p.ut : p.dzt;
   const bf16* b = p.ut ? p.hs : p.h;
   const long apad = (long)p.Npad * p.Vp;
   const GemmOperand A{a, p.Vp, p.N, p.V, apad, 0, SPLIT ? apad : 0};
   const GemmOperand B = head_operand<SPLIT>(b, p.N, p.d, (long)p.N * p.d);
-  floatx16 acc[HC::MB][HC::NB];
-  gemm_mainloop<MNMAJOR, MNMAJOR, HC, SPLIT>(s0, s1, A, B, m0, n0, kbeg, kend, acc);
+  floatx16 acc[C::MB][C::NB];
+  bf16* stage = gemm_tile<MNMAJOR, MNMAJOR, C, SPLIT>(A, B, m0, n0, kbeg, kend, acc);
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
-  wave_coords<HC>(wm, wn);
+  wave_coords<C>(wm, wn);
   if (unit >= 0) {  // one token range of a split tile: the whole f32 tile, row-major
-    float* part = p.de_part + (size_t)unit * HT_M * HT_N;
+    float* part = p.de_part + (size_t)unit * C::TM * C::TN;
 #pragma unroll
-    for (int mb = 0; mb < HC::MB; ++mb)
+    for (int mb = 0; mb < C::MB; ++mb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int r = wm * HC::WTM + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+        const int r = wm * C::WTM + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
 #pragma unroll
-        for (int nb = 0; nb < HC::NB; ++nb) part[r * HT_N + wn * HC::WTN + nb * 32 + l32] = acc[mb][nb][i];
+        for (int nb = 0; nb < C::NB; ++nb) part[r * C::TN + wn * C::WTN + nb * 32 + l32] = acc[mb][nb][i];
       }
     return;
   }
-  if (!p.dE_f32 && m0 + HT_M <= p.V && n0 + HT_N <= p.d) {  // interior tile, bf16 output
+  if (!p.dE_f32 && m0 + C::TM <= p.V && n0 + C::TN <= p.d) {  // interior tile, bf16 output
     __syncthreads();  // every wave is done with the pipeline buffers
-    store_block_bf16(acc, wave_stage(s0, s1, wm, wn),
-                     reinterpret_cast<bf16*>(p.dE) + (size_t)(m0 + wm * HC::WTM) * p.d + n0 + wn * HC::WTN, p.d,
+    store_block_bf16<C>(acc, stage,
+                     reinterpret_cast<bf16*>(p.dE) + (size_t)(m0 + wm * C::WTM) * p.d + n0 + wn * C::WTN, p.d,
                      [](int) { return 1.0f; });
     return;
   }
 #pragma unroll
-  for (int mb = 0; mb < HC::MB; ++mb) {
+  for (int mb = 0; mb < C::MB; ++mb) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int v = m0 + wm * HC::WTM + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+      const int v = m0 + wm * C::WTM + mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
       if (v >= p.V) continue;
 #pragma unroll
-      for (int nb = 0; nb < HC::NB; ++nb) {
-        const int col = n0 + wn * HC::WTN + nb * 32 + l32;
+      for (int nb = 0; nb < C::NB; ++nb) {
+        const int col = n0 + wn * C::WTN + nb * 32 + l32;
         if (col >= p.d) continue;
         const size_t o = (size_t)v * p.d + col;
         if (p.dE_f32) reinterpret_cast<float*>(p.dE)[o] = acc[mb][nb][i];
@@ -884,16 +862,24 @@ __global__ __launch_bounds__(256) void head_de_tail_kernel(HeadParams p) {
   }
 }
 
-int head_vocab_tiles(int V) { return (V + HT_M - 1) / HT_M; }
 int head_token_pad(int N) { return ((N + HT_N - 1) / HT_N) * HT_N; }
 int head_vocab_pitch(int V) { return (V + 7) / 8 * 8; }
 int head_stat_blocks(int N) { return (N + 63) / 64; }
 
-// Vocabulary splits of the dh product: minimise the rounds of 256 workgroups per unit of
-// k work (ceil(tiles*S/256)/S) for products with fewer than two rounds of tiles, keeping at
-// least 512 vocabulary entries per split; ties keep the smaller split count.
-int head_dh_split(int N, int d, int V) {
-  const int tiles = (head_token_pad(N) / HT_M) * ((d + HT_N - 1) / HT_N);
+static int head_tiles(int tile, int M, int N) { return ((M + tile - 1) / tile) * ((N + tile - 1) / tile); }
+
+// Tile side of the logit products (forward, dZ, evaluation): 128 where its tiles still run in one
+// round. Then 256 x 256 tiles leave half the CUs idle or multiply padding (us, 256 / 128; N 128,
+// d 1024, V 32768: forward 37 / 23, evaluation 46 / 24; N 512, d 512, V 8192: 22 / 15, 29 / 17);
+// past one round the 128 tiles' epilogues, with nothing beside them on a CU, cost more than that
+// (N 200, d 2048, V 32000: 59 / 74, 65 / 84; N 1000, d 1024, V 32768: 79 / 134, 93 / 163).
+int head_logit_tile(int N, int V) { return head_tiles(128, V, N) <= 256 ? 128 : 256; }
+
+// Vocabulary splits of the dh product on 256 x 256 tiles: minimise the rounds of 256 workgroups
+// per unit of k work (ceil(tiles*S/256)/S) for products with fewer than two rounds of tiles,
+// keeping at least 512 vocabulary entries per split; ties keep the smaller split count.
+static int head_dh_split(int N, int d, int V) {
+  const int tiles = head_tiles(HT_M, N, d);
   if (tiles >= 512) return 1;
   int best = 1;
   double best_cost = std::ceil(tiles / 256.0);
@@ -903,6 +889,29 @@ int head_dh_split(int N, int d, int V) {
   }
   return best;
 }
+
+// The dh product: that split, or, for few tokens, 128 x 128 tiles with up to 32 vocabulary splits
+// when gemm_tile_time says so. A split costs its f32 partials written and read (about 4.5
+// TB/s) and the summing launch.
+HeadDhPlan head_dh_plan(int N, int d, int V, int passes) {
+  auto time = [&](int tile, int s) {
+    return gemm_tile_time(tile, head_tiles(tile, N, d) * s, (double)head_dh_kchunk(V, s) * passes) +
+           (s > 1 ? 5.0 + 8e-6 / 4.5 * s * N * d : 0.0);
+  };
+  // us, 256 / 128, with the summing launch (N, d, V): 128 1024 32768 77 / 44; 512 512 8192 46 / 32;
+  // 300 768 50257 117 / 108; 700 320 32000 79 / 76; 1000 1024 32768 93 / 138.
+  HeadDhPlan pl{256, head_dh_split(N, d, V), 0};
+  double best = time(256, pl.split);
+  if (head_tiles(256, N, d) < 256)
+    for (int s = 1; s <= 32 && V / s >= 256; s *= 2)
+      if (const double t = time(128, s); t < best) {
+        best = t;
+        pl.tile = 128;
+        pl.split = s;
+      }
+  pl.kchunk = head_dh_kchunk(V, pl.split);
+  return pl;
+}
 int head_dh_kchunk(int V, int split) { return ((V + split - 1) / split + 127) / 128 * 128; }
 
 // dE tiles past the last complete round of 256 workgroups are split over the tokens when that
@@ -910,9 +919,11 @@ int head_dh_kchunk(int V, int split) { return ((V + split - 1) / split + 127) / 
 // instead of one (C2's 591 tiles: two full rounds, then 79 tiles x 3 ranges in a third of a
 // tile's time). A range keeps at least 1024 tokens, and a split must save a quarter of a round
 // (its f32 tiles are written and summed by head_de_tail_kernel); ties keep the smaller split.
-HeadDePlan head_de_plan(int N, int d, int V) {
+// Products that do not fill a round take 128 x 128 tiles, unsplit, when gemm_tile_time says so.
+HeadDePlan head_de_plan(int N, int d, int V, int passes) {
   HeadDePlan pl;
-  pl.tiles = head_vocab_tiles(V) * ((d + HT_N - 1) / HT_N);
+  pl.tile = 256;
+  pl.tiles = head_tiles(256, V, d);
   pl.full = pl.tiles;
   pl.split = 1;
   pl.kchunk = 0;
@@ -924,21 +935,34 @@ HeadDePlan head_de_plan(int N, int d, int V) {
     const double cost = std::ceil(tail * (double)s / 256.0) / s;
     if (cost < best_cost - 1e-9) { best = s; best_cost = cost; }
   }
-  if (best == 1 || best_cost > 0.75) return pl;
-  pl.full = full;
-  pl.split = best;
-  pl.kchunk = ((N + best - 1) / best + 127) / 128 * 128;
+  if (best > 1 && best_cost <= 0.75) {
+    pl.full = full;
+    pl.split = best;
+    pl.kchunk = ((N + best - 1) / best + 127) / 128 * 128;
+    return pl;
+  }
+  const double K = (double)N * passes;
+  const int tiles128 = head_tiles(128, V, d);
+  if (full == 0 && gemm_tile_time(128, tiles128, K) < gemm_tile_time(256, pl.tiles, K)) {
+    pl.tile = 128;
+    pl.tiles = pl.full = tiles128;
+  }
   return pl;
 }
 
+template <class C, bool SPLIT>
+static void launch_fwd_cfg(const HeadParams& p, hipStream_t st) {
+  const dim3 grid(head_tiles(C::TM, p.V, p.N)), nt(C::THREADS);
+  KTimer t(SPLIT ? "head_fwd_split" : "head_fwd", st);
+  if (p.log2n == 3) hipLaunchKernelGGL((head_fwd_kernel<C, 3, SPLIT>), grid, nt, 0, st, p);
+  else hipLaunchKernelGGL((head_fwd_kernel<C, 0, SPLIT>), grid, nt, 0, st, p);
+}
+
 hipError_t launch_head_fwd(const HeadParams& p, hipStream_t st) {
-  const int tiles = head_vocab_tiles(p.V) * (p.Npad / HT_N);
-  {
-    KTimer t("head_fwd", st);
-    if (p.log2n == 3) hipLaunchKernelGGL((head_fwd_kernel<3, false>), dim3(tiles), dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL((head_fwd_kernel<0, false>), dim3(tiles), dim3(NT), 0, st, p);
-  }
-  return launch_head_stats(p, head_vocab_tiles(p.V), st);
+  const int tile = head_logit_tile(p.N, p.V);
+  if (tile == 128) launch_fwd_cfg<HC128, false>(p, st);
+  else launch_fwd_cfg<HC, false>(p, st);
+  return launch_head_stats(p, (p.V + tile - 1) / tile, st);
 }
 
 // Statistics, telemetry and objective from the forward's per-tile partial sums (any tiling:
@@ -956,24 +980,29 @@ hipError_t launch_head_eval_stats(const HeadParams& p, int vocab_tiles, hipStrea
   return hipGetLastError();
 }
 
+template <class C>
+static void launch_eval_cfg(const HeadParams& p, hipStream_t st) {
+  const dim3 grid(head_tiles(C::TM, p.V, p.N)), nt(C::THREADS);
+  KTimer t("head_eval", st);
+  if (p.log2n == 3) hipLaunchKernelGGL((head_eval_kernel<C, 3>), grid, nt, 0, st, p);
+  else hipLaunchKernelGGL((head_eval_kernel<C, 0>), grid, nt, 0, st, p);
+}
+
 hipError_t launch_head_eval(const HeadParams& p, hipStream_t st) {
-  const int tiles = head_vocab_tiles(p.V) * (p.Npad / HT_N);
-  {
-    KTimer t("head_eval", st);
-    if (p.log2n == 3) hipLaunchKernelGGL(head_eval_kernel<3>, dim3(tiles), dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL(head_eval_kernel<0>, dim3(tiles), dim3(NT), 0, st, p);
-  }
-  return launch_head_eval_stats(p, head_vocab_tiles(p.V), st);
+  const int tile = head_logit_tile(p.N, p.V);
+  if (tile == 128) launch_eval_cfg<HC128>(p, st);
+  else launch_eval_cfg<HC>(p, st);
+  return launch_head_eval_stats(p, (p.V + tile - 1) / tile, st);
 }
 
 // dh = (U' or dZ) E, and the sum over vocabulary splits when the product is split.
 static void launch_head_dh(const HeadParams& p, hipStream_t st) {
-  const int dtiles = (p.d + HT_N - 1) / HT_N;
   {
     KTimer t("head_dh", st);
-    const dim3 grid((p.Npad / HT_M) * dtiles * p.dh_split);
-    if (p.dh_accum) hipLaunchKernelGGL((head_dh_kernel<true, false>), grid, dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL((head_dh_kernel<false, false>), grid, dim3(NT), 0, st, p);
+    const dim3 grid(head_tiles(p.dh_tile, p.N, p.d) * p.dh_split);
+    if (p.dh_accum) hipLaunchKernelGGL((head_dh_kernel<HC, true, false>), grid, dim3(HC::THREADS), 0, st, p);
+    else if (p.dh_tile == 128) hipLaunchKernelGGL((head_dh_kernel<HC128, false, false>), grid, dim3(HC128::THREADS), 0, st, p);
+    else hipLaunchKernelGGL((head_dh_kernel<HC, false, false>), grid, dim3(HC::THREADS), 0, st, p);
   }
   if (p.dh_split > 1) {
     const size_t chunks = (size_t)p.N * p.d / 8;
@@ -984,20 +1013,21 @@ static void launch_head_dh(const HeadParams& p, hipStream_t st) {
 }
 
 // dE = (U' or dZ)^T (hs or h), with the token split of head_de_plan when p carries one.
+template <bool SPLIT>
 static void launch_head_de(const HeadParams& p, hipStream_t st) {
-  const int de_tiles = head_vocab_tiles(p.V) * ((p.d + HT_N - 1) / HT_N);
   HeadParams q = p;
+  const int tiles = head_tiles(p.de_tile, p.V, p.d);
   const bool split = p.de_split > 1 && p.de_part;
   if (!split) {
-    q.de_full = de_tiles;
+    q.de_full = tiles;
     q.de_split = 1;
   }
-  const int tail = de_tiles - q.de_full;
+  const int tail = tiles - q.de_full;
   {
     KTimer t("head_de", st);
     const dim3 grid(q.de_full + tail * q.de_split);
-    if (p.split_bad) hipLaunchKernelGGL(head_de_kernel<true>, grid, dim3(NT), 0, st, q);
-    else hipLaunchKernelGGL(head_de_kernel<false>, grid, dim3(NT), 0, st, q);
+    if (p.de_tile == 128) hipLaunchKernelGGL((head_de_kernel<HC128, SPLIT>), grid, dim3(HC128::THREADS), 0, st, q);
+    else hipLaunchKernelGGL((head_de_kernel<HC, SPLIT>), grid, dim3(HC::THREADS), 0, st, q);
   }
   if (split) {
     KTimer t("head_de_tail", st);
@@ -1005,11 +1035,17 @@ static void launch_head_de(const HeadParams& p, hipStream_t st) {
   }
 }
 
+template <class C, bool SPLIT>
+static void launch_dz_cfg(const HeadParams& p, hipStream_t st) {
+  const dim3 grid(head_tiles(C::TM, p.V, p.N)), nt(C::THREADS);
+  KTimer t(SPLIT ? "head_dz_split" : "head_dz", st);
+  if (p.log2n == 3) hipLaunchKernelGGL((head_dz_kernel<C, 3, SPLIT>), grid, nt, 0, st, p);
+  else hipLaunchKernelGGL((head_dz_kernel<C, 0, SPLIT>), grid, nt, 0, st, p);
+}
+
 static void launch_head_dz(const HeadParams& p, hipStream_t st) {
-  const int tiles = head_vocab_tiles(p.V) * (p.Npad / HT_N);
-  KTimer t("head_dz", st);
-  if (p.log2n == 3) hipLaunchKernelGGL((head_dz_kernel<3, false>), dim3(tiles), dim3(NT), 0, st, p);
-  else hipLaunchKernelGGL((head_dz_kernel<0, false>), dim3(tiles), dim3(NT), 0, st, p);
+  if (head_logit_tile(p.N, p.V) == 128) launch_dz_cfg<HC128, false>(p, st);
+  else launch_dz_cfg<HC, false>(p, st);
 }
 
 hipError_t launch_head_bwd(const HeadParams& p, hipStream_t st) {
@@ -1021,7 +1057,7 @@ hipError_t launch_head_bwd(const HeadParams& p, hipStream_t st) {
     launch_head_dz(p, st);
   }
   launch_head_dh(p, st);
-  launch_head_de(p, st);
+  launch_head_de<false>(p, st);
   return hipGetLastError();
 }
 
@@ -1071,28 +1107,23 @@ static void launch_head_split3(const HeadParams& p, hipStream_t st) {
 
 void launch_head_fwd_split(const HeadParams& p, hipStream_t st) {
   launch_head_split3(p, st);
-  const int tiles = head_vocab_tiles(p.V) * (p.Npad / HT_N);
-  KTimer t("head_fwd_split", st);
-  if (p.log2n == 3) hipLaunchKernelGGL((head_fwd_kernel<3, true>), dim3(tiles), dim3(NT), 0, st, p);
-  else hipLaunchKernelGGL((head_fwd_kernel<0, true>), dim3(tiles), dim3(NT), 0, st, p);
+  if (head_logit_tile(p.N, p.V) == 128) launch_fwd_cfg<HC128, true>(p, st);
+  else launch_fwd_cfg<HC, true>(p, st);
 }
 
 void launch_head_bwd_split(const HeadParams& p, hipStream_t st) {
   launch_head_split3(p, st);
-  const int tiles = head_vocab_tiles(p.V) * (p.Npad / HT_N);
-  {
-    KTimer t("head_dz_split", st);
-    if (p.log2n == 3) hipLaunchKernelGGL((head_dz_kernel<3, true>), dim3(tiles), dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL((head_dz_kernel<0, true>), dim3(tiles), dim3(NT), 0, st, p);
-  }
+  if (head_logit_tile(p.N, p.V) == 128) launch_dz_cfg<HC128, true>(p, st);
+  else launch_dz_cfg<HC, true>(p, st);
   {
     HeadParams q = p;
     if (p.dh_split == 1) q.dh_part = p.dh32;
     KTimer t("head_dh_split", st);
-    const dim3 grid((p.Npad / HT_M) * ((p.d + HT_N - 1) / HT_N) * p.dh_split);
-    hipLaunchKernelGGL((head_dh_kernel<false, true>), grid, dim3(NT), 0, st, q);
+    const dim3 grid(head_tiles(p.dh_tile, p.N, p.d) * p.dh_split);
+    if (p.dh_tile == 128) hipLaunchKernelGGL((head_dh_kernel<HC128, false, true>), grid, dim3(HC128::THREADS), 0, st, q);
+    else hipLaunchKernelGGL((head_dh_kernel<HC, false, true>), grid, dim3(HC::THREADS), 0, st, q);
   }
-  launch_head_de(p, st);
+  launch_head_de<true>(p, st);
 }
 
 HeadParams head_vocab_chunk(const HeadParams& p, int v0, int vc) {
@@ -1111,17 +1142,19 @@ hipError_t launch_head_bwd_streamed(const HeadParams& p, int chunk, hipStream_t 
   const int nchunks = (p.V + chunk - 1) / chunk;
   for (int k = 0; k < nchunks; ++k) {
     HeadParams q = head_vocab_chunk(p, k * chunk, std::min(chunk, p.V - k * chunk));
+    q.dh_tile = 256;
     q.dh_split = 1;
     q.dh_kchunk = head_dh_kchunk(q.V, 1);
     q.dh_part = nchunks > 1 ? p.dh_part : nullptr;
     q.dh_accum = k == 0 ? 0 : (k == nchunks - 1 ? 2 : 1);
-    const HeadDePlan de = head_de_plan(p.N, p.d, q.V);
+    const HeadDePlan de = head_de_plan(p.N, p.d, q.V, 1);
+    q.de_tile = de.tile;
     q.de_full = de.full;
     q.de_split = de.split;
     q.de_kchunk = de.kchunk;
     launch_head_dz(q, st);
     launch_head_dh(q, st);
-    launch_head_de(q, st);
+    launch_head_de<false>(q, st);
   }
   return hipGetLastError();
 }

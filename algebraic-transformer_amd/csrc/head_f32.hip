@@ -159,12 +159,13 @@ struct F32Wave {
 
 // Forward: z^T = E h^T (m = vocabulary, n = tokens), per-token partial sums of w over the tile's
 // vocabulary rows and the target logit (fused_head.py:83-103).
+template <bool FALLBACK>
 __global__ __launch_bounds__(F_NT) void head_fwd_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   __shared__ float red[F_WM][F_TN];
   const int nbm = (p.V + F_TM - 1) / F_TM, nbn = (p.N + F_TN - 1) / F_TN;
-  if (p.split_bad && !*p.split_bad) return;
-  for (int bid = blockIdx.x; bid < nbm * nbn; bid += gridDim.x) {
+  if (FALLBACK && !*p.split_bad) return;
+  for (int bid = blockIdx.x; FALLBACK ? bid < nbm * nbn : bid == (int)blockIdx.x; bid += gridDim.x) {
   int tm, tn;
   xcd_tile(bid, nbm, nbn, tm, tn);
   const int m0 = tm * F_TM, n0 = tn * F_TN;
@@ -203,11 +204,12 @@ __global__ __launch_bounds__(F_NT) void head_fwd_f32_kernel(HeadParams p) {
 
 // Backward, logit gradient: z = h E^T (m = tokens, n = vocabulary, so the f32 stores run along
 // the vocabulary), dZ = ((p - y) r) s with p = (rho(x) stat)^n (fused_head.py:133-146).
+template <bool FALLBACK>
 __global__ __launch_bounds__(F_NT) void head_dz_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   const int nbm = (p.N + F_TM - 1) / F_TM, nbn = (p.V + F_TN - 1) / F_TN;
-  if (p.split_bad && !*p.split_bad) return;
-  for (int bid = blockIdx.x; bid < nbm * nbn; bid += gridDim.x) {
+  if (FALLBACK && !*p.split_bad) return;
+  for (int bid = blockIdx.x; FALLBACK ? bid < nbm * nbn : bid == (int)blockIdx.x; bid += gridDim.x) {
   int tm, tn;
   xcd_tile(bid, nbm, nbn, tm, tn);
   const int m0 = tm * F_TM, n0 = tn * F_TN;
@@ -239,11 +241,12 @@ __global__ __launch_bounds__(F_NT) void head_dz_f32_kernel(HeadParams p) {
 
 // dh = dZ E: A = dZ stored [token][v] (k contiguous), B = E stored [v][d] (n contiguous). With
 // several vocabulary splits each workgroup writes its f32 partial for head_dh_f32_reduce_kernel.
+template <bool FALLBACK>
 __global__ __launch_bounds__(F_NT) void head_dh_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   const int nbm = (p.N + F_TM - 1) / F_TM, nbn = (p.d + F_TN - 1) / F_TN;
-  if (p.split_bad && !*p.split_bad) return;
-  for (int bid = blockIdx.x; bid < nbm * p.dh_split * nbn; bid += gridDim.x) {
+  if (FALLBACK && !*p.split_bad) return;
+  for (int bid = blockIdx.x; FALLBACK ? bid < nbm * p.dh_split * nbn : bid == (int)blockIdx.x; bid += gridDim.x) {
   int tr, tn;
   xcd_tile_rowmajor(bid, nbm * p.dh_split, nbn, tr, tn);
   const int tm = tr / p.dh_split, split = tr - tm * p.dh_split;
@@ -285,11 +288,12 @@ __global__ __launch_bounds__(256) void head_dh_f32_reduce_kernel(HeadParams p) {
 }
 
 // dE = dZ^T h: A = dZ stored [token][v] (m contiguous), B = h stored [token][d] (n contiguous).
+template <bool FALLBACK>
 __global__ __launch_bounds__(F_NT) void head_de_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   const int nbm = (p.V + F_TM - 1) / F_TM, nbn = (p.d + F_TN - 1) / F_TN;
-  if (p.split_bad && !*p.split_bad) return;
-  for (int bid = blockIdx.x; bid < nbm * nbn; bid += gridDim.x) {
+  if (FALLBACK && !*p.split_bad) return;
+  for (int bid = blockIdx.x; FALLBACK ? bid < nbm * nbn : bid == (int)blockIdx.x; bid += gridDim.x) {
   int tm, tn;
   xcd_tile_rowmajor(bid, nbm, nbn, tm, tn);
   const int m0 = tm * F_TM, n0 = tn * F_TN;
@@ -395,20 +399,39 @@ __global__ __launch_bounds__(F_NT) void head_eval_f32_kernel(HeadParams p) {
 
 int head_f32_vocab_tiles(int V) { return (V + F_TM - 1) / F_TM; }
 
+// Whether the products run on the bf16 matrix cores, as three bf16 planes an operand. Splitting E
+// costs two passes over it a step, which fewer than two 128-token tiles do not pay back (forward +
+// backward kernels, us, f32 / split; N, d, V: 100 256 4096 151 / 186; 128 1024 32768 452 / 519;
+// 200 2048 32000 1474 / 1457; 300 768 50257 1395 / 1308; 512 512 8192 275 / 252; 1000 1024 32768
+// 3149 / 1559; 2048 768 32768 4151 / 2158).
+bool head_f32_split(int N) { return N >= 256; }
+
+// Vocabulary splits of the f32 dh product: double them while the product has fewer than about
+// 1024 workgroups (4 per CU) and each split keeps at least 256 vocabulary entries.
+int head_f32_dh_split(int N, int d, int V) {
+  const long tiles = (long)((N + F_TM - 1) / F_TM) * ((d + F_TN - 1) / F_TN);
+  int s = 1;
+  while (s < 32 && tiles * s < 1024 && V / (2 * s) >= 256) s *= 2;
+  return s;
+}
 // Vocabulary entries per split: a multiple of the k step (so every split starts 16-byte aligned).
 int head_f32_dh_kchunk(int V, int split) { return ((V + split - 1) / split + F_TK - 1) / F_TK * F_TK; }
 
-// Workgroups of an f32 kernel: one per tile, or, where the split kernels have done the work unless
-// an input was not finite, at most four per CU looping over the tiles (a launch that returns at
-// once costs its workgroups).
-static dim3 f32_grid(const HeadParams& p, int tiles) { return dim3(p.split_bad ? std::min(tiles, 1024) : tiles); }
+// An f32 kernel over `tiles` tiles: a workgroup each, or, as the fallback of the split kernels
+// (which have done the work unless an input was not finite), at most four workgroups per CU looping
+// over the tiles (a launch that returns at once costs its workgroups).
+typedef void (*F32Kernel)(HeadParams);
+static void launch_f32(F32Kernel fallback, F32Kernel plain, const HeadParams& p, hipStream_t st, int tiles) {
+  if (p.split_bad) hipLaunchKernelGGL(fallback, dim3(std::min(tiles, 1024)), dim3(F_NT), 0, st, p);
+  else hipLaunchKernelGGL(plain, dim3(tiles), dim3(F_NT), 0, st, p);
+}
 
 hipError_t launch_head_fwd_f32(const HeadParams& p, hipStream_t st) {
   const int tiles = head_f32_vocab_tiles(p.V) * ((p.N + F_TN - 1) / F_TN);
   if (p.split_bad) launch_head_fwd_split(p, st);
   {
     KTimer t("head_fwd_f32", st);
-    hipLaunchKernelGGL(head_fwd_f32_kernel, f32_grid(p, tiles), dim3(F_NT), 0, st, p);
+    launch_f32(head_fwd_f32_kernel<true>, head_fwd_f32_kernel<false>, p, st, (tiles));
   }
   return launch_head_stats(p, head_f32_vocab_tiles(p.V), st);
 }
@@ -418,11 +441,11 @@ hipError_t launch_head_bwd_f32(const HeadParams& p, hipStream_t st) {
   if (p.split_bad) launch_head_bwd_split(p, st);
   {
     KTimer t("head_dz_f32", st);
-    hipLaunchKernelGGL(head_dz_f32_kernel, f32_grid(p, ntok * head_f32_vocab_tiles(p.V)), dim3(F_NT), 0, st, p);
+    launch_f32(head_dz_f32_kernel<true>, head_dz_f32_kernel<false>, p, st, (ntok * head_f32_vocab_tiles(p.V)));
   }
   {
     KTimer t("head_dh_f32", st);
-    hipLaunchKernelGGL(head_dh_f32_kernel, f32_grid(p, ntok * nd * p.dh_split), dim3(F_NT), 0, st, p);
+    launch_f32(head_dh_f32_kernel<true>, head_dh_f32_kernel<false>, p, st, (ntok * nd * p.dh_split));
   }
   if (p.dh_split > 1) {
     const size_t chunks = (size_t)p.N * p.d / 4;
@@ -432,7 +455,7 @@ hipError_t launch_head_bwd_f32(const HeadParams& p, hipStream_t st) {
   }
   {
     KTimer t("head_de_f32", st);
-    hipLaunchKernelGGL(head_de_f32_kernel, f32_grid(p, head_f32_vocab_tiles(p.V) * nd), dim3(F_NT), 0, st, p);
+    launch_f32(head_de_f32_kernel<true>, head_de_f32_kernel<false>, p, st, (head_f32_vocab_tiles(p.V) * nd));
   }
   return hipGetLastError();
 }
@@ -450,9 +473,9 @@ hipError_t launch_head_bwd_f32_streamed(const HeadParams& p, int chunk, hipStrea
     q.dh_part = nullptr;
     q.dh_accum = k > 0;
     const int vt = head_f32_vocab_tiles(q.V);
-    { KTimer t("head_dz_f32", st); hipLaunchKernelGGL(head_dz_f32_kernel, dim3(ntok * vt), dim3(F_NT), 0, st, q); }
-    { KTimer t("head_dh_f32", st); hipLaunchKernelGGL(head_dh_f32_kernel, dim3(ntok * nd), dim3(F_NT), 0, st, q); }
-    { KTimer t("head_de_f32", st); hipLaunchKernelGGL(head_de_f32_kernel, dim3(vt * nd), dim3(F_NT), 0, st, q); }
+    { KTimer t("head_dz_f32", st); hipLaunchKernelGGL(head_dz_f32_kernel<false>, dim3(ntok * vt), dim3(F_NT), 0, st, q); }
+    { KTimer t("head_dh_f32", st); hipLaunchKernelGGL(head_dh_f32_kernel<false>, dim3(ntok * nd), dim3(F_NT), 0, st, q); }
+    { KTimer t("head_de_f32", st); hipLaunchKernelGGL(head_de_f32_kernel<false>, dim3(vt * nd), dim3(F_NT), 0, st, q); }
   }
   return hipGetLastError();
 }

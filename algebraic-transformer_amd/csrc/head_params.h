@@ -23,7 +23,7 @@ struct HeadParams {
   int Vp;               // row pitch of the token-major U / dZ: V rounded up to 8
   int log2n;
   float inv_c, c, clamp;
-  float* partial;       // (ceil(V/HT_M), N) per-vocab-tile row sums
+  float* partial;       // (ceil(V/128), N) at most: per-vocab-tile row sums
   float* stat;          // (N,)
   float* zt;            // (N,)
   float* pt;            // (N,)
@@ -36,10 +36,12 @@ struct HeadParams {
   bf16* hs;             // residual path workspace (N, d): bf16(s h / l)
   bf16* dh;             // (N, d)
   float* dh_part;       // split-K partials of dh (dh_split, N, d) f32, or nullptr (one split)
+  int dh_tile;          // tile side of the dh product (head_dh_plan)
   int dh_split;         // k splits of the dh product (1: none)
   int dh_kchunk;        // vocabulary entries per split (a multiple of 128)
   void* dE;             // (V, d) bf16 or f32
   int dE_f32;
+  int de_tile = 256;    // tile side of the dE product (head_de_plan)
   // dE tiles past the last complete round of workgroups, split over the tokens (head_de_plan):
   float* de_part = nullptr;  // (tiles - de_full) * de_split f32 tiles of HT_M x HT_N, or nullptr
   int de_full = 0;      // tiles computed whole (all of them when de_split is 1)
