@@ -165,7 +165,7 @@ __global__ __launch_bounds__(F_NT) void head_fwd_f32_kernel(HeadParams p) {
   __shared__ float red[F_WM][F_TN];
   const int nbm = (p.V + F_TM - 1) / F_TM, nbn = (p.N + F_TN - 1) / F_TN;
   if (FALLBACK && !*p.split_bad) return;
-  for (int bid = blockIdx.x; FALLBACK ? bid < nbm * nbn : bid == (int)blockIdx.x; bid += gridDim.x) {
+  auto tile = [&](int bid) __attribute__((always_inline)) {
   int tm, tn;
   xcd_tile(bid, nbm, nbn, tm, tn);
   const int m0 = tm * F_TM, n0 = tn * F_TN;
@@ -198,7 +198,14 @@ __global__ __launch_bounds__(F_NT) void head_fwd_f32_kernel(HeadParams p) {
     const int tok = n0 + t;
     if (tok < p.N) p.partial[(size_t)tm * p.N + tok] = red[0][t] + red[1][t];
   }
-  __syncthreads();  // the next tile reuses the LDS
+  };
+  if constexpr (FALLBACK) {
+    for (int bid = blockIdx.x; bid < nbm * nbn; bid += gridDim.x) {
+      tile(bid);
+      __syncthreads();  // the next tile reuses the LDS
+    }
+  } else {
+    tile(blockIdx.x);
   }
 }
 
@@ -209,7 +216,7 @@ __global__ __launch_bounds__(F_NT) void head_dz_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   const int nbm = (p.N + F_TM - 1) / F_TM, nbn = (p.V + F_TN - 1) / F_TN;
   if (FALLBACK && !*p.split_bad) return;
-  for (int bid = blockIdx.x; FALLBACK ? bid < nbm * nbn : bid == (int)blockIdx.x; bid += gridDim.x) {
+  auto tile = [&](int bid) __attribute__((always_inline)) {
   int tm, tn;
   xcd_tile(bid, nbm, nbn, tm, tn);
   const int m0 = tm * F_TM, n0 = tn * F_TN;
@@ -236,6 +243,14 @@ __global__ __launch_bounds__(F_NT) void head_dz_f32_kernel(HeadParams p) {
         p.dz32[(size_t)tok * p.Vp + v] = (t - y) * r * scale;
       }
     }
+  };
+  if constexpr (FALLBACK) {
+    for (int bid = blockIdx.x; bid < nbm * nbn; bid += gridDim.x) {
+      tile(bid);
+      __syncthreads();  // the next tile reuses the LDS
+    }
+  } else {
+    tile(blockIdx.x);
   }
 }
 
@@ -246,7 +261,7 @@ __global__ __launch_bounds__(F_NT) void head_dh_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   const int nbm = (p.N + F_TM - 1) / F_TM, nbn = (p.d + F_TN - 1) / F_TN;
   if (FALLBACK && !*p.split_bad) return;
-  for (int bid = blockIdx.x; FALLBACK ? bid < nbm * p.dh_split * nbn : bid == (int)blockIdx.x; bid += gridDim.x) {
+  auto tile = [&](int bid) __attribute__((always_inline)) {
   int tr, tn;
   xcd_tile_rowmajor(bid, nbm * p.dh_split, nbn, tr, tn);
   const int tm = tr / p.dh_split, split = tr - tm * p.dh_split;
@@ -271,6 +286,14 @@ __global__ __launch_bounds__(F_NT) void head_dh_f32_kernel(HeadParams p) {
         else out[(size_t)tok * p.d + col] = acc[mb][nb][i];
       }
     }
+  };
+  if constexpr (FALLBACK) {
+    for (int bid = blockIdx.x; bid < nbm * p.dh_split * nbn; bid += gridDim.x) {
+      tile(bid);
+      __syncthreads();  // the next tile reuses the LDS
+    }
+  } else {
+    tile(blockIdx.x);
   }
 }
 
@@ -293,7 +316,7 @@ __global__ __launch_bounds__(F_NT) void head_de_f32_kernel(HeadParams p) {
   __shared__ __attribute__((aligned(16))) float sA[2][F_TILE], sB[2][F_TILE];
   const int nbm = (p.V + F_TM - 1) / F_TM, nbn = (p.d + F_TN - 1) / F_TN;
   if (FALLBACK && !*p.split_bad) return;
-  for (int bid = blockIdx.x; FALLBACK ? bid < nbm * nbn : bid == (int)blockIdx.x; bid += gridDim.x) {
+  auto tile = [&](int bid) __attribute__((always_inline)) {
   int tm, tn;
   xcd_tile_rowmajor(bid, nbm, nbn, tm, tn);
   const int m0 = tm * F_TM, n0 = tn * F_TN;
@@ -316,6 +339,14 @@ __global__ __launch_bounds__(F_NT) void head_de_f32_kernel(HeadParams p) {
         else reinterpret_cast<bf16*>(p.dE)[o] = f2bf(acc[mb][nb][i]);
       }
     }
+  };
+  if constexpr (FALLBACK) {
+    for (int bid = blockIdx.x; bid < nbm * nbn; bid += gridDim.x) {
+      tile(bid);
+      __syncthreads();  // the next tile reuses the LDS
+    }
+  } else {
+    tile(blockIdx.x);
   }
 }
 
@@ -431,7 +462,7 @@ hipError_t launch_head_fwd_f32(const HeadParams& p, hipStream_t st) {
   if (p.split_bad) launch_head_fwd_split(p, st);
   {
     KTimer t("head_fwd_f32", st);
-    launch_f32(head_fwd_f32_kernel<true>, head_fwd_f32_kernel<false>, p, st, (tiles));
+    launch_f32(head_fwd_f32_kernel<true>, head_fwd_f32_kernel<false>, p, st, tiles);
   }
   return launch_head_stats(p, head_f32_vocab_tiles(p.V), st);
 }
@@ -441,11 +472,11 @@ hipError_t launch_head_bwd_f32(const HeadParams& p, hipStream_t st) {
   if (p.split_bad) launch_head_bwd_split(p, st);
   {
     KTimer t("head_dz_f32", st);
-    launch_f32(head_dz_f32_kernel<true>, head_dz_f32_kernel<false>, p, st, (ntok * head_f32_vocab_tiles(p.V)));
+    launch_f32(head_dz_f32_kernel<true>, head_dz_f32_kernel<false>, p, st, ntok * head_f32_vocab_tiles(p.V));
   }
   {
     KTimer t("head_dh_f32", st);
-    launch_f32(head_dh_f32_kernel<true>, head_dh_f32_kernel<false>, p, st, (ntok * nd * p.dh_split));
+    launch_f32(head_dh_f32_kernel<true>, head_dh_f32_kernel<false>, p, st, ntok * nd * p.dh_split);
   }
   if (p.dh_split > 1) {
     const size_t chunks = (size_t)p.N * p.d / 4;
@@ -455,7 +486,7 @@ hipError_t launch_head_bwd_f32(const HeadParams& p, hipStream_t st) {
   }
   {
     KTimer t("head_de_f32", st);
-    launch_f32(head_de_f32_kernel<true>, head_de_f32_kernel<false>, p, st, (head_f32_vocab_tiles(p.V) * nd));
+    launch_f32(head_de_f32_kernel<true>, head_de_f32_kernel<false>, p, st, head_f32_vocab_tiles(p.V) * nd);
   }
   return hipGetLastError();
 }
