@@ -55,6 +55,10 @@ _SIGNATURES = {
     "alg_ffn_alu_glu_dy": (_I, [_P, _I, _I, _I, _P, _P, _P, _P, _F, _P]),
     "alg_ffn_gemm_workspace_size": (_S, [_I, _I, _I]),
     "alg_ffn_gemm": (_I, [_P, _I, _I, _I, _P, _L, _I, _P, _L, _I, _P, _L, _P, _S]),
+    "alg_ffn_block_workspace_size": (_S, [_I, _I, _I, _I, _I]),
+    "alg_ffn_block_fwd": (_I, [_P, _I, _I, _I, _I, _P, _P, _I, _P, _I, _P, _I, _F, _P, _P, _P, _P, _P, _P, _P, _S]),
+    "alg_ffn_block_bwd": (_I, [_P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _F, _P, _P, _I, _P, _I, _P, _I, _P,
+                               _S]),
     "alg_rms_norm_fwd": (_I, [_P, _I, _I, _P, _P, _F, _P, _P]),
     "alg_rms_norm_bwd": (_I, [_P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _S]),
     "alg_timer_enable": (None, [_I]),

@@ -3,13 +3,15 @@
 ``alu_glu_ffn(h2, w_g, w_u, w_d, beta)`` is ``(h2 @ w_g * alu(h2 @ w_u, beta)) @ w_d`` as the
 model's block computes it (src/algebraic/model.py:185-193, ffn="alu_glu"; alu and its custom VJP
 src/algebraic/algebraic.py:86-113), differentiable in h2 and the three weights. The gate/up
-product over the concatenated weights [w_g | w_u] carries the activation in its epilogue (one
+product over the packed weights [w_g | w_u] carries the activation in its epilogue (one
 HIP kernel writes y = gate*alu(up) and the gate/up residuals); in the backward, the product
 dout @ w_d^T carries the activation's VJP in its epilogue (one HIP kernel writes
-[d_gate | d_up]). The four remaining products are plain GEMMs on the same MFMA core
-(``alg_ffn_gemm``), each operand read in its stored layout (no transposed copies): y @ w_d,
-[d_gate | d_up] @ [w_g | w_u]^T, h2^T @ [d_gate | d_up], y^T @ dout. bf16 only; d_ff must be a
-multiple of 128 and the widths multiples of 8. No CPU fallback.
+[d_gate | d_up]). The four remaining products are plain GEMMs on the same MFMA core, each operand
+read in its stored layout (no transposed copies): y @ w_d, [d_gate | d_up] @ [w_g | w_u]^T,
+h2^T @ [d_gate | d_up], y^T @ dout. Each direction is one library call (``alg_ffn_block_fwd``,
+``alg_ffn_block_bwd``). Activations in bf16, products in bf16 with f32 sums; bf16 or f32 weights
+(others go through bf16), whose gradients come back in their dtype, f32 ones as the f32 sum. d_ff
+must be a multiple of 128 and the widths multiples of 8. No CPU fallback.
 """
 
 import torch
@@ -17,19 +19,20 @@ import torch
 from .. import _lib
 
 
-def _gemm(a, b, a_trans=False, b_trans=False):
-    """C = op(A) op(B) in bf16 (f32 accumulation) through alg_ffn_gemm. ``a`` is stored (M, K),
-    or (K, M) with ``a_trans``; ``b`` is stored (K, N), or (N, K) with ``b_trans``; both
-    contiguous row-major."""
-    lib = _lib.load()
-    M, K = (a.shape[1], a.shape[0]) if a_trans else a.shape
-    N = b.shape[0] if b_trans else b.shape[1]
-    c = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-    ws_b = lib.alg_ffn_gemm_workspace_size(M, N, K)
-    ws = torch.empty(max(ws_b, 1), dtype=torch.uint8, device=a.device)
-    _lib.check(lib.alg_ffn_gemm(_lib.stream_of(a), M, N, K, _lib.ptr(a), a.shape[1], int(a_trans), _lib.ptr(b),
-                                b.shape[1], int(b_trans), _lib.ptr(c), N, _lib.ptr(ws), ws_b), "alu_glu_ffn product")
-    return c
+_DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float32: _lib.DTYPE_F32}
+
+
+def _weight(w):
+    """``w`` as the library reads it (bf16 or f32, contiguous, aligned) and its dtype code."""
+    if w.dtype not in _DTYPES:
+        w = w.to(torch.bfloat16)
+    return _lib.aligned16(w), _DTYPES[w.dtype]
+
+
+def _grad_like(w_dtype, rows, cols, dev):
+    """An empty weight gradient in the weight's dtype (bf16 where the library writes no other)."""
+    dt = w_dtype if w_dtype in _DTYPES else torch.bfloat16
+    return torch.empty((rows, cols), dtype=dt, device=dev), _DTYPES[dt]
 
 
 class _FfnFn(torch.autograd.Function):
@@ -39,32 +42,41 @@ class _FfnFn(torch.autograd.Function):
         shape = h2.shape
         d = shape[-1]
         x = _lib.aligned16(h2).reshape(-1, d)
-        N, F = x.shape[0], w_g.shape[1]
-        w_gu = torch.cat([w_g, w_u], dim=1).to(torch.bfloat16).contiguous()
-        wd = _lib.aligned16(w_d.to(torch.bfloat16))
-        y, gate, up = (torch.empty((N, F), dtype=torch.bfloat16, device=x.device) for _ in range(3))
-        _lib.check(lib.alg_ffn_alu_glu_fwd(_lib.stream_of(x), N, d, F, _lib.ptr(x), _lib.ptr(w_gu), float(beta),
-                                           _lib.ptr(y), _lib.ptr(gate), _lib.ptr(up)), "alu_glu_ffn")
-        out = _gemm(y, wd)
-        ctx.save_for_backward(x, w_gu, wd, y, gate, up)
+        dev, bf = x.device, torch.bfloat16
+        N, F, dm = x.shape[0], w_g.shape[1], w_d.shape[1]
+        (wg, gt), (wu, ut), (wd, dt) = _weight(w_g), _weight(w_u), _weight(w_d)
+        w_gu = torch.empty((d, 2 * F), dtype=bf, device=dev)
+        wd16 = torch.empty((F, dm), dtype=bf, device=dev) if dt == _lib.DTYPE_F32 else None
+        y, gate, up = (torch.empty((N, F), dtype=bf, device=dev) for _ in range(3))
+        out = torch.empty((N, dm), dtype=bf, device=dev)
+        nbytes = lib.alg_ffn_block_workspace_size(N, d, F, dm, 0)
+        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
+        p = _lib.ptr
+        _lib.check(lib.alg_ffn_block_fwd(_lib.stream_of(x), N, d, F, dm, p(x), p(wg), gt, p(wu), ut, p(wd), dt,
+                                         float(beta), p(w_gu), p(wd16), p(y), p(gate), p(up), p(out), p(ws), nbytes),
+                   "alu_glu_ffn")
+        ctx.save_for_backward(x, w_gu, wd if wd16 is None else wd16, y, gate, up)
         ctx.meta = (shape, beta, w_g.dtype, w_u.dtype, w_d.dtype)
-        return out.reshape(*shape[:-1], wd.shape[1])
+        return out.reshape(*shape[:-1], dm)
 
     @staticmethod
     def backward(ctx, dout):
         x, w_gu, wd, y, gate, up = ctx.saved_tensors
         shape, beta, tg, tu, td = ctx.meta
         lib = _lib.load()
+        dev = x.device
         N, d = x.shape
         F, dm = wd.shape
         do = _lib.aligned16(dout.to(torch.bfloat16)).reshape(N, dm)
-        d_gu = torch.empty((N, 2 * F), dtype=torch.bfloat16, device=x.device)
-        _lib.check(lib.alg_ffn_alu_glu_dy(_lib.stream_of(x), N, dm, F, _lib.ptr(do), _lib.ptr(wd), _lib.ptr(gate),
-                                          _lib.ptr(up), float(beta), _lib.ptr(d_gu)), "alu_glu_ffn backward")
-        dh2 = _gemm(d_gu, w_gu, b_trans=True).reshape(shape)
-        dw_gu = _gemm(x, d_gu, a_trans=True)
-        dw_d = _gemm(y, do, a_trans=True)
-        return dh2, dw_gu[:, :F].to(tg), dw_gu[:, F:].to(tu), dw_d.to(td), None
+        dx = torch.empty_like(x)
+        (dwg, gt), (dwu, ut), (dwd, dt) = (_grad_like(t, r, c, dev) for t, r, c in ((tg, d, F), (tu, d, F), (td, F, dm)))
+        nbytes = lib.alg_ffn_block_workspace_size(N, d, F, dm, 1)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        p = _lib.ptr
+        _lib.check(lib.alg_ffn_block_bwd(_lib.stream_of(x), N, d, F, dm, p(x), p(w_gu), p(wd), p(y), p(gate), p(up),
+                                         p(do), float(beta), p(dx), p(dwg), gt, p(dwu), ut, p(dwd), dt, p(ws), nbytes),
+                   "alu_glu_ffn backward")
+        return dx.reshape(shape), dwg.to(tg), dwu.to(tu), dwd.to(td), None
 
 
 def alu_glu_ffn(h2, w_g, w_u, w_d, beta: float = 0.5):

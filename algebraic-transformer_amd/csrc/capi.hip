@@ -804,21 +804,27 @@ size_t alg_ffn_gemm_workspace_size(int M, int N, int K) {
   return alg::ffn_gemm_plan(M, N, K).ws_bytes;
 }
 
-int alg_ffn_gemm(alg_stream_t stream, int M, int N, int K, const void* A, long lda, int a_trans, const void* B,
-                 long ldb, int b_trans, void* C, long ldc, void* workspace, size_t workspace_bytes) {
-  if (M <= 0 || N <= 0 || K <= 0) return fail(ALG_ERR_INVALID, "M, N, K must be positive (got %d, %d, %d)", M, N, K);
-  if (!A || !B || !C) return fail(ALG_ERR_INVALID, "null argument");
-  if (!aligned16({A, B, C})) return fail(ALG_ERR_INVALID, "A, B and C must be 16-byte aligned");
+// Where a product's columns go: all of them, or those below n2, to C, the others to C2.
+struct FfnOut {
+  void* C;
+  int c_f32;
+  void* C2;
+  int c2_f32, n2;
+  long ldc;
+};
+static int ffn_product(alg_stream_t stream, int M, int N, int K, const void* A, long lda, int a_trans, const void* B,
+                       long ldb, int b_trans, const FfnOut& out, void* workspace, size_t workspace_bytes,
+                       const char* what) {
   // Stored row lengths: A (M, K) or (K, M); B (K, N) or (N, K).
   const int a_cols = a_trans ? M : K, a_rows = a_trans ? K : M;
   const int b_cols = b_trans ? K : N, b_rows = b_trans ? N : K;
   if (a_cols % 8 || b_cols % 8 || N % 8)
     return fail(ALG_ERR_INVALID, "stored row lengths (%d, %d) and N = %d must be multiples of 8", a_cols, b_cols, N);
-  if (lda < a_cols || ldb < b_cols || ldc < N || lda % 8 || ldb % 8 || ldc % 8)
+  if (lda < a_cols || ldb < b_cols || out.ldc < out.n2 || lda % 8 || ldb % 8 || out.ldc % 8)
     return fail(ALG_ERR_INVALID, "leading dimensions (%ld, %ld, %ld) must cover the rows and be multiples of 8", lda,
-                ldb, ldc);
+                ldb, out.ldc);
   if ((double)(a_rows - 1) * lda + a_cols > 2.0e9 || (double)(b_rows - 1) * ldb + b_cols > 2.0e9 ||
-      (double)(M - 1) * ldc + N > 2.0e9)
+      (double)(M - 1) * out.ldc + N > 2.0e9)
     return fail(ALG_ERR_INVALID, "matrices too large");
   const alg::FfnGemmPlan pl = alg::ffn_gemm_plan(M, N, K);
   const size_t need = pl.ws_bytes;
@@ -829,15 +835,113 @@ int alg_ffn_gemm(alg_stream_t stream, int M, int N, int K, const void* A, long l
   std::memset(&g, 0, sizeof g);
   g.A = alg::GemmOperand{static_cast<const bf16*>(A), lda, a_rows, a_cols, (long)(a_rows - 1) * lda + a_cols};
   g.B = alg::GemmOperand{static_cast<const bf16*>(B), ldb, b_rows, b_cols, (long)(b_rows - 1) * ldb + b_cols};
-  g.C = static_cast<bf16*>(C);
-  g.ldc = ldc;
+  g.C = out.C; g.c_f32 = out.c_f32; g.C2 = out.C2; g.c2_f32 = out.c2_f32; g.n2 = out.n2; g.ldc = out.ldc;
   g.M = M; g.N = N; g.K = K;
   g.tile = pl.tile; g.full = pl.full; g.split = pl.split; g.kchunk = pl.kchunk;
   g.part = need ? static_cast<float*>(workspace) : nullptr;
   // A stored (M, K) is k-contiguous; B stored (N, K) is k-contiguous.
   return hip_status(alg::launch_ffn_gemm(g, a_trans ? alg::MNMAJOR : alg::KMAJOR, b_trans ? alg::KMAJOR : alg::MNMAJOR,
                                          (hipStream_t)stream),
-                    "alg_ffn_gemm");
+                    what);
+}
+
+int alg_ffn_gemm(alg_stream_t stream, int M, int N, int K, const void* A, long lda, int a_trans, const void* B,
+                 long ldb, int b_trans, void* C, long ldc, void* workspace, size_t workspace_bytes) {
+  if (M <= 0 || N <= 0 || K <= 0) return fail(ALG_ERR_INVALID, "M, N, K must be positive (got %d, %d, %d)", M, N, K);
+  if (!A || !B || !C) return fail(ALG_ERR_INVALID, "null argument");
+  if (!aligned16({A, B, C})) return fail(ALG_ERR_INVALID, "A, B and C must be 16-byte aligned");
+  return ffn_product(stream, M, N, K, A, lda, a_trans, B, ldb, b_trans, FfnOut{C, 0, nullptr, 0, N, ldc}, workspace,
+                     workspace_bytes, "alg_ffn_gemm");
+}
+
+// Whole block. Backward workspace: [d_gu bf16 N*2F][f32 tiles of the largest split product].
+struct FfnBlockWs {
+  size_t part, total;
+};
+static FfnBlockWs ffn_block_ws(int N, int d, int F, int dm, bool backward) {
+  FfnBlockWs w;
+  w.part = backward ? align256((size_t)N * 2 * F * 2) : 0;
+  w.total = w.part;
+  auto product = [&](int m, int n, int k) { w.total = std::max(w.total, w.part + alg::ffn_gemm_plan(m, n, k).ws_bytes); };
+  if (!backward) {
+    product(N, dm, F);
+  } else {
+    product(N, d, 2 * F);
+    product(d, 2 * F, N);
+    product(F, dm, N);
+  }
+  return w;
+}
+
+static int check_ffn_block(int N, int d, int F, int dm) {
+  if (dm <= 0 || dm % 8) return fail(ALG_ERR_INVALID, "output width %d must be a positive multiple of 8", dm);
+  return check_ffn(N, d, F);
+}
+
+static bool is_weight_dtype(int dt) { return dt == ALG_DTYPE_BF16 || dt == ALG_DTYPE_F32; }
+
+size_t alg_ffn_block_workspace_size(int N, int d, int F, int dm, int backward) {
+  if (N <= 0 || d <= 0 || F <= 0 || dm <= 0) return 0;
+  return ffn_block_ws(N, d, F, dm, backward != 0).total;
+}
+
+int alg_ffn_block_fwd(alg_stream_t stream, int N, int d, int F, int dm, const void* x, const void* w_g, int g_dtype,
+                      const void* w_u, int u_dtype, const void* w_d, int d_dtype, float beta, void* w_gu, void* w_d16,
+                      void* y, void* gate, void* up, void* out, void* workspace, size_t workspace_bytes) {
+  int rc = check_ffn_block(N, d, F, dm);
+  if (rc) return rc;
+  if (!x || !w_g || !w_u || !w_d || !w_gu || !y || !gate || !up || !out) return fail(ALG_ERR_INVALID, "null argument");
+  if (!is_weight_dtype(g_dtype) || !is_weight_dtype(u_dtype) || !is_weight_dtype(d_dtype))
+    return fail(ALG_ERR_INVALID, "weights must be bf16 or f32");
+  if (d_dtype == ALG_DTYPE_F32 && !w_d16) return fail(ALG_ERR_INVALID, "f32 w_d needs w_d16");
+  if (!aligned16({x, w_g, w_u, w_d, w_gu, w_d16, y, gate, up, out, workspace}))
+    return fail(ALG_ERR_INVALID, "matrices must be 16-byte aligned");
+  if (!std::isfinite(beta)) return fail(ALG_ERR_INVALID, "beta must be finite");
+  const FfnBlockWs ws = ffn_block_ws(N, d, F, dm, false);
+  if (ws.total && (!workspace || workspace_bytes < ws.total))
+    return fail(ALG_ERR_INVALID, "workspace too small: need %zu bytes", ws.total);
+  alg::FfnPackParams p;
+  std::memset(&p, 0, sizeof p);
+  p.w_g = w_g; p.w_u = w_u; p.w_d = w_d;
+  p.w_gu = static_cast<bf16*>(w_gu);
+  p.w_d16 = static_cast<bf16*>(w_d16);
+  p.g_f32 = g_dtype == ALG_DTYPE_F32; p.u_f32 = u_dtype == ALG_DTYPE_F32; p.d_f32 = d_dtype == ALG_DTYPE_F32;
+  p.d = d; p.F = F; p.dm = dm;
+  rc = hip_status(alg::launch_ffn_pack(p, (hipStream_t)stream), "alg_ffn_block_fwd");
+  if (!rc) rc = alg_ffn_alu_glu_fwd(stream, N, d, F, x, w_gu, beta, y, gate, up);
+  if (rc) return rc;
+  return ffn_product(stream, N, dm, F, y, F, 0, w_d16 ? w_d16 : w_d, dm, 0, FfnOut{out, 0, nullptr, 0, dm, dm},
+                     workspace, workspace_bytes, "alg_ffn_block_fwd");
+}
+
+int alg_ffn_block_bwd(alg_stream_t stream, int N, int d, int F, int dm, const void* x, const void* w_gu,
+                      const void* w_d16, const void* y, const void* gate, const void* up, const void* dout, float beta,
+                      void* dx, void* dw_g, int g_dtype, void* dw_u, int u_dtype, void* dw_d, int d_dtype,
+                      void* workspace, size_t workspace_bytes) {
+  int rc = check_ffn_block(N, d, F, dm);
+  if (rc) return rc;
+  if (!x || !w_gu || !w_d16 || !y || !gate || !up || !dout || !dx || !dw_g || !dw_u || !dw_d)
+    return fail(ALG_ERR_INVALID, "null argument");
+  if (!is_weight_dtype(g_dtype) || !is_weight_dtype(u_dtype) || !is_weight_dtype(d_dtype))
+    return fail(ALG_ERR_INVALID, "weight gradients must be bf16 or f32");
+  if (!aligned16({x, w_gu, w_d16, y, gate, up, dout, dx, dw_g, dw_u, dw_d, workspace}))
+    return fail(ALG_ERR_INVALID, "matrices must be 16-byte aligned");
+  const FfnBlockWs ws = ffn_block_ws(N, d, F, dm, true);
+  if (!workspace || workspace_bytes < ws.total)
+    return fail(ALG_ERR_INVALID, "workspace too small: need %zu bytes", ws.total);
+  char* w = static_cast<char*>(workspace);
+  void* part = w + ws.part;
+  const size_t part_bytes = workspace_bytes - ws.part;
+  const char* what = "alg_ffn_block_bwd";
+  rc = alg_ffn_alu_glu_dy(stream, N, dm, F, dout, w_d16, gate, up, beta, w);
+  if (!rc) rc = ffn_product(stream, N, d, 2 * F, w, 2L * F, 0, w_gu, 2L * F, 1, FfnOut{dx, 0, nullptr, 0, d, d}, part,
+                            part_bytes, what);
+  if (!rc) rc = ffn_product(stream, d, 2 * F, N, x, d, 1, w, 2L * F, 0,
+                            FfnOut{dw_g, g_dtype == ALG_DTYPE_F32, dw_u, u_dtype == ALG_DTYPE_F32, F, F}, part,
+                            part_bytes, what);
+  if (!rc) rc = ffn_product(stream, F, dm, N, y, F, 1, dout, dm, 0,
+                            FfnOut{dw_d, d_dtype == ALG_DTYPE_F32, nullptr, 0, dm, dm}, part, part_bytes, what);
+  return rc;
 }
 
 int alg_head_eval(alg_stream_t stream, int dtype, int N, int d, int V, const void* h, const void* E,

@@ -66,6 +66,33 @@ __device__ __forceinline__ void ffn_tile(const GemmOperand& A, const GemmOperand
 
 }  // namespace
 
+// The weights in bf16, [w_g | w_u] side by side: one pass in place of a concatenation, its
+// conversion and w_d's (bound by memory; f32 weights of d 768, d_ff 2048: 20 us of three kernels,
+// FFN_PACK_US us so).
+__global__ __launch_bounds__(256) void ffn_pack_kernel(FfnPackParams p) {
+  const int n1 = p.d * (p.F / 8), n2 = p.w_d16 ? p.F * (p.dm / 8) : 0;  // 8-element chunks
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < 2 * n1 + n2; i += gridDim.x * 256) {
+    const int part = i < n1 ? 0 : i < 2 * n1 ? 1 : 2;
+    const int c = i - part * n1;
+    const void* src = part == 0 ? p.w_g : part == 1 ? p.w_u : p.w_d;
+    bf16x8 v;
+    if (part == 0 ? p.g_f32 : part == 1 ? p.u_f32 : p.d_f32) {
+      const floatx4 x = static_cast<const floatx4*>(src)[2 * (size_t)c], y = static_cast<const floatx4*>(src)[2 * (size_t)c + 1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = f2bf(x[e]);
+        v[4 + e] = f2bf(y[e]);
+      }
+    } else {
+      v = static_cast<const bf16x8*>(src)[c];
+    }
+    const int row = c / (p.F / 8);
+    bf16* dst = part == 2 ? p.w_d16 + 8 * (size_t)c
+                          : p.w_gu + (size_t)row * 2 * p.F + part * p.F + 8 * (c - row * (p.F / 8));
+    *reinterpret_cast<bf16x8*>(dst) = v;
+  }
+}
+
 template <class C>
 __global__ __launch_bounds__(C::THREADS, 2) void ffn_gate_up_kernel(FfnParams p) {
   const int nbm = (p.N + C::TM - 1) / C::TM, nbn = 2 * p.F / C::TN;
@@ -220,6 +247,25 @@ __global__ __launch_bounds__(C::THREADS, 2) void ffn_gemm_kernel(FfnGemmParams g
         }
       return;
     }
+    // n2 is a multiple of 64, so a wave's columns lie on one side of it.
+    const int mw = m0 + wm * C::WTM, nw = n0 + wn * W;
+    const bool second = nw >= g.n2;
+    const int nc = second ? nw - g.n2 : nw, ncols = second ? g.N - g.n2 : g.n2;
+    void* base = second ? g.C2 : g.C;
+    if (second ? g.c2_f32 : g.c_f32) {
+      float* out = static_cast<float*>(base) + (size_t)mw * g.ldc + nc;
+#pragma unroll
+      for (int mb = 0; mb < C::MB; ++mb) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int row = mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+#pragma unroll
+          for (int nb = 0; nb < C::NB; ++nb)
+            if (mw + row < g.M && nc + nb * 32 + l32 < ncols) out[(size_t)row * g.ldc + nb * 32 + l32] = acc[mb][nb][i];
+        }
+      }
+      return;
+    }
     // Staged 16-byte row stores; N is a multiple of 8, so a chunk lies inside a row or past it.
 #pragma unroll
     for (int mb = 0; mb < C::MB; ++mb) {
@@ -230,13 +276,12 @@ __global__ __launch_bounds__(C::THREADS, 2) void ffn_gemm_kernel(FfnGemmParams g
         for (int nb = 0; nb < C::NB; ++nb) stg[stage_at<W>(row, nb * 32 + l32)] = f2bf(acc[mb][nb][i]);
       }
     }
-    const int mw = m0 + wm * C::WTM, nw = n0 + wn * W;
-    bf16* out = g.C + (size_t)mw * g.ldc + nw;
+    bf16* out = static_cast<bf16*>(base) + (size_t)mw * g.ldc + nc;
     const bool inside = m0 + C::TM <= g.M && n0 + C::TN <= g.N;
 #pragma unroll 4
     for (int it = 0; it < C::WTM * CH / 64; ++it) {
       const int idx = it * 64 + lane, row = idx / CH, ch = idx % CH;
-      if (inside || (mw + row < g.M && nw + 8 * ch < g.N))
+      if (inside || (mw + row < g.M && nc + 8 * ch < ncols))
         *reinterpret_cast<bf16x8*>(out + (size_t)row * g.ldc + 8 * ch) =
             *reinterpret_cast<const bf16x8*>(stg + stage_at<W>(row, 8 * ch));
     }
@@ -266,11 +311,20 @@ __global__ __launch_bounds__(256) void ffn_gemm_tail_kernel(FfnGemmParams g) {
       a.x += x.x; a.y += x.y; a.z += x.z; a.w += x.w;
       b.x += y.x; b.y += y.y; b.z += y.z; b.w += y.w;
     }
+    const bool second = n >= g.n2;
+    const size_t at = (size_t)m * g.ldc + (second ? n - g.n2 : n);
+    void* base = second ? g.C2 : g.C;
+    if (second ? g.c2_f32 : g.c_f32) {
+      float4* out = reinterpret_cast<float4*>(static_cast<float*>(base) + at);
+      out[0] = a;
+      out[1] = b;
+      continue;
+    }
     const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
     bf16x8 o8;
 #pragma unroll
     for (int t = 0; t < 8; ++t) o8[t] = f2bf(v[t]);
-    *reinterpret_cast<bf16x8*>(g.C + (size_t)m * g.ldc + n) = o8;
+    *reinterpret_cast<bf16x8*>(static_cast<bf16*>(base) + at) = o8;
   }
 }
 
@@ -365,6 +419,13 @@ hipError_t launch_ffn_gemm(const FfnGemmParams& g, int a_mode, int b_mode, hipSt
   if (g.tile == 64) launch_ffn_gemm_cfg<FC64>(g, a_mode, b_mode, st);
   else if (g.tile == 128) launch_ffn_gemm_cfg<FC128>(g, a_mode, b_mode, st);
   else launch_ffn_gemm_cfg<FC>(g, a_mode, b_mode, st);
+  return hipGetLastError();
+}
+
+hipError_t launch_ffn_pack(const FfnPackParams& p, hipStream_t st) {
+  const long chunks = 2L * p.d * (p.F / 8) + (p.w_d16 ? (long)p.F * (p.dm / 8) : 0);
+  KTimer t("ffn_pack", st);
+  hipLaunchKernelGGL(ffn_pack_kernel, dim3((int)std::min(2048L, (chunks + 255) / 256)), dim3(256), 0, st, p);
   return hipGetLastError();
 }
 

@@ -88,10 +88,24 @@ struct FfnParams {
   float beta;
 };
 
+// The block's weights as its products read them: w_gu (d, 2F) = [w_g | w_u] and w_d16 (F, dm), in
+// bf16, from weights in bf16 or f32.
+struct FfnPackParams {
+  const void *w_g, *w_u, *w_d;
+  bf16* w_gu;
+  bf16* w_d16;          // or nullptr (w_d is bf16 and read in place)
+  int g_f32, u_f32, d_f32;
+  int d, F, dm;
+};
+
 // Plain bf16 products of the feed-forward block: C (M, N) row-major = A B, f32 accumulation.
+// Columns from n2 on (a multiple of 64) belong to C2; each part is bf16, or f32 (the sum itself).
 struct FfnGemmParams {
   GemmOperand A, B;     // A: M x K, B: K x N, each k- or m/n-contiguous as stored
-  bf16* C;              // (M, ldc)
+  void* C;              // (M, ldc): columns below n2
+  void* C2;             // (M, ldc): columns n2 .. N - 1 (n2 == N: none)
+  int c_f32, c2_f32;
+  int n2;
   long ldc;
   int M, N, K;
   float* part;          // f32 tiles of the split tiles (ffn_gemm_plan), or nullptr

@@ -81,6 +81,7 @@ int rms_norm_max_d();
 int rms_norm_blocks(int rows);
 int rms_norm_gain_groups(int rows);
 hipError_t launch_rms_norm_fwd(const RmsNormParams& p, hipStream_t st);
+hipError_t launch_ffn_pack(const FfnPackParams& p, hipStream_t st);
 hipError_t launch_ffn_fwd(const FfnParams& p, hipStream_t st);
 hipError_t launch_ffn_dy(const FfnParams& p, hipStream_t st);
 struct FfnGemmPlan {

@@ -261,6 +261,22 @@ size_t alg_ffn_gemm_workspace_size(int M, int N, int K);
 int alg_ffn_gemm(alg_stream_t stream, int M, int N, int K, const void* A, long lda, int a_trans, const void* B,
                  long ldb, int b_trans, void* C, long ldc, void* workspace, size_t workspace_bytes);
 
+/* The whole block, (x w_g alu(x w_u, beta)) w_d, model.py:185-193 with ffn = "alu_glu". x, y, gate,
+ * up, out, dout, dx in bf16; each weight, and its gradient, in bf16 or f32 (ALG_DTYPE_*): the products
+ * run in bf16 (the cast of the reference's compute dtype), an f32 gradient is the f32 sum.
+ * Forward: writes w_gu (d, 2F) = bf16 [w_g | w_u], w_d16 (F, dm) = bf16 w_d (NULL if w_d is bf16 and
+ * read in place), y, gate, up (N, F) and out (N, dm). Backward: reads what the forward wrote (w_d16:
+ * bf16 w_d) and dout (N, dm); writes dx (N, d), dw_g, dw_u (d, F) and dw_d (F, dm). Every matrix is
+ * row-major, contiguous and 16-byte aligned; workspace: alg_ffn_block_workspace_size bytes. */
+size_t alg_ffn_block_workspace_size(int N, int d, int F, int dm, int backward);
+int alg_ffn_block_fwd(alg_stream_t stream, int N, int d, int F, int dm, const void* x, const void* w_g, int g_dtype,
+                      const void* w_u, int u_dtype, const void* w_d, int d_dtype, float beta, void* w_gu,
+                      void* w_d16, void* y, void* gate, void* up, void* out, void* workspace, size_t workspace_bytes);
+int alg_ffn_block_bwd(alg_stream_t stream, int N, int d, int F, int dm, const void* x, const void* w_gu,
+                      const void* w_d16, const void* y, const void* gate, const void* up, const void* dout, float beta,
+                      void* dx, void* dw_g, int g_dtype, void* dw_u, int u_dtype, void* dw_d, int d_dtype,
+                      void* workspace, size_t workspace_bytes);
+
 /* Head backward, fused_head.py:120-156, 194-216, 247-254:
  * in h, E (of dtype ALG_DTYPE_BF16 or ALG_DTYPE_F32), targets, stat, g (1) f32 on the device
  * (cotangent of obj) and optionally the forward's residual (bf16 only); out dh (N,d) in h's

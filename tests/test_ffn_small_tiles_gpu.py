@@ -38,22 +38,32 @@ def test_small_products(M, N, K, a_trans, b_trans):
     assert bool(c[M].isnan().all())  # nothing past the last row
 
 
+@pytest.mark.parametrize("dtypes", ["bbb", "fff", "bfb", "fbf"])
 @pytest.mark.parametrize("N,d,F", [(1, 64, 128), (64, 72, 128), (65, 128, 256), (129, 192, 640), (1000, 256, 1024),
                                    (1025, 320, 2048)])
-def test_small_block(N, d, F):
+def test_small_block(N, d, F, dtypes):
+    """Weights in bf16 (b) or f32 (f): the products run on their bf16 values, an f32 weight's gradient
+    is the f32 sum, which the oracle rounds to bf16."""
     from algebraic_amd.kernels.ffn import alu_glu_ffn
     from oracle import ffn as OF
     from oracle.numerics import round_bf16
-    print(f"[ffn small block] N={N} d={d} F={F}", flush=True)
+    print(f"[ffn small block] N={N} d={d} F={F} {dtypes}", flush=True)
     rng = np.random.default_rng(N + d + F)
     mk = lambda *s: round_bf16(rng.standard_normal(s).astype(np.float32) / np.sqrt(s[0] if len(s) == 2 else 1))
     x = round_bf16(rng.standard_normal((N, d)).astype(np.float32))
     do = round_bf16(rng.standard_normal((N, d)).astype(np.float32))
     wg, wu, wd = mk(d, F), mk(d, F), mk(F, d)
-    tx, tg, tu, td = (torch.tensor(a, device="cuda").to(torch.bfloat16).requires_grad_(True) for a in (x, wg, wu, wd))
+    dt = {"b": torch.bfloat16, "f": torch.float32}
+    tx, tg, tu, td = (torch.tensor(a, device="cuda").to(dt[c]).requires_grad_(True)
+                      for a, c in zip((x, wg, wu, wd), "b" + dtypes))
+    with torch.no_grad():  # f32 weights that bf16 does not hold
+        for w in (tg, tu, td):
+            if w.dtype == torch.float32:
+                w.mul_(1 + 2.0 ** -12)
     y = alu_glu_ffn(tx, tg, tu, td)
     got = [y.detach(), *torch.autograd.grad(y, (tx, tg, tu, td), torch.tensor(do, device="cuda").to(torch.bfloat16))]
     out, *_ = OF.ffn_forward(x, wg, wu, wd)
     want = [out, *OF.ffn_backward(x, wg, wu, wd, do)[:4]]
-    for name, a, b in zip(("out", "dx", "dw_g", "dw_u", "dw_d"), got, want):
+    for name, a, b, w in zip(("out", "dx", "dw_g", "dw_u", "dw_d"), got, want, (tx, tx, tg, tu, td)):
+        assert a.dtype == w.dtype and a.is_contiguous()
         assert rel_l2(a.float().cpu().numpy(), b) < 1e-2, name
