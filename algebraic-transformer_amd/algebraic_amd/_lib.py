@@ -35,6 +35,8 @@ _SIGNATURES = {
                                   _P, _S]),
     "alg_attn_bwd": (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _F, _I, _I, _F,
                           _P, _P, _P, _P, _P, _P, _S]),
+    "alg_attn_bwd_sink_logit": (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _F, _I, _I,
+                                     _F, _F, _P, _P, _P, _P, _P, _P, _S]),
     "alg_attn_bwd_noalloc": (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _F, _I, _I,
                                   _F, _P, _P, _P, _P, _P]),
     "alg_attn_prologue_workspace_size": (_S, [_I, _I, _I, _I]),
@@ -134,10 +136,18 @@ def aligned16(t):
 
 
 def ptr(t):
-    """Device pointer of a tensor (or None)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """Device pointer of a tensor (or None), as an integer: the declared argument types make it a
+    void pointer, without a ctypes object per argument."""
+    return None if t is None else t.data_ptr()
 
 
 def stream_of(t):
+    """Handle of the current stream on ``t``'s device, without a torch Stream object (which took
+    2 to 13 us to make, in the backward's thread above all)."""
     import torch
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+def align256(nbytes):
+    """The next multiple of 256: parts of one scratch allocation start there."""
+    return (nbytes + 255) & ~255

@@ -35,6 +35,12 @@ def _grad_like(w_dtype, rows, cols, dev):
     return torch.empty((rows, cols), dtype=dt, device=dev), _DTYPES[dt]
 
 
+def _parts(act):
+    """Pointers of the three (N, F) bf16 matrices of one (3, N, F) allocation."""
+    base, step = act.data_ptr(), act.numel() // 3 * 2
+    return base, base + step, base + 2 * step
+
+
 class _FfnFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, h2, w_g, w_u, w_d, beta):
@@ -47,21 +53,21 @@ class _FfnFn(torch.autograd.Function):
         (wg, gt), (wu, ut), (wd, dt) = _weight(w_g), _weight(w_u), _weight(w_d)
         w_gu = torch.empty((d, 2 * F), dtype=bf, device=dev)
         wd16 = torch.empty((F, dm), dtype=bf, device=dev) if dt == _lib.DTYPE_F32 else None
-        y, gate, up = (torch.empty((N, F), dtype=bf, device=dev) for _ in range(3))
+        act = torch.empty((3, N, F), dtype=bf, device=dev)  # y, gate, up
         out = torch.empty((N, dm), dtype=bf, device=dev)
         nbytes = lib.alg_ffn_block_workspace_size(N, d, F, dm, 0)
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
         p = _lib.ptr
         _lib.check(lib.alg_ffn_block_fwd(_lib.stream_of(x), N, d, F, dm, p(x), p(wg), gt, p(wu), ut, p(wd), dt,
-                                         float(beta), p(w_gu), p(wd16), p(y), p(gate), p(up), p(out), p(ws), nbytes),
+                                         float(beta), p(w_gu), p(wd16), *_parts(act), p(out), p(ws), nbytes),
                    "alu_glu_ffn")
-        ctx.save_for_backward(x, w_gu, wd if wd16 is None else wd16, y, gate, up)
+        ctx.save_for_backward(x, w_gu, wd if wd16 is None else wd16, act)
         ctx.meta = (shape, beta, w_g.dtype, w_u.dtype, w_d.dtype)
         return out.reshape(*shape[:-1], dm)
 
     @staticmethod
     def backward(ctx, dout):
-        x, w_gu, wd, y, gate, up = ctx.saved_tensors
+        x, w_gu, wd, act = ctx.saved_tensors
         shape, beta, tg, tu, td = ctx.meta
         lib = _lib.load()
         dev = x.device
@@ -73,8 +79,8 @@ class _FfnFn(torch.autograd.Function):
         nbytes = lib.alg_ffn_block_workspace_size(N, d, F, dm, 1)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         p = _lib.ptr
-        _lib.check(lib.alg_ffn_block_bwd(_lib.stream_of(x), N, d, F, dm, p(x), p(w_gu), p(wd), p(y), p(gate), p(up),
-                                         p(do), float(beta), p(dx), p(dwg), gt, p(dwu), ut, p(dwd), dt, p(ws), nbytes),
+        _lib.check(lib.alg_ffn_block_bwd(_lib.stream_of(x), N, d, F, dm, p(x), p(w_gu), p(wd), *_parts(act), p(do),
+                                         float(beta), p(dx), p(dwg), gt, p(dwu), ut, p(dwd), dt, p(ws), nbytes),
                    "alu_glu_ffn backward")
         return dx.reshape(shape), dwg.to(tg), dwu.to(tu), dwd.to(td), None
 

@@ -95,6 +95,64 @@ class _Plan(NamedTuple):
     layout: int = 0     # _lib.LAYOUT_BHTD or _lib.LAYOUT_BTHD
 
 
+def _sink_input(sink_logit, H, dev):
+    """The sink logits as (1,) or (H,) f32 on ``dev`` (flash.py:826-828), or None."""
+    if sink_logit is None:
+        return None
+    s = sink_logit.detach()
+    if s.dtype != torch.float32 or s.device != dev:
+        s = s.to(device=dev, dtype=torch.float32)
+    s = s.reshape(-1).contiguous()
+    if s.numel() not in (1, H):
+        raise ValueError(f"sink_logit must broadcast to ({H},)")
+    return s
+
+
+def _row_state(B, H, T, dev):
+    """One f32 allocation for the forward's per-row statistic (B H T), sink/c (H) and guard flag
+    (one int32), which the backward reads, and the pointers of the three."""
+    aux = torch.empty(B * H * T + H + 1, dtype=torch.float32, device=dev)
+    return aux, *_row_state_ptrs(aux, B, H, T)
+
+
+def _row_state_ptrs(aux, B, H, T):
+    base = aux.data_ptr()
+    return base, base + 4 * B * H * T, base + 4 * (B * H * T + H)
+
+
+def _attn_backward(plan, q_s, k, v, o, aux, do, has_sink, what):
+    """dq, dk, dv and the sink logits' gradient (H,) f32 or None, for the cotangent ``do``."""
+    B, H, T, D = _bhtd(q_s.shape, plan.layout)
+    lib = _lib.load()
+    dt = _DTYPES[q_s.dtype]
+    dev = q_s.device
+    if do.dtype != q_s.dtype:
+        do = do.to(q_s.dtype)
+    do = _lib.aligned16(do)
+    stat, sink, flag = _row_state_ptrs(aux, B, H, T)
+    ws_bytes = lib.alg_attn_workspace_size(dt, B, H, T, D)
+    di = _lib.align256(ws_bytes)
+    ws = torch.empty(di + 4 * B * H * T, dtype=torch.uint8, device=dev)  # workspace, then di
+    dq, dk, dv = torch.empty_like(q_s), torch.empty_like(k), torch.empty_like(v)
+    dsink = torch.empty(H, dtype=torch.float32, device=dev) if has_sink else None
+    p = _lib.ptr
+    _lib.check(lib.alg_attn_bwd_sink_logit(
+        _lib.stream_of(q_s), dt, plan.layout, B, H, T, D, p(q_s), p(k), p(v), sink if has_sink else None, p(o), stat,
+        p(do), plan.n, plan.variant, flag, plan.clamp, int(plan.fast_rho), int(plan.inv_stat),
+        1.0 / (math.sqrt(D) * plan.c), plan.c, p(dq), p(dk), p(dv), p(ws) + di, p(dsink), p(ws), ws_bytes), what)
+    return dq, dk, dv, dsink
+
+
+def _sink_gradient(dsink, shape, dtype):
+    """The gradient of a sink given as ``shape`` (broadcast over the heads where it has one entry)."""
+    if dsink is None:
+        return None
+    numel = math.prod(shape) if shape else 1
+    if numel != dsink.numel():
+        dsink = dsink.sum()
+    return dsink.reshape(shape).to(dtype)
+
+
 class _FlashFn(torch.autograd.Function):
     """Custom VJP of flash.py:708-729 over the HIP kernels."""
 
@@ -107,71 +165,38 @@ class _FlashFn(torch.autograd.Function):
         st = _lib.stream_of(q)
         q, k, v = _lib.aligned16(q), _lib.aligned16(k), _lib.aligned16(v)
         has_sink = sink_logit is not None
-        sink_in = None
-        if has_sink:
-            sink_in = sink_logit.detach().to(device=dev, dtype=torch.float32).reshape(-1).contiguous()
-            if sink_in.numel() not in (1, H):
-                raise ValueError(f"sink_logit must broadcast to ({H},)")
+        sink_in = _sink_input(sink_logit, H, dev)
+        nsink = sink_in.numel() if has_sink else 0
         ws_bytes = lib.alg_attn_workspace_size(dt, B, H, T, D)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        q_s = torch.empty_like(q)
-        sink = torch.empty(H, dtype=torch.float32, device=dev) if has_sink else None
-        flag = torch.empty(1, dtype=torch.int32, device=dev)
-        o = torch.empty_like(q)
-        stat = torch.empty((B, H, T), dtype=torch.float32, device=dev)
-        nsink = sink_in.numel() if has_sink else 0
+        q_s, o = torch.empty_like(q), torch.empty_like(q)
+        aux, stat, sink, flag = _row_state(B, H, T, dev)
+        if not has_sink:
+            sink = None
+        p = _lib.ptr
         if plan.variant == _lib.ATTN_GUARDED:
             # q_s, sink/c, the guard and the guarded forward (flash.py:823-856) in one call.
             _lib.check(lib.alg_attn_fwd_guarded(
-                st, dt, plan.layout, B, H, T, D, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(sink_in), nsink,
-                plan.c, plan.n, _lib.ptr(q_s), _lib.ptr(sink), _lib.ptr(flag), _lib.ptr(o), None, _lib.ptr(stat),
-                _lib.ptr(ws), ws_bytes), "flash_attention forward")
+                st, dt, plan.layout, B, H, T, D, p(q), p(k), p(v), p(sink_in), nsink, plan.c, plan.n, p(q_s), sink,
+                flag, p(o), None, stat, p(ws), ws_bytes), "flash_attention forward")
         else:
             _lib.check(lib.alg_attn_prepare(
-                st, dt, B, H, T, D, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(sink_in), nsink, plan.c, plan.n,
-                int(plan.range_guard), _lib.ptr(q_s), _lib.ptr(sink), _lib.ptr(flag), _lib.ptr(ws), ws_bytes),
-                "flash_attention prologue")
+                st, dt, B, H, T, D, p(q), p(k), p(v), p(sink_in), nsink, plan.c, plan.n, int(plan.range_guard), p(q_s),
+                sink, flag, p(ws), ws_bytes), "flash_attention prologue")
             _lib.check(lib.alg_attn_fwd(
-                st, dt, plan.layout, B, H, T, D, _lib.ptr(q_s), _lib.ptr(k), _lib.ptr(v), _lib.ptr(sink), plan.n,
-                plan.variant, _lib.ptr(flag), plan.clamp, int(plan.fast_rho), int(plan.inv_stat),
-                _lib.ptr(o), None, _lib.ptr(stat)), "flash_attention forward")
+                st, dt, plan.layout, B, H, T, D, p(q_s), p(k), p(v), sink, plan.n, plan.variant, flag, plan.clamp,
+                int(plan.fast_rho), int(plan.inv_stat), p(o), None, stat), "flash_attention forward")
         ctx.plan = plan
-        ctx.sink_shape = None if not has_sink else tuple(sink_logit.shape)
-        ctx.sink_dtype = None if not has_sink else sink_logit.dtype
-        ctx.save_for_backward(q_s, k, v, sink, o, stat, flag)
+        ctx.sink_meta = None if not has_sink else (tuple(sink_logit.shape), sink_logit.dtype)
+        ctx.save_for_backward(q_s, k, v, o, aux)
         return o
 
     @staticmethod
     def backward(ctx, do):
-        q_s, k, v, sink, o, stat, flag = ctx.saved_tensors
-        plan = ctx.plan
-        B, H, T, D = _bhtd(q_s.shape, plan.layout)
-        lib = _lib.load()
-        dt = _DTYPES[q_s.dtype]
-        dev = q_s.device
-        st = _lib.stream_of(q_s)
-        do = _lib.aligned16(do.to(q_s.dtype))
-        ws_bytes = lib.alg_attn_workspace_size(dt, B, H, T, D)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        dq = torch.empty_like(q_s)
-        dk = torch.empty_like(k)
-        dv = torch.empty_like(v)
-        di = torch.empty((B, H, T), dtype=torch.float32, device=dev)
-        dbeta = torch.empty(H, dtype=torch.float32, device=dev) if sink is not None else None
-        alpha = 1.0 / (math.sqrt(D) * plan.c)
-        _lib.check(lib.alg_attn_bwd(
-            st, dt, plan.layout, B, H, T, D, _lib.ptr(q_s), _lib.ptr(k), _lib.ptr(v), _lib.ptr(sink), _lib.ptr(o),
-            _lib.ptr(stat), _lib.ptr(do), plan.n, plan.variant, _lib.ptr(flag), plan.clamp,
-            int(plan.fast_rho), int(plan.inv_stat), alpha, _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(di),
-            _lib.ptr(dbeta), _lib.ptr(ws), ws_bytes), "flash_attention backward")
-        dsink = None
-        if sink is not None:
-            # sink = broadcast(reshape(sink_logit, -1), (H,)) / c  (flash.py:826-828)
-            g = dbeta / plan.c
-            numel = math.prod(ctx.sink_shape) if ctx.sink_shape else 1
-            g = g if numel == H else g.sum().reshape(1)
-            dsink = g.reshape(ctx.sink_shape).to(ctx.sink_dtype)
-        return dq, dk, dv, dsink, None
+        q_s, k, v, o, aux = ctx.saved_tensors
+        dq, dk, dv, dsink = _attn_backward(ctx.plan, q_s, k, v, o, aux, do, ctx.sink_meta is not None,
+                                           "flash_attention backward")
+        return dq, dk, dv, _sink_gradient(dsink, *ctx.sink_meta) if ctx.sink_meta else None, None
 
 
 def flash_attention(q, k, v, sink_logit=None, *, kind: str = "softmax",

@@ -59,9 +59,9 @@ class _HeadFn(torch.autograd.Function):
         if SCHEDULE == "streamed" and (VOCAB_CHUNK < 0 or VOCAB_CHUNK % 256):
             raise ValueError(f"vocab chunk {VOCAB_CHUNK}: 0 or a positive multiple of 256")
         ws_bytes = lib.alg_head_workspace_size(dt, N, d, V, 0)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        zt = _lib.align256(ws_bytes)
+        ws = torch.empty(zt + 4 * N, dtype=torch.uint8, device=dev)  # workspace, then the target logits
         stat = torch.empty(N, dtype=torch.float32, device=dev)
-        zt = torch.empty(N, dtype=torch.float32, device=dev)
         pt = torch.empty(N, dtype=torch.float32, device=dev)
         obj = torch.empty((), dtype=torch.float32, device=dev)
         residual = None
@@ -71,7 +71,7 @@ class _HeadFn(torch.autograd.Function):
         if SCHEDULE == "residual" and dt == _lib.DTYPE_BF16 and n > 1 and any(ctx.needs_input_grad[:2]):
             residual = torch.empty(lib.alg_head_residual_size(N, d, V), dtype=torch.uint8, device=dev)
         _lib.check(lib.alg_head_fwd(st, dt, N, d, V, _lib.ptr(h), _lib.ptr(e), _lib.ptr(t), n, c, _lib.ptr(stat),
-                                    _lib.ptr(zt), _lib.ptr(pt), _lib.ptr(obj), _lib.ptr(residual),
+                                    _lib.ptr(ws) + zt, _lib.ptr(pt), _lib.ptr(obj), _lib.ptr(residual),
                                     _lib.ptr(ws), ws_bytes),
                    "fused_head forward")
         ctx.n, ctx.c = n, c
@@ -80,6 +80,7 @@ class _HeadFn(torch.autograd.Function):
         ctx.embed_dtype = embed.dtype
         ctx.save_for_backward(h, e, t, stat, residual)
         ctx.mark_non_differentiable(pt)
+        ctx.set_materialize_grads(False)  # no zeros for the telemetry's gradient
         return obj, pt
 
     @staticmethod

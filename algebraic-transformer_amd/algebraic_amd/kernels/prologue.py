@@ -21,7 +21,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
-from .flash import _DTYPES, _bhtd, _make_plan
+from .flash import _DTYPES, _attn_backward, _bhtd, _make_plan, _row_state, _sink_gradient, _sink_input
 
 
 def cayley_powers(w: torch.Tensor, seq_len: int):
@@ -82,76 +82,57 @@ class _PrologueFlashFn(torch.autograd.Function):
             if g is not None and g.numel() != D:
                 raise ValueError(f"{name} must have {D} entries")
         has_sink = sink_logit is not None
-        sink_in = None
-        if has_sink:
-            sink_in = sink_logit.detach().to(device=dev, dtype=torch.float32).reshape(-1).contiguous()
-            if sink_in.numel() not in (1, H):
-                raise ValueError(f"sink_logit must broadcast to ({H},)")
+        sink_in = _sink_input(sink_logit, H, dev)
         ws_bytes = lib.alg_attn_prologue_workspace_size(B, H, T, D)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        q_s, k_r = torch.empty_like(q), torch.empty_like(k)
-        tau_q = torch.empty((B, H, T), dtype=torch.float32, device=dev)
-        tau_k = torch.empty_like(tau_q)
-        sink = torch.empty(H, dtype=torch.float32, device=dev) if has_sink else None
-        flag = torch.empty(1, dtype=torch.int32, device=dev)
+        q_s, k_r, o = torch.empty_like(q), torch.empty_like(k), torch.empty_like(q)
+        tau = torch.empty((2, B, H, T), dtype=torch.float32, device=dev)  # 1/rms of the rows of q and of k
+        tau_q, tau_k = _tau_ptrs(tau)
+        aux, stat, sink, flag = _row_state(B, H, T, dev)
+        if not has_sink:
+            sink = None
+        p = _lib.ptr
         _lib.check(lib.alg_attn_qk_prologue(
-            st, dt, plan.layout, B, H, T, D, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(gq), _lib.ptr(gk),
-            _lib.ptr(cs), _lib.ptr(sn), float(eps), _lib.ptr(sink_in), sink_in.numel() if has_sink else 0, plan.c,
-            plan.n, int(plan.range_guard), _lib.ptr(q_s), _lib.ptr(k_r), _lib.ptr(tau_q), _lib.ptr(tau_k),
-            _lib.ptr(sink), _lib.ptr(flag), _lib.ptr(ws), ws_bytes), "attention prologue")
-        o = torch.empty_like(q)
-        stat = torch.empty((B, H, T), dtype=torch.float32, device=dev)
+            st, dt, plan.layout, B, H, T, D, p(q), p(k), p(v), p(gq), p(gk), p(cs), p(sn), float(eps), p(sink_in),
+            sink_in.numel() if has_sink else 0, plan.c, plan.n, int(plan.range_guard), p(q_s), p(k_r), tau_q, tau_k,
+            sink, flag, p(ws), ws_bytes), "attention prologue")
         _lib.check(lib.alg_attn_fwd(
-            st, dt, plan.layout, B, H, T, D, _lib.ptr(q_s), _lib.ptr(k_r), _lib.ptr(v), _lib.ptr(sink), plan.n, plan.variant,
-            _lib.ptr(flag), plan.clamp, int(plan.fast_rho), int(plan.inv_stat),
-            _lib.ptr(o), None, _lib.ptr(stat)), "attention forward")
+            st, dt, plan.layout, B, H, T, D, p(q_s), p(k_r), p(v), sink, plan.n, plan.variant, flag, plan.clamp,
+            int(plan.fast_rho), int(plan.inv_stat), p(o), None, stat), "attention forward")
         ctx.plan = plan
-        ctx.sink_shape = None if not has_sink else tuple(sink_logit.shape)
-        ctx.sink_dtype = None if not has_sink else sink_logit.dtype
+        ctx.sink_meta = None if not has_sink else (tuple(sink_logit.shape), sink_logit.dtype)
         ctx.gain_meta = [None if g is None else (g.shape, g.dtype) for g in (q_gain, k_gain)]
-        ctx.save_for_backward(q, k, v, gq, gk, cs, sn, q_s, k_r, tau_q, tau_k, sink, o, stat, flag)
+        ctx.save_for_backward(q, k, v, gq, gk, cs, sn, q_s, k_r, tau, o, aux)
         return o
 
     @staticmethod
     def backward(ctx, do):
-        q, k, v, gq, gk, cs, sn, q_s, k_r, tau_q, tau_k, sink, o, stat, flag = ctx.saved_tensors
+        q, k, v, gq, gk, cs, sn, q_s, k_r, tau, o, aux = ctx.saved_tensors
         plan = ctx.plan
         B, H, T, D = _bhtd(q.shape, plan.layout)
         lib = _lib.load()
-        dt = _DTYPES[q.dtype]
         dev = q.device
-        st = _lib.stream_of(q)
-        do = _lib.aligned16(do.to(q.dtype))
-        ws_bytes = lib.alg_attn_workspace_size(dt, B, H, T, D)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        dq_r, dk_r, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        di = torch.empty((B, H, T), dtype=torch.float32, device=dev)
-        dbeta = torch.empty(H, dtype=torch.float32, device=dev) if sink is not None else None
-        alpha = 1.0 / (math.sqrt(D) * plan.c)
-        _lib.check(lib.alg_attn_bwd(
-            st, dt, plan.layout, B, H, T, D, _lib.ptr(q_s), _lib.ptr(k_r), _lib.ptr(v), _lib.ptr(sink), _lib.ptr(o),
-            _lib.ptr(stat), _lib.ptr(do), plan.n, plan.variant, _lib.ptr(flag), plan.clamp,
-            int(plan.fast_rho), int(plan.inv_stat), alpha, _lib.ptr(dq_r), _lib.ptr(dk_r), _lib.ptr(dv),
-            _lib.ptr(di), _lib.ptr(dbeta), _lib.ptr(ws), ws_bytes), "attention backward")
-        pws_bytes = lib.alg_attn_prologue_workspace_size(B, H, T, D)
-        pws = torch.empty(pws_bytes, dtype=torch.uint8, device=dev)
+        dq_r, dk_r, dv, dsink = _attn_backward(plan, q_s, k_r, v, o, aux, do, ctx.sink_meta is not None,
+                                               "attention backward")
+        nbytes = lib.alg_attn_prologue_workspace_size(B, H, T, D)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         dq, dk = torch.empty_like(q), torch.empty_like(k)
         dgq = torch.empty(D, dtype=torch.float32, device=dev) if gq is not None else None
         dgk = torch.empty(D, dtype=torch.float32, device=dev) if gk is not None else None
+        p = _lib.ptr
         _lib.check(lib.alg_attn_qk_prologue_bwd(
-            st, dt, plan.layout, B, H, T, D, _lib.ptr(q), _lib.ptr(k), _lib.ptr(gq), _lib.ptr(gk), _lib.ptr(cs),
-            _lib.ptr(sn), _lib.ptr(tau_q), _lib.ptr(tau_k), _lib.ptr(dq_r), _lib.ptr(dk_r), _lib.ptr(dq),
-            _lib.ptr(dk), _lib.ptr(dgq), _lib.ptr(dgk), _lib.ptr(pws), pws_bytes), "attention prologue backward")
-        dsink = None
-        if sink is not None:
-            g = dbeta / plan.c
-            numel = math.prod(ctx.sink_shape) if ctx.sink_shape else 1
-            g = g if numel == H else g.sum().reshape(1)
-            dsink = g.reshape(ctx.sink_shape).to(ctx.sink_dtype)
-        gains = []
-        for dg, meta in zip((dgq, dgk), ctx.gain_meta):
-            gains.append(None if meta is None else dg.reshape(meta[0]).to(meta[1]))
+            _lib.stream_of(q), _DTYPES[q.dtype], plan.layout, B, H, T, D, p(q), p(k), p(gq), p(gk), p(cs), p(sn),
+            *_tau_ptrs(tau), p(dq_r), p(dk_r), p(dq), p(dk), p(dgq), p(dgk), p(ws), nbytes),
+            "attention prologue backward")
+        gains = [None if meta is None else dg.reshape(meta[0]).to(meta[1])
+                 for dg, meta in zip((dgq, dgk), ctx.gain_meta)]
+        dsink = _sink_gradient(dsink, *ctx.sink_meta) if ctx.sink_meta else None
         return dq, dk, dv, dsink, gains[0], gains[1], None, None, None, None
+
+
+def _tau_ptrs(tau):
+    base = tau.data_ptr()
+    return base, base + 2 * tau.numel()  # half of its 4-byte entries
 
 
 def qk_norm_rotary_flash_attention(q, k, v, sink_logit=None, q_gain=None, k_gain=None, cos=None, sin=None, *,

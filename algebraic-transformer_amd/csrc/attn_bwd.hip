@@ -493,7 +493,7 @@ __device__ __forceinline__ void attn_sink_grad(const AttnBwdParams& p, int nblk)
     rho_exact(bb, r);
     float sl = (float)(1 << p.log2n) * r;
     if (clipped && !(beta < p.clamp)) sl = 0.0f;  // flash.py:703-704
-    p.dbeta[hh] = -s * sl;
+    p.dbeta[hh] = -s * sl / p.sink_c;
   }
 }
 

@@ -65,7 +65,7 @@ struct AttnBwdParams {
   void* dq;            // (B,H,T,D) output
   void* dk;
   void* dv;
-  float* dbeta;        // (H,) gradient w.r.t. sink/c
+  float* dbeta;        // (H,) gradient w.r.t. sink/c, divided by sink_c
   int B, H, T;
   int log2n;
   float clamp;
@@ -74,6 +74,7 @@ struct AttnBwdParams {
   int mode;            // AttnMode selected by the host when flag is nullptr
   float dq_scale;      // chain-rule factor applied after the slope (alpha), or 1
   int layout;          // storage of q, k, v, o, dO, dq, dk, dv (see head_base)
+  float sink_c = 1.0f; // c: dbeta is the gradient w.r.t. the sink logit; 1: w.r.t. sink/c
 };
 
 __host__ __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }

@@ -509,11 +509,11 @@ int alg_attn_fwd_guarded(alg_stream_t stream, int dtype, int layout, int B, int 
   return hip_status(alg::launch_attn_fwd(ps, D, bf, alg::MODE_SHIFTED, st), "alg_attn_fwd_guarded");
 }
 
-int alg_attn_bwd(alg_stream_t stream, int dtype, int layout, int B, int H, int T, int D, const void* q_s,
-                 const void* k, const void* v, const float* sink_scaled, const void* o, const float* stat,
-                 const void* dO, int n, int variant, const int* guard_flag, float clamp, int fast_rho, int inv_stat,
-                 float dq_scale, void* dq, void* dk, void* dv, float* di, float* dsink_scaled, void* workspace,
-                 size_t workspace_bytes) {
+static int attn_bwd(alg_stream_t stream, int dtype, int layout, int B, int H, int T, int D, const void* q_s,
+                    const void* k, const void* v, const float* sink_scaled, const void* o, const float* stat,
+                    const void* dO, int n, int variant, const int* guard_flag, float clamp, int fast_rho, int inv_stat,
+                    float dq_scale, void* dq, void* dk, void* dv, float* di, float* dsink, float sink_c,
+                    void* workspace, size_t workspace_bytes) {
   int rc = check_attn_shape(dtype, B, H, T, D);
   if (rc) return rc;
   if ((rc = check_layout(layout, H, T, D))) return rc;
@@ -534,7 +534,8 @@ int alg_attn_bwd(alg_stream_t stream, int dtype, int layout, int B, int H, int T
   p.di = di;
   p.dq_acc = dtype == ALG_DTYPE_F32 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + ws.dq_acc) : nullptr;
   p.sink_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + ws.sink_part);
-  p.dq = dq; p.dk = dk; p.dv = dv; p.dbeta = dsink_scaled;
+  p.dq = dq; p.dk = dk; p.dv = dv; p.dbeta = dsink;
+  p.sink_c = sink_c;
   p.B = B; p.H = H; p.T = T;
   p.log2n = log2_pow2(n);
   p.clamp = clamp; p.fast_rho = fast_rho; p.inv_stat = inv_stat;
@@ -552,6 +553,25 @@ int alg_attn_bwd(alg_stream_t stream, int dtype, int layout, int B, int H, int T
   }
   const int modes[1] = {variant};
   return hip_status(alg::launch_attn_bwd(p, D, bf, modes, 1, st), "alg_attn_bwd");
+}
+
+int alg_attn_bwd(alg_stream_t stream, int dtype, int layout, int B, int H, int T, int D, const void* q_s,
+                 const void* k, const void* v, const float* sink_scaled, const void* o, const float* stat,
+                 const void* dO, int n, int variant, const int* guard_flag, float clamp, int fast_rho, int inv_stat,
+                 float dq_scale, void* dq, void* dk, void* dv, float* di, float* dsink_scaled, void* workspace,
+                 size_t workspace_bytes) {
+  return attn_bwd(stream, dtype, layout, B, H, T, D, q_s, k, v, sink_scaled, o, stat, dO, n, variant, guard_flag, clamp,
+                  fast_rho, inv_stat, dq_scale, dq, dk, dv, di, dsink_scaled, 1.0f, workspace, workspace_bytes);
+}
+
+int alg_attn_bwd_sink_logit(alg_stream_t stream, int dtype, int layout, int B, int H, int T, int D, const void* q_s,
+                            const void* k, const void* v, const float* sink_scaled, const void* o, const float* stat,
+                            const void* dO, int n, int variant, const int* guard_flag, float clamp, int fast_rho,
+                            int inv_stat, float dq_scale, float c, void* dq, void* dk, void* dv, float* di,
+                            float* dsink_logit, void* workspace, size_t workspace_bytes) {
+  if (!(c > 0.0f) || !std::isfinite(c)) return fail(ALG_ERR_INVALID, "c must be positive and finite");
+  return attn_bwd(stream, dtype, layout, B, H, T, D, q_s, k, v, sink_scaled, o, stat, dO, n, variant, guard_flag, clamp,
+                  fast_rho, inv_stat, dq_scale, dq, dk, dv, di, dsink_logit, c, workspace, workspace_bytes);
 }
 
 int alg_attn_bwd_noalloc(alg_stream_t stream, int dtype, int layout, int B, int H, int T, int D, const void* q_s,

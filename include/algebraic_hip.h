@@ -127,6 +127,16 @@ int alg_attn_bwd(alg_stream_t stream, int dtype, int layout, int B, int H, int T
                  void* dq, void* dk, void* dv, float* di, float* dsink_scaled,
                  void* workspace, size_t workspace_bytes);
 
+/* alg_attn_bwd with the sink's gradient taken on to the sink logit, flash.py:826-828:
+ * dsink_logit (H) f32 = dL/d(sink/c) / c (may be NULL). */
+int alg_attn_bwd_sink_logit(alg_stream_t stream, int dtype, int layout, int B, int H, int T, int D,
+                            const void* q_s, const void* k, const void* v, const float* sink_scaled,
+                            const void* o, const float* stat, const void* dO,
+                            int n, int variant, const int* guard_flag, float clamp, int fast_rho, int inv_stat,
+                            float dq_scale, float c,
+                            void* dq, void* dk, void* dv, float* di, float* dsink_logit,
+                            void* workspace, size_t workspace_bytes);
+
 /* Allocation-free variant of alg_attn_bwd. It has no counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture, tight serving or
  * training loops, harnesses that forbid allocation). Same arguments, results and errors as

@@ -12,20 +12,20 @@ from oracle import attention as OA
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
+VARIANTS = {"guarded": dict(range_guard=True), "shifted": dict(shift=True), "clipped": dict()}
 # (B, H, T, D): one key, blocks one short, whole and one over, an odd number of query tiles; the
-# last has 1152 key blocks, two to a CU.
+# last has 1152 key blocks, two to a CU (run once).
 CASES = [(1, 2, 1, 64), (1, 3, 63, 64), (2, 1, 64, 128), (1, 2, 65, 64), (1, 1, 97, 128), (1, 2, 130, 64),
          (1, 2, 320, 128), (1, 2, 321, 64), (8, 16, 520, 64)]
+RUNS = [(c, v, lay) for c in CASES for v in VARIANTS for lay in ("bhtd", "bthd")
+        if c[0] * c[1] < 100 or (v, lay) == ("guarded", "bhtd")]
 
 
-@pytest.mark.parametrize("layout", ["bhtd", "bthd"])
-@pytest.mark.parametrize("kw", [dict(range_guard=True), dict(shift=True), dict()], ids=["guarded", "shifted", "clipped"])
-@pytest.mark.parametrize("shape", CASES, ids=lambda s: "x".join(map(str, s)))
-def test_f32_backward(shape, kw, layout):
+@pytest.mark.parametrize("shape,variant,layout", RUNS, ids=lambda x: "x".join(map(str, x)) if isinstance(x, tuple) else x)
+def test_f32_backward(shape, variant, layout):
     from algebraic_amd.kernels.flash import flash_attention
     B, H, T, D = shape
-    if B * H > 100 and (layout == "bthd" or not kw.get("range_guard")):
-        pytest.skip("the large case runs once")
+    kw = VARIANTS[variant]
     print(f"[f32 bwd] {shape} {kw} {layout}", flush=True)
     rng = np.random.default_rng(B + H + T + D)
     q, k, v, do = (rng.standard_normal((B, H, T, D)).astype(np.float32) for _ in range(4))
