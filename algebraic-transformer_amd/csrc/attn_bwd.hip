@@ -164,15 +164,15 @@ struct RowTile {
 // are added through LDS at the end, and for dQ each wave takes 32 queries and half of D. At
 // D = 64 the LDS (70 KB) lets two workgroups run on a CU. Against 128 keys per workgroup with one
 // wave per SIMD and the next tile's registers spilled (us, B H T D): 2 12 1024 64: 219 -> 119;
-// 4 12 2048 64: 726 -> 607; 8 16 1024 64: 496 -> 432; 1 4 300 64: 70 -> 40; 2 12 1024 128:
+// 4 12 2048 64: 726 -> 607 to 655 by run; 8 16 1024 64: 496 -> 432; 1 4 300 64: 70 -> 40; 2 12 1024 128:
 // 526 -> 212. (Two workgroups per key block, its query tiles dealt between them, took 2 12 1024 64
 // to 109 us, but dQ's addends then arrive in an order that changes from call to call.)
 constexpr int F32_BK = 64, F32_BQ = 64;
 // Barrier for LDS alone: __syncthreads() also waits for every global access in flight, here the
 // dQ atomics and the next tile's loads.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-template <int D, int MODE, int L2N>
-__global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_f32_kernel(AttnBwdParams p) {
+template <int D, int MODE, int L2N, int WPS>
+__global__ __launch_bounds__(256, WPS) void attn_bwd_f32_kernel(AttnBwdParams p) {
   static_assert(D == 64 || D == 128, "head_dim");
   constexpr int PITCH = D + F32_PAD;
   constexpr int SPITCH = F32_BQ + F32_PAD;
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_f32_kernel(Attn
       floatx16 dqa[DBW];
 #pragma unroll
       for (int j = 0; j < DBW; ++j) dqa[j] = floatx16{};
-      // The operands of 8 MFMA steps are read together, one group ahead of their MFMAs.
+      // The operands of G MFMA steps are read together, one group ahead of their MFMAs.
       constexpr int G = 8;
       float a[2][G], b[2][G][DBW];
       auto operands = [&](int ks0, int to) __attribute__((always_inline)) {
@@ -1555,26 +1555,33 @@ static hipError_t launch_bwd_bf16(const AttnBwdParams& p, int mode, bool dq, hip
 // key blocks, then start on a CU each and the short ones follow, where two to a CU put long
 // blocks together and left CUs idle (384 key blocks, B H T D: 2 12 1024 64 142 -> 119 us,
 // 1 12 2048 64 253 -> 210). With more blocks than that, two to a CU hide each other's waits
-// (1536, 4 12 2048 64: 607 us, one to a CU 672).
+// (1536, 4 12 2048 64: 607 us, one to a CU 672). The form for one to a CU has the registers of one wave
+// per SIMD and spills nothing (384 blocks, 2 12 1024 64: 131 -> 120 us).
 template <int D>
 static hipError_t launch_bwd_f32(const AttnBwdParams& p, int mode, hipStream_t st) {
+  constexpr int WPS = D == 64 ? 2 : 1;  // waves per SIMD
   const int nbh = p.B * p.H, nkb = ceil_div(p.T, F32_BK);
   dim3 block(256);
   switch (mode) {
     case MODE_INRANGE: {
       KTimer t("attn_bwd_inrange", st);
       dim3 grid(nbh, nkb);
-      const int pad = D == 64 && (long)nbh * nkb <= 512 ? 16 << 10 : 0;  // 70 + 16 KB: over half of 160
-      if (p.log2n == 4) hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_INRANGE, 4>), grid, block, pad, st, p);
-      else hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_INRANGE, 0>), grid, block, pad, st, p);
+      const bool alone = D == 128 || (long)nbh * nkb <= 512;
+      const int pad = D == 64 && alone ? 16 << 10 : 0;  // 70 + 16 KB: over half of 160
+      if (p.log2n == 4) {
+        if (alone) hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_INRANGE, 4, 1>), grid, block, pad, st, p);
+        else hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_INRANGE, 4, WPS>), grid, block, 0, st, p);
+      } else {
+        hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_INRANGE, 0, WPS>), grid, block, pad, st, p);
+      }
     } break;
     case MODE_CLIPPED: {
       KTimer t("attn_bwd_clipped", st);
-      hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_CLIPPED, 0>), dim3(fallback_grid(p, nbh * nkb)), block, 0, st, p);
+      hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_CLIPPED, 0, WPS>), dim3(fallback_grid(p, nbh * nkb)), block, 0, st, p);
     } break;
     case MODE_SHIFTED: {
       KTimer t("attn_bwd_shifted", st);
-      hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_SHIFTED, 0>), dim3(fallback_grid(p, nbh * nkb)), block, 0, st, p);
+      hipLaunchKernelGGL((attn_bwd_f32_kernel<D, MODE_SHIFTED, 0, WPS>), dim3(fallback_grid(p, nbh * nkb)), block, 0, st, p);
     } break;
     default: return hipErrorInvalidValue;
   }
