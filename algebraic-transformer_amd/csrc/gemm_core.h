@@ -512,13 +512,19 @@ constexpr int gemm_share() {
 }
 
 
+// Position of workgroup `bid` of `total` in an order that gives each XCD (ids congruent mod 8 run
+// on the same one) a contiguous share: total / 8 positions, the first total % 8 XCDs one more.
+__device__ __forceinline__ int xcd_contiguous(int bid, int total) {
+  const int x = bid % 8;
+  return x * (total / 8) + min(x, total % 8) + bid / 8;
+}
+
 // Map a linear workgroup id to (tile_m, tile_n) so that the workgroups one XCD runs
 // (ids congruent mod 8 are dispatched to the same XCD) cover a compact group of tiles
 // that share A row panels and B column panels in that XCD's L2.
 __device__ __forceinline__ void xcd_tile(int bid, int nbm, int nbn, int& tm, int& tn) {
   const int total = nbm * nbn;
-  int lin = bid;
-  if (total % 8 == 0) lin = (bid % 8) * (total / 8) + bid / 8;
+  const int lin = xcd_contiguous(bid, total);
   constexpr int GROUP = 8;  // tiles of M per group, swept across N
   const int group_size = GROUP * nbn;
   const int g = lin / group_size;
@@ -533,8 +539,7 @@ __device__ __forceinline__ void xcd_tile(int bid, int nbm, int nbn, int& tm, int
 // together cover a few A row panels with every B column panel, so each A panel is streamed
 // from memory once (for products whose A operand is large and B small).
 __device__ __forceinline__ void xcd_tile_rowmajor(int bid, int nbm, int nbn, int& tm, int& tn) {
-  const int total = nbm * nbn;
-  const int lin = total % 8 == 0 ? (bid % 8) * (total / 8) + bid / 8 : bid;
+  const int lin = xcd_contiguous(bid, nbm * nbn);
   tm = lin / nbn;
   tn = lin - tm * nbn;
 }

@@ -802,7 +802,7 @@ __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_de_
   const int bid = blockIdx.x;
   int lin, kbeg = 0, kend = p.N, unit = -1;
   if (bid < p.de_full) {
-    lin = p.de_full % 8 == 0 ? (bid % 8) * (p.de_full / 8) + bid / 8 : bid;
+    lin = xcd_contiguous(bid, p.de_full);
   } else {
     unit = bid - p.de_full;
     lin = p.de_full + unit / p.de_split;
@@ -909,18 +909,21 @@ static int head_tiles(int tile, int M, int N) { return ((M + tile - 1) / tile) *
 // (N 200, d 2048, V 32000: 59 / 74, 65 / 84; N 1000, d 1024, V 32768: 79 / 134, 93 / 163).
 int head_logit_tile(int N, int V) { return head_tiles(128, V, N) <= 256 ? 128 : 256; }
 
-// Vocabulary splits of the dh product on 256 x 256 tiles: minimise the rounds of 256 workgroups
-// per unit of k work (ceil(tiles*S/256)/S) for products with fewer than two rounds of tiles,
-// keeping at least 512 vocabulary entries per split; ties keep the smaller split count.
+// Vocabulary splits of the dh product on 256 x 256 tiles, for products with fewer than two rounds
+// of tiles: minimise the rounds of 256 workgroups, ceil(tiles*S/256)/S of the whole product's k at
+// 23.4 ns each, plus the f32 partials written and read at about 4.5 TB/s, keeping at least 512
+// vocabulary entries per split; ties keep the smaller split count. (N 8192, d 768, V 50257, product
+// and summing launch, us: S = 2 731 + 13, 4 777 + 21, 5 654 + 25, 8 657 + 37, 16 719 + 90.)
 static int head_dh_split(int N, int d, int V) {
   const int tiles = head_tiles(HT_M, N, d);
   if (tiles >= 512) return 1;
+  auto cost = [&](int s) {
+    return std::ceil(tiles * (double)s / 256.0) / s * V * 0.0234 + (s > 1 ? 8e-6 / 4.5 * s * N * d : 0.0);
+  };
   int best = 1;
-  double best_cost = std::ceil(tiles / 256.0);
-  for (int s = 2; s <= 16 && V / s >= 512; ++s) {
-    const double cost = std::ceil(tiles * (double)s / 256.0) / s;
-    if (cost < best_cost - 1e-9) { best = s; best_cost = cost; }
-  }
+  double best_cost = cost(1);
+  for (int s = 2; s <= 16 && V / s >= 512; ++s)
+    if (const double c = cost(s); c < best_cost - 1e-9) { best = s; best_cost = c; }
   return best;
 }
 
