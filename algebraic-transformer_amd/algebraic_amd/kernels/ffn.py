@@ -94,4 +94,7 @@ def alu_glu_ffn(h2, w_g, w_u, w_d, beta: float = 0.5):
         raise ValueError("w_g, w_u must be (d, d_ff) and w_d (d_ff, d_out)")
     if not h2.is_cuda:
         raise RuntimeError("alu_glu_ffn needs GPU tensors (no CPU fallback)")
+    # The library packs the weights by pointer, so nothing else would notice one on another device.
+    if any(w.device != h2.device for w in (w_g, w_u, w_d)):
+        raise RuntimeError(f"alu_glu_ffn needs its weights on {h2.device}")
     return _FfnFn.apply(h2, w_g, w_u, w_d, float(beta))

@@ -67,3 +67,14 @@ def test_small_block(N, d, F, dtypes):
     for name, a, b, w in zip(("out", "dx", "dw_g", "dw_u", "dw_d"), got, want, (tx, tx, tg, tu, td)):
         assert a.dtype == w.dtype and a.is_contiguous()
         assert rel_l2(a.float().cpu().numpy(), b) < 1e-2, name
+
+
+@pytest.mark.parametrize("host", [0, 1, 2])
+def test_weight_on_the_host_is_refused(host):
+    """A weight on another device than the input is refused before any pointer reaches a kernel."""
+    from algebraic_amd.kernels.ffn import alu_glu_ffn
+    x = torch.zeros(8, 64, dtype=torch.bfloat16, device="cuda")
+    w = [torch.zeros(s, dtype=torch.bfloat16, device="cuda") for s in ((64, 128), (64, 128), (128, 64))]
+    w[host] = w[host].cpu()
+    with pytest.raises(RuntimeError, match="weights"):
+        alu_glu_ffn(x, *w)
