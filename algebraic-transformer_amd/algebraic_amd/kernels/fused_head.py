@@ -165,10 +165,11 @@ def head_logprob(h, embed, targets, *, head="alg_ce", n=8, c=2.0, argmax=True):
     E = _lib.aligned16(embed.to(h.dtype))  # the cast of fused_head.py:168
     t = targets.to(device=h.device, dtype=torch.int32).contiguous()
     logprob = torch.empty(N, dtype=torch.float32, device=h.device)
-    am = torch.empty(N, dtype=torch.int32, device=h.device) if argmax else None
+    am = torch.empty(N, dtype=torch.int64, device=h.device) if argmax else None
     dt = _DTYPES[h.dtype]
     nbytes = lib.alg_head_workspace_size(dt, N, d, V, 3)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=h.device)
-    _lib.check(lib.alg_head_eval(_lib.stream_of(h), dt, N, d, V, _lib.ptr(h), _lib.ptr(E), _lib.ptr(t), int(n), float(c),
-                                 _lib.ptr(logprob), _lib.ptr(am), _lib.ptr(ws), nbytes), "head_logprob")
-    return logprob, (am.long() if argmax else None)
+    _lib.check(lib.alg_head_eval_index64(_lib.stream_of(h), dt, N, d, V, _lib.ptr(h), _lib.ptr(E), _lib.ptr(t), int(n),
+                                         float(c), _lib.ptr(logprob), _lib.ptr(am), _lib.ptr(ws), nbytes),
+               "head_logprob")
+    return logprob, am

@@ -964,9 +964,9 @@ int alg_ffn_block_bwd(alg_stream_t stream, int N, int d, int F, int dm, const vo
   return rc;
 }
 
-int alg_head_eval(alg_stream_t stream, int dtype, int N, int d, int V, const void* h, const void* E,
-                  const int32_t* targets, int n, float c, float* logprob, int32_t* argmax, void* workspace,
-                  size_t workspace_bytes) {
+static int head_eval(alg_stream_t stream, int dtype, int N, int d, int V, const void* h, const void* E,
+                     const int32_t* targets, int n, float c, float* logprob, int32_t* argmax, int64_t* argmax64,
+                     void* workspace, size_t workspace_bytes) {
   int rc = check_head(N, d, V, n, c);
   if (!rc) rc = check_head_dtype(dtype, nullptr);
   if (rc) return rc;
@@ -986,8 +986,21 @@ int alg_head_eval(alg_stream_t stream, int dtype, int N, int d, int V, const voi
   p.zt = reinterpret_cast<float*>(logprob);  // the target logit is staged in the output
   p.logprob = logprob;
   p.argmax = argmax;
+  p.argmax64 = argmax64;
   if (f32) return hip_status(alg::launch_head_eval_f32(p, (hipStream_t)stream), "alg_head_eval");
   return hip_status(alg::launch_head_eval(p, (hipStream_t)stream), "alg_head_eval");
+}
+
+int alg_head_eval(alg_stream_t stream, int dtype, int N, int d, int V, const void* h, const void* E,
+                  const int32_t* targets, int n, float c, float* logprob, int32_t* argmax, void* workspace,
+                  size_t workspace_bytes) {
+  return head_eval(stream, dtype, N, d, V, h, E, targets, n, c, logprob, argmax, nullptr, workspace, workspace_bytes);
+}
+
+int alg_head_eval_index64(alg_stream_t stream, int dtype, int N, int d, int V, const void* h, const void* E,
+                          const int32_t* targets, int n, float c, float* logprob, int64_t* argmax, void* workspace,
+                          size_t workspace_bytes) {
+  return head_eval(stream, dtype, N, d, V, h, E, targets, n, c, logprob, nullptr, argmax, workspace, workspace_bytes);
 }
 
 int alg_head_bwd(alg_stream_t stream, int dtype, int N, int d, int V, const void* h, const void* E,

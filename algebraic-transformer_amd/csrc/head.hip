@@ -424,7 +424,10 @@ __global__ __launch_bounds__(64 * EVQ) void head_eval_stats_kernel(HeadParams p,
   const float zt = tgt >= 0 && tgt < p.V ? p.zt[tok] : 0.0f;
   const float rel = zt == m ? 0.0f : logf(rho_exact(zt * p.inv_c)) + logf(rho_exact(-m * p.inv_c));
   p.logprob[tok] = (float)(1 << p.log2n) * rel - logf(l);
-  if (p.argmax) p.argmax[tok] = ix == EVAL_NO_INDEX ? 0 : ix;  // every logit -inf: index 0
+  // Both widths here: widening the indices afterwards was a launch of 7 us (N 1531).
+  const int best = ix == EVAL_NO_INDEX ? 0 : ix;  // every logit -inf: index 0
+  if (p.argmax) p.argmax[tok] = best;
+  if (p.argmax64) p.argmax64[tok] = best;
 }
 
 // Per-token statistics and telemetry (fused_head.py:116-117, 219-229); with the residual

@@ -56,7 +56,8 @@ struct HeadParams {
   float* pmax;          // eval: (ceil(V/HT_M), N) per-vocab-tile maximum logit
   int* pidx;            // eval: (ceil(V/HT_M), N) its vocabulary index
   float* logprob;       // eval: (N,) log p(target)
-  int* argmax;          // eval: (N,) argmax_v z
+  int* argmax;          // eval: (N,) argmax_v z, or nullptr
+  int64_t* argmax64;    // eval: the same as 64-bit indices, or nullptr
   // f32 hidden states. With split_bad set, h, E and dzt above are three bf16 planes each (the
   // products run on the bf16 matrix cores) and the f32 kernels run only where *split_bad says
   // that an input was not finite; without it the f32 kernels always run and h, E, dzt are unused.

@@ -231,6 +231,10 @@ int alg_head_fwd(alg_stream_t stream, int dtype, int N, int d, int V,
 int alg_head_eval(alg_stream_t stream, int dtype, int N, int d, int V,
                   const void* h, const void* E, const int32_t* targets, int n, float c,
                   float* logprob, int32_t* argmax, void* workspace, size_t workspace_bytes);
+/* The same with argmax (N) int64 (or NULL), as index types of torch are. */
+int alg_head_eval_index64(alg_stream_t stream, int dtype, int N, int d, int V,
+                          const void* h, const void* E, const int32_t* targets, int n, float c,
+                          float* logprob, int64_t* argmax, void* workspace, size_t workspace_bytes);
 
 /* Row RMS norm with a learned gain, bf16 rows of d elements (d % 8 == 0, d <= 4096): the
  * model's final norm ahead of the head (model.py:208; rms_norm at algebraic.py:76-83).

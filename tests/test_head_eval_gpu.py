@@ -154,3 +154,29 @@ def test_head_argmax_takes_the_first_nan():
     lp, am = _run(h, E, t)
     assert am[5] == 0
     np.testing.assert_array_equal(am[np.arange(N) != 5], 300)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N", [1, 64, 65, 257])
+def test_both_index_widths_agree(N, dtype):
+    """The 32-bit and 64-bit entries write the same tokens and log-probabilities, and neither
+    writes past N (guard entries behind the output stay)."""
+    from algebraic_amd import _lib as L
+    lib = L.load()
+    print(f"[eval index] N={N} {dtype}", flush=True)
+    d, V = 64, 700
+    h, E, t = head_inputs(N, d, V, seed=23, e_std=0.05)
+    th, tE = (torch.tensor(a, device="cuda").to(dtype) for a in (h, E))
+    tt = torch.tensor(t, device="cuda", dtype=torch.int32)
+    dt = L.DTYPE_BF16 if dtype == torch.bfloat16 else L.DTYPE_F32
+    nbytes = lib.alg_head_workspace_size(dt, N, d, V, 3)
+    out = []
+    for name, it in (("alg_head_eval", torch.int32), ("alg_head_eval_index64", torch.int64)):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        lp = torch.full((N,), -7.0, device="cuda")
+        am = torch.full((N + 8,), -7, dtype=it, device="cuda")
+        L.check(getattr(lib, name)(L.stream_of(th), dt, N, d, V, L.ptr(th), L.ptr(tE), L.ptr(tt), 8, 2.0, L.ptr(lp),
+                                   L.ptr(am), L.ptr(ws), nbytes), name)
+        assert (am[N:] == -7).all() and (am[:N] >= 0).all() and (am[:N] < V).all()
+        out.append((lp, am[:N].long()))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
