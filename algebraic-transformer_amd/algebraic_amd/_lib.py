@@ -11,7 +11,7 @@ from pathlib import Path
 _HERE = Path(__file__).resolve().parent
 LIB_PATH = Path(os.environ.get("ALGEBRAIC_HIP_LIB", _HERE / "libalgebraic_hip.so"))
 
-ABI_VERSION = 2  # ALG_ABI_VERSION of include/algebraic_hip.h these signatures follow
+ABI_VERSION = 3  # ALG_ABI_VERSION of include/algebraic_hip.h these signatures follow
 
 ALG_OK, ALG_ERR_INVALID, ALG_ERR_UNSUPPORTED, ALG_ERR_HIP = 0, 1, 2, 3
 DTYPE_BF16, DTYPE_F32 = 0, 1
@@ -95,7 +95,9 @@ def load():
         raise HipLibraryMissing(f"{LIB_PATH} has ABI version {lib.alg_abi_version()}, these bindings "
                                 f"expect {ABI_VERSION}: rebuild it")
     for name, (res, args) in _SIGNATURES.items():
-        fn = getattr(lib, name)
+        fn = getattr(lib, name, None)
+        if fn is None:
+            raise HipLibraryMissing(f"{LIB_PATH} has no {name}: rebuild it")
         fn.restype = res
         fn.argtypes = args
     _lib = lib

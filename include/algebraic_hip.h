@@ -61,8 +61,10 @@ enum { ALG_LAYOUT_BHTD = 0, ALG_LAYOUT_BTHD = 1 };
 enum { ALG_ATTN_INRANGE = 0, ALG_ATTN_CLIPPED = 1, ALG_ATTN_SHIFTED = 2, ALG_ATTN_GUARDED = 3 };
 
 /* Version 2: alg_attn_workspace_size and alg_head_* take a leading dtype argument and
- * alg_attn_bwd has no o_precise argument (version 1 had one). */
-#define ALG_ABI_VERSION 2
+ * alg_attn_bwd has no o_precise argument (version 1 had one).
+ * Version 3: adds alg_attn_bwd_sink_logit, alg_head_eval_index64 and alg_ffn_block_*; nothing
+ * else changed. */
+#define ALG_ABI_VERSION 3
 
 const char* alg_last_error(void);
 const char* alg_version(void);

@@ -5,7 +5,10 @@ launch is exercised through calls whose arguments fail validation.
 """
 
 import ctypes
+import os
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -51,6 +54,22 @@ def test_abi_version_matches_the_header():
     assert m, "ALG_ABI_VERSION missing from the header"
     assert lib().alg_abi_version() == int(m.group(1)) == _lib.ABI_VERSION
     assert f"ABI {_lib.ABI_VERSION}" in lib().alg_version().decode()
+
+
+@pytest.mark.parametrize("version,what", [(2, "ABI version 2"), (None, "has no alg_")])
+def test_a_library_without_the_bound_symbols_is_refused(version, what, tmp_path):
+    """A library built for an older header (version 2 lacks entry points these bindings call), or
+    one of this version without them, raises HipLibraryMissing when it is loaded."""
+    from algebraic_amd import _lib
+    src = tmp_path / "old.c"
+    src.write_text(f"int alg_abi_version(void) {{ return {version or _lib.ABI_VERSION}; }}\n")
+    so = tmp_path / "libold.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    code = ("from algebraic_amd import _lib\ntry:\n    _lib.load()\n"
+            "except _lib.HipLibraryMissing as e:\n    print(e)")
+    env = dict(os.environ, ALGEBRAIC_HIP_LIB=str(so), PYTHONPATH=str(ROOT / "algebraic-transformer_amd"))
+    res = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True)
+    assert res.returncode == 0 and what in res.stdout, res.stdout + res.stderr
 
 
 def test_workspace_sizes():
