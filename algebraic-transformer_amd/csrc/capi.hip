@@ -895,7 +895,11 @@ static FfnBlockWs ffn_block_ws(int N, int d, int F, int dm, bool backward) {
 
 static int check_ffn_block(int N, int d, int F, int dm) {
   if (dm <= 0 || dm % 8) return fail(ALG_ERR_INVALID, "output width %d must be a positive multiple of 8", dm);
-  return check_ffn(N, d, F);
+  if (const int rc = check_ffn(N, d, F)) return rc;
+  // The products' own limit, before anything is launched (the packing pass counts w_d's chunks in
+  // 32 bits).
+  if ((double)F * dm > 2.0e9 || (double)N * dm > 2.0e9) return fail(ALG_ERR_INVALID, "matrices too large");
+  return ALG_OK;
 }
 
 static bool is_weight_dtype(int dt) { return dt == ALG_DTYPE_BF16 || dt == ALG_DTYPE_F32; }

@@ -273,6 +273,21 @@ def test_neighbour_entry_points_validate_before_launch():
     assert handle.alg_ffn_gemm_workspace_size(4224, 1536, 16384) == 102 * 5 * 256 * 256 * 4
 
 
+@pytest.mark.parametrize("N,d,F,dm", [(16, 64, 1 << 20, 2048), (1 << 20, 64, 512, 2048)])
+def test_ffn_block_rejects_large_products_before_any_launch(N, d, F, dm):
+    """w_d or the output over the products' 2e9 elements (gate and up alone are not)."""
+    from algebraic_amd import _lib
+    handle = lib()
+    p = [ctypes.c_void_p(16 << i) for i in range(12)]
+    big = 1 << 40
+    rc = handle.alg_ffn_block_fwd(None, N, d, F, dm, p[0], p[1], 1, p[2], 1, p[3], 1, 0.5, p[4], p[5], p[6], p[7],
+                                  p[8], p[9], p[10], big)
+    assert rc == _lib.ALG_ERR_INVALID and b"too large" in handle.alg_last_error()
+    rc = handle.alg_ffn_block_bwd(None, N, d, F, dm, p[0], p[1], p[2], p[3], p[4], p[5], p[6], 0.5, p[7], p[8], 1,
+                                  p[9], 1, p[10], 1, p[11], big)
+    assert rc == _lib.ALG_ERR_INVALID and b"too large" in handle.alg_last_error()
+
+
 def test_noalloc_backward_rejects_scratch_beyond_its_limit():
     """alg_attn_bwd_noalloc refuses, before any launch or device call, a shape whose scratch
     (here an f32 dQ accumulator of 2 x 12 x 1024 x 128 floats) exceeds the per-GPU array."""
