@@ -226,11 +226,15 @@ __device__ __forceinline__ void wave_coords(int& wm, int& wn) {
   wn = wave % C::WN;
 }
 
-// f32 products on the bf16 matrix cores: an f32 value is the exact sum of three bf16 values
-// (8 significant bits each, nearest first), and the product of two such sums drops only the
-// terms of planes (1,2), (2,1) and (2,2), together under 2^-25 of the product. The six kept terms run
-// as six passes over k, smallest first, so the large (0,0) pass alone sets the rounding of the
-// f32 accumulator: plane of A and of B for each pass, one hex digit each.
+// f32 products on the bf16 matrix cores: an f32 value of SPLIT3_MIN or more is the exact sum of three
+// bf16 values (8 significant bits each, nearest first), none of them subnormal. The product of two
+// such sums drops the terms of planes (1,2), (2,1) and (2,2): planes 1 and 2 are at most 2^-8 and
+// 2^-17 of the value, so together they are at most 2^-24 of the product, reached for mantissas
+// just above 1 (half a unit in the last place of an f32 product, beside the rounding of the sums).
+// The six kept terms run as six passes over k, smallest first, so the large (0,0) pass alone sets
+// the rounding of the f32 accumulator: plane of A and of B for each pass, one hex digit each.
+constexpr float SPLIT3_MIN = 0x1p-103f;  // last bit 2^-126, the smallest normal bf16
+constexpr float SPLIT3_MAX = 0x1p+64f;   // products of scaled planes and their sums stay far from overflow
 constexpr int SPLIT3_PASSES = 6;
 __device__ __forceinline__ int split3_a(int pass) { return (0x001102 >> (4 * pass)) & 15; }
 __device__ __forceinline__ int split3_b(int pass) { return (0x010120 >> (4 * pass)) & 15; }

@@ -111,7 +111,7 @@ __device__ __forceinline__ float select_row(const floatx16 (&acc)[C::MB][C::NB],
 
 // SPLIT: f32 h and E as three bf16 planes each (gemm_mainloop's six passes); no residual, and
 // the row sums are kept per 128 vocabulary entries, the tiling of the f32 kernels that run
-// instead when an input is not finite (p.split_bad).
+// instead when a value is out of the planes' range (p.split_bad).
 template <class C, int L2N, bool SPLIT>
 __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_fwd_kernel(HeadParams p) {
   if (SPLIT && *p.split_bad) return;
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(256) void head_obj_kernel(HeadParams p, int nblocks
 }
 
 // Recompute schedules: z^T again, dZ^T = s (p - y) r, token-major: rounded to bf16, or (SPLIT,
-// f32 hidden states) as three bf16 planes whose sum is the f32 value. L2N > 0 fixes
+// f32 hidden states) as three bf16 planes whose sum is the f32 value times 2^split3_dz_exp(s). L2N > 0 fixes
 // n = 2^L2N at compile time (0: taken from the parameters). Each wave's block is staged and
 // written in whole token rows with 16-byte stores (default cache policy: the dh and dE products
 // read dZ right after); edge tiles write the rows up to Npad and the columns up to Vp too, of
@@ -520,7 +520,8 @@ __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_dz_
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
   wave_coords<C>(wm, wn);
-  const float scale = head_grad_scale(p);
+  float scale = head_grad_scale(p);
+  if constexpr (SPLIT) scale = ldexpf(scale, split3_dz_exp(scale));
   const float inv_c = p.inv_c, clamp = p.clamp;
   const int vrow0 = m0 + wm * C::WTM;  // first vocab row of this wave
   __syncthreads();  // every wave is done reading the pipeline buffers
@@ -689,7 +690,7 @@ __device__ __forceinline__ void store_block_bf16(const floatx16 (&acc)[C::MB][C:
 // whole after the main loop (all loads issued before the first add) and added to the product,
 // which then goes back to the accumulator (dh_accum 1) or, rounded, to dh (dh_accum 2).
 // SPLIT (f32 hidden states): dZ and E as three bf16 planes each, the f32 result or its
-// vocabulary partials in p.dh_part.
+// vocabulary partials, scaled back by 2^-split3_dz_exp, in p.dh_part.
 template <class C, bool ACC, bool SPLIT>
 __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_dh_kernel(HeadParams p) {
   if (SPLIT && *p.split_bad) return;
@@ -738,6 +739,7 @@ __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_dh_
     if (back) return;
   }
   const float s = p.ut ? head_grad_scale(p) : 1.0f;
+  const float unscale = SPLIT ? ldexpf(1.0f, -split3_dz_exp(head_grad_scale(p))) : 1.0f;
   const bool to_dh = !part || ACC;  // bf16 output (ACC here: the last chunk)
   if (to_dh && m0 + C::TM <= p.N && n0 + C::TN <= p.d) {
     // Interior tile, bf16 output: the row scales s/l once per row (the expression of
@@ -763,7 +765,7 @@ __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_dh_
         if (col >= p.d) continue;
         const size_t o = (size_t)tok * p.d + col;
         if (to_dh) p.dh[o] = f2bf(acc[mb][nb][i] * f);
-        else part[o] = acc[mb][nb][i];
+        else part[o] = SPLIT ? acc[mb][nb][i] * unscale : acc[mb][nb][i];
       }
     }
   }
@@ -797,7 +799,8 @@ __global__ __launch_bounds__(256) void head_dh_reduce_kernel(HeadParams p) {
 // XCD's share (U panels streamed once); the rest compute token range (id - de_full) % de_split
 // of tile de_full + (id - de_full) / de_split into an f32 tile of de_part, which
 // head_de_tail_kernel sums.
-// SPLIT (f32 hidden states): dZ and h as three bf16 planes each.
+// SPLIT (f32 hidden states): dZ and h as three bf16 planes each, the products scaled back by
+// 2^-split3_dz_exp.
 template <class C, bool SPLIT>
 __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_de_kernel(HeadParams p) {
   if (SPLIT && *p.split_bad) return;
@@ -822,6 +825,15 @@ __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_de_
   const GemmOperand B = head_operand<SPLIT>(b, p.N, p.d, (long)p.N * p.d);
   floatx16 acc[C::MB][C::NB];
   bf16* stage = gemm_tile<MNMAJOR, MNMAJOR, C, SPLIT>(A, B, m0, n0, kbeg, kend, acc);
+  if constexpr (SPLIT) {
+    const float unscale = ldexpf(1.0f, -split3_dz_exp(head_grad_scale(p)));
+#pragma unroll
+    for (int mb = 0; mb < C::MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < C::NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[mb][nb][i] *= unscale;
+  }
   const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
   int wm, wn;
   wave_coords<C>(wm, wn);
@@ -1102,27 +1114,30 @@ hipError_t launch_head_bwd(const HeadParams& p, hipStream_t st) {
 }
 
 // f32 hidden states on the bf16 matrix cores (p.E, p.h, p.dzt: three planes each; p.split_bad
-// set): every launch returns at once when an input was not finite, and the f32 kernels of
-// head_f32.hip, launched after it, run instead.
+// set): every launch returns at once when a value was out of the planes' range, and the f32
+// kernels of head_f32.hip, launched after it, run instead.
 //
 // f32 values into three bf16 planes, each the bf16 nearest to what the planes before it leave;
-// with 8 significant bits a plane the third leaves nothing (values under 2^-110 aside, whose
-// last planes would be subnormal). An infinity or NaN, or a value that rounds to infinity in
-// bf16, has no such planes: it sets *bad. Bound by memory: 4 bytes read and 6 written an element.
+// with 8 significant bits a plane the third leaves nothing. A value that is not zero and under
+// SPLIT3_MIN (its last planes would be subnormal) or over SPLIT3_MAX, an infinity and a NaN set
+// *bad. Bound by memory: 4 bytes read and 6 written an element.
 __global__ __launch_bounds__(256) void head_split3_kernel(const float* src, bf16* dst, size_t n, int* bad) {
   bool off = false;
   for (size_t c = (size_t)blockIdx.x * 256 + threadIdx.x; c < n / 8; c += (size_t)gridDim.x * 256) {
     const float4 x = reinterpret_cast<const float4*>(src)[2 * c], y = reinterpret_cast<const float4*>(src)[2 * c + 1];
     float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
 #pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float a = __builtin_fabsf(v[e]);
+      off |= !((a >= SPLIT3_MIN && a <= SPLIT3_MAX) || a == 0.0f);
+    }
+#pragma unroll
     for (int pl = 0; pl < 3; ++pl) {
       bf16x8 o;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         o[e] = f2bf(v[e]);
-        const float b = (float)o[e];
-        if (pl == 0) off |= !(__builtin_fabsf(b) < INFINITY);
-        v[e] -= b;
+        v[e] -= (float)o[e];
       }
       *reinterpret_cast<bf16x8*>(dst + pl * n + 8 * c) = o;
     }
@@ -1130,13 +1145,16 @@ __global__ __launch_bounds__(256) void head_split3_kernel(const float* src, bf16
   if (__builtin_amdgcn_ballot_w64(off) && (threadIdx.x & 63) == 0) *bad = 1;
 }
 
-__global__ void head_split_clear_kernel(int* bad) { *bad = 0; }
+// In the backward an upstream gradient that is not finite has no planes either.
+__global__ void head_split_clear_kernel(HeadParams p, int* bad, bool backward) {
+  *bad = backward && !(__builtin_fabsf(head_grad_scale(p)) < INFINITY);
+}
 
 // Planes of h and E, and *p.split_bad.
-static void launch_head_split3(const HeadParams& p, hipStream_t st) {
+static void launch_head_split3(const HeadParams& p, bool backward, hipStream_t st) {
   KTimer t("head_split3", st);
   int* bad = const_cast<int*>(p.split_bad);
-  hipLaunchKernelGGL(head_split_clear_kernel, dim3(1), dim3(1), 0, st, bad);
+  hipLaunchKernelGGL(head_split_clear_kernel, dim3(1), dim3(1), 0, st, p, bad, backward);
   auto split = [&](const float* src, const bf16* dst, size_t n) {
     const int blocks = (int)std::min<size_t>((n / 8 + 255) / 256, 4096);
     hipLaunchKernelGGL(head_split3_kernel, dim3(blocks), dim3(256), 0, st, src, const_cast<bf16*>(dst), n, bad);
@@ -1146,13 +1164,13 @@ static void launch_head_split3(const HeadParams& p, hipStream_t st) {
 }
 
 void launch_head_fwd_split(const HeadParams& p, hipStream_t st) {
-  launch_head_split3(p, st);
+  launch_head_split3(p, false, st);
   if (head_logit_tile(p.N, p.V) == 128) launch_fwd_cfg<HC128, true>(p, st);
   else launch_fwd_cfg<HC, true>(p, st);
 }
 
 void launch_head_bwd_split(const HeadParams& p, hipStream_t st) {
-  launch_head_split3(p, st);
+  launch_head_split3(p, true, st);
   if (head_logit_tile(p.N, p.V) == 128) launch_dz_cfg<HC128, true>(p, st);
   else launch_dz_cfg<HC, true>(p, st);
   {

@@ -60,7 +60,7 @@ struct HeadParams {
   int64_t* argmax64;    // eval: the same as 64-bit indices, or nullptr
   // f32 hidden states. With split_bad set, h, E and dzt above are three bf16 planes each (the
   // products run on the bf16 matrix cores) and the f32 kernels run only where *split_bad says
-  // that an input was not finite; without it the f32 kernels always run and h, E, dzt are unused.
+  // that a value is out of the planes' range; without it the f32 kernels always run and h, E, dzt are unused.
   const int* split_bad;
   const float* h32;     // (N, d)
   const float* E32;     // (V, d), already cast to f32
@@ -73,6 +73,14 @@ typedef GemmCfg<HT_M, HT_N, ALG_HEAD_WM, ALG_HEAD_WN> HeadGemm;
 // Scale of the logit gradient, g n / (c N) (fused_head.py:249-251).
 __device__ __forceinline__ float head_grad_scale(const HeadParams& p) {
   return p.g[0] * (((float)(1 << p.log2n) * p.inv_c) / (float)p.N);
+}
+
+// k of the power of two 2^k that the planes of dZ are scaled by (f32 hidden states), and the
+// products scaled back by: the gradient scale becomes 2^24 to 2^25, so (p - y) r down to 2^-127
+// keeps its 24 bits however small the upstream gradient is; powers of two round nothing.
+__device__ __forceinline__ int split3_dz_exp(float scale) {
+  const int e = scale == 0.0f ? 0 : __builtin_amdgcn_frexp_expf(scale) - 1;
+  return max(-100, min(100, 24 - e));
 }
 
 // ALU-GLU feed-forward products with fused activation epilogues (model.py:185-193).

@@ -60,6 +60,42 @@ def test_small_values_keep_their_precision():
     assert rel_l2(dh, dh_r) < 3e-6 and rel_l2(dE, dE_r) < 3e-6
 
 
+@pytest.mark.parametrize("h_scale,E_scale,g", [(1.0, 1.0, 1e-32), (1e16, 1e-35, 1e4), (1e-30, 1e30, 1.0),
+                                               (1e-35, 1e16, 1e4)])
+def test_whole_f32_range_keeps_its_precision(h_scale, E_scale, g):
+    """Upstream gradients, hidden states and embeddings whose planes would be subnormal bf16 (or whose
+    scaled products would overflow): the results keep the f32 bar."""
+    rng = np.random.default_rng(5)
+    h = (rng.standard_normal((300, 128)) * h_scale).astype(np.float32)
+    E = (rng.standard_normal((500, 128)) * 0.15 * E_scale).astype(np.float32)
+    t = rng.integers(0, 500, 300).astype(np.int32)
+    _, pt, dh, dE = _run(h, E, t, g=g)
+    _, pt_r = OH.dense_forward(h, E, t, n=8, c=2.0)
+    dh_r, dE_r = OH.dense_backward(h, E, t, g, n=8, c=2.0)
+    np.testing.assert_allclose(pt, pt_r, rtol=1e-5)
+    # The norms of such values underflow: scaled to about 1 first.
+    for got, want in ((dh, dh_r), (dE, dE_r)):
+        m = np.abs(want).max()
+        assert rel_l2(got / m, want / m) < 3e-6
+
+
+@pytest.mark.parametrize("g", [float("inf"), float("nan")])
+def test_upstream_gradient_not_finite(g, monkeypatch):
+    """As the f32 kernels (the streamed schedule) give it."""
+    from algebraic_amd.kernels import fused_head as FH
+    rng = np.random.default_rng(6)
+    h = np.abs(rng.standard_normal((300, 64))).astype(np.float32)  # one sign: infinities stay infinities
+    E = (rng.standard_normal((500, 64)) * 0.15).astype(np.float32)
+    t = rng.integers(0, 250, 300).astype(np.int32)
+    _, _, dh, dE = _run(h, E, t, g=g)
+    monkeypatch.setattr(FH, "SCHEDULE", "streamed")
+    _, _, dh_s, dE_s = _run(h, E, t, g=g)
+    np.testing.assert_array_equal(dh, dh_s)
+    np.testing.assert_array_equal(dE, dE_s)
+    if g > 0:
+        assert np.isinf(dE[300:]).all()  # entries that are no token's target
+
+
 @pytest.mark.parametrize("where", ["h_inf", "h_nan", "E_inf", "E_huge"])
 def test_not_finite_inputs(where, monkeypatch):
     from algebraic_amd.kernels import fused_head as FH
