@@ -109,7 +109,7 @@ struct OperandTile {
   // its rows' scalar byte offsets stay under 2^31 (a 256-row tile: rows of up to 2^22 elements;
   // the checked copies form every row's address in 64 bits).
   static __device__ __forceinline__ bool whole(const GemmOperand& op, int mn0) {
-    return (MODE == KMAJOR ? op.rows_valid : op.cols_valid) >= mn0 + TMN && op.ld <= (1L << 30) / ROWS;
+    return ((MODE == KMAJOR ? op.rows_valid : op.cols_valid) >= mn0 + TMN) & (op.ld <= (1L << 30) / ROWS);
   }
 
   // Asynchronous global -> LDS copy of the tile at (mn0, k0); the tile must lie inside the
@@ -282,7 +282,7 @@ __device__ __forceinline__ void gemm_mainloop(GemmStage<AM, BM, C>& s0, GemmStag
   // Pipelined part of the k range (of every pass: six passes make an even number of k steps of
   // any number per pass).
   const int kmain = SPLIT3 ? klen - klen % GT_K : klen >= 2 * GT_K ? klen - klen % (2 * GT_K) : 0;
-  const bool a_full = TA::whole(A, m0), b_full = TB::whole(B, n0);
+  const bool whole = TA::whole(A, m0) & TB::whole(B, n0);
   if (kmain > 0) {
     uint32_t aoff[2], boff[2];
     TA::lane_offsets(A, aoff);
@@ -370,7 +370,7 @@ __device__ __forceinline__ void gemm_mainloop(GemmStage<AM, BM, C>& s0, GemmStag
       step(s0, s1, kt, std::false_type{});
       last(s1);
     };
-    if (a_full && b_full) pipelined(std::false_type{});
+    if (whole) pipelined(std::false_type{});
     else pipelined(std::true_type{});
   }
   // Remaining partial k tiles (and short k ranges): register copies with zero fill.
@@ -429,7 +429,7 @@ __device__ __forceinline__ void gemm_ring(GemmStage<AM, BM, C>& s0, GemmStage<AM
   };
   const int nk1 = K > kbeg ? (K - kbeg) / GT_K : 0;  // k steps of one pass
   const int nk = SPLIT3 ? SPLIT3_PASSES * nk1 : nk1;
-  const bool a_full = TA::whole(A, m0), b_full = TB::whole(B, n0);
+  const bool whole = TA::whole(A, m0) & TB::whole(B, n0);
   auto pipelined = [&](auto checked) {
     constexpr bool CHK = decltype(checked)::value;
     constexpr int NG = TA::PER_WAVE + TB::PER_WAVE;
@@ -475,7 +475,7 @@ __device__ __forceinline__ void gemm_ring(GemmStage<AM, BM, C>& s0, GemmStage<AM
       if (kt + 3 < nk) step(s3, s2, kt + 3);
     }
   };
-  if (a_full && b_full) pipelined(std::false_type{});
+  if (whole) pipelined(std::false_type{});
   else pipelined(std::true_type{});
   // The remaining partial k tile: register copies with zero fill.
   if (const int k0 = kbeg + nk1 * GT_K; k0 < K) {
