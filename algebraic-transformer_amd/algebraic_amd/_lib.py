@@ -15,6 +15,8 @@ ABI_VERSION = 3  # ALG_ABI_VERSION of include/algebraic_hip.h these signatures f
 
 ALG_OK, ALG_ERR_INVALID, ALG_ERR_UNSUPPORTED, ALG_ERR_HIP = 0, 1, 2, 3
 DTYPE_BF16, DTYPE_F32 = 0, 1
+FFN_GEMM, FFN_GATE_UP, FFN_DY = 0, 1, 2
+HEAD_LOGITS, HEAD_DH, HEAD_DE = 0, 1, 2
 ATTN_INRANGE, ATTN_CLIPPED, ATTN_SHIFTED, ATTN_GUARDED = 0, 1, 2, 3
 LAYOUT_BHTD, LAYOUT_BTHD = 0, 1
 
@@ -46,6 +48,7 @@ _SIGNATURES = {
     "alg_attn_qk_prologue_bwd": (_I, [_P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P,
                                       _P, _P, _P, _S]),
     "alg_head_workspace_size": (_S, [_I, _I, _I, _I, _I]),
+    "alg_head_plan": (_I, [_I, _I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "alg_head_residual_size": (_S, [_I, _I, _I]),
     "alg_head_fwd": (_I, [_P, _I, _I, _I, _I, _P, _P, _P, _I, _F, _P, _P, _P, _P, _P, _P, _S]),
     "alg_head_bwd": (_I, [_P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _F, _P, _P, _P, _I, _P, _S]),
@@ -58,6 +61,7 @@ _SIGNATURES = {
     "alg_ffn_alu_glu_dy": (_I, [_P, _I, _I, _I, _P, _P, _P, _P, _F, _P]),
     "alg_ffn_gemm_workspace_size": (_S, [_I, _I, _I]),
     "alg_ffn_gemm": (_I, [_P, _I, _I, _I, _P, _L, _I, _P, _L, _I, _P, _L, _P, _S]),
+    "alg_ffn_plan": (_I, [_I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "alg_ffn_block_workspace_size": (_S, [_I, _I, _I, _I, _I]),
     "alg_ffn_block_fwd": (_I, [_P, _I, _I, _I, _I, _P, _P, _I, _P, _I, _P, _I, _F, _P, _P, _P, _P, _P, _P, _P, _S]),
     "alg_ffn_block_bwd": (_I, [_P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _F, _P, _P, _I, _P, _I, _P, _I, _P,

@@ -602,6 +602,28 @@ size_t alg_head_workspace_size(int dtype, int N, int d, int V, int pass) {
   return head_ws(N, d, V, pass ? 1 : 0, pass == 2).total;
 }
 
+int alg_head_plan(int dtype, int product, int N, int d, int V, int* tile, int* split) {
+  if (N <= 0 || d <= 0 || V <= 0) return fail(ALG_ERR_INVALID, "N, d, V must be positive (got %d, %d, %d)", N, d, V);
+  if (dtype != ALG_DTYPE_BF16 && dtype != ALG_DTYPE_F32) return fail(ALG_ERR_INVALID, "dtype must be bf16 or f32");
+  if (!tile || !split) return fail(ALG_ERR_INVALID, "null argument");
+  const bool f32 = dtype == ALG_DTYPE_F32, plain_f32 = f32 && !alg::head_f32_split(N);
+  const HeadWs w = f32 ? head_ws_f32(N, d, V, 1) : head_ws(N, d, V, 1, false);
+  *split = 1;
+  if (product == ALG_HEAD_LOGITS) {
+    *tile = alg::head_logit_tile(N, V);
+  } else if (product == ALG_HEAD_DH) {
+    *tile = w.dh.tile;
+    *split = w.dh.split;
+  } else if (product == ALG_HEAD_DE) {
+    *tile = w.de.tile;
+    *split = w.de.split;
+  } else {
+    return fail(ALG_ERR_INVALID, "unknown product %d", product);
+  }
+  if (plain_f32) *tile = 0;
+  return ALG_OK;
+}
+
 // Streamed backward (alg_head_bwd_streamed): the vocabulary in chunks of `chunk` rows. The
 // default chunk gives one chunk's dE product at least 256 tiles of 256 x 256 (one per CU).
 // Workspace: [logit gradient of one chunk: bf16 Npad x pitch(chunk), or f32 N x pitch(chunk)]
@@ -822,6 +844,24 @@ int alg_ffn_alu_glu_dy(alg_stream_t stream, int N, int dm, int F, const void* do
 size_t alg_ffn_gemm_workspace_size(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   return alg::ffn_gemm_plan(M, N, K).ws_bytes;
+}
+
+int alg_ffn_plan(int product, int M, int N, int K, int* tile, int* split) {
+  if (M <= 0 || N <= 0 || K <= 0) return fail(ALG_ERR_INVALID, "M, N, K must be positive (got %d, %d, %d)", M, N, K);
+  if (!tile || !split) return fail(ALG_ERR_INVALID, "null argument");
+  *split = 1;
+  if (product == ALG_FFN_GEMM) {
+    const alg::FfnGemmPlan pl = alg::ffn_gemm_plan(M, N, K);
+    *tile = pl.tile;
+    *split = pl.split;
+  } else if (product == ALG_FFN_GATE_UP) {
+    *tile = alg::ffn_gate_up_tile(M, N, K);
+  } else if (product == ALG_FFN_DY) {
+    *tile = alg::ffn_dy_tile(M, N, K);
+  } else {
+    return fail(ALG_ERR_INVALID, "unknown product %d", product);
+  }
+  return ALG_OK;
 }
 
 // Where a product's columns go: all of them, or those below n2, to C, the others to C2.

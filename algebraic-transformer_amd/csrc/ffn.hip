@@ -330,13 +330,27 @@ __global__ __launch_bounds__(256) void ffn_gemm_tail_kernel(FfnGemmParams g) {
 
 static int ffn_tiles(int tile, int M, int N) { return ((M + tile - 1) / tile) * ((N + tile - 1) / tile); }
 
-// Tile of an unsplit product with an epilogue of its own (allowed: 256, 128 and, if `min_tile`
-// lets it, 64).
-static int ffn_epilogue_tile(int M, int N, int K, int min_tile) {
-  int best = 256;
-  for (int t = 128; t >= min_tile; t /= 2)
-    if (gemm_tile_time(t, ffn_tiles(t, M, N), K) < gemm_tile_time(best, ffn_tiles(best, M, N), K)) best = t;
-  return best;
+// Tile of the gate/up product: 128 where its tiles run in one round of the CUs, or, when no tile is
+// ragged in the tokens, in two, or in more when gemm_tile_time says so. Its weights come in 64-byte pieces (gate and up columns alternate), so
+// later rounds of 128 tiles, and ragged ones above all, cost more than those of 256 (N d F, us,
+// 256 / 128; 2048 512 1408: 22.0 / 20.4; 1000 1024 2816: 36 / 40; 400 2048 5632: 57 / 89;
+// 3500 1024 2816: 67 / 120; 6528 960 1280: 64 / 52).
+int ffn_gate_up_tile(int N, int F, int d) {
+  const int tiles = ffn_tiles(128, N, 2 * F);
+  if (tiles <= 256) return 128;
+  if (N % 128) return 256;
+  return tiles <= 512 || gemm_tile_time(128, tiles, d, N, 2 * F) <
+                             gemm_tile_time(256, ffn_tiles(256, N, 2 * F), d, N, 2 * F) ? 128 : 256;
+}
+
+// Tile of the dout w_d^T product with the activation's VJP: 64 while gemm_tile_time says so. The
+// epilogue reads gate and up and writes their gradients, 9.9 us a round of 256 tiles, where two
+// workgroups of 64 tiles to a CU hide each other's (N dm F, us, 256 / 128 / 64; 1500 1024 2816:
+// 41.6 / 46.8 / 27.7; 2500 768 2048: 36.2 / 39.2 / 25.3; 4096 1024 2816: 43.7 / 54.1 / 47.3; 128 tiles
+// were the best nowhere by more than 0.6 us).
+int ffn_dy_tile(int N, int F, int dm) {
+  const int t256 = ffn_tiles(256, N, F), rounds = (t256 + 255) / 256;
+  return gemm_tile_time(64, ffn_tiles(64, N, F), dm, N, F) < gemm_tile_time(256, t256, dm, N, F) + 9.9 * rounds ? 64 : 256;
 }
 
 // Plan of a plain product. With 256 x 256 tiles, those past the last complete round of 256
@@ -346,8 +360,9 @@ static int ffn_epilogue_tile(int M, int N, int K, int min_tile) {
 // its f32 tile written, read and summed (512 KiB at about 5 TB/s over the chip, 0.1 us) plus 5 us
 // for the summing launch. A range keeps at least 1024 of K (so every range is non-empty). The
 // workspace is that of this split. A product that fills less of the chip runs on smaller tiles
-// when gemm_tile_time says so; 64 x 64 tiles are split over k (ranges of at least 512) as far as
-// the same workspace goes, which pays where few tiles have a long k (304 1024 4096: 26.9 us
+// when gemm_tile_time says so (a split: 3 us for its summing launch and its f32 tiles written and
+// read at 15 TB/s, out of the caches); 64 x 64 tiles are split over k (ranges of at least 512) as
+// far as the same workspace goes, which pays where few tiles have a long k (304 1024 4096: 26.9 us
 // whole, 15.0 us in four ranges).
 FfnGemmPlan ffn_gemm_plan(int M, int N, int K) {
   FfnGemmPlan pl;
@@ -377,12 +392,14 @@ FfnGemmPlan ffn_gemm_plan(int M, int N, int K) {
     }
   }
   if (base) return pl;  // a whole round of 256 tiles: the chip is full
-  double best_time = pl.split == 1 ? gemm_tile_time(256, pl.tiles, K)
-                                   : gemm_tile_time(256, pl.tiles * pl.split, pl.kchunk) + 5.0;
+  auto time = [&](int tile, int units, int s, int chunk) {
+    return gemm_tile_time(tile, units, chunk, M, N) + (s > 1 ? 3.0 + 8e-6 * 0.067 * units * tile * tile : 0.0);
+  };
+  double best_time = time(256, pl.tiles * pl.split, pl.split, pl.split == 1 ? K : pl.kchunk);
   auto consider = [&](int tile, int s) {
     const int tiles = ffn_tiles(tile, M, N);
     const int chunk = s > 1 ? ((K + s - 1) / s + 127) / 128 * 128 : K;
-    const double t = gemm_tile_time(tile, tiles * s, chunk) + (s > 1 ? 5.0 : 0.0);
+    const double t = time(tile, tiles * s, s, chunk);
     if (t >= best_time) return;
     best_time = t;
     pl.tile = tile;
@@ -431,7 +448,7 @@ hipError_t launch_ffn_pack(const FfnPackParams& p, hipStream_t st) {
 
 hipError_t launch_ffn_fwd(const FfnParams& p, hipStream_t st) {
   KTimer t("ffn_gate_up", st);
-  if (ffn_epilogue_tile(p.N, 2 * p.F, p.d, 128) == 128)
+  if (ffn_gate_up_tile(p.N, p.F, p.d) == 128)
     hipLaunchKernelGGL(ffn_gate_up_kernel<FC128>, dim3(ffn_tiles(128, p.N, 2 * p.F)), dim3(FC128::THREADS), 0, st, p);
   else
     hipLaunchKernelGGL(ffn_gate_up_kernel<FC>, dim3(ffn_tiles(256, p.N, 2 * p.F)), dim3(FC::THREADS), 0, st, p);
@@ -440,10 +457,9 @@ hipError_t launch_ffn_fwd(const FfnParams& p, hipStream_t st) {
 
 hipError_t launch_ffn_dy(const FfnParams& p, hipStream_t st) {
   KTimer t("ffn_dy", st);
-  const int tile = ffn_epilogue_tile(p.N, p.F, p.dm, 64);
+  const int tile = ffn_dy_tile(p.N, p.F, p.dm);
   const dim3 grid(ffn_tiles(tile, p.N, p.F));
   if (tile == 64) hipLaunchKernelGGL(ffn_dy_kernel<FC64>, grid, dim3(FC64::THREADS), 0, st, p);
-  else if (tile == 128) hipLaunchKernelGGL(ffn_dy_kernel<FC128>, grid, dim3(FC128::THREADS), 0, st, p);
   else hipLaunchKernelGGL(ffn_dy_kernel<FC>, grid, dim3(FC::THREADS), 0, st, p);
   return hipGetLastError();
 }

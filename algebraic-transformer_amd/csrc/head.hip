@@ -942,20 +942,27 @@ static int head_dh_split(int N, int d, int V) {
   return best;
 }
 
-// The dh product: that split, or, for few tokens, 128 x 128 tiles with up to 32 vocabulary splits
-// when gemm_tile_time says so. A split costs its f32 partials written and read (about 4.5
-// TB/s) and the summing launch.
+// The dh product: that split, or, for few tokens, 128 x 128 tiles with up to 32 vocabulary splits,
+// whichever takes less time. The time of a split is gemm_tile_time's form (rounds of 256 workgroups,
+// a constant and a rate per k each), with constants of its own: f32 partials stored an element a
+// lane, E read in rows of d, then the partials written and read and the summing launch. Fitted
+// with it to 777 products: 0.3 % over the best form on average. A range of 128 tiles keeps 384 k at
+// least. us, 256 / 128, with the summing launch (N, d, V): 128 1024 32768 77 / 44; 512 512 8192
+// 46 / 32; 512 1024 50257 117 / 105; 700 1536 8192 56 / 77; 2500 1536 8192 87 / 125.
 HeadDhPlan head_dh_plan(int N, int d, int V, int passes) {
   auto time = [&](int tile, int s) {
-    return gemm_tile_time(tile, head_tiles(tile, N, d) * s, (double)head_dh_kchunk(V, s) * passes) +
-           (s > 1 ? 5.0 + 8e-6 / 4.5 * s * N * d : 0.0);
+    const bool ragged = N % tile || d % tile;
+    const int units = head_tiles(tile, N, d) * s, full = units / 256, rest = units % 256, rounds = full + (rest > 0);
+    const double K = (double)head_dh_kchunk(V, s) * passes;
+    const double t = tile == 256 ? 2.3 + rounds * 14.0 +
+                                       K * (full * 0.025 + (rest > 0) * ((ragged ? 0.019 : 0.016) + 0.0076 * rest / 256.0))
+                                 : 1.2 + rounds * (6.0 + K * (ragged ? 0.012 : 0.010));
+    return t + (s > 1 ? 5.8 + 8e-6 * 0.087 * s * N * d : 0.0);
   };
-  // us, 256 / 128, with the summing launch (N, d, V): 128 1024 32768 77 / 44; 512 512 8192 46 / 32;
-  // 300 768 50257 117 / 108; 700 320 32000 79 / 76; 1000 1024 32768 93 / 138.
   HeadDhPlan pl{256, head_dh_split(N, d, V), 0};
   double best = time(256, pl.split);
   if (head_tiles(256, N, d) < 256)
-    for (int s = 1; s <= 32 && V / s >= 256; s *= 2)
+    for (int s = 1; s <= 32 && V / s >= (passes == 1 ? 384 : 256); s *= 2)
       if (const double t = time(128, s); t < best) {
         best = t;
         pl.tile = 128;
@@ -971,7 +978,9 @@ int head_dh_kchunk(int V, int split) { return ((V + split - 1) / split + 127) / 
 // instead of one (C2's 591 tiles: two full rounds, then 79 tiles x 3 ranges in a third of a
 // tile's time). A range keeps at least 1024 tokens, and a split must save a quarter of a round
 // (its f32 tiles are written and summed by head_de_tail_kernel); ties keep the smaller split.
-// Products that do not fill a round take 128 x 128 tiles, unsplit, when gemm_tile_time says so.
+// Products that do not fill a round take 128 x 128 tiles, unsplit, when gemm_tile_time says so; 6 us
+// more for 256 tiles that reach past the matrix, which store an element a lane (N d V, us, 256 /
+// 128: 100 896 8192 21.4 / 15.0; 128 1920 4096 19.6 / 12.8; 200 256 50257 22.7 / 35.1).
 HeadDePlan head_de_plan(int N, int d, int V, int passes) {
   HeadDePlan pl;
   pl.tile = 256;
@@ -995,7 +1004,8 @@ HeadDePlan head_de_plan(int N, int d, int V, int passes) {
   }
   const double K = (double)N * passes;
   const int tiles128 = head_tiles(128, V, d);
-  if (full == 0 && gemm_tile_time(128, tiles128, K) < gemm_tile_time(256, pl.tiles, K)) {
+  if (full == 0 && gemm_tile_time(128, tiles128, K, V, d) <
+                       gemm_tile_time(256, pl.tiles, K, V, d) + (V % 256 || d % 256 ? 6.0 : 0.0)) {
     pl.tile = 128;
     pl.tiles = pl.full = tiles128;
   }

@@ -11,24 +11,31 @@
 namespace alg {
 
 // The tile configurations of the bf16 products (gemm_core.h) are 256 x 256, 128 x 128 and, for the
-// feed-forward, 64 x 64.
-// Time in us of `units` workgroups of a tile configuration over k steps of K in all, fitted to
-// the products of one short sequence and of the 1b block (M N K, measured us for tiles of 256 /
-// 128 / 64, each in a captured graph with its launch):
+// feed-forward, 64 x 64. gemm_tile_time is the time in us of `units` workgroups of one of them over
+// K, for an M x N result: rounds of 256 workgroups (512 of the 64 tiles, two to a CU), each a
+// constant (the first copies and the epilogue, with nothing beside them) and a rate per k. The
+// rates are lower while CUs stand idle (256 tiles: power; 64 tiles: one to a CU), and higher
+// where tiles reach past the matrix, whose copies take a descriptor each. Fitted to 2876 products
+// of the feed-forward (100 to 8000 tokens) and of the head (32 to 4096 tokens, V 1000 to 50257),
+// each configuration timed on its own: the one chosen takes 1.0 % more than the best on average,
+// and more than 1.04 times the 256 tiles in 13 of them (at most 1.26). Without the constant of each round and the ragged rates
+// the same rule took up to 1.8 times the 256 tiles (dh of N d V 2500 1536 8192: 87 us, 126 on 240
+// tiles of 128). M N K, us for tiles of 256 / 128 / 64:
 //   1024  768 2048   39.3 / 20.8 / 11.0     768 4096 1024   25.4 / 14.7 / 19.6
 //   1024  768 4096   69.5 / 37.2 / 19.2    2048  768 1024   23.2 / 12.6 /  8.3
-//    512  512 2048   37.5 / 20.2 / 10.5    2048 2048 2048   41.8 / 25.1 / 36.7
-// A 256 tile needs 14.8 ns per k alone on the chip and 23.4 ns when all CUs hold one (power); 128
-// tiles 8 to 10 ns; 64 tiles 4 ns while a CU holds one, 8 ns for two. Small tiles move two or four
-// times the operand bytes per multiplication, so they win only while the larger ones leave
-// CUs idle.
-inline double gemm_tile_time(int tile, int units, double K) {
-  const double fill = std::min(1.0, units / 256.0), rounds = std::ceil(units / 256.0);
-  if (tile == 256) return 9.0 + rounds * K * (0.0148 + 0.0086 * fill);
-  if (tile == 128) return 4.4 + rounds * K * (0.008 + 0.002 * fill);
-  return 2.8 + K * (units <= 512 ? 0.004 + 0.004 * std::max(0, units - 256) / 256.0 : std::ceil(units / 512.0) * 0.008);
+//   1024 8192  300   18.6 / 23.0 / 25.9    2048 1536 4224   42.8 / 39.5 / 58.4
+inline double gemm_tile_time(int tile, int units, double K, int M, int N) {
+  const bool ragged = M % tile || N % tile;
+  if (tile == 256) {
+    const int full = units / 256, rest = units % 256;
+    return 1.4 + (full + (rest > 0)) * 9.0 +
+           K * (full * 0.025 + (rest > 0) * ((ragged ? 0.017 : 0.014) + 0.0076 * rest / 256.0));
+  }
+  if (tile == 128) return 1.2 + std::ceil(units / 256.0) * (5.2 + K * (ragged ? 0.014 : 0.0088));
+  const int full = units / 512, rest = units % 512;
+  return 4.9 + (full + (rest > 0)) * 0.88 +
+         K * ((full + (rest > 256)) * (ragged ? 0.0071 : 0.0068) + (rest > 0 && rest <= 256) * (ragged ? 0.0052 : 0.0042));
 }
-
 
 int attn_fwd_f32_query_block(int B, int H, int T);
 hipError_t launch_attn_fwd(const AttnFwdParams& p, int D, bool bf16_io, int mode, hipStream_t st);
@@ -89,6 +96,8 @@ struct FfnGemmPlan {
   size_t ws_bytes;  // f32 tiles of the split tiles
 };
 FfnGemmPlan ffn_gemm_plan(int M, int N, int K);
+int ffn_gate_up_tile(int N, int F, int d);
+int ffn_dy_tile(int N, int F, int dm);
 hipError_t launch_ffn_gemm(const FfnGemmParams& g, int a_mode, int b_mode, hipStream_t st);
 hipError_t launch_rms_norm_bwd(const RmsNormParams& p, float* dgain, hipStream_t st);
 

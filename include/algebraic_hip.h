@@ -62,8 +62,8 @@ enum { ALG_ATTN_INRANGE = 0, ALG_ATTN_CLIPPED = 1, ALG_ATTN_SHIFTED = 2, ALG_ATT
 
 /* Version 2: alg_attn_workspace_size and alg_head_* take a leading dtype argument and
  * alg_attn_bwd has no o_precise argument (version 1 had one).
- * Version 3: adds alg_attn_bwd_sink_logit, alg_head_eval_index64 and alg_ffn_block_*; nothing
- * else changed. */
+ * Version 3: adds alg_attn_bwd_sink_logit, alg_head_eval_index64, alg_ffn_block_*, alg_head_plan
+ * and alg_ffn_plan; nothing else changed. */
 #define ALG_ABI_VERSION 3
 
 const char* alg_last_error(void);
@@ -200,6 +200,11 @@ int alg_attn_qk_prologue_bwd(alg_stream_t stream, int dtype, int layout, int B, 
  * alg_head_bwd with a residual (pass 2) and alg_head_eval (pass 3), for hidden states of
  * dtype ALG_DTYPE_BF16 or ALG_DTYPE_F32 (0 for f32 pass 2: the residual is bf16 only). */
 size_t alg_head_workspace_size(int dtype, int N, int d, int V, int pass);
+/* Side of the square tiles (256 or 128; 0: f32 hidden states on the f32 matrix instructions) and
+ * ranges per tile (1: whole; dE: of the tiles past the last complete round) of the head's products
+ * E h^T, dh and dE, the last two outside alg_head_bwd_streamed. */
+enum { ALG_HEAD_LOGITS = 0, ALG_HEAD_DH = 1, ALG_HEAD_DE = 2 };
+int alg_head_plan(int dtype, int product, int N, int d, int V, int* tile, int* split);
 
 /* Bytes of the optional forward->backward residual: the token-major bf16 block
  * U = w*r (target entries (w_t - l) r_t) of Npad x Vp entries (U[tok, v] at tok * Vp + v,
@@ -276,6 +281,12 @@ int alg_ffn_alu_glu_dy(alg_stream_t stream, int N, int dm, int F, const void* do
 size_t alg_ffn_gemm_workspace_size(int M, int N, int K);
 int alg_ffn_gemm(alg_stream_t stream, int M, int N, int K, const void* A, long lda, int a_trans, const void* B,
                  long ldb, int b_trans, void* C, long ldc, void* workspace, size_t workspace_bytes);
+
+/* Side of the square tiles (256, 128 or 64) and k ranges per tile (1: whole; with 256 tiles, of the
+ * tiles past the last complete round) that a product of these sizes runs on: alg_ffn_gemm's,
+ * alg_ffn_alu_glu_fwd's (M tokens, N = d_ff, K = d) or alg_ffn_alu_glu_dy's (N = d_ff, K = dm). */
+enum { ALG_FFN_GEMM = 0, ALG_FFN_GATE_UP = 1, ALG_FFN_DY = 2 };
+int alg_ffn_plan(int product, int M, int N, int K, int* tile, int* split);
 
 /* The whole block, (x w_g alu(x w_u, beta)) w_d, model.py:185-193 with ffn = "alu_glu". x, y, gate,
  * up, out, dout, dx in bf16; each weight, and its gradient, in bf16 or f32 (ALG_DTYPE_*): the products
