@@ -221,7 +221,10 @@ __global__ __launch_bounds__(C::THREADS, 2) void ffn_gemm_kernel(FfnGemmParams g
   const int bid = blockIdx.x;
   int lin, kbeg = 0, kend = g.K, unit = -1;
   if (bid < g.full) {
-    lin = xcd_contiguous(bid, g.full);
+    // A share of rows per XCD reads all of B on every XCD. Where B is the larger operand and the row
+    // length lets the plain order give an XCD every fourth column, or fewer, that is the better one
+    // (M N K 1600 3328 1536: 44 us in shares, 33 plain; 704 5888 2115: 45 / 37).
+    lin = g.full % 8 && nbn % 4 == 0 && g.N > g.M ? bid : xcd_contiguous(bid, g.full);
   } else {
     unit = bid - g.full;
     lin = g.full + unit / g.split;

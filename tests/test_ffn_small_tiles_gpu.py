@@ -1,6 +1,7 @@
 """The feed-forward products on 64 x 64 and 128 x 128 tiles (short inputs): one row and column of
 tiles more or less than whole, k of one step, under one, and with a remainder, each stored layout,
-k splits; the two fused epilogues around the sizes where the tile changes. Products against a
+k splits, a row length and tile count that take the plain tile order; the two fused epilogues around
+the sizes where the tile changes. Products against a
 float32 product of the same bf16 operands (one bf16 rounding, and the order of the f32 sums).
 """
 
@@ -15,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("a_trans,b_trans", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("M,N,K", [(64, 64, 64), (72, 56, 40), (128, 192, 320), (200, 136, 1000), (8, 520, 192),
-                                   (304, 1024, 4096), (1016, 776, 2056), (776, 4088, 1016)])
+                                   (304, 1024, 4096), (1016, 776, 2056), (776, 4088, 1016), (320, 768, 136)])
 def test_small_products(M, N, K, a_trans, b_trans):
     from algebraic_amd import _lib as L
     lib = L.load()
