@@ -261,7 +261,7 @@ def test_neighbour_entry_points_validate_before_launch():
     rc = handle.alg_ffn_gemm(None, 256, 256, 512, P(16), 512, 0, P(24), 256, 0, P(16), 256, None, 0)
     assert rc == _lib.ALG_ERR_INVALID and b"aligned" in err()
     assert handle.alg_ffn_gemm_workspace_size(256, 256, 512) == 0       # one tile, short k: no split
-    need = handle.alg_ffn_gemm_workspace_size(296, 264, 5000)           # 4 tiles, k split 4 ways
+    need = handle.alg_ffn_gemm_workspace_size(296, 264, 5000)           # sized for 4 tiles of 256, k split 4 ways
     assert need == 4 * 4 * 256 * 256 * 4
     rc = handle.alg_ffn_gemm(None, 296, 264, 5000, P(16), 5000, 0, P(16), 264, 0, P(16), 264, P(16), need - 1)
     assert rc == _lib.ALG_ERR_INVALID and b"workspace" in err()

@@ -2,12 +2,14 @@
 plain PyTorch float32 product of the same bf16 operands: every output element within one bf16
 rounding of the f32 sum plus the f32 accumulation-order slack, bounded by the sum of |a||b|.
 
-Covers the four stored layouts of A and B, ragged tiles in m and n, whole-tile plans, plans
-whose every tile is split over k (fewer tiles than CUs), and plans that compute a first round
-of whole tiles and split the rest (the 1b block's y w_d and d_gu w_gu^T shapes).
+Covers the four stored layouts of A and B with ragged tiles in m and n on 64 x 64 tiles, whole and
+in k ranges (the sizes of 256 x 256 tiles are in test_large_tiles_gpu.py), and plans of 256 x 256
+tiles that compute a first round of whole tiles and split the rest (the 1b block's y w_d and
+d_gu w_gu^T shapes).
 """
 
-import numpy as np
+import ctypes
+
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -32,8 +34,12 @@ def _run(a, b, a_trans, b_trans, M, N, K, calls=2):
 
 
 @pytest.mark.parametrize("a_trans,b_trans", LAYOUTS)
-@pytest.mark.parametrize("M,N,K,split", [(296, 264, 5000, True), (264, 512, 640, False), (512, 256, 1032, False)])
+@pytest.mark.parametrize("M,N,K,split", [(296, 264, 5000, 8), (264, 512, 640, 1), (512, 256, 1032, 1)])
 def test_ffn_gemm_matches_f32(M, N, K, split, a_trans, b_trans):
+    from algebraic_amd import _lib as L
+    tile, ranges = ctypes.c_int(), ctypes.c_int()
+    L.check(L.load().alg_ffn_plan(L.FFN_GEMM, M, N, K, tile, ranges), "alg_ffn_plan")
+    assert (tile.value, ranges.value) == (64, split)
     print(f"[ffn_gemm] M={M} N={N} K={K} a_trans={a_trans} b_trans={b_trans}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     A = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
@@ -41,7 +47,7 @@ def test_ffn_gemm_matches_f32(M, N, K, split, a_trans, b_trans):
     a = A.t().contiguous() if a_trans else A
     b = B.t().contiguous() if b_trans else B
     outs, ws_b = _run(a, b, a_trans, b_trans, M, N, K)
-    assert (ws_b > 0) == split
+    assert (ws_b > 0) == (split > 1)
     ref = A.float() @ B.float()
     slack = A.float().abs() @ B.float().abs()
     for c in outs:
