@@ -165,8 +165,10 @@ struct RowTile {
 // D = 64 the LDS (70 KB) lets two workgroups run on a CU. Against 128 keys per workgroup with one
 // wave per SIMD and the next tile's registers spilled (us, B H T D): 2 12 1024 64: 219 -> 119;
 // 4 12 2048 64: 726 -> 607 to 655 by run; 8 16 1024 64: 496 -> 432; 1 4 300 64: 70 -> 40; 2 12 1024 128:
-// 526 -> 212. (Two workgroups per key block, its query tiles dealt between them, took 2 12 1024 64
-// to 109 us, but dQ's addends then arrive in an order that changes from call to call.)
+// 526 -> 212. dQ's addends (one per key block, by f32 atomics) meet in no fixed order, so dQ may
+// differ from call to call in its last bits; dK and dV, which no atomics form, are the same bits.
+// (Two workgroups per key block, its query tiles dealt between them, took 2 12 1024 64 to 109 us, but
+// dK and dV would then be such sums as well.)
 constexpr int F32_BK = 64, F32_BQ = 64;
 // Barrier for LDS alone: __syncthreads() also waits for every global access in flight, here the
 // dQ atomics and the next tile's loads.
@@ -1553,10 +1555,13 @@ static hipError_t launch_bwd_bf16(const AttnBwdParams& p, int mode, bool dq, hip
 // f32: the key-stationary kernel with dQ atomics. Up to 512 key blocks, the in-range launch asks
 // for LDS it does not use, so that a CU takes one workgroup at a time: the first 256, the longest
 // key blocks, then start on a CU each and the short ones follow, where two to a CU put long
-// blocks together and left CUs idle (384 key blocks, B H T D: 2 12 1024 64 142 -> 119 us,
-// 1 12 2048 64 253 -> 210). With more blocks than that, two to a CU hide each other's waits
-// (1536, 4 12 2048 64: 607 us, one to a CU 672). The form for one to a CU has the registers of one wave
-// per SIMD and spills nothing (384 blocks, 2 12 1024 64: 131 -> 120 us).
+// blocks together and left CUs idle. With more blocks than that, two to a CU hide each other's
+// waits. At n = 16 the form for one to a CU also has the registers of one wave per SIMD and spills
+// nothing; at other n it is the two-wave form with the LDS pad. One box, us, one / two to a CU, n = 16
+// then n = 8 (T = 1024, D = 64; key blocks): 192 112 / 123, 127 / 127; 384 113 / 146, 131 / 151;
+// 512 126 / 157, 145 / 163; 576 154 / 162, 176 / 171; 640 173 / 167, 197 / 173; 1152 284 / 251,
+// 322 / 261; T = 2048: 384 214 / 278, 246 / 288; 512 234 / 302, 268 / 312; 640 319 / 320, 364 / 334;
+// 1536 676 / 625, 774 / 644.
 template <int D>
 static hipError_t launch_bwd_f32(const AttnBwdParams& p, int mode, hipStream_t st) {
   constexpr int WPS = D == 64 ? 2 : 1;  // waves per SIMD

@@ -192,7 +192,7 @@ HeadWs head_ws_f32(int N, int d, int V, int pass) {
 struct HeadEvalWs {
   size_t partial, pmax, pidx, total;
 };
-HeadEvalWs head_eval_ws(int N, int d, int V, bool f32) {
+HeadEvalWs head_eval_ws(int N, int V, bool f32) {
   const size_t cells = (size_t)(f32 ? alg::head_f32_vocab_tiles(V) : alg::ceil_div(V, alg::head_logit_tile(N, V))) * N;
   HeadEvalWs w;
   w.partial = 0;
@@ -597,7 +597,7 @@ size_t alg_head_workspace_size(int dtype, int N, int d, int V, int pass) {
   if (dtype != ALG_DTYPE_BF16 && dtype != ALG_DTYPE_F32) return 0;
   const bool f32 = dtype == ALG_DTYPE_F32;
   // pass 0: forward; 1: backward without a residual; 2: backward with a residual; 3: eval
-  if (pass == 3) return head_eval_ws(N, d, V, f32).total;
+  if (pass == 3) return head_eval_ws(N, V, f32).total;
   if (f32) return pass == 2 ? 0 : head_ws_f32(N, d, V, pass ? 1 : 0).total;  // no residual in f32
   return head_ws(N, d, V, pass ? 1 : 0, pass == 2).total;
 }
@@ -1017,7 +1017,7 @@ static int head_eval(alg_stream_t stream, int dtype, int N, int d, int V, const 
   const bool f32 = dtype == ALG_DTYPE_F32;
   if (!h || !E || !targets || !logprob) return fail(ALG_ERR_INVALID, "null argument");
   if (!aligned16({h, E, workspace})) return fail(ALG_ERR_INVALID, "matrices must be 16-byte aligned");
-  const HeadEvalWs ws = head_eval_ws(N, d, V, f32);
+  const HeadEvalWs ws = head_eval_ws(N, V, f32);
   if (!workspace || workspace_bytes < ws.total)
     return fail(ALG_ERR_INVALID, "workspace too small: need %zu bytes", ws.total);
   const HeadWs hw = f32 ? head_ws_f32(N, d, V, 0) : head_ws(N, d, V, 0, false);

@@ -1,4 +1,4 @@
-// bf16 MFMA GEMM main loop for gfx950, shared by the fused-head kernels.
+// bf16 MFMA GEMM main loops for gfx950, shared by the fused-head and feed-forward kernels.
 //
 // C[M][N] = sum_k A[m][k] B[k][n] with f32 accumulation. A configuration fixes the
 // workgroup tile TM x TN, 64-deep k steps and a WM x WN grid of waves; each wave owns a
@@ -10,14 +10,15 @@
 //
 // Global -> LDS copies are buffer loads that write LDS (each lane of a wave instruction
 // writes 16 bytes at base + 16*lane), so no VGPRs stage the tiles and the next tile's copy is
-// in flight while the current one feeds the MFMAs; tiles are double-buffered with one barrier
-// per k step. Because the copy writes rows without padding, 16-byte chunks are placed with an
+// in flight while the current one feeds the MFMAs. Tiles of 256 x 256 (8 waves) are double-buffered,
+// smaller ones (4 waves) go round a ring of four stages; both take one barrier per k step. Because the copy writes rows without padding, 16-byte chunks are placed with an
 // XOR swizzle that keeps the fragment reads free of bank conflicts:
 //   k-contiguous rows (128 B):      chunk c of row r lives at chunk c ^ ((r >> 1) & 7)
 //   mn-contiguous rows (2*TMN B):   chunk c of row r lives at chunk c ^ (4 * (r & 3))
 //     (rows of 128 B: c ^ (4 * ((r >> 1) & 1)), two rows to a period of the banks)
-// The pipelined loop covers the largest multiple of 128 in the k range; a remaining partial
-// k tile is copied through registers with zero fill. Tiles that reach past the matrix edge in
+// The double-buffered loop covers the largest multiple of 128 in the k range, its six-pass form
+// (SPLIT3) and the ring the largest multiple of 64; the rest is copied through registers with zero
+// fill. Tiles that reach past the matrix edge in
 // m or n stay on the pipelined loop with range-checked copies: every copy instruction gets a
 // descriptor whose range ends at the operand's allocation, so reads past it return zeros, and
 // the values read past a row's logical end (the next row's data) only reach output rows or

@@ -133,9 +133,9 @@ __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_fwd
   // WITH_U also stores the residual. U is token-major (element (tok, v) at tok * Vp + v),
   // staged per wave and written with 16-byte stores marked non-temporal so the 1 GB stream of U
   // does not evict the E / h panels the GEMM is reusing from L2. EDGE (tiles that reach past V
-  // or N): rows past V add nothing to the sums; U's rows up to Npad and its columns up to Vp
-  // are all written, as finite values wherever h is finite (operand rows past the end read as
-  // zeros). Edge tiles once stored U an element at a time, 2 bytes a lane: at N = 1000 their
+  // or N): rows past V add nothing to the sums; U's rows up to the end of the last tile and its
+  // columns up to Vp are all written, as finite values wherever h is finite (operand rows past the
+  // end read as zeros); nothing reads a row past N. Edge tiles once stored U an element at a time, 2 bytes a lane: at N = 1000 their
   // quarter of the tiles took most of the kernel.
   static_assert(C::WTM * C::WTN <= gemm_share<KMAJOR, KMAJOR, C>(), "a wave's block fits its share");
   auto epilogue = [&](auto with_u, auto edge) {
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_fwd
       part += xor32(part);
       if (h == 0) red[wm][col] = part;
     }
-    // Rows of this wave's block: tokens n0 + wn*64 + (0..63), vocabulary vrow0 + (0..127).
+    // Rows of this wave's block: tokens n0 + wn*WTN + (0..WTN-1), vocabulary vrow0 + (0..WTM-1).
     if constexpr (WITH_U) store_staged_tokmajor<C, BUF_NT, EDGE>(ub, p.ut, p.Npad, p.Vp, n0 + wn * C::WTN, vrow0, lane);
   };
   const bool inside = m0 + C::TM <= p.V && n0 + C::TN <= p.N;
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(256) void head_obj_kernel(HeadParams p, int nblocks
 // f32 hidden states) as three bf16 planes whose sum is the f32 value times 2^split3_dz_exp(s). L2N > 0 fixes
 // n = 2^L2N at compile time (0: taken from the parameters). Each wave's block is staged and
 // written in whole token rows with 16-byte stores (default cache policy: the dh and dE products
-// read dZ right after); edge tiles write the rows up to Npad and the columns up to Vp too, of
+// read dZ right after); edge tiles write the rows up to their end and the columns up to Vp too, of
 // which nothing is read.
 template <class C, int L2N, bool SPLIT>
 __global__ __launch_bounds__(C::THREADS, head_waves_per_simd<C>()) void head_dz_kernel(HeadParams p) {

@@ -53,8 +53,8 @@ struct HeadParams {
   int v_off = 0;        // vocabulary index of E's first row (targets are compared with v + v_off)
   int dh_accum = 0;     // dh product: 0 writes, 1 adds into the f32 accumulator (dh_part, or
                         // dh32 for f32 hidden states), 2 writes bf16(accumulator + product)
-  float* pmax;          // eval: (ceil(V/HT_M), N) per-vocab-tile maximum logit
-  int* pidx;            // eval: (ceil(V/HT_M), N) its vocabulary index
+  float* pmax;          // eval: (ceil(V/128), N) at most: per-vocab-tile maximum logit
+  int* pidx;            // eval: (ceil(V/128), N) at most: its vocabulary index
   float* logprob;       // eval: (N,) log p(target)
   int* argmax;          // eval: (N,) argmax_v z, or nullptr
   int64_t* argmax64;    // eval: the same as 64-bit indices, or nullptr
