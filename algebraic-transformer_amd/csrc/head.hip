@@ -962,7 +962,7 @@ HeadDhPlan head_dh_plan(int N, int d, int V, int passes) {
   HeadDhPlan pl{256, head_dh_split(N, d, V), 0};
   double best = time(256, pl.split);
   if (head_tiles(256, N, d) < 256)
-    for (int s = 1; s <= 32 && V / s >= (passes == 1 ? 384 : 256); s *= 2)
+    for (int s = 1; s <= 32 && (s == 1 || V / s >= (passes == 1 ? 384 : 256)); s *= 2)
       if (const double t = time(128, s); t < best) {
         best = t;
         pl.tile = 128;

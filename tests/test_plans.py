@@ -50,6 +50,7 @@ HEAD = [
     ("BF16", "DH", 700, 1536, 8192, 256, 56.2, 76.9),
     ("BF16", "DH", 300, 2048, 16384, 256, 61.7, 76.9),
     ("BF16", "DH", 512, 512, 8192, 128, 33.9, 46.2),
+    ("BF16", "DH", 127, 72, 129, 128, None, None),  # a vocabulary shorter than a range keeps the choice
     ("BF16", "DH", 128, 1024, 32000, 128, 44.4, 76.7),
     ("BF16", "DE", 200, 256, 50257, 256, 22.7, 35.1),
     ("BF16", "DE", 300, 768, 16384, 256, 21.1, 27.3),
