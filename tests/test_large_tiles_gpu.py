@@ -1,7 +1,8 @@
-"""The feed-forward's products on 256 x 256 tiles where these are ragged: rows, columns and k past a
-tile, whole and split over k, each stored layout; the block's direct and summed stores into one or
-two weight gradients, in bf16 and f32. Every case states the tile and the k ranges it is meant for
-and checks them, so that a change of the rule that chooses them cannot take the test elsewhere.
+"""The products of the feed-forward and of the bf16 head on 256 x 256 tiles where these are ragged:
+rows, columns and k past a tile, whole and split over k, each stored layout; the block's direct and
+summed stores into one or two weight gradients, in bf16 and f32. Every case states the tile and the
+k ranges it is meant for and checks them, so that a change of the rule that chooses them cannot take
+the test elsewhere.
 """
 
 import ctypes
@@ -79,3 +80,36 @@ def test_ragged_block(N, d, F, dw_splits, dtypes):
         a = a.float().cpu().numpy()
         assert rel_l2(a, b) < 1e-2, name
         assert rel_l2(a[e], np.asarray(b)[e]) < 1e-2, f"{name} in the ragged tiles"
+
+
+@pytest.mark.parametrize("schedule", ["residual", "recompute"])
+@pytest.mark.parametrize("e_dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+@pytest.mark.parametrize("N,d,V,dh_split,de_split", [(1030, 1032, 8200, 10, 1), (2060, 1032, 4104, 5, 2)])
+def test_ragged_head(N, d, V, dh_split, de_split, e_dtype, schedule, monkeypatch):
+    from algebraic_amd import _lib as L
+    from algebraic_amd.kernels import fused_head as FH
+    from oracle import head as OH
+    from oracle.numerics import round_bf16
+    monkeypatch.setattr(FH, "SCHEDULE", schedule)
+    tile, split = ctypes.c_int(), ctypes.c_int()
+    for product, ranges in ((L.HEAD_LOGITS, 1), (L.HEAD_DH, dh_split), (L.HEAD_DE, de_split)):
+        L.check(L.load().alg_head_plan(L.DTYPE_BF16, product, N, d, V, tile, split), "alg_head_plan")
+        assert (tile.value, split.value) == (256, ranges)
+    print(f"head large tiles N{N} d{d} V{V} {e_dtype} {schedule}", flush=True)
+    rng = np.random.default_rng(N + d + V)
+    h = round_bf16(rng.standard_normal((N, d)).astype(np.float32))
+    E = round_bf16((rng.standard_normal((V, d)) * 0.05).astype(np.float32))
+    t = rng.integers(0, V, N).astype(np.int32)
+    th = torch.tensor(h, device="cuda").to(torch.bfloat16).requires_grad_(True)
+    tE = torch.tensor(E, device="cuda").to(e_dtype).requires_grad_(True)
+    obj, pt = FH.fused_head(th, tE, torch.tensor(t, device="cuda"), kind="alg_ce", n=8, c=2.0, block_n=N)
+    dh, dE = torch.autograd.grad(obj * 0.7, (th, tE))
+    obj_r, pt_r = OH.dense_forward(h, E, t, n=8, c=2.0)
+    dh_r, dE_r = OH.dense_backward(h, E, t, 0.7, n=8, c=2.0)
+    np.testing.assert_allclose(obj.item(), obj_r, rtol=2e-3, atol=2e-4)
+    np.testing.assert_allclose(pt.cpu().numpy(), pt_r, rtol=1e-4, atol=1e-9)  # f32 sums of exact products
+    for got, want, rows in ((dh, dh_r, N), (dE, dE_r, V)):
+        got = got.float().cpu().numpy()
+        assert rel_l2(got, want) < 1e-2
+        edge = np.s_[-(rows % 256):, :], np.s_[:, -(d % 256):]
+        assert all(rel_l2(got[e], want[e]) < 1e-2 for e in edge)
