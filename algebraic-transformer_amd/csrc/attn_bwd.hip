@@ -1162,7 +1162,7 @@ __global__ __launch_bounds__(64 * NW, dkdv16_waves_per_simd<D>() * 4 / NW) void 
 // f32 rounding however the weights are spread. In exact arithmetic both are <dO_i, o_i>.
 // Waves per SIMD the dQ kernel is built for: at D = 64 the in-range kernel with n fixed at
 // compile time fits 168 VGPRs (16 bytes spilled) and runs three (C3 dQ 0.158 -> 0.152 ms,
-// measured A/B on one box); the other variants spill far more at that bound and keep two.
+// measured in turn on one card); the other variants spill far more at that bound and keep two.
 template <int D, int MODE, int L2N>
 constexpr int dq_waves_per_simd() { return D == 64 && MODE == MODE_INRANGE && L2N > 0 ? 3 : 2; }
 
@@ -1557,7 +1557,7 @@ static hipError_t launch_bwd_bf16(const AttnBwdParams& p, int mode, bool dq, hip
 // key blocks, then start on a CU each and the short ones follow, where two to a CU put long
 // blocks together and left CUs idle. With more blocks than that, two to a CU hide each other's
 // waits. At n = 16 the form for one to a CU also has the registers of one wave per SIMD and spills
-// nothing; at other n it is the two-wave form with the LDS pad. One box, us, one / two to a CU, n = 16
+// nothing; at other n it is the two-wave form with the LDS pad. Timed in turn, us, one / two to a CU, n = 16
 // then n = 8 (T = 1024, D = 64; key blocks): 192 112 / 123, 127 / 127; 384 113 / 146, 131 / 151;
 // 512 126 / 157, 145 / 163; 576 154 / 162, 176 / 171; 640 173 / 167, 197 / 173; 1152 284 / 251,
 // 322 / 261; T = 2048: 384 214 / 278, 246 / 288; 512 234 / 302, 268 / 312; 640 319 / 320, 364 / 334;

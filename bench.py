@@ -570,7 +570,7 @@ def cpu_baseline(c1_gpu_ms=None):
     of the step (attention fwd+bwd on a few heads, head fwd+bwd on a few tokens, scaled to the
     full step) and of BASELINE config 1 (attention forward, fp32, B2 H12 T1024 D64) at full
     shape. BLAS threads: the affinity mask's cores, capped at OMP_NUM_THREADS when the host
-    sets it (a GPU box's share of the host)."""
+    sets it (a share of the host)."""
     import numpy as np
     from oracle import attention as OA
     from oracle import head as OH

@@ -1,5 +1,5 @@
 """CPU: bench.py's command-line contract without a GPU. One GPU is the only supported count
-(the driver may ask for more; the line must say why it refuses), and with no GPU visible the
+(a launcher may ask for more; the line must say why it refuses), and with no GPU visible the
 bench fails loudly rather than timing anything on the host."""
 
 import subprocess
