@@ -19,8 +19,8 @@ namespace alg {
 // of the feed-forward (100 to 8000 tokens) and of the head (32 to 4096 tokens, V 1000 to 50257),
 // each configuration timed on its own: the one chosen takes 1.0 % more than the best on average,
 // and more than 1.04 times the 256 tiles in 13 of them (at most 1.26). Without the constant of each round and the ragged rates
-// the same rule took up to 1.8 times the 256 tiles (dh of N d V 2500 1536 8192: 87 us, 126 on 240
-// tiles of 128). M N K, us for tiles of 256 / 128 / 64:
+// the same rule took up to 1.6 times the 256 tiles (M N K 1536 8448 197: 20.5 us, 32 on 792 tiles
+// of 128). M N K, us for tiles of 256 / 128 / 64:
 //   1024  768 2048   39.3 / 20.8 / 11.0     768 4096 1024   25.4 / 14.7 / 19.6
 //   1024  768 4096   69.5 / 37.2 / 19.2    2048  768 1024   23.2 / 12.6 /  8.3
 //   1024 8192  300   18.6 / 23.0 / 25.9    2048 1536 4224   42.8 / 39.5 / 58.4
