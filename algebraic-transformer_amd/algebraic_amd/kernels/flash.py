@@ -109,20 +109,20 @@ def _sink_input(sink_logit, H, dev):
 
 
 def _row_state(B, H, T, dev):
-    """What the backward reads of the forward: one f32 allocation for the per-row statistic (B H T)
-    and sink/c (H), the guard flag (one int32, not a part of it: a saved-tensor hook may store
-    floating tensors in fewer bits, which would turn the flag's bits to 0), and their pointers."""
-    aux = torch.empty(B * H * T + H, dtype=torch.float32, device=dev)
-    flag = torch.empty(1, dtype=torch.int32, device=dev)
-    return aux, flag, *_row_state_ptrs(aux, flag, B, H, T)
+    """What the backward reads of the forward in one allocation, and pointers to its parts: the
+    per-row statistic (B H T, f32), sink/c (H, f32) and the guard flag (int32). Its type is the
+    flag's: a saved-tensor hook may store floating tensors in fewer bits, which would turn the
+    flag's bits to 0, and leaves whole numbers as they are."""
+    aux = torch.empty(B * H * T + H + 1, dtype=torch.int32, device=dev)
+    return aux, *_row_state_ptrs(aux, B, H, T)
 
 
-def _row_state_ptrs(aux, flag, B, H, T):
+def _row_state_ptrs(aux, B, H, T):
     base = aux.data_ptr()
-    return base, base + 4 * B * H * T, flag.data_ptr()
+    return base, base + 4 * B * H * T, base + 4 * (B * H * T + H)
 
 
-def _attn_backward(plan, q_s, k, v, o, aux, flag, do, has_sink, what):
+def _attn_backward(plan, q_s, k, v, o, aux, do, has_sink, what):
     """dq, dk, dv and the sink logits' gradient (H,) f32 or None, for the cotangent ``do``."""
     B, H, T, D = _bhtd(q_s.shape, plan.layout)
     lib = _lib.load()
@@ -131,7 +131,7 @@ def _attn_backward(plan, q_s, k, v, o, aux, flag, do, has_sink, what):
     if do.dtype != q_s.dtype:
         do = do.to(q_s.dtype)
     do = _lib.aligned16(do)
-    stat, sink, flag = _row_state_ptrs(aux, flag, B, H, T)
+    stat, sink, flag = _row_state_ptrs(aux, B, H, T)
     ws_bytes = lib.alg_attn_workspace_size(dt, B, H, T, D)
     di = _lib.align256(ws_bytes)
     ws = torch.empty(di + 4 * B * H * T, dtype=torch.uint8, device=dev)  # workspace, then di
@@ -172,7 +172,7 @@ class _FlashFn(torch.autograd.Function):
         ws_bytes = lib.alg_attn_workspace_size(dt, B, H, T, D)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         q_s, o = torch.empty_like(q), torch.empty_like(q)
-        aux, guard, stat, sink, flag = _row_state(B, H, T, dev)
+        aux, stat, sink, flag = _row_state(B, H, T, dev)
         if not has_sink:
             sink = None
         p = _lib.ptr
@@ -190,13 +190,13 @@ class _FlashFn(torch.autograd.Function):
                 int(plan.fast_rho), int(plan.inv_stat), p(o), None, stat), "flash_attention forward")
         ctx.plan = plan
         ctx.sink_meta = None if not has_sink else (tuple(sink_logit.shape), sink_logit.dtype)
-        ctx.save_for_backward(q_s, k, v, o, aux, guard)
+        ctx.save_for_backward(q_s, k, v, o, aux)
         return o
 
     @staticmethod
     def backward(ctx, do):
-        q_s, k, v, o, aux, guard = ctx.saved_tensors
-        dq, dk, dv, dsink = _attn_backward(ctx.plan, q_s, k, v, o, aux, guard, do, ctx.sink_meta is not None,
+        q_s, k, v, o, aux = ctx.saved_tensors
+        dq, dk, dv, dsink = _attn_backward(ctx.plan, q_s, k, v, o, aux, do, ctx.sink_meta is not None,
                                            "flash_attention backward")
         return dq, dk, dv, _sink_gradient(dsink, *ctx.sink_meta) if ctx.sink_meta else None, None
 

@@ -88,7 +88,7 @@ class _PrologueFlashFn(torch.autograd.Function):
         q_s, k_r, o = torch.empty_like(q), torch.empty_like(k), torch.empty_like(q)
         tau = torch.empty((2, B, H, T), dtype=torch.float32, device=dev)  # 1/rms of the rows of q and of k
         tau_q, tau_k = _tau_ptrs(tau)
-        aux, guard, stat, sink, flag = _row_state(B, H, T, dev)
+        aux, stat, sink, flag = _row_state(B, H, T, dev)
         if not has_sink:
             sink = None
         p = _lib.ptr
@@ -102,17 +102,17 @@ class _PrologueFlashFn(torch.autograd.Function):
         ctx.plan = plan
         ctx.sink_meta = None if not has_sink else (tuple(sink_logit.shape), sink_logit.dtype)
         ctx.gain_meta = [None if g is None else (g.shape, g.dtype) for g in (q_gain, k_gain)]
-        ctx.save_for_backward(q, k, v, gq, gk, cs, sn, q_s, k_r, tau, o, aux, guard)
+        ctx.save_for_backward(q, k, v, gq, gk, cs, sn, q_s, k_r, tau, o, aux)
         return o
 
     @staticmethod
     def backward(ctx, do):
-        q, k, v, gq, gk, cs, sn, q_s, k_r, tau, o, aux, guard = ctx.saved_tensors
+        q, k, v, gq, gk, cs, sn, q_s, k_r, tau, o, aux = ctx.saved_tensors
         plan = ctx.plan
         B, H, T, D = _bhtd(q.shape, plan.layout)
         lib = _lib.load()
         dev = q.device
-        dq_r, dk_r, dv, dsink = _attn_backward(plan, q_s, k_r, v, o, aux, guard, do, ctx.sink_meta is not None,
+        dq_r, dk_r, dv, dsink = _attn_backward(plan, q_s, k_r, v, o, aux, do, ctx.sink_meta is not None,
                                                "attention backward")
         nbytes = lib.alg_attn_prologue_workspace_size(B, H, T, D)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)

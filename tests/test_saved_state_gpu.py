@@ -42,5 +42,5 @@ def test_guard_flag_survives_reduced_precision_storage(prologue, range_guard):
         got = grads()
     for a, b in zip(got, want):
         a, b = a.float(), b.float()
-        # The row statistic, sink and 1/rms in bf16: 2^-9 each, a few of them in a weight.
+        # The prologue's 1/rms and gains in bf16: 2^-9 each.
         assert float((a - b).norm() / b.norm()) < 2e-2
